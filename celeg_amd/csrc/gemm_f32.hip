@@ -1,72 +1,176 @@
 // True 32-bit matrix product for the 32-bit path: Y[M,N] = X[M,K] W[N,K]^T (+ bias).
-// No reduced-precision matrix mode: plain fused multiply-adds in float, and every
-// output element is accumulated over k = 0..K-1 in that order whatever M, the tile or
-// the batch is, so the logits of a row do not depend on how rows were batched.
+// No reduced-precision matrix mode: the matrix cores' 32-bit instruction (16x16x4).  Every output
+// element is summed in the same order whatever M, the tile or the batch is, so the logits of a row do
+// not depend on how rows were batched: k in segments of 128, a segment as a chain of 32 instructions
+// (instruction i of a piece of 16 takes the values i, 4 + i, 8 + i and 12 + i), then the segments'
+// sums in order.
 // The reference's projections: y = x W^T, weights [out, in] row-major
 // (src/model/weight_plan.cpp:82-130).
+//
+// A workgroup owns a tile of 16 RT rows x 16 CT columns; its wavefronts take the segments in turn and
+// leave their sums in LDS, where the workgroup adds them in order.  Few rows are bound by reading W: one
+// column tile a workgroup, up to 16 wavefronts that each ask for a whole segment (8 KiB) at once, so
+// that even a 1024 x 1024 matrix is asked for by 512 wavefronts in one trip to memory.  Many rows are bound
+// by the matrix cores: larger tiles, operands straight from the caches (16 bytes a cycle and CU of them).
+// Measured in a chain over different matrices (before: 64 x 64 tiles of vector instructions, k in order,
+// 137 us for any product with K = 1,024): 2 rows, 1024 x 1024 4.5 us, 3072 x 1024 5.6 us, 1024 x 4608
+// 14.8 us (before 613), 65536 x 1024 54 us (4.9 TB/s; before 247); 64 rows, 3072 x 1024 13.7 us; 2,048 rows,
+// 4608 x 1024 256 us (76 TFLOP/s).  Error against 64 bits 2.1e-7 of the result (2-norm), before 3 times that.
 #include "common.h"
 
-#define BM 64
-#define BN 64
-#define BK 16
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
-__global__ __launch_bounds__(256) void gemm_f32_kernel(
+#define F32_SEGMENT 128
+#define F32_PIECES (F32_SEGMENT / 16)
+
+// GROUP: pieces of 16 values of k that are asked for together.  VEC: rows of X and W lie on 16 bytes
+// and K is a multiple of 4; the same sums in the same order without it.
+template <int RT, int CT, int GROUP, int MAX_THREADS, bool VEC>
+__global__ __launch_bounds__(MAX_THREADS) void gemm_f32_kernel(
     const float* __restrict__ X, int ldx, const float* __restrict__ W, int ldw,
-    const float* __restrict__ bias, float* __restrict__ Y, int ldy, int M, int N, int K) {
-    __shared__ float Xs[BK][BM + 1];
-    __shared__ float Ws[BK][BN + 1];
-    const int tid = threadIdx.x;
-    const int tx = tid % 16, ty = tid / 16;
-    const int row0 = blockIdx.y * BM, col0 = blockIdx.x * BN;
-    float acc[4][4];
+    const float* __restrict__ bias, float* __restrict__ Y, int ldy, int M, int N, int K, int wide_store) {
+    constexpr int TILES = RT * CT;
+    constexpr int ITEMS = TILES > 8 ? TILES / 4 : 1;      // sums of four a thread: at least min(TILES, 8) wavefronts, 4 if TILES > 8
+    extern __shared__ f32x4_t parts[];                    // [wavefront][tile][lane]
+    const int wave = threadIdx.x / CELEG_WAVE, lane = threadIdx.x % CELEG_WAVE;
+    const int n_waves = blockDim.x / CELEG_WAVE;
+    const int qd = lane >> 4, r16 = lane & 15;
+    const int row0 = blockIdx.y * (16 * RT), col0 = blockIdx.x * (16 * CT);
+    // rows and columns past the end repeat the last one: an output depends on its own row and column only
+    const float* x_row[RT];
+    const float* w_row[CT];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int rt = 0; rt < RT; ++rt) x_row[rt] = X + static_cast<size_t>(min(row0 + rt * 16 + r16, M - 1)) * ldx;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+    for (int ct = 0; ct < CT; ++ct) w_row[ct] = W + static_cast<size_t>(min(col0 + ct * 16 + r16, N - 1)) * ldw;
 
-    for (int k0 = 0; k0 < K; k0 += BK) {
+    auto four = [&](const float* row, int k, bool whole) __attribute__((always_inline)) {
+        f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+        if (VEC) {
+            if (whole || k < K) v = *reinterpret_cast<const f32x4_t*>(row + k);
+        } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int e = tid + i * 256;
-            const int r = e / BK, c = e % BK;
-            const int gr = row0 + r, gc = col0 + r, gk = k0 + c;
-            Xs[c][r] = (gr < M && gk < K) ? X[static_cast<size_t>(gr) * ldx + gk] : 0.f;
-            Ws[c][r] = (gc < N && gk < K) ? W[static_cast<size_t>(gc) * ldw + gk] : 0.f;
+            for (int i = 0; i < 4; ++i)
+                if (whole || k + i < K) v[i] = row[k + i];
         }
-        __syncthreads();
+        return v;
+    };
+    auto load = [&](int k0, bool whole, f32x4_t (&wv)[CT][GROUP], f32x4_t (&xv)[RT][GROUP]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int kk = 0; kk < BK; ++kk) {
-            float a[4], b[4];
+        for (int s = 0; s < GROUP; ++s) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = Xs[kk][ty * 4 + i];
+            for (int ct = 0; ct < CT; ++ct) wv[ct][s] = four(w_row[ct], k0 + 16 * s + 4 * qd, whole);
+        }
 #pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = Ws[kk][tx * 4 + j];
+        for (int s = 0; s < GROUP; ++s) {
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) xv[rt][s] = four(x_row[rt], k0 + 16 * s + 4 * qd, whole);
+        }
+    };
+    f32x4_t acc[CT][RT];
+    auto multiply = [&](const f32x4_t (&wv)[CT][GROUP], const f32x4_t (&xv)[RT][GROUP]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < GROUP; ++s)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
+                for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                    for (int rt = 0; rt < RT; ++rt)
+                        acc[ct][rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[ct][s][i], xv[rt][s][i], acc[ct][rt], 0, 0, 0);
+    };
+    auto segment = [&](int k0, bool whole) __attribute__((always_inline)) {
+        f32x4_t w0[CT][GROUP], x0[RT][GROUP];
+        load(k0, whole, w0, x0);
+        if (GROUP == F32_PIECES) {
+            multiply(w0, x0);
+            return;
         }
+        f32x4_t w1[CT][GROUP], x1[RT][GROUP];
+#pragma unroll
+        for (int g = 0; g < F32_PIECES / GROUP; g += 2) {
+            load(k0 + (g + 1) * 16 * GROUP, whole, w1, x1);
+            multiply(w0, x0);
+            if (g + 2 < F32_PIECES / GROUP) load(k0 + (g + 2) * 16 * GROUP, whole, w0, x0);
+            multiply(w1, x1);
+        }
+    };
+
+    f32x4_t total[ITEMS];
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) total[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const int segments = (K + F32_SEGMENT - 1) / F32_SEGMENT;
+    for (int first = 0; first < segments; first += n_waves) {
+        const int k0 = (first + wave) * F32_SEGMENT;
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) acc[ct][rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        if (k0 + F32_SEGMENT <= K) segment(k0, true);
+        else if (k0 < K) segment(k0, false);
+        if (first) __syncthreads();                       // the sums before have been read
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) parts[(wave * TILES + ct * RT + rt) * CELEG_WAVE + lane] = acc[ct][rt];
         __syncthreads();
-    }
+        const int n = min(n_waves, segments - first);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int gr = row0 + ty * 4 + i;
-        if (gr >= M) continue;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int gc = col0 + tx * 4 + j;
-            if (gc >= N) continue;
-            Y[static_cast<size_t>(gr) * ldy + gc] = acc[i][j] + (bias ? bias[gc] : 0.f);
+        for (int j = 0; j < ITEMS; ++j) {
+            const int item = static_cast<int>(threadIdx.x) + j * static_cast<int>(blockDim.x);
+            if (item < TILES * CELEG_WAVE)
+                for (int w = 0; w < n; ++w) total[j] += parts[w * TILES * CELEG_WAVE + item];
         }
     }
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+        const int item = static_cast<int>(threadIdx.x) + j * static_cast<int>(blockDim.x);
+        if (item >= TILES * CELEG_WAVE) continue;
+        const int tile = item / CELEG_WAVE, l = item % CELEG_WAVE;
+        const int row = row0 + (tile % RT) * 16 + (l & 15), col = col0 + (tile / RT) * 16 + 4 * (l >> 4);
+        if (row >= M) continue;
+        float* y = Y + static_cast<size_t>(row) * ldy + col;
+        if (wide_store && col + 3 < N) {
+            f32x4_t v = total[j];
+            if (bias) v += f32x4_t{bias[col], bias[col + 1], bias[col + 2], bias[col + 3]};
+            *reinterpret_cast<f32x4_t*>(y) = v;
+            continue;
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (col + r < N) y[r] = total[j][r] + (bias ? bias[col + r] : 0.f);
+    }
+}
+
+template <int RT, int CT, int GROUP, int MAX_THREADS>
+static int launch_f32(const float* X, int ldx, const float* W, int ldw, const float* bias, float* Y, int ldy,
+                      int M, int N, int K, hipStream_t stream) {
+    const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    const bool vec = K % 4 == 0 && ldx % 4 == 0 && ldw % 4 == 0 && aligned(X) && aligned(W);
+    const int wide_store = ldy % 4 == 0 && aligned(Y);
+    constexpr int most = MAX_THREADS / CELEG_WAVE, least = RT * CT > 8 ? 4 : (RT * CT > 4 ? RT * CT : 4);
+    const int segments = (K + F32_SEGMENT - 1) / F32_SEGMENT;
+    const int rounds = (segments + most - 1) / most;      // as even as it goes: 36 segments are 3 rounds of 12
+    const int waves = max(least, (segments + rounds - 1) / rounds);
+    const dim3 grid((N + 16 * CT - 1) / (16 * CT), (M + 16 * RT - 1) / (16 * RT)), block(waves * CELEG_WAVE);
+    const size_t lds = static_cast<size_t>(waves) * RT * CT * CELEG_WAVE * sizeof(f32x4_t);
+    if (vec)
+        hipLaunchKernelGGL((gemm_f32_kernel<RT, CT, GROUP, MAX_THREADS, true>), grid, block, lds, stream, X, ldx, W, ldw, bias, Y, ldy, M, N, K, wide_store);
+    else
+        hipLaunchKernelGGL((gemm_f32_kernel<RT, CT, GROUP, MAX_THREADS, false>), grid, block, lds, stream, X, ldx, W, ldw, bias, Y, ldy, M, N, K, wide_store);
+    return CELEG_LAUNCH_RESULT();
 }
 
 extern "C" int celeg_gemm_f32(const float* X, int ldx, const float* W, int ldw, const float* bias,
                               float* Y, int ldy, int M, int N, int K, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
     if (K <= 0) return static_cast<int>(hipErrorInvalidValue);
-    dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM), block(256);
-    hipLaunchKernelGGL(gemm_f32_kernel, grid, block, 0, stream, X, ldx, W, ldw, bias, Y, ldy, M, N,
-                       K);
-    return CELEG_LAUNCH_RESULT();
+    if (M <= 16) return launch_f32<1, 1, 8, 1024>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
+    if (M <= 32) return launch_f32<2, 1, 8, 512>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
+    if (M <= 64) return launch_f32<4, 1, 4, 512>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
+    // 64 x 64 tiles (an operand from the caches serves four products) once there are two for every CU; below
+    // that (350 rows: 96 of them at N = 1,024) half the tile and twice the wavefronts
+    if (static_cast<long long>((M + 63) / 64) * ((N + 63) / 64) >= 512)
+        return launch_f32<4, 4, 2, 256>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
+    return launch_f32<2, 4, 2, 512>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
 }

@@ -105,6 +105,38 @@ def test_gemm_f32_is_true_32bit_and_row_independent(ops, M, N, K):
     assert torch.equal(one[0], out[M // 2])
 
 
+@pytest.mark.parametrize("M", [1, 2, 16, 17, 32, 33, 64, 65, 130])
+@pytest.mark.parametrize("N,K", [(4, 4), (17, 77), (48, 128), (61, 132), (64, 2048), (70, 4612)])
+def test_gemm_f32_tiles(ops, M, N, K):
+    """Every tile of the 32-bit product at its edges: against 64 bits within the bound of a sum of 128 products and of the
+    segments' sums, rows on any alignment, and a row's bits whatever rows it is computed with."""
+    wide = randn(M, K + 5, seed=7)
+    w, b = randn(N, K, seed=8), randn(N, seed=9)
+    x = wide[:, 1:K + 1]                          # rows that lie on 4 bytes only
+    out, same = torch.empty(M, N, device=DEV), torch.empty(M, N + 3, device=DEV)
+    ops.linear(x, w, out, bias=b)
+    ops.linear(x.contiguous(), w, same[:, :N], bias=b)
+    assert torch.equal(out, same[:, :N])
+    ref = x.double() @ w.double().T + b.double()
+    bound = (min(K, 128) + K // 128 + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T + b.double().abs())
+    assert bool(((out.double() - ref).abs() <= bound).all())
+    for m in {0, M // 2, M - 1}:
+        one = torch.empty(1, N, device=DEV)
+        ops.linear(x[m:m + 1], w, one, bias=b)
+        assert torch.equal(one[0], out[m])
+
+
+@pytest.mark.parametrize("M,N,K", [(530, 4100, 132), (4097, 513, 260)])
+def test_gemm_f32_many_rows(ops, M, N, K):
+    x, w = randn(M, K, seed=7), randn(N, K, seed=8)
+    out, one = torch.empty(M, N, device=DEV), torch.empty(1, N, device=DEV)
+    ops.linear(x, w, out)
+    bound = (128 + K // 128 + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert bool(((out.double() - x.double() @ w.double().T).abs() <= bound).all())
+    ops.linear(x[M - 1:], w, one)
+    assert torch.equal(one[0], out[M - 1])
+
+
 def test_linear_bf16_and_stored_f32_matrix(ops):
     M, N, K = 9, 200, 96
     x = randn(M, K, seed=10, dtype=torch.bfloat16)
