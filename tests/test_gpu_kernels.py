@@ -470,6 +470,7 @@ def attention_case(ops, dtype, heads, kv_heads, head_dim, lengths, cuts, window=
         ref = plain.causal_attention(qf, kf, vf, window=window).reshape(n, -1)
         torch.testing.assert_close(torch.cat(got[i]), ref, **tol(dtype),
                                    msg=lambda m: f"request {i}: {m}")
+    return [torch.cat(g) for g in got]
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
@@ -568,6 +569,21 @@ def test_fast_and_general_attention_agree(ops):
         attention_case(ops, torch.bfloat16, 4, 2, 64, lengths=[333, 150], cuts=[300] + [1] * 40)
     finally:
         ops.attention_impl = "auto"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("head_dim,window", [(64, None), (64, 100), (96, 83), (128, None), (200, None), (256, 64), (20, 7)])
+def test_general_attention_wide_and_narrow_loads(ops, dtype, head_dim, window):
+    """Pages of 16 keys are read 16 bytes a load, pages of 5 a value a load: the same sums in the same order.  Cuts that put
+    rows at the edges of chunks of 64 keys and of the four wavefronts' turns of 256."""
+    ops.attention_impl = "general"
+    try:
+        got = [attention_case(ops, dtype, 2, 1, head_dim, lengths=[262, 65], cuts=[63, 1, 1, 190, 1, 1, 1], window=window,
+                              rotary_dim=0, page_tokens=page_tokens) for page_tokens in (16, 5)]
+    finally:
+        ops.attention_impl = "auto"
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
