@@ -150,6 +150,25 @@ def test_linear_bf16_and_stored_f32_matrix(ops):
     torch.testing.assert_close(out32.double().cpu(), ref, rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 16, 17, 33, 64, 65])
+@pytest.mark.parametrize("N,K", [(3, 8), (331, 96), (1000, 520), (16384, 64), (16388, 64)])
+def test_linear_few_rows(ops, M, N, K):
+    """Products of few bfloat16 rows at the edges of their route (rows, columns, inner sizes that are and are not multiples
+    of 32), rows that are not dense, rows that lie on two bytes only, with and without a bias."""
+    wide = randn(M, K + 16, seed=20, dtype=torch.bfloat16)
+    w, b = randn(N, K, seed=21, scale=0.1, dtype=torch.bfloat16), randn(N, seed=22)
+    for at in (8, 1):
+        x = wide[:, at:at + K]
+        for bias in (None, b):
+            out = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+            ops.linear(x, w, out, bias=bias)
+            ref = x.double() @ w.double().T
+            # the rounding of the result (and of the product in front of the bias, where that is added after it), 2^-9 each
+            bound = 2.0 ** -8 * (ref.abs() + (ref + bias.double()).abs() if bias is not None else ref.abs())
+            bound = bound + 2.0 ** -24 * (K + 8) * (x.double().abs() @ w.double().abs().T)
+            assert bool(((out.double() - ref - (0 if bias is None else bias.double())).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 331, 96), (77, 130, 96), (300, 1000, 352), (129, 48, 40),
                                    (512, 2048, 1024), (2041, 272, 4608)])
 def test_library_product_called_directly(ops, M, N, K):
