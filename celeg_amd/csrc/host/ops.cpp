@@ -72,6 +72,7 @@ const char* path_name(Path p) {
         case Path::RoutedExperts: return "routed_experts";
         case Path::LinearF32: return "linear_f32";
         case Path::LinearLibrary: return "linear_library";
+        case Path::LinearFewRows: return "linear_few_rows";
         case Path::LinearStandIn: return "linear_stand_in";
         case Path::FusedSliced: return "fused_sliced";
         case Path::FusedRows: return "fused_rows";
@@ -611,6 +612,7 @@ bool Ops::few_rows_product(const Tensor& x, const Tensor& w, const Tensor& out) 
     if (rows_of(x, "x") % 8 || rows_of(x, "x") > 0xfffff || !aligned(x) || !aligned(w)) return false;
     FusedArgs args;
     args.epilogue = Epilogue::Store;
+    args.plain = true;
     fused_linear(x, w, out, args);
     return true;
 }
@@ -1766,7 +1768,7 @@ void Ops::fused_linear(const Tensor& a, const Tensor& w, const Tensor& out, cons
         prm.row_best_ld = args.row_best_ld;
         prm.row_best_rows = args.row_best_rows;
     }
-    took(sliced ? Path::FusedSliced : streamed ? Path::FusedRows : Path::FusedStaged);
+    took(args.plain ? Path::LinearFewRows : sliced ? Path::FusedSliced : streamed ? Path::FusedRows : Path::FusedStaged);
     if (sliced) {
         kernel_check(celeg_gemv_slices(&prm, static_cast<int>(epi), stream), "fused_linear (k-sliced)");
     } else if (streamed) {

@@ -68,6 +68,7 @@ struct FusedArgs {
     const ConvOperands* conv = nullptr;
     Tensor out_bf16;              // residual: the bfloat16 copy of the stream
     bool packed = false;          // w is [K/32, rows, 32] (pack_weight)
+    bool plain = false;           // nothing is fused: counted as a plain product
     // 32-bit store of an output head: beside the logits, the best (logit, index) of every share of
     // columns [row_best_rows, row_best_ld >= parts]; Ops::last_best_parts then says how many parts
     // of every row were written
@@ -102,7 +103,7 @@ struct StepPrologue {
 // graph records; a replay counts nothing): what tests and tools ask to see that a size took the
 // path it was meant to take.
 enum class Path : int {
-    AttentionDecode = 0, AttentionDecodeFresh, AttentionRows, AttentionGeneral, AttentionSigmoid, AttentionSigmoidRows, AttentionSigmoidDecode, DeltaRule, AttentionLatent, AttentionLatentRows, AttentionLatentDecode, AttentionBiased, AttentionBiasedRows, AttentionBiasedDecode, ChannelScan, MatrixMemory, MatrixMemoryRows, MatrixMemoryStep, DecayScan, DecayScanRows, DecayScanStep, LinearRecurrentUnit, RoutedExperts, LinearF32, LinearLibrary, LinearStandIn,
+    AttentionDecode = 0, AttentionDecodeFresh, AttentionRows, AttentionGeneral, AttentionSigmoid, AttentionSigmoidRows, AttentionSigmoidDecode, DeltaRule, AttentionLatent, AttentionLatentRows, AttentionLatentDecode, AttentionBiased, AttentionBiasedRows, AttentionBiasedDecode, ChannelScan, MatrixMemory, MatrixMemoryRows, MatrixMemoryStep, DecayScan, DecayScanRows, DecayScanStep, LinearRecurrentUnit, RoutedExperts, LinearF32, LinearLibrary, LinearFewRows, LinearStandIn,
     FusedSliced, FusedRows, FusedStaged, Tiled, TiledQkv, ArgmaxMerged, Count
 };
 const char* path_name(Path p);
