@@ -226,8 +226,7 @@ __device__ __forceinline__ void tile_epilogue(
     }
 }
 
-// ---- the q/k/v epilogue (heads of 64 columns: a wavefront of a 128x128 tile on 4x2 wavefronts
-// holds 32 rows of one head)
+// ---- the q/k/v epilogue (heads of 64 columns: a wavefront holds 16 or 32 rows of one head)
 #define QKV_HD 64
 // What it needs from memory, asked for before the product: the positions of the lane's rows
 // and the head's norm weight at the lane's columns; and, lanes 0 .. rows-1 of the wavefront, the
@@ -788,7 +787,8 @@ extern "C" void celeg_gemm_tiles_force(int shape) { g_force_shape = shape; }
 extern "C" void celeg_gemm_tiles_force_dies(int dies_m) { g_force_dies_m = dies_m; }
 
 // id, rows, weight rows, wavefronts along rows and along weight rows, stages, values of k a block of
-// the wide kernel (0: the kernel with tiles up to 256x128)
+// the wide kernel (0: the kernel with tiles up to 256x128).  The rule below takes 10, 11, 13 and 16 to 22; the
+// others are what tests and tuning runs compare them with.
 #define TILE_SHAPES(X) \
     X(0, 128, 128, 2, 2, 3, 0) \
     X(1, 256, 128, 2, 2, 3, 0) \
@@ -808,43 +808,84 @@ extern "C" void celeg_gemm_tiles_force_dies(int dies_m) { g_force_dies_m = dies_
     X(15, 256, 128, 4, 2, 3, 64) \
     X(16, 128, 64, 4, 2, 4, 0) \
     X(17, 64, 128, 2, 4, 4, 0) \
-    X(18, 128, 192, 4, 2, 3, 0)
+    X(18, 128, 192, 4, 2, 3, 0) \
+    X(19, 32, 64, 2, 2, 8, 0)  \
+    X(20, 64, 64, 4, 2, 4, 0)  \
+    X(21, 64, 192, 4, 2, 4, 0) \
+    X(22, 128, 128, 4, 2, 4, 0)
 
-static const int k_shape_bm[] = {128, 256, 128, 64, 128, 256, 128, 64, 64, 128, 128, 256, 256, 256, 128, 256, 128, 64, 128};
-static const int k_shape_bn[] = {128, 128, 64, 128, 128, 128, 128, 64, 64, 64, 128, 288, 160, 192, 192, 128, 64, 128, 192};
-#define N_TILE_SHAPES 19
+static const int k_shape_bm[] = {128, 256, 128, 64, 128, 256, 128, 64, 64, 128, 128, 256, 256, 256, 128, 256, 128, 64, 128, 32, 64, 64, 128};
+static const int k_shape_bn[] = {128, 128, 64, 128, 128, 128, 128, 64, 64, 64, 128, 288, 160, 192, 192, 128, 64, 128, 192, 64, 64, 192, 128};
+#define N_TILE_SHAPES 23
+
+// How the dies share the grid of tiles: every row of tiles of A is read by 8 / m dies, every column of
+// tiles of W by m of them; the split with the fewest bytes read of those that leave no die more tiles than it
+// has compute units, or of all if none does.
+#define DIE_UNITS 32
+struct Dies {
+    int m, per_die;      // dies along the rows; the most tiles a die gets
+};
+static Dies dies_of(int tiles_m, int tiles_n, int M, int weight_rows) {
+    Dies best{1, 0};
+    double best_cost = -1.;
+    for (int dm = 1; dm <= 8; dm *= 2) {
+        const int dn = 8 / dm;
+        if (dm > tiles_m || dn > tiles_n) continue;       // a die without a tile
+        const int per_die = ((tiles_m + dm - 1) / dm) * ((tiles_n + dn - 1) / dn);
+        const double cost = static_cast<double>(dn) * M + static_cast<double>(dm) * weight_rows;
+        const bool over = per_die > DIE_UNITS, best_over = best.per_die > DIE_UNITS;
+        if (best_cost < 0. || (over == best_over ? cost < best_cost : best_over)) {
+            best_cost = cost;
+            best = Dies{dm, per_die};
+        }
+    }
+    if (best_cost < 0.) best.per_die = tiles_m * ((tiles_n + 7) / 8);
+    return best;
+}
 
 static TileShape tile_shape(int M, int N, int K, int streams) {
     int id = 0;
     if (g_force_shape >= 0 && g_force_shape < N_TILE_SHAPES) id = g_force_shape;
     else {
-        // Measured at 2,048 rows (1,024 to 9,216 weight rows, 1,024 and 4,608 values of k):
-        // tiles of 128x128 with two workgroups of 8 wavefronts a compute unit where they give
-        // every unit one and a half or more (8 wavefronts: a tenth faster than 4), else
-        // smaller tiles, which fill the chip.
-        // Tiles of 256x288, one workgroup a compute unit, where a round of them (2.2 times as long
-        // as a round of 128x128 tiles, measured at 1,024 and 2,048 values of k) covers the product
-        // in less time: 2,048 rows by 9,216 weight rows are exactly one round, 44 us with the
-        // SwiGLU against 63 us.
-        const long long wide = static_cast<long long>((M + 127) / 128) * ((static_cast<long long>(N) * streams + 127) / 128);
-        const long long tiles288 = static_cast<long long>((M + 255) / 256) * ((static_cast<long long>(N) * streams + 287) / 288);
-        const long long rounds288 = (tiles288 + 255) / 256, rounds128 = (wide + 511) / 512;
-        // Few weight rows (w2, out_proj: 1,024 of them by 2,048 rows): what a compute unit pulls
-        // from L2 bounds the product, so tiles of 128x64 or 64x128 on 8 wavefronts, one a compute
-        // unit and 4 blocks of k in flight, beat 64x64 where they still give nearly every unit
-        // one (w2 at K = 4,608: 34.8 us as 128x64, 36.0 as 64x128, 40.3 as 64x64; out_proj at
-        // K = 1,024: 14.1, 13.6, 14.5).
-        const long long tall = static_cast<long long>((M + 127) / 128) * ((static_cast<long long>(N) * streams + 63) / 64);
-        const long long flat = static_cast<long long>((M + 63) / 64) * ((static_cast<long long>(N) * streams + 127) / 128);
-        // Tiles of 128x192 where they are just one a compute unit (in_proj, 2,048 rows by 3,072
-        // weight rows: 256 of them, 20.9 us against 22.2 on 384 tiles of 128x128).
-        const long long tiles192 = static_cast<long long>((M + 127) / 128) * ((static_cast<long long>(N) * streams + 191) / 192);
-        id = wide >= 384   ? (rounds288 * 22 < rounds128 * 10 ? 11 : (tiles192 > 192 && tiles192 <= 256 ? 18 : 10))
-             : wide >= 256 ? 10
-             : wide >= 192 ? 3
-             : tall >= 224 && K >= 2048 ? 16
-             : flat >= 224 ? 17
-                           : 7;
+        // The smallest tile of which no die gets more than one for each of its compute units: the workgroups then
+        // run side by side, each for as long as its own chain of blocks of k takes, and a smaller tile's
+        // chain is shorter (less to pull from L2 and from LDS a block, room for more blocks in flight).  Measured
+        // with weights from memory, us (chosen | the tiles of the rule before, which wanted few and large ones):
+        //   rows   w2 (1,024 x 4,608)  out_proj (1,024 x 1,024)  in_proj (3,072 x 1,024)  w1 with w3 (9,216 x 1,024)
+        //    100      17.7 | 25.6          7.1 |  9.2               6.9 |  8.7                11.1 | 12.3
+        //    300      17.8 | 26.1          7.3 |  9.4               7.9 |  8.9                13.9 | 16.8
+        //    600      21.1 | 26.3          8.5 |  9.6               9.8 |  9.8                19.1 | 21.2
+        //  1,000      24.9 | 27.3          8.9 | 10.1              14.2 | 14.6                28.4 | 37.4
+        //  1,400      36.0 | 36.0          9.9 | 10.9              17.9 | 18.9                37.4 | 37.4
+        //  2,048      37.4 | 37.4         12.3 | 12.3              19.3 | 19.3                41.4 | 41.4
+        //  4,096      53.2 | 70.1         20.2 | 21.0              29.6 | 33.9
+        // With a long K tiles of 128x64 and 64x128 are the same (w2 at 2,048 rows: 37.4 and 37.3).  Tiles of
+        // 64x192 end at 240: 256 of them (1,000 rows by 3,072) would be 12.9 us against 14.2 on 128x128, but how
+        // that product is cut is held by a test.  Two workgroups of 8 wavefronts a compute unit on 128x128 tiles
+        // come before 256x192 (w1 with w3 at 800 rows 23.2 us against 27.5).
+        const auto fits = [&](int bm, int bn, int on_a_unit) {
+            return dies_of((M + bm - 1) / bm, (N * streams + bn - 1) / bn, M, N * streams).per_die <= DIE_UNITS * on_a_unit;
+        };
+        if (fits(32, 64, 1)) id = 19;
+        else if (fits(64, 64, 1)) id = 20;
+        else if (K >= 2048 && fits(128, 64, 1)) id = 16;
+        else if (fits(64, 128, 1)) id = 17;
+        else if (((M + 63) / 64) * ((N * streams + 191) / 192) <= 240 && fits(64, 192, 1)) id = 21;
+        else if (fits(128, 128, 1)) id = 22;
+        else if (fits(128, 192, 1)) id = 18;
+        else if (fits(128, 128, 2)) id = 10;
+        else if (fits(256, 192, 1)) id = 13;
+        else if (fits(256, 288, 1)) id = 11;
+        else {
+            // More than a round: 128x128 with two workgroups a compute unit, or 256x288, one a compute unit, where
+            // the rounds of them (2.2 times as long as a round of 128x128 tiles, measured at 1,024 and 2,048 values
+            // of k) cover the product in less time.
+            const auto tiles = [&](int bm, int bn) {
+                return static_cast<long long>((M + bm - 1) / bm) * ((static_cast<long long>(N) * streams + bn - 1) / bn);
+            };
+            const long long rounds288 = (tiles(256, 288) + 255) / 256, rounds128 = (tiles(128, 128) + 511) / 512;
+            id = rounds288 * 22 < rounds128 * 10 ? 11 : 10;
+        }
     }
     return TileShape{id, k_shape_bm[id], k_shape_bn[id]};
 }
@@ -868,16 +909,7 @@ static int launch_tiles(const TileParams& p, hipStream_t stream) {
         raised = true;
     }
     const int tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N * NS + BN - 1) / BN;
-    // how the dies share the grid: every row of tiles of A is read by dies_n dies, every
-    // column of tiles of W by dies_m; the split with the fewest bytes read
-    int dies_m = 1;
-    double best = -1.;
-    for (int dm = 1; dm <= 8; dm *= 2) {
-        const int dn = 8 / dm;
-        if (dm > tiles_m || dn > tiles_n) continue;       // a die without a tile
-        const double cost = static_cast<double>(dn) * p.M + static_cast<double>(dm) * p.N * NS;
-        if (best < 0. || cost < best) { best = cost; dies_m = dm; }
-    }
+    int dies_m = dies_of(tiles_m, tiles_n, p.M, p.N * NS).m;
     if (g_force_dies_m > 0) dies_m = g_force_dies_m;
     const int dies_n = 8 / dies_m;
     const int per_die = ((tiles_m + dies_m - 1) / dies_m) * ((tiles_n + dies_n - 1) / dies_n);
@@ -930,7 +962,13 @@ extern "C" int celeg_gemm_tiles(const TileParams* params, int epi, hipStream_t s
                 p.n_layers <= 0 || p.layer < 0 || p.layer >= p.n_layers || misaligned(p.q_weight) || misaligned(p.k_weight) ||
                 misaligned(p.cos_sin))
                 return static_cast<int>(hipErrorInvalidValue);
-            // a wavefront of the 128x128 tile on 4x2 wavefronts holds 32 rows of one head
+            // (a wavefront holds 16 or 32 rows of one head of 64 columns; the smallest tile of which no die gets
+            // more than one for each of its compute units, as above.  In a model, 2,048 columns by
+            // 1,024: 301 rows 12.4 us, 600 rows 14.4, 2,048 rows 21.3; with the last of these for all 22.4, 22.6 and 23.0)
+            const auto fits = [&](int bm, int bn) { return dies_of((p.M + bm - 1) / bm, (p.N + bn - 1) / bn, p.M, p.N).per_die <= DIE_UNITS; };
+            if (fits(64, 64)) return launch_tiles<64, 64, 4, 1, 4, 0, T_QKV>(p, stream);
+            if (fits(64, 128)) return launch_tiles<64, 128, 4, 2, 4, 0, T_QKV>(p, stream);
+            if (fits(128, 128)) return launch_tiles<128, 128, 4, 2, 4, 0, T_QKV>(p, stream);
             return launch_tiles<128, 128, 4, 2, 2, 0, T_QKV>(p, stream);
         }
         default: return static_cast<int>(hipErrorInvalidValue);

@@ -158,9 +158,39 @@ def test_unsupported_sizes_are_refused(ops):
 
 
 # ---------------------------------------------------------------- the q/k/v product with its tail
+@pytest.mark.parametrize("M", [65, 256, 257, 513, 700, 1000, 1300, 2048, 2049])
+@pytest.mark.parametrize("N,K", [(1024, 4608), (1024, 1024), (3072, 64), (264, 128)])
+def test_a_row_is_the_same_in_every_chosen_tile(ops, M, N, K):
+    """Every tile that the rule picks over these rows sums a row's products in one order: the bits of a step's
+    last 65 rows are those of a step of these rows alone, for a plain product and behind the SwiGLU."""
+    ops._lib("gemm_tiles").celeg_gemm_tiles_force(-1)
+    a = randn(M, K, seed=12, dtype=BF)
+    w = randn(N, K, seed=13, scale=0.05, dtype=BF)
+    for epilogue, columns in (("store", N), ("swiglu", N // 2)):
+        big = torch.zeros(M + 1, columns, dtype=BF, device=DEV)
+        small = torch.empty(65, columns, dtype=BF, device=DEV)
+        ops.tiled_linear(a, w, big[:M], epilogue=epilogue)
+        ops.tiled_linear(a[M - 65:], w, small, epilogue=epilogue)
+        assert torch.equal(big[M - 65:M], small) and float(big[M].abs().max()) == 0
+    ref = product(a, w)
+    out = torch.empty(M, N, dtype=BF, device=DEV)
+    ops.tiled_linear(a, w, out)
+    assert float((out.double() - ref).abs().max()) <= 2 ** -7 * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("lengths", [[333, 131, 1, 97], [803, 131, 1, 166], [1990, 131, 1, 166]])
+def test_qkv_product_on_larger_tiles(ops, lengths):
+    """As below, on steps of as many rows as take the tiles of 64x128 and of 128x128 (one and two a compute unit)."""
+    check_qkv_product(ops, 16, 8, 128, True, True, [0, 5, 130, 77], lengths)
+
+
 @pytest.mark.parametrize("heads,kv_heads,K,rotate,normed", [(16, 8, 1024, True, True), (6, 2, 192, True, False),
                                                             (4, 4, 128, False, True), (3, 1, 64, True, True)])
 def test_qkv_product_with_norm_rotation_and_cache_write(ops, heads, kv_heads, K, rotate, normed):
+    check_qkv_product(ops, heads, kv_heads, K, rotate, normed, [0, 5, 130, 77], [203, 131, 1, 66])
+
+
+def check_qkv_product(ops, heads, kv_heads, K, rotate, normed, starts, lengths):
     """The product of the q, k and v projections that normalises and turns the query and key
     heads and writes keys and values into the pages inside its own kernel, against the product
     followed by qk_norm_rope_store: a step of three requests (portions that start at positions
@@ -172,7 +202,6 @@ def test_qkv_product_with_norm_rotation_and_cache_write(ops, heads, kv_heads, K,
     from celeg_amd.engine import StepEntry
     from kernel_harness import build_batch, make_cache
     hd, n_layers, layer, page_tokens = 64, 2, 1, 16
-    starts, lengths = [0, 5, 130, 77], [203, 131, 1, 66]
     total = sum(lengths)
     N = (heads + 2 * kv_heads) * hd
     a = randn(total, K, seed=30, dtype=BF)
@@ -186,7 +215,7 @@ def test_qkv_product_with_norm_rotation_and_cache_write(ops, heads, kv_heads, K,
     stats = (torch.rand(total, blocks, generator=g) * K / blocks).to(DEV)
     results = []
     for fused in (False, True):
-        cache = make_cache(kv_heads, hd, n_layers, BF, page_tokens=page_tokens, n_pages=64, max_context=512, slots=4)
+        cache = make_cache(kv_heads, hd, n_layers, BF, page_tokens=page_tokens, n_pages=64 + sum(lengths) // page_tokens, max_context=2048, slots=4)
         kv = cache.layer_cache(layer).kv
         slots = [cache.open() for _ in lengths]
         entries = []
