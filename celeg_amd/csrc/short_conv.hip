@@ -138,46 +138,6 @@ __global__ void short_conv_fwd_vec_kernel(
                             token_seq, seq_start, seq_slot, cu_seqlens, width, taps);
 }
 
-// The state update for VEC neighbouring channels of one request, by the thread that has just
-// read the old state for the request's first tokens: entry j becomes bx at position
-// end - taps + j, from the step's rows where they reach that far back, else from the old state.
-template <typename T>
-__device__ __forceinline__ void short_conv_state_vec(
-    int s, int ch, const T* __restrict__ bcx, int ld_bcx, float* state, size_t state_slot_stride,
-    const int* __restrict__ seq_start, const int* __restrict__ seq_slot,
-    const int* __restrict__ cu_seqlens, int width, int taps) {
-    constexpr int VEC = ConvVec<T>::n;
-    typedef typename ConvVec<T>::raw raw;
-    const int start = seq_start[s];
-    const int row0 = cu_seqlens[s];
-    const int n = cu_seqlens[s + 1] - row0;
-    const int end = start + n;
-    float* st = state + static_cast<size_t>(seq_slot[s]) * state_slot_stride + ch;
-    float v[CONV_VEC_MAX_TAPS][VEC];
-#pragma unroll
-    for (int j = 0; j < CONV_VEC_MAX_TAPS; ++j) {
-        if (j >= taps) break;
-        const int q = end - taps + j;
-        if (q >= start) {
-            const T* row = bcx + static_cast<size_t>(row0 + (q - start)) * ld_bcx;
-            const raw bv = *reinterpret_cast<const raw*>(row + ch);
-            const raw xv = *reinterpret_cast<const raw*>(row + 2 * width + ch);
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) v[j][i] = ConvVec<T>::at(bv, i) * ConvVec<T>::at(xv, i);
-        } else {
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) v[j][i] = q >= 0 ? st[static_cast<size_t>(q - start + taps) * width + i] : 0.f;
-        }
-    }
-    // every old entry has been read: now the new ones
-#pragma unroll
-    for (int j = 0; j < CONV_VEC_MAX_TAPS; ++j) {
-        if (j >= taps) break;
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) st[static_cast<size_t>(j) * width + i] = v[j][i];
-    }
-}
-
 // The same for TT tokens in a row per thread: where they all belong to one request and every
 // tap lies in rows of this step, a row's B and x are read once for all the tokens that use it
 // (a window that slides down the rows) instead of once per tap.  The sums are formed in the
@@ -186,13 +146,29 @@ __device__ __forceinline__ void short_conv_state_vec(
 // This kernel also updates the state, with no kernel behind it: the first taps-1 tokens of a
 // request's rows, the only ones that read the old state, are all computed by the block that
 // holds the request's first row (also those that lie in the next block, which skips them), and
-// the same thread then writes the new state for its channels.
-#define CONV_BLOCK_TOKENS 2     // (2,048 tokens of 1,024 channels, with the state update: 8.8 us with 2, 9.4 with 1 and 10.1 with 4 a thread; more were slower)
+// the same thread then writes the new state for its channels.  What a block needs beside its own rows
+// where requests begin or end in it (their places, old states, last rows, the rows behind the block) is
+// asked for without conditions, in two trips to memory: such blocks, one for every two decoding
+// requests beside a prompt, set the kernel's time (2,048 rows of 1,024 channels: 20 decoding requests
+// and a prompt 14.8 us with a load at a time there, now 7.0; one prompt 9.0, now 5.8; 24 rows 7.1, now 3.3; the taps,
+// 16 bytes a load instead of 4, are in these too).
+#define CONV_BLOCK_TOKENS 2     // (more need more registers than leave room for a second wavefront; 1 and 4 were slower before)
+typedef float conv_f32x4 __attribute__((ext_vector_type(4)));
+template <int VEC>
+__device__ __forceinline__ void conv_load(float (&to)[VEC], const float* from) {
+#pragma unroll
+    for (int i = 0; i < VEC; i += 4) {
+        const conv_f32x4 v = *reinterpret_cast<const conv_f32x4*>(from + i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) to[i + e] = v[e];
+    }
+}
+
 template <typename T, int TAPS, int TT>
 __global__ __launch_bounds__(256) void short_conv_fwd_block_kernel(
     const T* __restrict__ bcx, int ld_bcx, const float* __restrict__ w,
     const float* __restrict__ bias, float* state, size_t state_slot_stride,
-    T* __restrict__ out, const int* __restrict__ positions, const int* __restrict__ token_seq,
+    T* __restrict__ out, const int* __restrict__ token_seq,
     const int* __restrict__ seq_start, const int* __restrict__ seq_slot,
     const int* __restrict__ cu_seqlens, int width, int n_tokens) {
     constexpr int VEC = ConvVec<T>::n;
@@ -208,58 +184,134 @@ __global__ __launch_bounds__(256) void short_conv_fwd_block_kernel(
     if (t0 >= n_tokens) return;
     const int n = min(TT, n_tokens - t0);
     // (asked for ahead of the rows; what depends on it is asked for while the rows are on their way)
-    const int s = token_seq[t0], s_end = token_seq[min(t0 + TT - 1, n_tokens - 1)];
+    int seq[TT];
+#pragma unroll
+    for (int j = 0; j < TT; ++j) seq[j] = token_seq[min(t0 + j, n_tokens - 1)];
+    auto load_row = [&](int t, raw& bv, raw& xv) __attribute__((always_inline)) {
+        const T* row = bcx + static_cast<size_t>(min(max(t, 0), n_tokens - 1)) * ld_bcx;
+        bv = *reinterpret_cast<const raw*>(row + ch);
+        xv = *reinterpret_cast<const raw*>(row + 2 * width + ch);
+    };
+    auto load_gate = [&](int t) __attribute__((always_inline)) {
+        return *reinterpret_cast<const raw*>(bcx + static_cast<size_t>(min(t, n_tokens - 1)) * ld_bcx + width + ch);
+    };
     raw bv[TT + TAPS - 1], xv[TT + TAPS - 1], cv[TT];
 #pragma unroll
-    for (int j = 0; j < TT + TAPS - 1; ++j) {
-        const T* row = bcx + static_cast<size_t>(min(max(t0 - (TAPS - 1) + j, 0), n_tokens - 1)) * ld_bcx;
-        bv[j] = *reinterpret_cast<const raw*>(row + ch);
-        xv[j] = *reinterpret_cast<const raw*>(row + 2 * width + ch);
-    }
+    for (int j = 0; j < TT + TAPS - 1; ++j) load_row(t0 - (TAPS - 1) + j, bv[j], xv[j]);
 #pragma unroll
-    for (int j = 0; j < TT; ++j)
-        cv[j] = *reinterpret_cast<const raw*>(bcx + static_cast<size_t>(min(t0 + j, n_tokens - 1)) * ld_bcx + width + ch);
-    float wt[VEC][TAPS], b0[VEC];
+    for (int j = 0; j < TT; ++j) cv[j] = load_gate(t0 + j);
+    float taps_flat[VEC * TAPS], b0[VEC];        // tap of channel ch + i: [i * TAPS + tap]
+    conv_load<VEC * TAPS>(taps_flat, w + static_cast<size_t>(ch) * TAPS);
 #pragma unroll
-    for (int i = 0; i < VEC; ++i) {
-        b0[i] = bias ? bias[ch + i] : 0.f;
+    for (int i = 0; i < VEC; ++i) b0[i] = bias ? bias[ch + i] : 0.f;
+    auto store = [&](int t, const raw& gate, const float (&conv)[VEC]) __attribute__((always_inline)) {
+        raw o;
 #pragma unroll
-        for (int tap = 0; tap < TAPS; ++tap) wt[i][tap] = w[static_cast<size_t>(ch + i) * TAPS + tap];
-    }
+        for (int i = 0; i < VEC; ++i) ConvVec<T>::set(o, i, ConvVec<T>::at(gate, i) * conv[i]);
+        *reinterpret_cast<raw*>(out + static_cast<size_t>(t) * width + ch) = o;
+    };
     // the same for the whole workgroup
-    if (n < TT || s_end != s || t0 - (TAPS - 1) < cu_seqlens[s]) {
-        for (int j = 0; j < n; ++j) {
-            const int t = t0 + j;
-            const int first = cu_seqlens[token_seq[t]];
-            if (t - first < TAPS - 1 && first < t0) continue;      // the block of the request's first row has it
-            short_conv_token_vec<T>(t, ch, bcx, ld_bcx, w, bias, state, state_slot_stride, out,
-                                    positions, token_seq, seq_start, seq_slot, cu_seqlens, width, TAPS);
+    if (n < TT || seq[TT - 1] != seq[0] || t0 - (TAPS - 1) < cu_seqlens[seq[0]]) {
+        // the requests of the block's rows
+        int first[TT], last[TT], start[TT], slot[TT];
+#pragma unroll
+        for (int j = 0; j < TT; ++j) {
+            first[j] = cu_seqlens[seq[j]];
+            last[j] = cu_seqlens[seq[j] + 1];
+            start[j] = seq_start[seq[j]];
+            slot[j] = seq_slot[seq[j]];
         }
-        for (int j = 0; j < n; ++j) {
-            const int t = t0 + j;
-            const int sj = token_seq[t];
-            if (cu_seqlens[sj] != t) continue;                     // requests that begin in this block:
-            const int last = min(t + TAPS - 1, cu_seqlens[sj + 1]);
-            for (int u = t0 + n; u < last; ++u)                    // their tokens in the next block that read the old state,
-                short_conv_token_vec<T>(u, ch, bcx, ld_bcx, w, bias, state, state_slot_stride, out,
-                                        positions, token_seq, seq_start, seq_slot, cu_seqlens, width, TAPS);
-            short_conv_state_vec<T>(sj, ch, bcx, ld_bcx, state, state_slot_stride, seq_start, seq_slot,      // then the new one
-                                    cu_seqlens, width, TAPS);
+        // rows behind the block that may read an old state (rows 1 .. TAPS-2 of a request that begins at its end)
+        constexpr int EXT = TAPS - 2;
+        raw ebv[EXT > 0 ? EXT : 1], exv[EXT > 0 ? EXT : 1], ecv[EXT > 0 ? EXT : 1];
+#pragma unroll
+        for (int e = 0; e < EXT; ++e) {
+            load_row(t0 + TT + e, ebv[e], exv[e]);
+            ecv[e] = load_gate(t0 + TT + e);
+        }
+        // every row's request: its old state, and the last rows it brings
+        float old[TT][TAPS][VEC];
+        raw lbv[TT][TAPS], lxv[TT][TAPS];
+#pragma unroll
+        for (int j = 0; j < TT; ++j) {
+            const float* st = state + static_cast<size_t>(slot[j]) * state_slot_stride + ch;
+#pragma unroll
+            for (int k = 0; k < TAPS; ++k) {
+                conv_load<VEC>(old[j][k], st + static_cast<size_t>(k) * width);
+                load_row(max(last[j] - TAPS + k, first[j]), lbv[j][k], lxv[j][k]);
+            }
+        }
+        // B x at `back` rows before row `at` of the request of row j: a row of the step (row r of the window
+        // t0 - (TAPS-1) ..), an old entry, or zero before position 0
+        auto window = [&](int r, int i) __attribute__((always_inline)) {       // r is known when this is compiled
+            return r < TT + TAPS - 1 ? ConvVec<T>::at(bv[r], i) * ConvVec<T>::at(xv[r], i)
+                                     : ConvVec<T>::at(ebv[r - (TT + TAPS - 1) < EXT ? r - (TT + TAPS - 1) : 0], i) *
+                                           ConvVec<T>::at(exv[r - (TT + TAPS - 1) < EXT ? r - (TT + TAPS - 1) : 0], i);
+        };
+        auto token = [&](int j, int u, const raw& gate) __attribute__((always_inline)) {     // row t0 + u, of row j's request
+            const int at = t0 + u - first[j];
+            float conv[VEC];
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) conv[i] = b0[i];
+#pragma unroll
+            for (int tap = 0; tap < TAPS; ++tap) {
+                const int from = at - (TAPS - 1 - tap);          // < 0: entry from + TAPS of the old state
+                // (positions before 0 add nothing, not even a zero: the sum of a short sequence keeps its bits)
+                if (start[j] + from < 0) continue;
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) {
+                    float bx = window(u + tap, i);
+#pragma unroll
+                    for (int k = 1; k < TAPS; ++k) bx = from + TAPS == k ? old[j][k][i] : bx;
+                    conv[i] = fmaf(taps_flat[i * TAPS + tap], bx, conv[i]);
+                }
+            }
+            store(t0 + u, gate, conv);
+        };
+#pragma unroll
+        for (int j = 0; j < TT; ++j) {
+            if (j >= n) continue;
+            // (the block of the request's first row has those of its rows that read the old state)
+            if (first[j] >= t0 || t0 + j - first[j] >= TAPS - 1) token(j, j, cv[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < TT; ++j) {
+            if (j >= n || first[j] != t0 + j) continue;          // requests that begin in this block:
+#pragma unroll
+            for (int e = 0; e < EXT; ++e)                        // their rows in the next block that read the old state,
+                if (t0 + TT + e < min(t0 + j + TAPS - 1, last[j])) token(j, TT + e, ecv[e]);
+            // then the new state: entry k is B x at position end - TAPS + k
+            const int rows = last[j] - first[j];
+            float* st = state + static_cast<size_t>(slot[j]) * state_slot_stride + ch;
+#pragma unroll
+            for (int k = 0; k < TAPS; ++k) {
+                const int from = rows - TAPS + k;                // < 0: entry from + TAPS of the old state
+                float v[VEC];
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) {
+                    v[i] = ConvVec<T>::at(lbv[j][k], i) * ConvVec<T>::at(lxv[j][k], i);
+#pragma unroll
+                    for (int m = 1; m < TAPS; ++m) v[i] = from + TAPS == m && from < 0 ? old[j][m][i] : v[i];
+                    if (start[j] + from < 0) v[i] = 0.f;
+                }
+#pragma unroll
+                for (int i = 0; i < VEC; i += 4)
+                    *reinterpret_cast<conv_f32x4*>(st + static_cast<size_t>(k) * width + i) = conv_f32x4{v[i], v[i + 1], v[i + 2], v[i + 3]};
+            }
         }
         return;
     }
 #pragma unroll
     for (int j = 0; j < TT; ++j) {
-        raw o;
+        float conv[VEC];
 #pragma unroll
         for (int i = 0; i < VEC; ++i) {
-            float conv = b0[i];
+            conv[i] = b0[i];
 #pragma unroll
             for (int tap = 0; tap < TAPS; ++tap)
-                conv = fmaf(wt[i][tap], ConvVec<T>::at(bv[j + tap], i) * ConvVec<T>::at(xv[j + tap], i), conv);
-            ConvVec<T>::set(o, i, ConvVec<T>::at(cv[j], i) * conv);
+                conv[i] = fmaf(taps_flat[i * TAPS + tap], ConvVec<T>::at(bv[j + tap], i) * ConvVec<T>::at(xv[j + tap], i), conv[i]);
         }
-        *reinterpret_cast<raw*>(out + static_cast<size_t>(t0 + j) * width + ch) = o;
+        store(t0 + j, cv[j], conv);
     }
 }
 
@@ -309,7 +361,7 @@ extern "C" int celeg_short_conv(const void* bcx, int ld_bcx, int dtype, const fl
         aligned(bcx) && aligned(out)) {
         const int threads = min(256, (width / vec + 63) / 64 * 64);
         dim3 vblock(threads), vgrid(n_tokens, (width / vec + threads - 1) / threads);
-        if (taps >= 2 && taps <= 4) {      // (n_tokens >= 16 here)
+        if (taps >= 2 && taps <= 4 && aligned(w) && aligned(state) && state_slot_stride % 4 == 0) {      // (n_tokens >= 16 here)
             const int tt = g_force_block_tokens == 4 ? 4 : CONV_BLOCK_TOKENS;
             dim3 bgrid(((n_tokens + tt - 1) / tt + 7) / 8 * 8, vgrid.y);      // (8 runs of tokens, one a die)
 #define CELEG_CONV_BLOCK(T_, TAPS_)                                                                \
@@ -317,8 +369,7 @@ extern "C" int celeg_short_conv(const void* bcx, int ld_bcx, int dtype, const fl
 #define CELEG_CONV_BLOCK_TT(T_, TAPS_, TT_)                                                        \
     hipLaunchKernelGGL((short_conv_fwd_block_kernel<T_, TAPS_, TT_>), bgrid, vblock, 0, stream,     \
                        static_cast<const T_*>(bcx), ld_bcx, w, bias, state, state_slot_stride,      \
-                       static_cast<T_*>(out), positions, token_seq, seq_start, seq_slot, cu_seqlens, \
-                       width, n_tokens)
+                       static_cast<T_*>(out), token_seq, seq_start, seq_slot, cu_seqlens, width, n_tokens)
 #define CELEG_CONV_BLOCK_T(T_)                                                                     \
     if (taps == 2) { CELEG_CONV_BLOCK(T_, 2); } else if (taps == 3) { CELEG_CONV_BLOCK(T_, 3); }     \
     else { CELEG_CONV_BLOCK(T_, 4); }

@@ -333,6 +333,27 @@ def test_short_conv_long_steps_with_single_tokens_and_short_portions(ops, dtype,
         torch.testing.assert_close(torch.cat(got[i]), ref, **tol(dtype))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_short_conv_taps_on_any_alignment(ops, dtype):
+    """Taps that do not lie on 16 bytes take the kernels without the wide loads: the same bits, outputs and state."""
+    from celeg_amd.engine import StepEntry
+    width, taps, n = 64, 3, 40
+    bcx, flat = randn(n, 3 * width, seed=80, dtype=dtype), randn(width * taps + 1, seed=90)
+    got = []
+    for w in (flat[1:].view(width, taps), flat[1:].clone().view(width, taps)):
+        cache = make_cache(0, 0, 0, dtype, states=[(0, "bx", (taps, width))], slots=3)
+        state, slots = cache.layer_cache(0).states["bx"], [cache.open(), cache.open()]
+        outs = []
+        for pos in (0, n // 2):
+            batch, keep = build_batch(ops, cache, [StepEntry(slots[0], pos, [0] * (n // 2 - 1)), StepEntry(slots[1], pos // 20, [0])])
+            rows = bcx[pos:pos + n // 2].contiguous()
+            out = torch.empty(n // 2, width, dtype=dtype, device=DEV)
+            ops.short_conv(rows, w, None, state, out, batch)
+            outs.append(out)
+        got.append((torch.cat(outs), state.clone()))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
 def test_short_conv_reference_vector(ops):
     # tests/reference_test.cpp:68-73: hidden 2, L 3, bcx {1,1 | 1,1 | 2,4}, weights
     # {1,2,3 ; 1,2,3} channel-major, position 0, zero state -> {6, 12}
