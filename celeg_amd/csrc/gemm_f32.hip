@@ -8,13 +8,13 @@
 // (src/model/weight_plan.cpp:82-130).
 //
 // A workgroup owns a tile of 16 RT rows x 16 CT columns; its wavefronts take the segments in turn and
-// leave their sums in LDS, where the workgroup adds them in order.  Few rows are bound by reading W: one
-// column tile a workgroup, up to 16 wavefronts that each ask for a whole segment (8 KiB) at once, so
+// leave their sums in LDS, where the workgroup adds them in order.  Few rows are bound by reading W: up to 16
+// columns a workgroup, up to 16 wavefronts that each ask for 8 KiB at once, so
 // that even a 1024 x 1024 matrix is asked for by 512 wavefronts in one trip to memory.  Many rows are bound
 // by the matrix cores: larger tiles, operands straight from the caches (16 bytes a cycle and CU of them).
 // Measured in a chain over different matrices (before: 64 x 64 tiles of vector instructions, k in order,
-// 137 us for any product with K = 1,024): 2 rows, 1024 x 1024 4.5 us, 3072 x 1024 5.6 us, 1024 x 4608
-// 14.8 us (before 613), 65536 x 1024 54 us (4.9 TB/s; before 247); 64 rows, 3072 x 1024 13.7 us; 2,048 rows,
+// 137 us for any product with K = 1,024): 2 rows, 1024 x 1024 3.3 us, 3072 x 1024 5.5 us, 1024 x 4608
+// 7.2 us (before 613), 65536 x 1024 54 us (5.0 TB/s; before 247); 64 rows, 3072 x 1024 13.7 us; 2,048 rows,
 // 4608 x 1024 256 us (76 TFLOP/s).  Error against 64 bits 2.1e-7 of the result (2-norm), before 3 times that.
 #include "common.h"
 
@@ -142,6 +142,99 @@ __global__ __launch_bounds__(MAX_THREADS) void gemm_f32_kernel(
     }
 }
 
+// The products of up to 16 rows.  The 16 x 16 tile of the instruction is cut into G x G blocks: its rows are
+// (segment g of G, column j of 16 / G) of W, its columns (segment g', row m of 16 / G) of X, so the blocks
+// g = g' on the diagonal are G segments' sums of the same outputs and the others are dropped.  A workgroup
+// then owns 16 / G columns, and a matrix of few columns (w2: 1,024) is spread over G times as many
+// workgroups; a segment's sum is formed by the same instructions, so the outputs keep their bits.
+// 2 rows: 1024 x 4608 7.2 us (on 16 columns a workgroup 14.8), 1024 x 1024 3.3 (4.5).
+template <int G, bool VEC>
+__global__ __launch_bounds__(1024) void gemm_f32_slices_kernel(
+    const float* __restrict__ X, int ldx, const float* __restrict__ W, int ldw,
+    const float* __restrict__ bias, float* __restrict__ Y, int ldy, int M, int N, int K, int wide_store) {
+    constexpr int MP = 16 / G, ITEMS = MP * MP / 4;      // sums of four neighbouring columns of a row
+    extern __shared__ f32x4_t parts[];                    // [segment of the round][item]
+    const int wave = threadIdx.x / CELEG_WAVE, lane = threadIdx.x % CELEG_WAVE;
+    const int n_waves = blockDim.x / CELEG_WAVE;
+    const int qd = lane >> 4, r16 = lane & 15;
+    const int col0 = blockIdx.x * MP;
+    const float* const x_row = X + static_cast<size_t>(min(r16 % MP, M - 1)) * ldx;
+    const float* const w_row = W + static_cast<size_t>(min(col0 + r16 % MP, N - 1)) * ldw;
+    // this lane's sums: row (lane % MP) and columns 4 (quad in its block) .. + 3, of segment `of`
+    const int of = qd / (MP / 4), item = (qd % (MP / 4)) * MP + lane % MP;
+    const bool on_diagonal = r16 / MP == of;
+    const int segments = (K + F32_SEGMENT - 1) / F32_SEGMENT;
+    f32x4_t total = {0.f, 0.f, 0.f, 0.f};
+    for (int first = 0; first < segments; first += n_waves * G) {
+        const int mine = first + wave * G;                // this wavefront's segments: G of them from here
+        const int k0 = (mine + r16 / MP) * F32_SEGMENT + 4 * qd;
+        f32x4_t wv[F32_PIECES], xv[F32_PIECES];
+        if (VEC && (mine + G) * F32_SEGMENT <= K) {
+#pragma unroll
+            for (int s = 0; s < F32_PIECES; ++s) wv[s] = *reinterpret_cast<const f32x4_t*>(w_row + k0 + 16 * s);
+#pragma unroll
+            for (int s = 0; s < F32_PIECES; ++s) xv[s] = *reinterpret_cast<const f32x4_t*>(x_row + k0 + 16 * s);
+        } else {
+#pragma unroll
+            for (int s = 0; s < F32_PIECES; ++s) {
+                const int k = k0 + 16 * s;
+                wv[s] = xv[s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+                if (VEC) {
+                    if (k < K) {
+                        wv[s] = *reinterpret_cast<const f32x4_t*>(w_row + k);
+                        xv[s] = *reinterpret_cast<const f32x4_t*>(x_row + k);
+                    }
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (k + i < K) {
+                            wv[s][i] = w_row[k + i];
+                            xv[s][i] = x_row[k + i];
+                        }
+                }
+            }
+        }
+        f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < F32_PIECES; ++s)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[s][i], xv[s][i], acc, 0, 0, 0);
+        if (first) __syncthreads();                       // the sums before have been read
+        if (on_diagonal) parts[(wave * G + of) * ITEMS + item] = acc;
+        __syncthreads();
+        const int n = min(n_waves * G, segments - first);
+        if (threadIdx.x < ITEMS)
+            for (int g = 0; g < n; ++g) total += parts[g * ITEMS + threadIdx.x];
+    }
+    const int row = threadIdx.x % MP, col = col0 + 4 * (threadIdx.x / MP);
+    if (threadIdx.x >= ITEMS || row >= M) return;
+    float* y = Y + static_cast<size_t>(row) * ldy + col;
+    if (wide_store && col + 3 < N) {
+        if (bias) total += f32x4_t{bias[col], bias[col + 1], bias[col + 2], bias[col + 3]};
+        *reinterpret_cast<f32x4_t*>(y) = total;
+        return;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        if (col + r < N) y[r] = total[r] + (bias ? bias[col + r] : 0.f);
+}
+
+template <int G>
+static int launch_f32_slices(const float* X, int ldx, const float* W, int ldw, const float* bias, float* Y, int ldy,
+                             int M, int N, int K, hipStream_t stream) {
+    const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    const bool vec = K % 4 == 0 && ldx % 4 == 0 && ldw % 4 == 0 && aligned(X) && aligned(W);
+    const int wide_store = ldy % 4 == 0 && aligned(Y);
+    constexpr int MP = 16 / G;
+    const int groups = ((K + F32_SEGMENT - 1) / F32_SEGMENT + G - 1) / G;
+    const int rounds = (groups + 15) / 16, waves = (groups + rounds - 1) / rounds;     // as even as it goes: 36 are 3 rounds of 12
+    const dim3 grid((N + MP - 1) / MP), block(waves * CELEG_WAVE);
+    const size_t lds = static_cast<size_t>(waves) * G * (MP * MP / 4) * sizeof(f32x4_t);
+    auto kernel = vec ? &gemm_f32_slices_kernel<G, true> : &gemm_f32_slices_kernel<G, false>;
+    hipLaunchKernelGGL(kernel, grid, block, lds, stream, X, ldx, W, ldw, bias, Y, ldy, M, N, K, wide_store);
+    return CELEG_LAUNCH_RESULT();
+}
+
 template <int RT, int CT, int GROUP, int MAX_THREADS>
 static int launch_f32(const float* X, int ldx, const float* W, int ldw, const float* bias, float* Y, int ldy,
                       int M, int N, int K, hipStream_t stream) {
@@ -165,7 +258,11 @@ extern "C" int celeg_gemm_f32(const float* X, int ldx, const float* W, int ldw, 
                               float* Y, int ldy, int M, int N, int K, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
     if (K <= 0) return static_cast<int>(hipErrorInvalidValue);
-    if (M <= 16) return launch_f32<1, 1, 8, 1024>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
+    // (blocks of 4 or 8 columns while tiles of 16 would leave compute units without a second workgroup)
+    if (M <= 16) {
+        const int g = N >= 512 * 16 || M > 8 ? 1 : M > 4 ? 2 : 4;
+        return (g == 4 ? launch_f32_slices<4> : g == 2 ? launch_f32_slices<2> : launch_f32_slices<1>)(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
+    }
     if (M <= 32) return launch_f32<2, 1, 8, 512>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
     if (M <= 64) return launch_f32<4, 1, 4, 512>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
     // 64 x 64 tiles (an operand from the caches serves four products) once there are two for every CU; below

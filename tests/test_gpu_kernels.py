@@ -105,8 +105,8 @@ def test_gemm_f32_is_true_32bit_and_row_independent(ops, M, N, K):
     assert torch.equal(one[0], out[M // 2])
 
 
-@pytest.mark.parametrize("M", [1, 2, 16, 17, 32, 33, 64, 65, 130])
-@pytest.mark.parametrize("N,K", [(4, 4), (17, 77), (48, 128), (61, 132), (64, 2048), (70, 4612)])
+@pytest.mark.parametrize("M", [1, 2, 4, 5, 8, 9, 16, 17, 32, 33, 64, 65, 130])
+@pytest.mark.parametrize("N,K", [(8200, 68), (4, 4), (17, 77), (48, 128), (61, 132), (64, 2048), (70, 4612)])
 def test_gemm_f32_tiles(ops, M, N, K):
     """Every tile of the 32-bit product at its edges: against 64 bits within the bound of a sum of 128 products and of the
     segments' sums, rows on any alignment, and a row's bits whatever rows it is computed with."""
