@@ -206,9 +206,7 @@ __global__ __launch_bounds__(ROPE_WAVES * CELEG_WAVE) void qk_norm_rope_store_qu
     }
 #pragma unroll
     for (int i = 0; i < TOKENS; ++i) {
-        float sum = x[i][0] * x[i][0] + x[i][1] * x[i][1] + x[i][2] * x[i][2] + x[i][3] * x[i][3];
-#pragma unroll
-        for (int off = LPH / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, CELEG_WAVE);
+        const float sum = lanes_sum<LPH>(x[i][0] * x[i][0] + x[i][1] * x[i][1] + x[i][2] * x[i][2] + x[i][3] * x[i][3]);
         if (weight) {
             const float inv = 1.0f / sqrtf(sum / static_cast<float>(HD) + eps);
 #pragma unroll

@@ -33,31 +33,6 @@ __device__ __forceinline__ size_t kv_block(int page, int n_layers, int layer, in
 
 
 
-// Combining a value with the one that lane ^ 16 (lane ^ 32) holds, by the lane-swap
-// instructions of gfx950: both operands start as x; the swap leaves (row 0, row 0, row 2,
-// row 2) in one and (row 1, row 1, row 3, row 3) in the other (rows of 16 lanes; halves of
-// 32 lanes likewise), so the two results are the lane's own value and its partner's.
-__device__ __forceinline__ float max_row16(float x) {
-    const unsigned u = __float_as_uint(x);
-    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float max_half32(float x) {
-    const unsigned u = __float_as_uint(x);
-    const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float sum_row16(float x) {
-    const unsigned u = __float_as_uint(x);
-    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-__device__ __forceinline__ float sum_half32(float x) {
-    const unsigned u = __float_as_uint(x);
-    const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
 // ================================================================ rows of portions
 // A workgroup takes a tile of 64*RT rows of one request for one query head.  Its 8
 // wavefronts are two halves of 4; the wavefronts of a half each own RT tiles of 16 rows of
@@ -640,8 +615,7 @@ __device__ __forceinline__ void decode_prepare_head(float (&x)[KS][8], const boo
         for (int s = 0; s < KS; ++s)
 #pragma unroll
             for (int e = 0; e < 8; ++e) ssq += x[s][e] * x[s][e];
-        ssq += __shfl_xor(ssq, 16, 64);
-        ssq += __shfl_xor(ssq, 32, 64);
+        ssq = sum_half32(sum_row16(ssq));
         const float inv = 1.0f / sqrtf(ssq / static_cast<float>(HD) + eps);
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
@@ -804,8 +778,7 @@ __global__ __launch_bounds__(WAVES * 64) void attention_decode_heads_kernel(
             if (chunk == 0 && c == 0)        // one copy into the page
                 *reinterpret_cast<bf16x8_t*>(fresh.k_pool + block + static_cast<size_t>(pos & page_mask) * HD + s * 32 + qd * 8) = kb16;
         }
-        dot += __shfl_xor(dot, 16, 64);
-        dot += __shfl_xor(dot, 32, 64);
+        dot = sum_half32(sum_row16(dot));
         const float s_new = dot * scale;
         const float m_new = fmaxf(m_run, s_new);
         const float keep = expf(m_run - m_new);         // e^(-inf) = 0 where the part holds no other key
@@ -874,8 +847,7 @@ __global__ __launch_bounds__(WAVES * 64) void attention_decode_heads_kernel(
                 mx = fmaxf(mx, sc[T][i]);
             }
         }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));        // finite: the round holds a key
+        mx = max_half32(max_row16(mx));        // finite: the round holds a key
         const float m_new = fmaxf(m_run, mx);
         const float keep = expf(m_run - m_new);         // e^(-inf) = 0 the first time
         float psum = 0.f;
@@ -886,8 +858,7 @@ __global__ __launch_bounds__(WAVES * 64) void attention_decode_heads_kernel(
                 sc[T][i] = expf(sc[T][i] - m_new);
                 psum += sc[T][i];
             }
-        psum += __shfl_xor(psum, 16, 64);
-        psum += __shfl_xor(psum, 32, 64);
+        psum = sum_half32(sum_row16(psum));
         l_run = l_run * keep + psum;
         m_run = m_new;
 #pragma unroll

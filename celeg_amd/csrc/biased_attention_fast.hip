@@ -148,8 +148,7 @@ __device__ __forceinline__ void bf_block(const __bf16* ks, const __bf16* vs, con
             sacc[kt][i] = x;
             top = fmaxf(top, x);
         }
-    top = fmaxf(top, __shfl_xor(top, 16, CELEG_WAVE));
-    top = fmaxf(top, __shfl_xor(top, 32, CELEG_WAVE));
+    top = max_half32(max_row16(top));
     const float new_top = fmaxf(row.top, top);
     const float base = new_top == -INFINITY ? 0.f : new_top;      // (a row that has seen no key yet: every weight 0)
     const float keep = bf_exp2(row.top - base);
@@ -326,8 +325,7 @@ __global__ __launch_bounds__(BF_WAVES * CELEG_WAVE) void biased_attention_rows_k
         bf_block<D, V>(ks, vs, qreg, row, kb, my_pos, a.window, a.keep_first, blocks.kept(i), r, quad, s2, b1, b2, biased, cap2);
     }
     float total = row.sum;
-    total += __shfl_xor(total, 16, CELEG_WAVE);
-    total += __shfl_xor(total, 32, CELEG_WAVE);
+    total = sum_half32(sum_row16(total));
     if (r >= rows_here) return;
     const size_t at = static_cast<size_t>(row0 + my_row);
     bf_store<V, FULL>(row, total, a.gate ? a.gate + at * a.ldg + static_cast<size_t>(h) * vd : nullptr, a.out + at * a.ldo + static_cast<size_t>(h) * vd,
@@ -426,8 +424,7 @@ __global__ __launch_bounds__(WAVES * CELEG_WAVE) void biased_attention_tile_kern
 #pragma unroll
             for (int i = 0; i < 4; ++i) row.acc[dt][i] = fmaf(theirs[(2 + dt * 4 + i) * CELEG_WAVE + lane], f, row.acc[dt][i]);
     }
-    total += __shfl_xor(total, 16, CELEG_WAVE);
-    total += __shfl_xor(total, 32, CELEG_WAVE);
+    total = sum_half32(sum_row16(total));
     if (r >= rows_here) return;
     const size_t at = static_cast<size_t>(row0 + my_row);
     bf_store<V, FULL>(row, total, a.gate ? a.gate + at * a.ldg + static_cast<size_t>(h) * vd : nullptr, a.out + at * a.ldo + static_cast<size_t>(h) * vd,

@@ -287,9 +287,7 @@ void gemm_rows_kernel(const void* const a_, const bf16* const w_, const int* con
             v = finish_output<EPI>(p, rc, nc, sum, early_fetch<EPI>(p, rc, nc));
         }
         if (EPI == E_RESIDUAL && p.stats_out) {
-            float sq = v * v;               // the COLS columns of a row sit in COLS neighbouring lanes
-#pragma unroll
-            for (int off = COLS / 2; off > 0; off >>= 1) sq += __shfl_xor(sq, off, 64);
+            const float sq = lanes_sum<COLS>(v * v);   // the COLS columns of a row sit in COLS neighbouring lanes
             if (j == 0 && r < M) p.stats_out[static_cast<size_t>(r) * p.stats_ld_out + blockIdx.x] = sq;
         }
         if (EPI == E_STORE_F32 && p.row_best) {

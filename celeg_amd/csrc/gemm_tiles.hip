@@ -91,8 +91,7 @@ __device__ __forceinline__ void tile_row_scales(const TileParams& p, const int f
 #pragma unroll
     for (int tm = 0; tm < FM; ++tm) {
         float t = ssq[tm];
-        t += __shfl_xor(t, 16, 64);
-        t += __shfl_xor(t, 32, 64);
+        t = sum_half32(sum_row16(t));
         scale[tm] = 1.0f / sqrtf(t / static_cast<float>(p.K) + p.eps);
     }
 }
@@ -212,8 +211,7 @@ __device__ __forceinline__ void tile_epilogue(
 #pragma unroll
         for (int tm = 0; tm < FM; ++tm) {
             float s = sq[tm];
-            s += __shfl_xor(s, 16, 64);
-            s += __shfl_xor(s, 32, 64);
+            s = sum_half32(sum_row16(s));
             if (q == 0) red[wn * BM + wm * WTM + tm * 16 + r16] = s;
         }
         __syncthreads();
@@ -314,8 +312,7 @@ __device__ __forceinline__ void qkv_epilogue(const TileParams& p, floatx4_t (&ac
                 ssq += x[j][i] * x[j][i];
             }
         if (normed) {
-            ssq += __shfl_xor(ssq, 16, 64);
-            ssq += __shfl_xor(ssq, 32, 64);
+            ssq = sum_half32(sum_row16(ssq));
             const float inv = 1.0f / sqrtf(ssq / static_cast<float>(QKV_HD) + p.qk_eps);
 #pragma unroll
             for (int j = 0; j < 4; ++j)

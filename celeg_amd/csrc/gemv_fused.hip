@@ -163,11 +163,7 @@ __device__ __forceinline__ void gemv_epilogue(const GemvParams& p, floatx4_t (&a
         if (EPI == E_RESIDUAL && p.stats_out) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                float s = sq[r];
-                s += __shfl_xor(s, 1, 64);
-                s += __shfl_xor(s, 2, 64);
-                s += __shfl_xor(s, 4, 64);
-                s += __shfl_xor(s, 8, 64);
+                const float s = lanes_sum<16>(sq[r]);
                 const int m = mt * 16 + 4 * q + r;
                 if (c16 == 0 && m < M)
                     p.stats_out[static_cast<size_t>(m) * p.stats_ld_out + tile] = s;

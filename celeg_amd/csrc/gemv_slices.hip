@@ -185,8 +185,7 @@ void gemv_slices_kernel(const void* const a_, const bf16* const w_, const int* c
     }
     float scale = 1.f;
     if (p.stats) {
-#pragma unroll
-        for (int off = LPR / 2; off > 0; off >>= 1) ssq += __shfl_xor(ssq, off, 64);
+        ssq = lanes_sum<LPR>(ssq);
         // the lanes of row em - fw * ROWS_FW hold its sum
         const float total = __shfl(ssq, ((em - (ROWS_BY_WAVE ? fw * ROWS_FW : 0)) & (ROWS_FW - 1)) * LPR, 64);
         scale = 1.0f / sqrtf(total / static_cast<float>(K) + p.eps);
@@ -225,9 +224,7 @@ void gemv_slices_kernel(const void* const a_, const bf16* const w_, const int* c
             if (p.out_bf16) static_cast<bf16*>(p.out_bf16)[static_cast<size_t>(em) * p.ld_bf16 + en] = from_float<bf16>(v);
         }
         if (p.stats_out) {
-            float sq = v * v;                   // the MP columns of a row and tile sit in MP neighbouring lanes
-#pragma unroll
-            for (int off = MP / 2; off > 0; off >>= 1) sq += __shfl_xor(sq, off, 64);
+            const float sq = lanes_sum<MP>(v * v);   // the MP columns of a row and tile sit in MP neighbouring lanes
             // (one partial sum a tile: CT of them a workgroup)
             if (t % MP == 0 && em < M && t < MP * MP * CT)
                 p.stats_out[static_cast<size_t>(em) * p.stats_ld_out + blockIdx.x * CT + tile_ct] = sq;

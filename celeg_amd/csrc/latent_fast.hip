@@ -30,12 +30,10 @@ typedef unsigned int lat_u32x4 __attribute__((ext_vector_type(4)));
 #define LOG2E 1.4426950408889634f
 
 __device__ __forceinline__ float quad_max(float v) {      // over the four lanes that share a column
-    v = fmaxf(v, __shfl_xor(v, 16, 64));
-    return fmaxf(v, __shfl_xor(v, 32, 64));
+    return max_half32(max_row16(v));
 }
 __device__ __forceinline__ float quad_sum(float v) {
-    v += __shfl_xor(v, 16, 64);
-    return v + __shfl_xor(v, 32, 64);
+    return sum_half32(sum_row16(v));
 }
 
 template <int FORM, int KSMAX, int DTMAX, int RT, bool EXACT>

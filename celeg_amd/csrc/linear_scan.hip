@@ -193,14 +193,6 @@ __global__ void gla_prepare_kernel(const T* __restrict__ q, int ldq, const T* __
     if (c < v_cols) v32[static_cast<size_t>(t) * v_cols + c] = to_float(v[static_cast<size_t>(t) * ldv + c]);
 }
 
-// the sum of x over the P neighbouring lanes of a column, in all of them
-template <int P>
-__device__ __forceinline__ float ls_part_sum(float x) {
-#pragma unroll
-    for (int off = 1; off < P; off <<= 1) x += __shfl_xor(x, off, CELEG_WAVE);
-    return x;
-}
-
 // One wavefront per (request, value head, 64 / P columns).  qk: [rows, 2 * G * D] (query heads, then
 // key heads); v, out: [rows, H * V]; decay: [rows, H * D]; beta: value [t * ld_beta + h], or null
 // (no correction: u = v); state [slots, H, D, V].
@@ -257,7 +249,7 @@ __global__ __launch_bounds__(CELEG_WAVE) void channel_scan_kernel(
                 S[i] *= a[i];
                 kv = fmaf(k[i], S[i], kv);
             }
-            u = b * (vj - ls_part_sum<P>(kv));
+            u = b * (vj - lanes_sum<P>(kv));
         } else {
 #pragma unroll
             for (int i = 0; i < DPL; ++i) S[i] *= a[i];
@@ -268,7 +260,7 @@ __global__ __launch_bounds__(CELEG_WAVE) void channel_scan_kernel(
             S[i] = fmaf(k[i], u, S[i]);
             o = fmaf(q[i], S[i], o);
         }
-        o = ls_part_sum<P>(o);
+        o = lanes_sum<P>(o);
         if (live && p == 0) out[static_cast<size_t>(row0 + r) * ldv + static_cast<size_t>(h) * V + j] = o;
     }
     if (live) {

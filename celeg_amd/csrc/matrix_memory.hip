@@ -404,8 +404,7 @@ __global__ __launch_bounds__(256) void mm_chunk_out_kernel(const MmArgs a) {
                 if (d + e < D) qn = fmaf(q[g][e], n0[d + e], qn);
         }
     }
-    qn += __shfl_xor(qn, 16, CELEG_WAVE);
-    qn += __shfl_xor(qn, 32, CELEG_WAVE);
+    qn = sum_half32(sum_row16(qn));
     if (quad == 0) Qn[16 * wave + c] = qn;
     for (int i = tid; i < MM_ROWS * (Dp / 4); i += 256) {
         const int r = i / (Dp / 4), d = 4 * (i % (Dp / 4));

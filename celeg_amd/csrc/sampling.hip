@@ -314,10 +314,7 @@ __device__ __forceinline__ bool top_k_ranked(
     const int c = (top_k + SAMPLE_THREADS / CELEG_WAVE - 1) / (SAMPLE_THREADS / CELEG_WAVE);
     uint32_t left = my_max, cth = 0u;
     for (int round = 0; round < c; ++round) {
-        uint32_t m = left;
-#pragma unroll
-        for (int off = CELEG_WAVE / 2; off > 0; off >>= 1)
-            m = max(m, static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), off, CELEG_WAVE)));
+        const uint32_t m = group_max_u32<CELEG_WAVE>(left);
         cth = m;
         const unsigned long long holders = __ballot(left == m);
         if (lane == __ffsll(static_cast<long long>(holders)) - 1) left = 0u;
@@ -417,10 +414,7 @@ __device__ __forceinline__ bool top_k_from_parts(
     const int c = (top_k + SAMPLE_THREADS / CELEG_WAVE - 1) / (SAMPLE_THREADS / CELEG_WAVE);
     uint32_t left = my_max, cth = 0u;
     for (int round = 0; round < c; ++round) {
-        uint32_t m = left;
-#pragma unroll
-        for (int off = CELEG_WAVE / 2; off > 0; off >>= 1)
-            m = max(m, static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), off, CELEG_WAVE)));
+        const uint32_t m = group_max_u32<CELEG_WAVE>(left);
         cth = m;
         const unsigned long long holders = __ballot(left == m);
         if (lane == __ffsll(static_cast<long long>(holders)) - 1) left = 0u;
@@ -685,11 +679,7 @@ __global__ __launch_bounds__(ARGMAX_THREADS) void argmax_parts_kernel(
         if (sn[j]) x = x >= 0.0f ? x / penalty : x * penalty;
         if (i < vocab) mine = max(mine, packed_logit(x, i));
     }
-#pragma unroll
-    for (int off = CELEG_WAVE / 2; off > 0; off >>= 1) {
-        const unsigned long long other = __shfl_xor(mine, off, CELEG_WAVE);
-        mine = max(mine, other);
-    }
+    mine = wave_max_u64(mine);
     if (lane == 0) s_best[wave] = mine;
     __syncthreads();
     if (tid != 0) return;
@@ -744,8 +734,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void argmax_merge_kernel(
 #pragma unroll
         for (int j = 0; j < 16; ++j) mine = max(mine, v[j]);
     }
-#pragma unroll
-    for (int off = CELEG_WAVE / 2; off > 0; off >>= 1) mine = max(mine, __shfl_xor(mine, off, CELEG_WAVE));
+    mine = wave_max_u64(mine);
     if (lane == 0) s_best[wave] = mine;
     __syncthreads();
     if (tid != 0) return;
