@@ -1,12 +1,14 @@
 """Each HIP kernel alone against a plain torch / plain-implementation reference, at sizes
 other than the engine's tiny configurations (widths and vocabularies that are no power
 of two, head sizes in steps of 16, odd head counts and groups)."""
+import ctypes
 import math
 
 import pytest
 import torch
 
 import plain_lfm2 as plain
+from celeg_amd import native
 
 pytestmark = pytest.mark.gpu
 
@@ -90,6 +92,51 @@ def test_swiglu(ops, dtype, rows, ff):
     out0 = torch.empty(2, ff, dtype=dtype, device=DEV)
     ops.swiglu(zero, out0)   # gate 0 -> 0
     assert float(out0.abs().max()) == 0.0
+
+
+class NormArgument(ctypes.Structure):
+    """A norm as the kernel takes it; mode 0: none, 2: RMS, 3: layer, 4: tanh."""
+    _fields_ = [("w", ctypes.c_void_p), ("b", ctypes.c_void_p), ("eps", ctypes.c_float), ("mode", ctypes.c_int),
+                ("alpha", ctypes.c_float), ("gain", ctypes.c_float)]
+
+
+@pytest.mark.parametrize("width", [1, 6, 1020, 1022, 1024, 1028, 2046, 2048, 2052])
+@pytest.mark.parametrize("post,pre", [(3, 2), (2, 3), (None, 2), (0, None), (4, 4), (2, None)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_norm_step_on_any_width(width, post, pre, shift):
+    """h += post(y), out = pre(h): rows read as groups of four neighbours, or one by one where the width or an
+    address (shift) does not allow that; rows of few and of many registers, and rows staged in LDS."""
+    lib, rows = ctypes.CDLL(native.library_path()), 3
+    h, y = randn(rows * width + 1, seed=61), randn(rows * width + 1, seed=62, dtype=torch.bfloat16)
+    w, b = randn(4, width, seed=63), randn(4, width, seed=64)
+    out = torch.zeros(rows * width + 1, dtype=torch.bfloat16, device=DEV)
+    hv, yv, ov = (t[shift:shift + rows * width].view(rows, width) for t in (h, y, out))
+
+    def argument(mode, i, gain):
+        return NormArgument(w[i].data_ptr(), b[i].data_ptr() if i else None, 1e-5, mode or 0, 0.7, gain)
+
+    def normed(x, mode, i, gain):
+        if mode in (2, 3):
+            x = x - x.mean(dim=1, keepdim=True) if mode == 3 else x
+            x = x / torch.sqrt((x * x).mean(dim=1, keepdim=True) + 1e-5)
+        elif mode == 4:
+            x = torch.tanh(x * 0.7)
+        return (x * w[i].double().cpu() + (b[i].double().cpu() if i else 0.0)) * gain
+
+    stream = hv.double().cpu()
+    if post is not None:
+        stream = stream + normed(yv.double().cpu(), post, 0, 0.5)
+    status = lib.celeg_norm_step(
+        ctypes.c_void_p(hv.data_ptr()), ctypes.c_void_p(yv.data_ptr() if post is not None else None), 1,
+        argument(post, 0, 0.5), argument(pre, 1, 1.0), ctypes.c_void_p(ov.data_ptr() if pre is not None else None), 1,
+        None, rows, width, 1 if post is not None else 0, None)
+    torch.cuda.synchronize()
+    assert status == 0
+    # 32-bit sums of up to `width` values, two norms: a few units of 2^-24 of the largest value (a layer norm of one
+    # value divides rounding by sqrt(eps))
+    torch.testing.assert_close(hv.double().cpu(), stream, rtol=2e-6, atol=2e-5)
+    if pre is not None:
+        torch.testing.assert_close(ov.double().cpu(), normed(stream, pre, 1, 1.0), **tol(torch.bfloat16))
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 331, 96), (67, 130, 77), (200, 65, 1030), (5, 1000, 64)])
