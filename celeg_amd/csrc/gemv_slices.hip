@@ -71,7 +71,7 @@ void gemv_slices_kernel(const void* const a_, const bf16* const w_, const int* c
     constexpr bool ROWS_BY_WAVE = MP * MP > 64;
     static_assert(CT == 1 || !ROWS_BY_WAVE, "several tiles of columns go with tiles of up to 64 outputs");
     __shared__ floatx4_t red[NS][CT][KW][64];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int n0 = blockIdx.x * cols;       // the workgroup owns `cols` <= CT * MP columns
 
     if (wave < KW) {
@@ -98,23 +98,8 @@ void gemv_slices_kernel(const void* const a_, const bf16* const w_, const int* c
         for (int s = 0; s < NS; ++s)
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct) acc[s][ct] = floatx4_t{0.f, 0.f, 0.f, 0.f};
-        for (int c0 = c_begin; c0 < c_end; c0 += U) {
-            Frag2 wv[U][NS][CT][2], av[U][2];
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-#pragma unroll
-                for (int v = 0; v < 2; ++v) {
-                    const int k = (c0 + u) * 64 + v * 32 + q * 8;
-                    const bool in = c0 + u < c_end && k + 8 <= Ks;
-                    const int kw_ = k_slice + k;      // 8 values from here never leave a block of 32
-                    const size_t w_off = static_cast<size_t>(kw_ >> 5) * w_kb_stride_ + (kw_ & 31);
-                    av[u][v] = in ? *reinterpret_cast<const Frag2*>(arow + k) : Frag2{};
-#pragma unroll
-                    for (int s = 0; s < NS; ++s)
-#pragma unroll
-                        for (int ct = 0; ct < CT; ++ct)
-                            wv[u][s][ct][v] = in ? *reinterpret_cast<const Frag2*>(wrow[s][ct] + w_off) : Frag2{};
-                }
+        Frag2 wv[U][NS][CT][2], av[U][2];
+        const auto multiply = [&] {
 #pragma unroll
             for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -126,6 +111,67 @@ void gemv_slices_kernel(const void* const a_, const bf16* const w_, const int* c
                             acc[s][ct] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av[u][v].lo, wv[u][s][ct][v].lo, acc[s][ct], 0, 0, 0);
                             acc[s][ct] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av[u][v].hi, wv[u][s][ct][v].hi, acc[s][ct], 0, 0, 0);
                         }
+        };
+        if ((Ks & 63) == 0) {
+            // whole chunks: whether a wavefront has one more is the same for all its lanes, and a lane's
+            // places differ from chunk to chunk by the same number of bytes in every lane.  The places of
+            // the chunks are kept as scalar offsets: the compiler would keep (and first compute) a pointer
+            // a lane for each load of the loop, in front of the first of them.  (Against the form below, with a
+            // condition and two 64-bit products a load: 8 requests of a model of 2,048 wide 51.8 -> 49.0 ms
+            // for their 64 tokens, of 1,024 wide 77.2 -> 76.0 ms for 128; one request the same.)
+            const bf16* ap = arow + q * 8;
+            const long long w_step = w_kb_stride_;
+#pragma unroll
+            for (int s = 0; s < NS; ++s)
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) wrow[s][ct] += static_cast<size_t>(k_slice >> 5) * w_kb_stride_ + q * 8;
+            for (int c0 = c_begin; c0 < c_end; c0 += U) {
+                long long w_at = 2 * w_step * c0, a_at = 64 * c0;
+                asm("" : "+s"(w_at), "+s"(a_at));
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    if (u == 0 || c0 + u < c_end) {
+#pragma unroll
+                        for (int v = 0; v < 2; ++v) {
+                            av[u][v] = *reinterpret_cast<const Frag2*>(ap + a_at + u * 64 + v * 32);
+#pragma unroll
+                            for (int s = 0; s < NS; ++s)
+#pragma unroll
+                                for (int ct = 0; ct < CT; ++ct)
+                                    wv[u][s][ct][v] = *reinterpret_cast<const Frag2*>(wrow[s][ct] + w_at + (2 * u + v) * w_step);
+                        }
+                    } else {
+#pragma unroll
+                        for (int v = 0; v < 2; ++v) {
+                            av[u][v] = Frag2{};
+#pragma unroll
+                            for (int s = 0; s < NS; ++s)
+#pragma unroll
+                                for (int ct = 0; ct < CT; ++ct) wv[u][s][ct][v] = Frag2{};
+                        }
+                    }
+                }
+                multiply();
+            }
+        } else {
+            for (int c0 = c_begin; c0 < c_end; c0 += U) {
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+#pragma unroll
+                    for (int v = 0; v < 2; ++v) {
+                        const int k = (c0 + u) * 64 + v * 32 + q * 8;
+                        const bool in = c0 + u < c_end && k + 8 <= Ks;
+                        const int kw_ = k_slice + k;      // 8 values from here never leave a block of 32
+                        const size_t w_off = static_cast<size_t>(kw_ >> 5) * w_kb_stride_ + (kw_ & 31);
+                        av[u][v] = in ? *reinterpret_cast<const Frag2*>(arow + k) : Frag2{};
+#pragma unroll
+                        for (int s = 0; s < NS; ++s)
+#pragma unroll
+                            for (int ct = 0; ct < CT; ++ct)
+                                wv[u][s][ct][v] = in ? *reinterpret_cast<const Frag2*>(wrow[s][ct] + w_off) : Frag2{};
+                    }
+                multiply();
+            }
         }
         // acc: lane l holds column l%16 of rows 4*(l/16)..+3 of the 16x16 tile
 #pragma unroll
@@ -152,25 +198,36 @@ void gemv_slices_kernel(const void* const a_, const bf16* const w_, const int* c
     // row, every lane takes each LPR-th partial sum; all are asked for at once.  (Loads are
     // made without conditions, from clamped places, and masked afterwards: a load under a
     // condition of its own is waited for before the next one is asked for.)
+    // Four neighbouring partial sums are one load where the rows allow it (the last four of a row may
+    // reach past the valid ones, never past the row): 256 of them at 8 rows are then one trip to memory
+    // instead of three.
     constexpr int LPR = 64 / ROWS_FW;
-    constexpr int NFIRST = 16;
+    constexpr int QUADS = 8;
     float ssq = 0.f;
     if (p.stats) {
         const int nb = p.n_stat_blocks;
         const int sm = min((ROWS_BY_WAVE ? fw * ROWS_FW : 0) + lane / LPR, M - 1), sj = lane % LPR;
         const float* srow = p.stats + static_cast<size_t>(rows_ ? rows_[sm] : sm) * p.stats_ld;
-        float part[NFIRST];
+        if ((p.stats_ld & 3) == 0 && (reinterpret_cast<uintptr_t>(p.stats) & 15) == 0) {
+            const int last = (nb - 1) >> 2;
+            for (int i0 = 0; i0 * LPR <= last; i0 += QUADS) {    // the same for every lane
+                float part[QUADS][4];
 #pragma unroll
-        for (int i = 0; i < NFIRST; ++i) part[i] = srow[min(sj + LPR * i, nb - 1)];
-        for (int i0 = NFIRST; i0 * LPR < nb; i0 += 8) {   // the same for every lane; rare
-            float rest[8];
+                for (int i = 0; i < QUADS; ++i) Vec4<float>::load(srow + 4 * min(sj + LPR * (i0 + i), last), part[i]);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) rest[i] = srow[min(sj + LPR * (i0 + i), nb - 1)];
+                for (int i = 0; i < QUADS; ++i)
 #pragma unroll
-            for (int i = 0; i < 8; ++i) ssq += sj + LPR * (i0 + i) < nb ? rest[i] : 0.f;
+                    for (int e = 0; e < 4; ++e) ssq += 4 * (sj + LPR * (i0 + i)) + e < nb ? part[i][e] : 0.f;
+            }
+        } else {
+            for (int i0 = 0; i0 * LPR < nb; i0 += 8) {
+                float part[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) part[i] = srow[min(sj + LPR * (i0 + i), nb - 1)];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) ssq += sj + LPR * (i0 + i) < nb ? part[i] : 0.f;
+            }
         }
-#pragma unroll
-        for (int i = 0; i < NFIRST; ++i) ssq += sj + LPR * i < nb ? part[i] : 0.f;
     }
     if (EPI == E_RESIDUAL)
         old = static_cast<const float*>(p.out)[static_cast<size_t>(emc) * p.ldo + en];

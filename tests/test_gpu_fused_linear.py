@@ -153,6 +153,23 @@ def test_the_32bit_store_leaves_the_best_of_every_share_of_a_row(ops, M, N, K, f
     assert tokens.tolist() == want
 
 
+@pytest.mark.parametrize("M,K,blocks,ld", [(1, 1024, 256, 256), (4, 4608, 511, 512), (3, 1000, 5, 8), (8, 1024, 256, 256),
+                                           (8, 1160, 257, 260), (7, 512, 130, 131), (16, 2048, 512, 512), (12, 64, 1, 4)])
+def test_sliced_products_on_any_partial_sums(ops, M, K, blocks, ld):
+    """Partial sums read four at a time (rows on boundaries of four, the last of them partly valid) and one by one; K of
+    whole chunks a slice and not; a workgroup's share of chunks that is less than it keeps in flight."""
+    N = 136
+    x, w = randn(M, K, seed=45), randn(N, K, seed=46, scale=K ** -0.5, dtype=BF)
+    stats = torch.full((M, ld), float("nan"), device=DEV)        # beyond the valid ones: not to be used
+    stats[:, :blocks] = torch.rand(M, blocks, generator=torch.Generator().manual_seed(47)).to(DEV) * K / blocks
+    out = torch.empty(M, N, device=DEV)
+    ops.fused_linear(x.to(BF), w, out, epilogue="store_f32", eps=1e-5, stats=stats, stat_blocks=blocks)
+    scale = 1.0 / torch.sqrt(stats[:, :blocks].double().cpu().sum(dim=1, keepdim=True) / K + 1e-5)
+    # products of bfloat16 operands in 32-bit sums: exact up to K units of 2^-24 of the sum of magnitudes
+    ref = x.to(BF).double().cpu() @ w.double().cpu().T * scale
+    torch.testing.assert_close(out.double().cpu(), ref, rtol=1e-4, atol=1e-4)
+
+
 @pytest.mark.parametrize("M,ff,K", [(1, 192, 64), (8, 4608, 1024), (19, 352, 128), (64, 200, 96)])
 def test_swiglu_epilogue(ops, M, ff, K):
     h = randn(M, K, seed=11)
