@@ -137,10 +137,11 @@ __global__ void rmsnorm_kernel(TX* __restrict__ x, const TD* __restrict__ delta,
     }
 }
 
-// The same with the row kept in registers: groups of 4 values, up to RMS_NV groups a
-// thread (width <= 4 * RMS_NV * 256), every load of a row asked for before the first is used.
+// The same with the row kept in registers: groups of 4 values, NV groups a thread (width <=
+// 4 * NV * 256), every load of a row asked for before the first is used.  NV is as small as the width
+// allows: a launch of few rows spends its time on fetching the code and on the chain through it.
 #define RMS_NV 4
-template <typename TX, typename TD, typename TO>
+template <typename TX, typename TD, typename TO, int NV>
 __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(
     TX* __restrict__ x, const TD* __restrict__ delta, const float* __restrict__ w,
     TO* __restrict__ out, const int* __restrict__ rows, int width, float eps, int write_back) {
@@ -148,9 +149,9 @@ __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(
     const int r = blockIdx.x;
     const size_t src = static_cast<size_t>(rows ? rows[r] : r) * width;
     const int groups = width >> 2;
-    float v[RMS_NV][4], d[RMS_NV][4], wv[RMS_NV][4];
+    float v[NV][4], d[NV][4], wv[NV][4];
 #pragma unroll
-    for (int j = 0; j < RMS_NV; ++j) {
+    for (int j = 0; j < NV; ++j) {
         const int g = min(static_cast<int>(threadIdx.x) + j * 256, groups - 1);   // clamped, masked below
         Vec4<TX>::load(x + src + 4 * g, v[j]);
         if (delta) Vec4<TD>::load(delta + src + 4 * g, d[j]);
@@ -158,7 +159,7 @@ __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(
     }
     float sum = 0.f;
 #pragma unroll
-    for (int j = 0; j < RMS_NV; ++j) {
+    for (int j = 0; j < NV; ++j) {
         const bool in = static_cast<int>(threadIdx.x) + j * 256 < groups;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -171,7 +172,7 @@ __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(
     const float inv = 1.0f / sqrtf(sum / static_cast<float>(width) + eps);
     TO* dst = out + static_cast<size_t>(r) * width;
 #pragma unroll
-    for (int j = 0; j < RMS_NV; ++j) {
+    for (int j = 0; j < NV; ++j) {
         if (static_cast<int>(threadIdx.x) + j * 256 < groups) {
             float o[4];
 #pragma unroll
@@ -243,12 +244,18 @@ static int rmsnorm_dispatch_out(TX* x, const TD* delta, const float* w, void* ou
                                    delta, w, static_cast<bf16*>(out), rows, n_rows, width, eps, write_back);
             return CELEG_LAUNCH_RESULT();
         }
-        if (out_dtype == CELEG_F32)
-            hipLaunchKernelGGL((rmsnorm_vec_kernel<TX, TD, float>), grid, dim3(256), 0, stream, x, delta,
-                               w, static_cast<float*>(out), rows, width, eps, write_back);
-        else
-            hipLaunchKernelGGL((rmsnorm_vec_kernel<TX, TD, bf16>), grid, dim3(256), 0, stream, x, delta,
-                               w, static_cast<bf16*>(out), rows, width, eps, write_back);
+#define CELEG_RMSNORM_VEC(TO, NV)                                                                                          \
+    hipLaunchKernelGGL((rmsnorm_vec_kernel<TX, TD, TO, NV>), grid, dim3(256), 0, stream, x, delta, w,                      \
+                       static_cast<TO*>(out), rows, width, eps, write_back)
+        const bool f32 = out_dtype == CELEG_F32;
+        if (width <= 1024) {
+            if (f32) CELEG_RMSNORM_VEC(float, 1); else CELEG_RMSNORM_VEC(bf16, 1);
+        } else if (width <= 2048) {
+            if (f32) CELEG_RMSNORM_VEC(float, 2); else CELEG_RMSNORM_VEC(bf16, 2);
+        } else {
+            if (f32) CELEG_RMSNORM_VEC(float, RMS_NV); else CELEG_RMSNORM_VEC(bf16, RMS_NV);
+        }
+#undef CELEG_RMSNORM_VEC
         return CELEG_LAUNCH_RESULT();
     }
     if (out_dtype == CELEG_F32)
@@ -299,63 +306,67 @@ __device__ __forceinline__ float swiglu_of(float g, float u, float limit, float 
     return (g / (1.0f + expf(-g))) * u;
 }
 
+// Workgroup (row, part of the row): no division to find a value's row.
 template <typename T>
-__global__ void swiglu_kernel(const T* __restrict__ gu, T* __restrict__ out, int ff,
-                              size_t total, float limit, float alpha) {
-    const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= total) return;
-    const size_t t = i / ff;
-    const int c = static_cast<int>(i - t * ff);
-    const float g = to_float(gu[t * 2 * ff + c]);
-    const float u = to_float(gu[t * 2 * ff + ff + c]);
-    out[i] = from_float<T>(swiglu_of(g, u, limit, alpha));
+__global__ __launch_bounds__(256) void swiglu_kernel(const T* __restrict__ gu, T* __restrict__ out, int ff, float limit, float alpha) {
+    const size_t t = blockIdx.x;
+    for (int c = blockIdx.y * 256 + threadIdx.x; c < ff; c += gridDim.y * 256) {
+        const float g = to_float(gu[t * 2 * ff + c]);
+        const float u = to_float(gu[t * 2 * ff + ff + c]);
+        out[t * ff + c] = from_float<T>(swiglu_of(g, u, limit, alpha));
+    }
 }
 
 // groups of 8 values a thread (ff % 8 == 0)
 template <typename T>
-__global__ __launch_bounds__(256) void swiglu_vec_kernel(const T* __restrict__ gu, T* __restrict__ out,
-                                                         int ff, size_t groups, float limit, float alpha) {
-    const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= groups) return;
-    const int per_row = ff >> 3;
-    const size_t t = i / per_row;
-    const int c = static_cast<int>(i - t * per_row) * 8;
-    float g[2][4], u[2][4], o[2][4];
+__global__ __launch_bounds__(256) void swiglu_vec_kernel(const T* __restrict__ gu, T* __restrict__ out, int ff, float limit, float alpha) {
+    const size_t t = blockIdx.x;
+    for (int c = (blockIdx.y * blockDim.x + threadIdx.x) * 8; c < ff; c += gridDim.y * blockDim.x * 8) {
+        float g[2][4], u[2][4], o[2][4];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        Vec4<T>::load(gu + t * 2 * ff + c + 4 * h, g[h]);
-        Vec4<T>::load(gu + t * 2 * ff + ff + c + 4 * h, u[h]);
-    }
+        for (int h = 0; h < 2; ++h) {
+            Vec4<T>::load(gu + t * 2 * ff + c + 4 * h, g[h]);
+            Vec4<T>::load(gu + t * 2 * ff + ff + c + 4 * h, u[h]);
+        }
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+        for (int h = 0; h < 2; ++h) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[h][e] = swiglu_of(g[h][e], u[h][e], limit, alpha);
-        Vec4<T>::store(out + t * ff + c + 4 * h, o[h]);
+            for (int e = 0; e < 4; ++e) o[h][e] = swiglu_of(g[h][e], u[h][e], limit, alpha);
+            Vec4<T>::store(out + t * ff + c + 4 * h, o[h]);
+        }
     }
 }
+
+// Few values, up to a workgroup of 256 on every compute unit, go one a thread: such a launch is a chain in
+// which the code itself, 2.9 KB of it for eight values and 0.7 KB for one, is fetched anew, and eight
+// exponentials after one another take longer than one (4 rows of 2,048: 2.3 -> 2.0 us).
+#define SWIGLU_FEW_VALUES (256 * 256)
+#define SWIGLU_MAX_PARTS 65535
 
 extern "C" int celeg_swiglu(const void* gu, void* out, int dtype, int rows, int ff, float limit, float alpha,
                             hipStream_t stream) {
     const size_t total = static_cast<size_t>(rows) * ff;
     if (total == 0) return 0;
-    if (ff % 8 == 0 && (reinterpret_cast<uintptr_t>(gu) & 15) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
-        const size_t groups = total / 8;
-        dim3 vblock(256), vgrid(static_cast<unsigned>((groups + 255) / 256));
+    const auto parts = [](int units, int size) { return static_cast<unsigned>(min((units + size - 1) / size, SWIGLU_MAX_PARTS)); };
+    if (total > SWIGLU_FEW_VALUES && ff % 8 == 0 && (reinterpret_cast<uintptr_t>(gu) & 15) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
+        // (workgroups of the size that shares a row out evenly: 576 groups are three times 192)
+        const int groups = ff / 8, n = (groups + 255) / 256, size = ((groups + n - 1) / n + 63) / 64 * 64;
+        dim3 vblock(size), vgrid(rows, parts(groups, size));
         if (dtype == CELEG_F32)
             hipLaunchKernelGGL(swiglu_vec_kernel<float>, vgrid, vblock, 0, stream,
-                               static_cast<const float*>(gu), static_cast<float*>(out), ff, groups, limit, alpha);
+                               static_cast<const float*>(gu), static_cast<float*>(out), ff, limit, alpha);
         else
             hipLaunchKernelGGL(swiglu_vec_kernel<bf16>, vgrid, vblock, 0, stream,
-                               static_cast<const bf16*>(gu), static_cast<bf16*>(out), ff, groups, limit, alpha);
+                               static_cast<const bf16*>(gu), static_cast<bf16*>(out), ff, limit, alpha);
         return CELEG_LAUNCH_RESULT();
     }
-    dim3 block(256), grid(static_cast<unsigned>((total + 255) / 256));
+    dim3 block(256), grid(rows, parts(ff, 256));
     if (dtype == CELEG_F32)
         hipLaunchKernelGGL(swiglu_kernel<float>, grid, block, 0, stream,
-                           static_cast<const float*>(gu), static_cast<float*>(out), ff, total, limit, alpha);
+                           static_cast<const float*>(gu), static_cast<float*>(out), ff, limit, alpha);
     else
         hipLaunchKernelGGL(swiglu_kernel<bf16>, grid, block, 0, stream,
-                           static_cast<const bf16*>(gu), static_cast<bf16*>(out), ff, total, limit, alpha);
+                           static_cast<const bf16*>(gu), static_cast<bf16*>(out), ff, limit, alpha);
     return CELEG_LAUNCH_RESULT();
 }
 
