@@ -139,6 +139,47 @@ def test_norm_step_on_any_width(width, post, pre, shift):
         torch.testing.assert_close(ov.double().cpu(), normed(stream, pre, 1, 1.0), **tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("rows", [1, 4, 16, 17, 65])
+@pytest.mark.parametrize("N,K,tail,gated", [(64, 256, 0, True), (256, 64, 32, False), (16, 96, 8, False), (80, 320, 0, False),
+                                            (64, 512, 4, True)])
+def test_headwise_products_of_few_and_many_rows(rows, N, K, tail, gated):
+    """A matrix a head on the matrix cores: up to 16 rows with all of a run of k in flight, more of them in tiles of 64;
+    the same bits for a row either way; the values that pass by the matrix, turned by the row's position or not."""
+    lib, heads, bf, rotary = ctypes.CDLL(native.library_path()), 3, torch.bfloat16, tail // 2
+    x_head, o_head, most = K + 8 * ((tail + 7) // 8), N + 8 * ((tail + 7) // 8), 65
+    x, w = randn(most, heads * x_head, seed=71, dtype=bf), randn(heads, N, K, seed=72, scale=K ** -0.5, dtype=bf)
+    gate = randn(most, heads * N, seed=73, dtype=bf)
+    freq, positions = torch.rand(max(rotary // 2, 1), device=DEV), torch.arange(most, dtype=torch.int32, device=DEV) * 3
+
+    def run(first, count):
+        out = torch.zeros(count, heads * o_head, dtype=bf, device=DEV)
+        status = lib.celeg_headwise_linear(
+            ctypes.c_void_p(x[first].data_ptr()), heads * x_head, x_head, ctypes.c_void_p(w.data_ptr()), 1, heads, N, K,
+            ctypes.c_void_p(out.data_ptr()), heads * o_head, o_head, tail,
+            ctypes.c_void_p(gate[first].data_ptr() if gated else None), heads * N, count, 1,
+            ctypes.c_void_p(freq.data_ptr() if tail else None), rotary, 1, ctypes.c_void_p(positions[first:].data_ptr()), None)
+        torch.cuda.synchronize()
+        assert status == 0
+        return out.view(count, heads, o_head)
+
+    out = run(0, rows)
+    xs = x[:rows].double().cpu().view(rows, heads, x_head)
+    # the product is rounded to bfloat16 before the gate and after it: 2^-8 of the value each, and 32-bit sums
+    ref = torch.einsum("thk,hnk->thn", xs[:, :, :K], w.double().cpu())
+    if gated:
+        ref = ref * torch.sigmoid(gate[:rows].double().cpu().view(rows, heads, N))
+    torch.testing.assert_close(out[:, :, :N].double().cpu(), ref, rtol=2 ** -7, atol=1e-4)
+    if tail:
+        passed = xs[:, :, K:K + tail].clone()
+        angle = (positions[:rows].double().cpu()[:, None, None] * freq[:rotary // 2].double().cpu())
+        u, v = passed[:, :, 0:rotary:2].clone(), passed[:, :, 1:rotary:2].clone()
+        passed[:, :, 0:rotary:2] = u * torch.cos(angle) - v * torch.sin(angle)
+        passed[:, :, 1:rotary:2] = u * torch.sin(angle) + v * torch.cos(angle)
+        torch.testing.assert_close(out[:, :, N:N + tail].double().cpu(), passed, rtol=2 ** -8, atol=2e-2)
+    assert torch.equal(run(0, most)[:rows], out)
+    assert torch.equal(run(rows - 1, 1)[0], out[rows - 1])
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 331, 96), (67, 130, 77), (200, 65, 1030), (5, 1000, 64)])
 def test_gemm_f32_is_true_32bit_and_row_independent(ops, M, N, K):
     x, w, b = randn(M, K, seed=7), randn(N, K, seed=8), randn(N, seed=9)
