@@ -94,6 +94,25 @@ def test_swiglu(ops, dtype, rows, ff):
     assert float(out0.abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,width", [(16, 4096), (17, 4104), (1, 70008), (3, 30001), (65, 1016)])
+def test_gated_and_plain_activations_of_few_and_many_values(ops, dtype, rows, width):
+    """One value a thread up to 65,536 values and where a row is no whole number of groups of eight; groups of eight,
+    shared out over workgroups of a part of a row, beyond."""
+    gu = randn(rows, 2 * width, seed=81, scale=2.0, dtype=dtype)
+    out = torch.empty(rows, width, dtype=dtype, device=DEV)
+    ops.swiglu(gu, out)
+    g, u = gu[:, :width].double().cpu(), gu[:, width:].double().cpu()
+    torch.testing.assert_close(out.double().cpu(), plain.silu(g) * u, **tol(dtype))
+    x, act = gu[:, :width].contiguous(), torch.empty(rows, width, dtype=dtype, device=DEV)
+    status = ctypes.CDLL(native.library_path()).celeg_activation_bias(
+        ctypes.c_void_p(x.data_ptr()), width, None, ctypes.c_void_p(act.data_ptr()), width, 0 if dtype == torch.float32 else 1,
+        rows, width, 0, ctypes.c_float(0.0), ctypes.c_float(0.0), None)
+    torch.cuda.synchronize()
+    assert status == 0
+    torch.testing.assert_close(act.double().cpu(), torch.nn.functional.gelu(g, approximate="tanh"), **tol(dtype))
+
+
 class NormArgument(ctypes.Structure):
     """A norm as the kernel takes it; mode 0: none, 2: RMS, 3: layer, 4: tanh."""
     _fields_ = [("w", ctypes.c_void_p), ("b", ctypes.c_void_p), ("eps", ctypes.c_float), ("mode", ctypes.c_int),
