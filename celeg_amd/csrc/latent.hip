@@ -54,7 +54,7 @@ __device__ __forceinline__ void latent_store_row(const T* dkv, int half, int rot
 }
 
 // ---------------------------------------------------------------- prepare
-// One workgroup per row.  proj[t] holds (q | dkv | ...): q is [heads, dim + rot] at column q_off,
+// proj[t] holds (q | dkv | ...): q is [heads, dim + rot] at column q_off,
 // dkv is [rank + rot] at column dkv_off.  The first `rank` values of dkv are RMS-normed with
 // `weight` and, with the rotated last `rot` values, written to the row's place in the pages; the
 // rotated part of every query head is turned in place (q_off < 0: no queries here).  The first `rotary`
