@@ -433,8 +433,10 @@ __global__ __launch_bounds__(ATT_WAVES * CELEG_WAVE) void paged_attention_kernel
             s = dot * scale;
         }
         const float m_new = fmaxf(m, wave_max(s));
-        const float p = valid ? expf(s - m_new) : 0.f;
-        const float corr = expf(m - m_new);  // m = -inf at the first chunk gives 0
+        // (keys that all score minus infinity weigh nothing, also where the wavefront has met no others yet)
+        const float at = m_new == -INFINITY ? 0.f : m_new;
+        const float p = valid ? expf(s - at) : 0.f;
+        const float corr = expf(m - at);  // m = -inf at the first chunk gives 0
         l = l * corr + wave_sum(p);
         // the wavefront's own part of LDS: its lanes only have to see each other's writes
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

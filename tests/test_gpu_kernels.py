@@ -734,6 +734,36 @@ def test_general_attention_wide_and_narrow_loads(ops, dtype, head_dim, window):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("keys,dead", [(65, (64, 65)), (200, (64, 128)), (400, (64, 320)), (130, (0, 64)), (130, (0, 129))])
+def test_general_attention_where_a_wavefront_sees_only_minus_infinity(ops, dtype, keys, dead):
+    """Keys whose scores overflow to minus infinity weigh nothing, also where a wavefront meets no others (its
+    maximum is then minus infinity too)."""
+    from celeg_amd.engine import StepEntry
+    heads, kv_heads, hd = 4, 2, 64
+    cache = make_cache(kv_heads, hd, 1, dtype, n_pages=32, max_context=512)
+    kv, slot = cache.layer_cache(0).kv, cache.open()
+    assert cache.prepare(slot, 0, keys)
+    q, k, v = (randn(keys, n * hd, seed=90 + i, dtype=dtype) for i, n in enumerate((heads, kv_heads, kv_heads)))
+    q.view(keys, heads, hd)[:, :, 0] = 1e20
+    k.view(keys, kv_heads, hd)[:, :, 0] = 0
+    k.view(keys, kv_heads, hd)[dead[0]:dead[1], :, 0] = -1e20
+    batch, keep = build_batch(ops, cache, [StepEntry(slot, 0, [0] * keys)])
+    ops.qk_norm_rope_store(q, k, v, None, None, 0.0, None, 0, heads, kv_heads, hd, batch, kv)
+    last, out = q[-1:].contiguous(), torch.empty(1, heads * hd, dtype=dtype, device=DEV)
+    batch, keep = build_batch(ops, cache, [StepEntry(slot, keys - 1, [0])])
+    ops.attention_impl = "general"
+    try:
+        ops.paged_attention(last, out, heads, kv_heads, hd, 0.125, None, batch, kv)
+    finally:
+        ops.attention_impl = "auto"
+    live = [i for i in range(keys) if not dead[0] <= i < dead[1]]
+    qf, kf, vf = (t.double().cpu().view(-1, n, hd) for t, n in ((last, heads), (k, kv_heads), (v, kv_heads)))
+    kf, vf = (t[live].repeat_interleave(heads // kv_heads, 1) for t in (kf, vf))
+    weights = torch.softmax(torch.einsum("hd,khd->hk", qf[0], kf) * 0.125, -1)
+    torch.testing.assert_close(out[0].double().cpu(), torch.einsum("hk,khd->hd", weights, vf).reshape(-1), **tol(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_attention_far_key_stands_out(ops, dtype):
     # query 299 is built to look at key 3, hundreds of keys back and in the first page
     attention_case(ops, dtype, 4, 2, 64, lengths=[300], cuts=[64, 1, 1, 50], boost=(3, 299),
