@@ -348,10 +348,10 @@ extern "C" int celeg_qk_norm_rope_store(
 }
 
 // ---------------------------------------------------------------- general attention
-// A workgroup of four wavefronts per (row, query head).  Keys at positions [first, pos] of the row's
+// A workgroup of up to four wavefronts per (row, query head).  Keys at positions [first, pos] of the row's
 // request, first = max(0, pos - window + 1) with a window, else 0; 64 keys at a time, the
 // wavefronts in turn: every lane scores one key, the chunk joins its wavefront's running (max, sum,
-// accumulator) in 32-bit, and the four are joined at the end, in order.  The chunking depends only
+// accumulator) in 32-bit, and they are joined at the end, in order.  The chunking depends only
 // on the row's own position, so a row's result is the same whatever else is in the batch.
 // scores = (q.k)*scale, scale applied once
 // (reference: src/backend/cpu/attention/paged_attention.cpp:229-283;
@@ -362,7 +362,12 @@ extern "C" int celeg_qk_norm_rope_store(
 // heads of 64: 15.3 us; their prompts (424 rows) 66.7 us; before, with one wavefront and a value a load, 91.7 and
 // 164 us.
 #define ATT_MAX_DIM_CHUNKS 4  // head_dim <= 256
-#define ATT_WAVES 4
+// Wavefronts a row: four, and with a window no more than it has chunks of 64 keys, so that each has a chunk and the
+// sums are those of four.  Idle wavefronts cost a prompt what live ones do: 1,024 rows, 16 heads of 64, bfloat16, a
+// window of 16 41 us with one wavefront and 94 with four, of 64 131 and 262, of 128 239 (two) and 278 (four).  Fewer
+// wavefronts than chunks would be faster for prompts (96: 187 us with one, 270 with four) but slower for single
+// tokens (25 against 17 us), and a row's sums must not depend on what else is in the step.
+#define ATT_MAX_WAVES 4
 
 template <typename T> struct Wide;      // 16 bytes as 32-bit numbers
 template <> struct Wide<float> {
@@ -380,8 +385,8 @@ template <> struct Wide<bf16> {
 };
 
 // DC: head_dim in pieces of 64, rounded up
-template <typename T, int DC, bool VEC>
-__global__ __launch_bounds__(ATT_WAVES * CELEG_WAVE) void paged_attention_kernel(
+template <typename T, int DC, int WAVES, bool VEC>
+__global__ __launch_bounds__(WAVES * CELEG_WAVE) void paged_attention_kernel(
     const T* __restrict__ q, int ldq, const T* __restrict__ k_pool, const T* __restrict__ v_pool,
     const int* __restrict__ table, int table_stride, const int* __restrict__ token_slot,
     const int* __restrict__ positions, T* __restrict__ out, int ldo, int q_heads, int kv_heads,
@@ -389,9 +394,9 @@ __global__ __launch_bounds__(ATT_WAVES * CELEG_WAVE) void paged_attention_kernel
     constexpr int W = Wide<T>::N;
     constexpr int AHEAD = 16 / W;                   // loads of values in flight: 16 keys
     __shared__ float qs[DC * CELEG_WAVE];
-    __shared__ float ps_all[ATT_WAVES][CELEG_WAVE];
-    __shared__ float joined[ATT_WAVES][DC * CELEG_WAVE];
-    __shared__ float stats[ATT_WAVES][2];
+    __shared__ float ps_all[WAVES][CELEG_WAVE];
+    __shared__ float joined[WAVES][DC * CELEG_WAVE];
+    __shared__ float stats[WAVES][2];
     const int t = blockIdx.x;
     const int h = blockIdx.y;
     const int wave = threadIdx.x / CELEG_WAVE, lane = threadIdx.x % CELEG_WAVE;
@@ -402,7 +407,7 @@ __global__ __launch_bounds__(ATT_WAVES * CELEG_WAVE) void paged_attention_kernel
     const int first = window > 0 ? max(0, pos - window + 1) : 0;
 
     const T* qrow = q + static_cast<size_t>(t) * ldq + static_cast<size_t>(h) * head_dim;
-    for (int d = threadIdx.x; d < head_dim; d += ATT_WAVES * CELEG_WAVE) qs[d] = to_float(qrow[d]);
+    for (int d = threadIdx.x; d < head_dim; d += WAVES * CELEG_WAVE) qs[d] = to_float(qrow[d]);
     __syncthreads();
 
     float m = -INFINITY, l = 0.f;
@@ -411,7 +416,7 @@ __global__ __launch_bounds__(ATT_WAVES * CELEG_WAVE) void paged_attention_kernel
     for (int j = 0; j < DC; ++j) acc[j] = 0.f;
     const bool wide_values = VEC && first % W == 0;        // (chunks start at first + 64 n)
 
-    for (int base = first + wave * CELEG_WAVE; base <= pos; base += ATT_WAVES * CELEG_WAVE) {
+    for (int base = first + wave * CELEG_WAVE; base <= pos; base += WAVES * CELEG_WAVE) {
         const int key = base + lane;
         const bool valid = key <= pos;
         const int page = pages[min(key, pos) / page_tokens];
@@ -487,6 +492,17 @@ __global__ __launch_bounds__(ATT_WAVES * CELEG_WAVE) void paged_attention_kernel
         }
         m = m_new;
     }
+    T* orow = out + static_cast<size_t>(t) * ldo + static_cast<size_t>(h) * head_dim;
+    if (WAVES == 1 || pos - first < CELEG_WAVE) {          // nothing to join: the same numbers as below
+        if (wave > 0) return;
+        const float inv = 1.0f / l;
+#pragma unroll
+        for (int j = 0; j < DC; ++j) {
+            const int d = lane + j * CELEG_WAVE;
+            if (d < head_dim) orow[d] = from_float<T>(acc[j] * inv);
+        }
+        return;
+    }
 #pragma unroll
     for (int j = 0; j < DC; ++j) joined[wave][lane + j * CELEG_WAVE] = acc[j];
     if (lane == 0) {
@@ -496,24 +512,23 @@ __global__ __launch_bounds__(ATT_WAVES * CELEG_WAVE) void paged_attention_kernel
     __syncthreads();
     float top = stats[0][0];                               // (wavefront 0 has always seen a key)
 #pragma unroll
-    for (int w = 1; w < ATT_WAVES; ++w) top = fmaxf(top, stats[w][0]);
-    float factor[ATT_WAVES], sum = 0.f;
+    for (int w = 1; w < WAVES; ++w) top = fmaxf(top, stats[w][0]);
+    float factor[WAVES], sum = 0.f;
 #pragma unroll
-    for (int w = 0; w < ATT_WAVES; ++w) {
+    for (int w = 0; w < WAVES; ++w) {
         factor[w] = expf(stats[w][0] - top);               // a wavefront without keys: 0
         sum = fmaf(factor[w], stats[w][1], sum);
     }
-    T* orow = out + static_cast<size_t>(t) * ldo + static_cast<size_t>(h) * head_dim;
     const float inv_l = 1.0f / sum;
-    for (int d = threadIdx.x; d < head_dim; d += ATT_WAVES * CELEG_WAVE) {
+    for (int d = threadIdx.x; d < head_dim; d += WAVES * CELEG_WAVE) {
         float x = 0.f;
 #pragma unroll
-        for (int w = 0; w < ATT_WAVES; ++w) x = fmaf(factor[w], joined[w][d], x);
+        for (int w = 0; w < WAVES; ++w) x = fmaf(factor[w], joined[w][d], x);
         orow[d] = from_float<T>(x * inv_l);
     }
 }
 
-template <typename T, int DC>
+template <typename T, int DC, int WAVES>
 static int launch_paged_attention(const void* q, int ldq, const void* k_pool, const void* v_pool, const int* table,
                                   int table_stride, const int* token_slot, const int* positions, void* out, int ldo,
                                   int n_tokens, int q_heads, int kv_heads, int head_dim, int page_tokens, int n_layers,
@@ -521,14 +536,26 @@ static int launch_paged_attention(const void* q, int ldq, const void* k_pool, co
     const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     const bool vec = head_dim % Wide<T>::N == 0 && page_tokens % Wide<T>::N == 0 && aligned(k_pool) && aligned(v_pool);
     auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(n_tokens, q_heads), dim3(ATT_WAVES * CELEG_WAVE), 0, stream,
+        hipLaunchKernelGGL(kernel, dim3(n_tokens, q_heads), dim3(WAVES * CELEG_WAVE), 0, stream,
                            static_cast<const T*>(q), ldq, static_cast<const T*>(k_pool), static_cast<const T*>(v_pool),
                            table, table_stride, token_slot, positions, static_cast<T*>(out), ldo, q_heads, kv_heads,
                            head_dim, page_tokens, n_layers, layer, scale, window);
     };
-    if (vec) launch(paged_attention_kernel<T, DC, true>);
-    else launch(paged_attention_kernel<T, DC, false>);
+    if (vec) launch(paged_attention_kernel<T, DC, WAVES, true>);
+    else launch(paged_attention_kernel<T, DC, WAVES, false>);
     return CELEG_LAUNCH_RESULT();
+}
+
+template <typename T, int WAVES>
+static int launch_paged_attention_of(const void* q, int ldq, const void* k_pool, const void* v_pool, const int* table,
+                                    int table_stride, const int* token_slot, const int* positions, void* out, int ldo,
+                                    int n_tokens, int q_heads, int kv_heads, int head_dim, int page_tokens, int n_layers,
+                                    int layer, float scale, int window, hipStream_t stream) {
+    const auto launch = head_dim <= 64 ? launch_paged_attention<T, 1, WAVES>
+                        : head_dim <= 128 ? launch_paged_attention<T, 2, WAVES>
+                                          : launch_paged_attention<T, ATT_MAX_DIM_CHUNKS, WAVES>;
+    return launch(q, ldq, k_pool, v_pool, table, table_stride, token_slot, positions, out, ldo, n_tokens, q_heads, kv_heads,
+                  head_dim, page_tokens, n_layers, layer, scale, window, stream);
 }
 
 template <typename T>
@@ -536,8 +563,9 @@ static int dispatch_paged_attention(const void* q, int ldq, const void* k_pool, 
                                     int table_stride, const int* token_slot, const int* positions, void* out, int ldo,
                                     int n_tokens, int q_heads, int kv_heads, int head_dim, int page_tokens, int n_layers,
                                     int layer, float scale, int window, hipStream_t stream) {
-    const auto launch = head_dim <= 64 ? launch_paged_attention<T, 1>
-                        : head_dim <= 128 ? launch_paged_attention<T, 2> : launch_paged_attention<T, ATT_MAX_DIM_CHUNKS>;
+    const auto launch = window > 0 && window <= CELEG_WAVE       ? launch_paged_attention_of<T, 1>
+                        : window > 0 && window <= 2 * CELEG_WAVE ? launch_paged_attention_of<T, 2>
+                                                                 : launch_paged_attention_of<T, ATT_MAX_WAVES>;
     return launch(q, ldq, k_pool, v_pool, table, table_stride, token_slot, positions, out, ldo, n_tokens, q_heads, kv_heads,
                   head_dim, page_tokens, n_layers, layer, scale, window, stream);
 }

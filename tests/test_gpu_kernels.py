@@ -734,6 +734,18 @@ def test_general_attention_wide_and_narrow_loads(ops, dtype, head_dim, window):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("head_dim", [40, 128, 256])
+@pytest.mark.parametrize("window", [1, 63, 64, 65, 128, 129])
+def test_general_attention_window_by_wavefronts(ops, dtype, head_dim, window):
+    """Windows at the edges of chunks of 64 keys and of the rule that gives a row one, two or four wavefronts."""
+    ops.attention_impl = "general"
+    try:
+        attention_case(ops, dtype, 4, 2, head_dim, lengths=[260, 66], cuts=[61, 1, 1, 1, 1, 70], window=window)
+    finally:
+        ops.attention_impl = "auto"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("keys,dead", [(65, (64, 65)), (200, (64, 128)), (400, (64, 320)), (130, (0, 64)), (130, (0, 129))])
 def test_general_attention_where_a_wavefront_sees_only_minus_infinity(ops, dtype, keys, dead):
     """Keys whose scores overflow to minus infinity weigh nothing, also where a wavefront meets no others (its
