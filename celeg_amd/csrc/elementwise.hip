@@ -306,33 +306,38 @@ __device__ __forceinline__ float swiglu_of(float g, float u, float limit, float 
     return (g / (1.0f + expf(-g))) * u;
 }
 
-// Workgroup (row, part of the row): no division to find a value's row.
+// Workgroup (rows, part of a row), a thread's row and column by its place in the workgroup: no division to find
+// a value's row.
 template <typename T>
-__global__ __launch_bounds__(256) void swiglu_kernel(const T* __restrict__ gu, T* __restrict__ out, int ff, float limit, float alpha) {
-    const size_t t = blockIdx.x;
-    for (int c = blockIdx.y * 256 + threadIdx.x; c < ff; c += gridDim.y * 256) {
-        const float g = to_float(gu[t * 2 * ff + c]);
-        const float u = to_float(gu[t * 2 * ff + ff + c]);
-        out[t * ff + c] = from_float<T>(swiglu_of(g, u, limit, alpha));
+__global__ __launch_bounds__(256) void swiglu_kernel(const T* __restrict__ gu, T* __restrict__ out, int rows, int ff, float limit,
+                                                     float alpha) {
+    for (size_t t = blockIdx.x * blockDim.y + threadIdx.y; t < rows; t += gridDim.x * blockDim.y) {
+        for (int c = blockIdx.y * blockDim.x + threadIdx.x; c < ff; c += gridDim.y * blockDim.x) {
+            const float g = to_float(gu[t * 2 * ff + c]);
+            const float u = to_float(gu[t * 2 * ff + ff + c]);
+            out[t * ff + c] = from_float<T>(swiglu_of(g, u, limit, alpha));
+        }
     }
 }
 
 // groups of 8 values a thread (ff % 8 == 0)
 template <typename T>
-__global__ __launch_bounds__(256) void swiglu_vec_kernel(const T* __restrict__ gu, T* __restrict__ out, int ff, float limit, float alpha) {
-    const size_t t = blockIdx.x;
-    for (int c = (blockIdx.y * blockDim.x + threadIdx.x) * 8; c < ff; c += gridDim.y * blockDim.x * 8) {
-        float g[2][4], u[2][4], o[2][4];
+__global__ __launch_bounds__(256) void swiglu_vec_kernel(const T* __restrict__ gu, T* __restrict__ out, int rows, int ff, float limit,
+                                                         float alpha) {
+    for (size_t t = blockIdx.x * blockDim.y + threadIdx.y; t < rows; t += gridDim.x * blockDim.y) {
+        for (int c = (blockIdx.y * blockDim.x + threadIdx.x) * 8; c < ff; c += gridDim.y * blockDim.x * 8) {
+            float g[2][4], u[2][4], o[2][4];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            Vec4<T>::load(gu + t * 2 * ff + c + 4 * h, g[h]);
-            Vec4<T>::load(gu + t * 2 * ff + ff + c + 4 * h, u[h]);
-        }
+            for (int h = 0; h < 2; ++h) {
+                Vec4<T>::load(gu + t * 2 * ff + c + 4 * h, g[h]);
+                Vec4<T>::load(gu + t * 2 * ff + ff + c + 4 * h, u[h]);
+            }
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+            for (int h = 0; h < 2; ++h) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[h][e] = swiglu_of(g[h][e], u[h][e], limit, alpha);
-            Vec4<T>::store(out + t * ff + c + 4 * h, o[h]);
+                for (int e = 0; e < 4; ++e) o[h][e] = swiglu_of(g[h][e], u[h][e], limit, alpha);
+                Vec4<T>::store(out + t * ff + c + 4 * h, o[h]);
+            }
         }
     }
 }
@@ -341,32 +346,38 @@ __global__ __launch_bounds__(256) void swiglu_vec_kernel(const T* __restrict__ g
 // which the code itself, 2.9 KB of it for eight values and 0.7 KB for one, is fetched anew, and eight
 // exponentials after one another take longer than one (4 rows of 2,048: 2.3 -> 2.0 us).
 #define SWIGLU_FEW_VALUES (256 * 256)
-#define SWIGLU_MAX_PARTS 65535
+#define SWIGLU_MAX_PARTS 65535u
+#define SWIGLU_MAX_GRID (1u << 23)      // (a launch holds fewer than 2^32 threads a dimension)
 
 extern "C" int celeg_swiglu(const void* gu, void* out, int dtype, int rows, int ff, float limit, float alpha,
                             hipStream_t stream) {
     const size_t total = static_cast<size_t>(rows) * ff;
     if (total == 0) return 0;
-    const auto parts = [](int units, int size) { return static_cast<unsigned>(min((units + size - 1) / size, SWIGLU_MAX_PARTS)); };
+    // Workgroups of the size that shares a row out evenly (576 groups are three times 192), or of several rows
+    // where a row is half a workgroup or less (131,072 rows of 8 3.0 us, with a workgroup a row 48; 16,384 of 64 2.9 and 8.7).
+    const auto shape = [rows](int units, dim3& grid, dim3& block) {
+        const int n = (units + 255) / 256, share = (units + n - 1) / n;
+        block = share <= 128 ? dim3(share, 256 / share) : dim3((share + 63) / 64 * 64);
+        grid = dim3(min((rows + block.y - 1) / block.y, SWIGLU_MAX_GRID), min((units + block.x - 1) / block.x, SWIGLU_MAX_PARTS));
+    };
+    dim3 grid, block;
     if (total > SWIGLU_FEW_VALUES && ff % 8 == 0 && (reinterpret_cast<uintptr_t>(gu) & 15) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
-        // (workgroups of the size that shares a row out evenly: 576 groups are three times 192)
-        const int groups = ff / 8, n = (groups + 255) / 256, size = ((groups + n - 1) / n + 63) / 64 * 64;
-        dim3 vblock(size), vgrid(rows, parts(groups, size));
+        shape(ff / 8, grid, block);
         if (dtype == CELEG_F32)
-            hipLaunchKernelGGL(swiglu_vec_kernel<float>, vgrid, vblock, 0, stream,
-                               static_cast<const float*>(gu), static_cast<float*>(out), ff, limit, alpha);
+            hipLaunchKernelGGL(swiglu_vec_kernel<float>, grid, block, 0, stream,
+                               static_cast<const float*>(gu), static_cast<float*>(out), rows, ff, limit, alpha);
         else
-            hipLaunchKernelGGL(swiglu_vec_kernel<bf16>, vgrid, vblock, 0, stream,
-                               static_cast<const bf16*>(gu), static_cast<bf16*>(out), ff, limit, alpha);
+            hipLaunchKernelGGL(swiglu_vec_kernel<bf16>, grid, block, 0, stream,
+                               static_cast<const bf16*>(gu), static_cast<bf16*>(out), rows, ff, limit, alpha);
         return CELEG_LAUNCH_RESULT();
     }
-    dim3 block(256), grid(rows, parts(ff, 256));
+    shape(ff, grid, block);
     if (dtype == CELEG_F32)
         hipLaunchKernelGGL(swiglu_kernel<float>, grid, block, 0, stream,
-                           static_cast<const float*>(gu), static_cast<float*>(out), ff, limit, alpha);
+                           static_cast<const float*>(gu), static_cast<float*>(out), rows, ff, limit, alpha);
     else
         hipLaunchKernelGGL(swiglu_kernel<bf16>, grid, block, 0, stream,
-                           static_cast<const bf16*>(gu), static_cast<bf16*>(out), ff, limit, alpha);
+                           static_cast<const bf16*>(gu), static_cast<bf16*>(out), rows, ff, limit, alpha);
     return CELEG_LAUNCH_RESULT();
 }
 

@@ -113,6 +113,20 @@ def test_gated_and_plain_activations_of_few_and_many_values(ops, dtype, rows, wi
     torch.testing.assert_close(act.double().cpu(), torch.nn.functional.gelu(g, approximate="tanh"), **tol(dtype))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,width", [(1, 1), (300, 7), (70001, 1), (9001, 8), (3000, 30), (2050, 64), (513, 128), (600, 129),
+                                        (700, 1024), (129, 1032), (77, 2056)])
+def test_swiglu_of_narrow_rows(ops, dtype, rows, width):
+    """Rows of half a workgroup or less share one: rows that do not fill the last workgroup, shares that are no whole
+    number of wavefronts, one value and eight values a thread."""
+    gu = randn(rows, 2 * width, seed=83, scale=2.0, dtype=dtype)
+    out = torch.zeros(rows + 1, width, dtype=dtype, device=DEV)
+    ops.swiglu(gu, out[:rows])
+    g, u = gu[:, :width].double().cpu(), gu[:, width:].double().cpu()
+    torch.testing.assert_close(out[:rows].double().cpu(), plain.silu(g) * u, **tol(dtype))
+    assert float(out[rows].abs().max()) == 0
+
+
 class NormArgument(ctypes.Structure):
     """A norm as the kernel takes it; mode 0: none, 2: RMS, 3: layer, 4: tanh."""
     _fields_ = [("w", ctypes.c_void_p), ("b", ctypes.c_void_p), ("eps", ctypes.c_float), ("mode", ctypes.c_int),
