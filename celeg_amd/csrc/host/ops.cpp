@@ -601,14 +601,42 @@ void Ops::library_product(const Tensor& x, const Tensor& w, const Tensor& out, W
 }
 
 // The bfloat16 products of few rows: the kernels for up to 16 and for 9 to 64 rows; false where the operands
-// are not what those read (16 bytes a load).  The library spreads a product of 4 rows over 64 workgroups.
-// 4 rows, 1,024 x 1,024 2.6 us against the library's 5.7, 1,024 x 2,048 3.4 against 9.1, 4,096 x 1,024 4.3 against
-// 7.5; 64 rows 4.0, 5.9 and 8.4 against 8.3, 8.8 and 11.6 (different weights in a chain).
-// Products of very many columns (output heads) stay with the library, which reads them at the rate of a copy.
+// are not what those read (16 bytes a load) or the library is the faster one.
+//
+// The library spreads a small product over few workgroups (4 rows, 1,024 x 1,024: 64 of them), these kernels over all
+// compute units.  But each of their workgroups has 4 to 16 columns and reads all rows of x beside them: with the rows
+// the traffic from L2 grows to four times the weights' own at 64, and with a long inner size the one chain of a
+// workgroup, which the library cuts.  So what they take ends at a size of the weights that falls with the rows.
+// Measured over 60 sizes with the weights in memory; these kernels' time over the library's at the largest sizes
+// that each line takes, and behind it:
+//   up to 4 rows   4,096 x 16,384 0.9, 2,048 x 16,384 1.0 (8,192 x 4,096 1.1 to 1.4)
+//   up to 8        4,096 x 12,288 0.8 to 0.9, 2,048 x 12,288 0.9 to 1.0; long: 16,384 x 2,048 0.7 to 0.9 (2,048 x 16,384
+//                  1.1; 8,192 x 4,096 1.1 to 1.4)
+//   up to 16       4,096 x 4,096 0.7 to 0.8, 1,024 x 14,336 0.9 to 1.0 (2,048 x 12,288 1.1; 1,024 x 16,384 1.1; 6,144 x 1,024 1.2)
+//   up to 24       1,024 x 9,216 0.8, 3,072 x 3,072 1.0 (1,536 x 8,192 1.1; 6,144 x 1,024 1.2)
+//   up to 32       1,024 x 12,288 0.9 to 1.0, 2,048 x 4,096 0.8 (1,024 x 16,384 1.2; 1,536 x 8,192 1.2; 3,072 x 2,048 1.1)
+//   up to 64       4,608 x 1,024 0.8, 1,024 x 4,096 0.8 to 0.9 (1,536 x 3,072 1.1; 1,024 x 6,144 1.0 to 1.2;
+//                  4,096 x 1,536 1.1 to 2.2; 4,096 x 16,384 2.6)
+// and, beyond 16 rows, at columns that are not too many for a short inner size (64 x 4,096: 1.1 at 24 rows, 1.6 at 64).
+// (inner size x columns)
+bool Ops::few_rows_faster(long long M, long long N, long long K) {
+    constexpr long long MI = 1 << 20, ANY = 1LL << 40;
+    struct Taken { long long rows, inner, columns, weights; };
+    static constexpr Taken taken[] = {
+        {4, 4608, 16384, 64 * MI}, {8, 4608, 12288, 48 * MI}, {8, ANY, 2048, 32 * MI}, {8, ANY, 16384, 16 * MI},
+        {16, 4608, 14336, 17 * MI}, {24, 4608, 16384, 9 * MI}, {32, 2048, 16384, 9 * MI}, {32, 1024, 14336, 14 * MI},
+        {64, 4608, 4096, 4 * MI}, {64, 4608, 1024, 9 * MI / 2}};
+    if (M > 16 && N > (M > 32 ? 16 : 32) * K) return false;
+    for (const Taken& t : taken)
+        if (M <= t.rows && K <= t.inner && N <= t.columns && N * K <= t.weights) return true;
+    return false;
+}
+
 bool Ops::few_rows_product(const Tensor& x, const Tensor& w, const Tensor& out) {
     const long long M = x.shape[0], K = x.shape[1], N = w.shape[0];
     const auto aligned = [](const Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data) & 15) == 0; };
-    if (M > 64 || N > FEW_ROWS_MAX_COLUMNS || K % 8 || !((M <= 16 && use_sliced) || rows_kernel_ok(static_cast<int>(M), {K}))) return false;
+    if (M > 64 || K <= 0 || K % 8 || !few_rows_faster(M, N, K)) return false;
+    if (!((M <= 16 && use_sliced) || rows_kernel_ok(static_cast<int>(M), {K}))) return false;
     if (rows_of(x, "x") % 8 || rows_of(x, "x") > 0xfffff || !aligned(x) || !aligned(w)) return false;
     FusedArgs args;
     args.epilogue = Epilogue::Store;

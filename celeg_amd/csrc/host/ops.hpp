@@ -421,7 +421,7 @@ private:
     const float* rope_table(const Tensor& inv_freq, int n_positions);
     void attention_decode(const Tensor& q, const Tensor& out, int heads, int kv_heads, int head_dim, float scale,
                           int window, const StepBatch& batch, const KVView& kv, int T, Workspace& ws, const FreshKV* fresh = nullptr);
-    static constexpr long long FEW_ROWS_MAX_COLUMNS = 16384;
+    static bool few_rows_faster(long long M, long long N, long long K);
     bool few_rows_product(const Tensor& x, const Tensor& w, const Tensor& out);
     void library_product(const Tensor& x, const Tensor& w, const Tensor& out, Workspace& ws);
 };

@@ -290,6 +290,25 @@ def test_linear_few_rows(ops, M, N, K):
             assert bool(((out.double() - ref - (0 if bias is None else bias.double())).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("K,N,most", [
+    (1024, 1024, 64), (4608, 1024, 64), (4608, 1280, 24), (1024, 4096, 64), (1024, 4097, 32), (2048, 4096, 32), (1536, 8192, 16),
+    (4096, 4096, 16), (4616, 1024, 8), (1024, 14336, 32), (1024, 16384, 8), (2048, 16384, 1), (3072, 8192, 8), (8192, 2048, 8), (8192, 4096, 0),
+    (64, 1024, 64), (64, 2048, 32), (64, 2049, 16), (1000, 2000, 16)])
+def test_linear_few_rows_and_the_library(ops, K, N, most):
+    """Products of up to `most` rows go to the kernels for few rows, of more (and of larger weights) to the library, which
+    is then faster; both within the rounding of the result."""
+    w = randn(N, K, seed=24, scale=K ** -0.5, dtype=torch.bfloat16)
+    for M in (1, 8, 9, 16, 17, 24, 25, 32, 33, 64):
+        x, out = randn(M, K, seed=23, dtype=torch.bfloat16), torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+        before = ops.paths()
+        ops.linear(x, w, out)
+        after = ops.paths()
+        assert after["linear_few_rows"] - before["linear_few_rows"] == int(M <= most), M
+        ref = x.double() @ w.double().T
+        bound = 2.0 ** -8 * ref.abs() + 2.0 ** -24 * (K + 8) * (x.double().abs() @ w.double().abs().T)
+        assert bool(((out.double() - ref).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 331, 96), (77, 130, 96), (300, 1000, 352), (129, 48, 40),
                                    (512, 2048, 1024), (2041, 272, 4608)])
 def test_library_product_called_directly(ops, M, N, K):
