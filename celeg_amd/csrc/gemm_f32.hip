@@ -254,6 +254,105 @@ static int launch_f32(const float* X, int ldx, const float* W, int ldw, const fl
     return CELEG_LAUNCH_RESULT();
 }
 
+// The products of many rows over a short K.  A wavefront has a tile of 16 RT x 16 CT outputs to itself and goes
+// through the segments one after the other, each summed and added as above, so the outputs have the same bits; there
+// is nothing to join, and a last segment that is not whole costs what it has.  2,048 x 4,096: K = 32 18 us (on the
+// kernel above, most of whose wavefronts then wait, 86; before that 26), K = 128 50 (95), K = 160 60 (100; 75).
+template <int RT, int CT, bool VEC>
+__global__ __launch_bounds__(256) void gemm_f32_short_kernel(
+    const float* __restrict__ X, int ldx, const float* __restrict__ W, int ldw,
+    const float* __restrict__ bias, float* __restrict__ Y, int ldy, int M, int N, int K, int wide_store) {
+    constexpr int GROUP = F32_PIECES / 2;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / CELEG_WAVE), lane = threadIdx.x % CELEG_WAVE;
+    const int qd = lane >> 4, r16 = lane & 15;
+    const int row0 = blockIdx.y * (16 * RT), col0 = (blockIdx.x * 4 + wave) * (16 * CT);
+    if (col0 >= N) return;
+    const float* x_row[RT];
+    const float* w_row[CT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) x_row[rt] = X + static_cast<size_t>(min(row0 + rt * 16 + r16, M - 1)) * ldx;
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) w_row[ct] = W + static_cast<size_t>(min(col0 + ct * 16 + r16, N - 1)) * ldw;
+    auto four = [&](const float* row, int k) __attribute__((always_inline)) {
+        f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+        if (VEC) {
+            if (k < K) v = *reinterpret_cast<const f32x4_t*>(row + k);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (k + i < K) v[i] = row[k + i];
+        }
+        return v;
+    };
+    f32x4_t acc[CT][RT], total[CT][RT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) total[ct][rt] = acc[ct][rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < K; k0 += 16 * GROUP) {
+        f32x4_t wv[CT][GROUP], xv[RT][GROUP];
+#pragma unroll
+        for (int s = 0; s < GROUP; ++s) {
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) wv[ct][s] = four(w_row[ct], k0 + 16 * s + 4 * qd);
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) xv[rt][s] = four(x_row[rt], k0 + 16 * s + 4 * qd);
+        }
+#pragma unroll
+        for (int s = 0; s < GROUP; ++s) {
+            if (k0 + 16 * s >= K) break;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                    for (int rt = 0; rt < RT; ++rt)
+                        acc[ct][rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[ct][s][i], xv[rt][s][i], acc[ct][rt], 0, 0, 0);
+        }
+        const int next = k0 + 16 * GROUP;
+        if (next % F32_SEGMENT == 0 || next >= K) {        // the segment is done
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) {
+                    total[ct][rt] += acc[ct][rt];
+                    acc[ct][rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+                }
+        }
+    }
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        const int row = row0 + rt * 16 + r16;
+        if (row >= M) continue;
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            const int col = col0 + ct * 16 + 4 * qd;
+            float* y = Y + static_cast<size_t>(row) * ldy + col;
+            f32x4_t v = total[ct][rt];
+            if (wide_store && col + 3 < N) {
+                if (bias) v += f32x4_t{bias[col], bias[col + 1], bias[col + 2], bias[col + 3]};
+                *reinterpret_cast<f32x4_t*>(y) = v;
+                continue;
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (col + r < N) y[r] = v[r] + (bias ? bias[col + r] : 0.f);
+        }
+    }
+}
+
+template <int RT, int CT>
+static int launch_f32_short(const float* X, int ldx, const float* W, int ldw, const float* bias, float* Y, int ldy,
+                            int M, int N, int K, hipStream_t stream) {
+    const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    const bool vec = K % 4 == 0 && ldx % 4 == 0 && ldw % 4 == 0 && aligned(X) && aligned(W);
+    const int wide_store = ldy % 4 == 0 && aligned(Y);
+    const dim3 grid((N + 64 * CT - 1) / (64 * CT), (M + 16 * RT - 1) / (16 * RT)), block(4 * CELEG_WAVE);
+    auto kernel = vec ? &gemm_f32_short_kernel<RT, CT, true> : &gemm_f32_short_kernel<RT, CT, false>;
+    hipLaunchKernelGGL(kernel, grid, block, 0, stream, X, ldx, W, ldw, bias, Y, ldy, M, N, K, wide_store);
+    return CELEG_LAUNCH_RESULT();
+}
+
 extern "C" int celeg_gemm_f32(const float* X, int ldx, const float* W, int ldw, const float* bias,
                               float* Y, int ldy, int M, int N, int K, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
@@ -265,9 +364,15 @@ extern "C" int celeg_gemm_f32(const float* X, int ldx, const float* W, int ldw, 
     }
     if (M <= 32) return launch_f32<2, 1, 8, 512>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
     if (M <= 64) return launch_f32<4, 1, 4, 512>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
+    // One segment of k is one wavefront's work in the kernel above and the others of its workgroup wait; with two, the
+    // wavefront to itself is the faster one once there are tiles enough for every CU (K = 256: 1,024 x 1,024
+    // 14.7 us against 16.9, 424 x 1,024 13.4 against 9.4; K = 384: 2,048 x 1,024 36 against 32).
+    const long long tiles = static_cast<long long>((M + 63) / 64) * ((N + 63) / 64);
+    if (M <= 32 * 65535 && (K <= F32_SEGMENT || (K <= 2 * F32_SEGMENT && tiles >= 256)))      // (a grid has 65,535 rows of tiles)
+        return launch_f32_short<2, 2>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
     // 64 x 64 tiles (an operand from the caches serves four products) once there are two for every CU; below
     // that (350 rows: 96 of them at N = 1,024) half the tile and twice the wavefronts
-    if (static_cast<long long>((M + 63) / 64) * ((N + 63) / 64) >= 512)
+    if (tiles >= 512)
         return launch_f32<4, 4, 2, 256>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
     return launch_f32<2, 4, 2, 512>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
 }

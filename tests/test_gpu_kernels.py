@@ -247,7 +247,25 @@ def test_gemm_f32_tiles(ops, M, N, K):
         assert torch.equal(one[0], out[m])
 
 
-@pytest.mark.parametrize("M,N,K", [(530, 4100, 132), (4097, 513, 260)])
+@pytest.mark.parametrize("M", [65, 96, 130])
+@pytest.mark.parametrize("N", [1, 31, 128, 129, 260])
+@pytest.mark.parametrize("K", [1, 4, 15, 16, 20, 64, 100, 127, 128, 129])
+def test_gemm_f32_short_inner_sizes(ops, M, N, K):
+    """Up to 128 values of k a wavefront keeps its tile to itself: every remainder of a piece of 16, rows and columns that
+    do not fill a tile, rows on any alignment, and the bits of a row alone."""
+    wide, out = randn(M, K + 3, seed=17), torch.zeros(M + 1, N, device=DEV)
+    w, b = randn(N, K, seed=18), randn(N, seed=19)
+    x, same, one = wide[:, 1:K + 1], torch.empty(M, N + 3, device=DEV), torch.empty(1, N, device=DEV)
+    ops.linear(x, w, out[:M], bias=b)
+    ops.linear(x.contiguous(), w, same[:, :N], bias=b)
+    ops.linear(x[M - 1:], w, one, bias=b)
+    assert torch.equal(out[:M], same[:, :N]) and torch.equal(out[M - 1], one[0]) and float(out[M].abs().max()) == 0
+    # a sum of K products and the bias, each step within 2^-24 of the magnitudes summed
+    bound = (K + 3) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T + b.double().abs())
+    assert bool(((out[:M].double() - x.double() @ w.double().T - b.double()).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(530, 4100, 132), (4097, 513, 260), (1025, 1000, 200), (1030, 1020, 256)])
 def test_gemm_f32_many_rows(ops, M, N, K):
     x, w = randn(M, K, seed=7), randn(N, K, seed=8)
     out, one = torch.empty(M, N, device=DEV), torch.empty(1, N, device=DEV)
