@@ -784,7 +784,7 @@ extern "C" void celeg_gemm_tiles_force(int shape) { g_force_shape = shape; }
 extern "C" void celeg_gemm_tiles_force_dies(int dies_m) { g_force_dies_m = dies_m; }
 
 // id, rows, weight rows, wavefronts along rows and along weight rows, stages, values of k a block of
-// the wide kernel (0: the kernel with tiles up to 256x128).  The rule below takes 10, 11, 13 and 16 to 22; the
+// the wide kernel (0: the kernel with tiles up to 256x128).  The rule below takes 3, 10, 11, 13 and 16 to 22; the
 // others are what tests and tuning runs compare them with.
 #define TILE_SHAPES(X) \
     X(0, 128, 128, 2, 2, 3, 0) \
@@ -852,34 +852,39 @@ static TileShape tile_shape(int M, int N, int K, int streams) {
         //    100      17.7 | 25.6          7.1 |  9.2               6.9 |  8.7                11.1 | 12.3
         //    300      17.8 | 26.1          7.3 |  9.4               7.9 |  8.9                13.9 | 16.8
         //    600      21.1 | 26.3          8.5 |  9.6               9.8 |  9.8                19.1 | 21.2
-        //  1,000      24.9 | 27.3          8.9 | 10.1              14.2 | 14.6                28.4 | 37.4
-        //  1,400      36.0 | 36.0          9.9 | 10.9              17.9 | 18.9                37.4 | 37.4
+        //  1,000      24.9 | 27.3          8.9 | 10.1              15.1 | 15.4                28.4 | 37.4
         //  2,048      37.4 | 37.4         12.3 | 12.3              19.3 | 19.3                41.4 | 41.4
-        //  4,096      53.2 | 70.1         20.2 | 21.0              29.6 | 33.9
-        // With a long K tiles of 128x64 and 64x128 are the same (w2 at 2,048 rows: 37.4 and 37.3).  Tiles of
-        // 64x192 end at 240: 256 of them (1,000 rows by 3,072) would be 12.9 us against 14.2 on 128x128, but how
-        // that product is cut is held by a test.  Two workgroups of 8 wavefronts a compute unit on 128x128 tiles
-        // come before 256x192 (w1 with w3 at 800 rows 23.2 us against 27.5).
+        // Where two shapes fit, both at 300 to 4,096 rows of 20 products in turn:
+        //   128x64 before 64x128 from 2,048 values of k on: 1 to 7 % faster in all of 56 (at 1,024 the same within 2 %)
+        //   64x192 before 128x128: 0 to 11 % faster in all of 51
+        //   64x128 on 4 wavefronts, two a compute unit, before 128x128 on 8, one: 2 to 6 % faster, up to 10 Mi weights;
+        //   with more than the dies' L2s hold beside the rows (2,048 x 8,192, 4,096 x 4,096) 10 to 25 % slower
+        //   128x128, two a compute unit, before 256x192: w1 with w3 at 800 rows 23.2 us against 27.5
+        //   256x192 before more than two of 128x128: 1 to 27 % faster in all of 45
+        //   256x288 likewise, where the work of a round pays for its long first loads and its end: values of k x tiles
+        //   of 128x128 from 1,152 Ki on 12 % faster to 2 % slower (29), below 5 to 20 % slower (12; w1 with w3 at
+        //   1,400 rows 39.7 us against 37.1)
+        const auto tiles = [&](int bm, int bn) {
+            return static_cast<long long>((M + bm - 1) / bm) * ((static_cast<long long>(N) * streams + bn - 1) / bn);
+        };
         const auto fits = [&](int bm, int bn, int on_a_unit) {
             return dies_of((M + bm - 1) / bm, (N * streams + bn - 1) / bn, M, N * streams).per_die <= DIE_UNITS * on_a_unit;
         };
+        const long long weights = static_cast<long long>(N) * streams * K;
         if (fits(32, 64, 1)) id = 19;
         else if (fits(64, 64, 1)) id = 20;
         else if (K >= 2048 && fits(128, 64, 1)) id = 16;
         else if (fits(64, 128, 1)) id = 17;
-        else if (((M + 63) / 64) * ((N * streams + 191) / 192) <= 240 && fits(64, 192, 1)) id = 21;
-        else if (fits(128, 128, 1)) id = 22;
+        else if (fits(64, 192, 1)) id = 21;
+        else if (fits(128, 128, 1)) id = weights <= (10 << 20) ? 3 : 22;
         else if (fits(128, 192, 1)) id = 18;
         else if (fits(128, 128, 2)) id = 10;
         else if (fits(256, 192, 1)) id = 13;
-        else if (fits(256, 288, 1)) id = 11;
+        else if (fits(256, 288, 1) && K * tiles(128, 128) >= (1152 << 10)) id = 11;
         else {
             // More than a round: 128x128 with two workgroups a compute unit, or 256x288, one a compute unit, where
             // the rounds of them (2.2 times as long as a round of 128x128 tiles, measured at 1,024 and 2,048 values
             // of k) cover the product in less time.
-            const auto tiles = [&](int bm, int bn) {
-                return static_cast<long long>((M + bm - 1) / bm) * ((static_cast<long long>(N) * streams + bn - 1) / bn);
-            };
             const long long rounds288 = (tiles(256, 288) + 255) / 256, rounds128 = (tiles(128, 128) + 511) / 512;
             id = rounds288 * 22 < rounds128 * 10 ? 11 : 10;
         }

@@ -103,7 +103,7 @@ def test_residual_adds_in_place_refreshes_the_copy_and_leaves_partial_sums(ops, 
 
 
 @pytest.mark.parametrize("M,N,K,blocks", [(2000, 1024, 2304, 16), (2000, 1024, 1024, 8), (2048, 2048, 1024, 16),
-                                          (2048, 3072, 1024, 16), (1024, 3072, 1024, 24)])
+                                          (2048, 3072, 1024, 16), (1024, 3072, 1024, 16)])
 def test_the_shapes_chosen_for_a_prefill(ops, M, N, K, blocks):
     """What the choice of shape gives at the sizes of a prefill of some 2,000 rows (few weight
     rows with a long and a short K, q/k/v, in_proj), against torch, with the residual epilogue;
@@ -174,6 +174,19 @@ def test_a_row_is_the_same_in_every_chosen_tile(ops, M, N, K):
         assert torch.equal(big[M - 65:M], small) and float(big[M].abs().max()) == 0
     ref = product(a, w)
     out = torch.empty(M, N, dtype=BF, device=DEV)
+    ops.tiled_linear(a, w, out)
+    assert float((out.double() - ref).abs().max()) <= 2 ** -7 * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("M,N,K,blocks", [
+    (1500, 1024, 1984, 8), (1500, 1024, 2048, 16),             # 64x128; 128x64 from 2,048 values of k on
+    (1024, 3072, 128, 16), (1089, 3072, 128, 24),              # 64x192 while it fits, then 128 columns
+    (3000, 1024, 64, 8)])
+def test_where_the_choice_of_shape_changes(ops, M, N, K, blocks):
+    ops._lib("gemm_tiles").celeg_gemm_tiles_force(-1)
+    assert ops.tiled_stat_blocks(M, N, K) == blocks
+    a, w = randn(M, K, seed=24, dtype=BF), randn(N, K, seed=25, scale=0.03, dtype=BF)
+    out, ref = torch.empty(M, N, dtype=BF, device=DEV), product(a, w)
     ops.tiled_linear(a, w, out)
     assert float((out.double() - ref).abs().max()) <= 2 ** -7 * float(ref.abs().max())
 
