@@ -565,6 +565,49 @@ __device__ __forceinline__ void lds_wait_rows(const int left, bf16x8_t& x, bf16x
     for (int tm = 0; tm < FM; ++tm) asm volatile("" : "+v"(rows[tm]));     // (behind the wait above: volatile statements keep their order)
 }
 
+// The reads from LDS of a block of the wide kernel, in the order of issue: the rows' operands of step 0,
+// weights 0 and 1; then with piece t = step * FN + j weights t + 2 and, for the first FM pieces of a step,
+// one of the rows' operands of the next step.  LDS answers in this order.
+template <int FM, int FN, int KS>
+struct WideReads {
+    static constexpr int PIECES = KS * FN;
+    static_assert(FM <= FN, "the rows' operands of a step are asked for with the pieces of the step before");
+    static constexpr bool row_with(int t) { return t / FN + 1 < KS && t % FN < FM; }
+    // reads that are asked for ahead of piece t
+    static constexpr int ahead_of(int t) {
+        int n = FM + 2;
+        for (int p = 0; p < t; ++p) n += (p + 2 < PIECES ? 1 : 0) + (row_with(p) ? 1 : 0);
+        return n;
+    }
+    static constexpr int weights(int t) { return t < 2 ? FM + t : ahead_of(t - 2); }           // the place of weights t
+    static constexpr int last_row(int t) {         // the place of the last of the rows' operands of piece t's step
+        const int with = (t / FN - 1) * FN + FM - 1;
+        return t < FN ? FM - 1 : ahead_of(with) + (with + 2 < PIECES ? 1 : 0);
+    }
+    // how many reads may still be out where piece t starts: those behind its weights and its step's rows, whichever
+    // is later (the rows where FM > FN - 2)
+    static constexpr int may_be_out(int t) {
+        const int needed = weights(t) > last_row(t) ? weights(t) : last_row(t);
+        return ahead_of(t) - 1 - needed;
+    }
+    // the reads replayed: where piece t starts, its weights and all rows' operands of its step are there
+    static constexpr bool sound() {
+        int weight_at[PIECES] = {}, row_at[KS][FM] = {}, asked = 0;
+        for (int r = 0; r < FM; ++r) row_at[0][r] = asked++;
+        weight_at[0] = asked++;
+        weight_at[1] = asked++;
+        for (int t = 0; t < PIECES; ++t) {
+            const int there = asked - may_be_out(t);
+            if (may_be_out(t) < 0 || may_be_out(t) > 3 || weight_at[t] >= there) return false;      // (lds_wait counts to 3)
+            for (int r = 0; r < FM; ++r)
+                if (row_at[t / FN][r] >= there) return false;
+            if (t + 2 < PIECES) weight_at[t + 2] = asked++;
+            if (row_with(t)) row_at[t / FN + 1][t % FN] = asked++;
+        }
+        return true;
+    }
+};
+
 // SwiGLU of a wide tile whose wavefronts each hold columns of one stream only: gate and up
 // (rounded to bfloat16, as where they are tensors of their own) meet in LDS, [stream][row], and
 // leave as whole rows, 16 bytes a lane.
@@ -651,6 +694,8 @@ void gemm_tiles_wide_kernel(const TileParams p, const int tiles_m, const int til
     static_assert(BN % (16 * WGN) == 0 && BN % (16 * NS) == 0 && PS % FN == 0 && WTM % 16 == 0 &&
                   (BM + BN) % 16 == 0 && STAGES >= 2 && FN >= 2 && FN <= 12 && FM <= 12 && (KB == 32 || KB == 64), "tile shape");
     static_assert(GPW * STAGES < 64, "more loads in flight than the counter holds");
+    using Reads = WideReads<FM, FN, KS>;
+    static_assert(Reads::sound(), "an operand is used ahead of its read");
     extern __shared__ __attribute__((aligned(1024))) char lds[];
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -733,10 +778,7 @@ void gemm_tiles_wide_kernel(const TileParams p, const int tiles_m, const int til
         }
         // The reads and the waits for them are written out (the compiler, left to count, waits for
         // every read in flight before each second piece).  Piece t = ks * FN + j of the block: step
-        // ks, column piece j.  In the order of issue: the rows' operands of step 0, weights 0 and 1;
-        // then behind the first matrix instruction of piece t weights t + 2 and, for the first FM
-        // pieces of a step, one of the rows' operands of the next step.  LDS answers in order, so
-        // piece t may start when no more reads are out than were issued behind weights t.
+        // ks, column piece j; its reads go behind its first matrix instruction (WideReads: their order).
         bf16x8_t a[2][FM], w[3];
 #pragma unroll
         for (int tm = 0; tm < FM; ++tm) lds_read<16 * ROW_BYTES>(a[0][tm], at_a[0], tm);
@@ -745,17 +787,11 @@ void gemm_tiles_wide_kernel(const TileParams p, const int tiles_m, const int til
 #pragma unroll
         for (int t = 0; t < KS * FN; ++t) {
             const int ks = t / FN, j = t % FN;
-            // reads issued behind weights t: weights t + 1 (if any) and the rows' operands that went
-            // with weights t and t + 1 (issued in pieces t - 2 and t - 1)
-            constexpr auto rows_with = [](int piece) {      // does piece `piece` issue one of the next step's rows' operands?
-                return piece >= 0 && piece / FN + 1 < KS && piece % FN < FM ? 1 : 0;
-            };
-            const int behind = (t + 1 < KS * FN ? 1 : 0) + (t >= 2 ? rows_with(t - 2) : 0) + (t >= 1 ? rows_with(t - 1) : 0);
-            if (j == 0) lds_wait_rows(behind, w[t % 3], a[ks & 1]);
-            else lds_wait(behind, w[t % 3]);
+            if (j == 0) lds_wait_rows(Reads::may_be_out(t), w[t % 3], a[ks & 1]);
+            else lds_wait(Reads::may_be_out(t), w[t % 3]);
             acc[j][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t % 3], a[ks & 1][0], acc[j][0], 0, 0, 0);
             if (t + 2 < KS * FN) lds_read<16 * ROW_BYTES>(w[(t + 2) % 3], at_w[(t + 2) / FN < KS ? (t + 2) / FN : 0], (t + 2) % FN);
-            if (rows_with(t)) lds_read<16 * ROW_BYTES>(a[(ks + 1) & 1][j < FM ? j : 0], at_a[ks + 1 < KS ? ks + 1 : 0], j);
+            if (Reads::row_with(t)) lds_read<16 * ROW_BYTES>(a[(ks + 1) & 1][j < FM ? j : 0], at_a[ks + 1 < KS ? ks + 1 : 0], j);
 #pragma unroll
             for (int tm = 1; tm < FM; ++tm)
                 acc[j][tm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t % 3], a[ks & 1][tm], acc[j][tm], 0, 0, 0);
