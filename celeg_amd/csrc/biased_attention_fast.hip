@@ -332,8 +332,12 @@ __global__ __launch_bounds__(BF_WAVES * CELEG_WAVE) void biased_attention_rows_k
                 quad, vd);
 }
 
+// Wavefronts a SIMD that the registers leave room for. Where the staging areas of two workgroups of eight
+// wavefronts fit LDS (heads of 32) they are four, so that two run on a compute unit (64 requests at 1,000 keys, 8
+// heads: 24.6 us; with the five registers more that the compiler takes by itself, and one workgroup, 33.1).
+constexpr int bf_tile_waves_a_simd(int d, int v, bool full) { return full && d <= 32 && v <= 32 ? 4 : 1; }
 template <int D, int V, int WAVES, bool FULL>
-__global__ __launch_bounds__(WAVES * CELEG_WAVE) void biased_attention_tile_kernel(const BfArgs a) {
+__global__ __launch_bounds__(WAVES * CELEG_WAVE, bf_tile_waves_a_simd(D, V, FULL)) void biased_attention_tile_kernel(const BfArgs a) {
     constexpr int KROW = D + 8, VROW = BF_KEYS + 8, KS = D / 32, DT = V / 16, BUF = BF_KEYS * KROW + V * VROW;
     const int kd = FULL ? D : a.kd, vd = FULL ? V : a.vd;
     extern __shared__ __attribute__((aligned(16))) unsigned char bf_lds[];
