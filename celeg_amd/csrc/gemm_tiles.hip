@@ -820,36 +820,28 @@ extern "C" void celeg_gemm_tiles_force(int shape) { g_force_shape = shape; }
 extern "C" void celeg_gemm_tiles_force_dies(int dies_m) { g_force_dies_m = dies_m; }
 
 // id, rows, weight rows, wavefronts along rows and along weight rows, stages, values of k a block of
-// the wide kernel (0: the kernel with tiles up to 256x128).  The rule below takes 3, 10, 11, 13 and 16 to 22; the
-// others are what tests and tuning runs compare them with.
+// the wide kernel (0: the kernel with tiles up to 128x192)
 #define TILE_SHAPES(X) \
-    X(0, 128, 128, 2, 2, 3, 0) \
-    X(1, 256, 128, 2, 2, 3, 0) \
-    X(2, 128, 64, 2, 2, 3, 0)  \
-    X(3, 64, 128, 2, 2, 3, 0)  \
-    X(4, 128, 128, 2, 2, 2, 0) \
-    X(5, 256, 128, 4, 2, 3, 0) \
-    X(6, 128, 128, 2, 2, 4, 0) \
-    X(7, 64, 64, 2, 2, 4, 0)   \
-    X(8, 64, 64, 2, 2, 2, 0)   \
-    X(9, 128, 64, 2, 2, 2, 0)  \
-    X(10, 128, 128, 4, 2, 2, 0) \
-    X(11, 256, 288, 4, 2, 2, 64) \
-    X(12, 256, 160, 4, 2, 3, 64) \
-    X(13, 256, 192, 4, 2, 2, 64) \
-    X(14, 128, 192, 2, 2, 3, 64) \
-    X(15, 256, 128, 4, 2, 3, 64) \
-    X(16, 128, 64, 4, 2, 4, 0) \
-    X(17, 64, 128, 2, 4, 4, 0) \
-    X(18, 128, 192, 4, 2, 3, 0) \
-    X(19, 32, 64, 2, 2, 8, 0)  \
-    X(20, 64, 64, 4, 2, 4, 0)  \
-    X(21, 64, 192, 4, 2, 4, 0) \
-    X(22, 128, 128, 4, 2, 4, 0)
+    X(0, 32, 64, 2, 2, 8, 0)  \
+    X(1, 64, 64, 4, 2, 4, 0)  \
+    X(2, 128, 64, 4, 2, 4, 0) \
+    X(3, 64, 128, 2, 4, 4, 0) \
+    X(4, 64, 192, 4, 2, 4, 0) \
+    X(5, 64, 128, 2, 2, 3, 0) \
+    X(6, 128, 128, 4, 2, 4, 0) \
+    X(7, 128, 192, 4, 2, 3, 0) \
+    X(8, 128, 128, 4, 2, 2, 0) \
+    X(9, 256, 192, 4, 2, 2, 64) \
+    X(10, 256, 288, 4, 2, 2, 64)
 
-static const int k_shape_bm[] = {128, 256, 128, 64, 128, 256, 128, 64, 64, 128, 128, 256, 256, 256, 128, 256, 128, 64, 128, 32, 64, 64, 128};
-static const int k_shape_bn[] = {128, 128, 64, 128, 128, 128, 128, 64, 64, 64, 128, 288, 160, 192, 192, 128, 64, 128, 192, 64, 64, 192, 128};
-#define N_TILE_SHAPES 23
+#define TILE_ROWS(ID, BM, BN, WGM, WGN, STAGES, KB) BM,
+#define TILE_COLUMNS(ID, BM, BN, WGM, WGN, STAGES, KB) BN,
+static const int k_shape_bm[] = {TILE_SHAPES(TILE_ROWS)};
+static const int k_shape_bn[] = {TILE_SHAPES(TILE_COLUMNS)};
+#undef TILE_ROWS
+#undef TILE_COLUMNS
+static constexpr int N_TILE_SHAPES = sizeof(k_shape_bm) / sizeof(k_shape_bm[0]);
+extern "C" int celeg_gemm_tiles_shapes() { return N_TILE_SHAPES; }      // (how many there are to force)
 
 // How the dies share the grid of tiles: every row of tiles of A is read by 8 / m dies, every column of
 // tiles of W by m of them; the split with the fewest bytes read of those that leave no die more tiles than it
@@ -907,22 +899,22 @@ static TileShape tile_shape(int M, int N, int K, int streams) {
             return dies_of((M + bm - 1) / bm, (N * streams + bn - 1) / bn, M, N * streams).per_die <= DIE_UNITS * on_a_unit;
         };
         const long long weights = static_cast<long long>(N) * streams * K;
-        if (fits(32, 64, 1)) id = 19;
-        else if (fits(64, 64, 1)) id = 20;
-        else if (K >= 2048 && fits(128, 64, 1)) id = 16;
-        else if (fits(64, 128, 1)) id = 17;
-        else if (fits(64, 192, 1)) id = 21;
-        else if (fits(128, 128, 1)) id = weights <= (10 << 20) ? 3 : 22;
-        else if (fits(128, 192, 1)) id = 18;
-        else if (fits(128, 128, 2)) id = 10;
-        else if (fits(256, 192, 1)) id = 13;
-        else if (fits(256, 288, 1) && K * tiles(128, 128) >= (1152 << 10)) id = 11;
+        if (fits(32, 64, 1)) id = 0;
+        else if (fits(64, 64, 1)) id = 1;
+        else if (K >= 2048 && fits(128, 64, 1)) id = 2;
+        else if (fits(64, 128, 1)) id = 3;
+        else if (fits(64, 192, 1)) id = 4;
+        else if (fits(128, 128, 1)) id = weights <= (10 << 20) ? 5 : 6;
+        else if (fits(128, 192, 1)) id = 7;
+        else if (fits(128, 128, 2)) id = 8;
+        else if (fits(256, 192, 1)) id = 9;
+        else if (fits(256, 288, 1) && K * tiles(128, 128) >= (1152 << 10)) id = 10;
         else {
             // More than a round: 128x128 with two workgroups a compute unit, or 256x288, one a compute unit, where
             // the rounds of them (2.2 times as long as a round of 128x128 tiles, measured at 1,024 and 2,048 values
             // of k) cover the product in less time.
             const long long rounds288 = (tiles(256, 288) + 255) / 256, rounds128 = (tiles(128, 128) + 511) / 512;
-            id = rounds288 * 22 < rounds128 * 10 ? 11 : 10;
+            id = rounds288 * 22 < rounds128 * 10 ? 10 : 8;
         }
     }
     return TileShape{id, k_shape_bm[id], k_shape_bn[id]};
