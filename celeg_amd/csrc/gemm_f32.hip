@@ -13,9 +13,9 @@
 // that even a 1024 x 1024 matrix is asked for by 512 wavefronts in one trip to memory.  Many rows are bound
 // by the matrix cores: larger tiles, operands straight from the caches (16 bytes a cycle and CU of them).
 // Measured in a chain over different matrices (before: 64 x 64 tiles of vector instructions, k in order,
-// 137 us for any product with K = 1,024): 2 rows, 1024 x 1024 3.3 us, 3072 x 1024 5.5 us, 1024 x 4608
-// 7.2 us (before 613), 65536 x 1024 54 us (5.0 TB/s; before 247); 64 rows, 3072 x 1024 13.7 us; 2,048 rows,
-// 4608 x 1024 256 us (76 TFLOP/s).  Error against 64 bits 2.1e-7 of the result (2-norm), before 3 times that.
+// 137 us for products of up to 64 rows and few columns with K = 1,024): 2 rows, 1024 x 1024 3.3 us, 3072 x 1024
+// 5.5 us, 1024 x 4608 7.2 us (before 613), 65536 x 1024 54 us (5.0 TB/s; before 247); 64 rows, 3072 x 1024
+// 13.7 us; 2,048 rows, 4608 x 1024 256 us (76 TFLOP/s).  Error against 64 bits 2.1e-7 of the result (2-norm), before 3 times that.
 #include "common.h"
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));

@@ -152,7 +152,9 @@ __global__ void short_conv_fwd_vec_kernel(
 // requests beside a prompt, set the kernel's time (2,048 rows of 1,024 channels: 20 decoding requests
 // and a prompt 14.8 us with a load at a time there, now 7.0; one prompt 9.0, now 5.8; 24 rows 7.1, now 3.3; the taps,
 // 16 bytes a load instead of 4, are in these too).
-#define CONV_BLOCK_TOKENS 2     // (more need more registers than leave room for a second wavefront; 1 and 4 were slower before)
+// (2,048 rows of one prompt 4.3 us, with 4 tokens a thread 5.8; beside 20 decoding requests 4.9 and 7.2; 64 decoding
+// requests 4.1 and 6.6; 24 rows 3.5 and 5.2: 1,024 channels, three taps, bfloat16, the same rows again and again)
+#define CONV_BLOCK_TOKENS 2
 typedef float conv_f32x4 __attribute__((ext_vector_type(4)));
 template <int VEC>
 __device__ __forceinline__ void conv_load(float (&to)[VEC], const float* from) {
