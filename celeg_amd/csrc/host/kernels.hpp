@@ -178,6 +178,11 @@ int celeg_delta_scan(const float* qk, const float* v, const float* beta_decay, f
                      int general, const int* token_seq, float* pairs, int n_tokens, hipStream_t stream);
 int celeg_delta_gated_norm(const float* o, const float* w, const void* gate, int ldg, int dtype, float eps, void* out,
                            int n_tokens, int H, int V, int act, hipStream_t stream);
+int celeg_delta_step_ok(int G, int H, int D, int V, int taps);
+int celeg_delta_step(const void* proj, int ld, int dtype, int col_b, int col_a, const float* conv_w, const float* a_log,
+                     const float* dt_bias, float* conv_state, size_t conv_stride, float* state, size_t state_stride,
+                     const int* seq_slot, const float* norm_w, const void* gate, int ldg, float eps, int act, void* out,
+                     int n_rows, int G, int H, int D, int V, int taps, hipStream_t stream);
 // layer_glue.hip
 int celeg_activation_bias(const void* x, int ldx, const float* bias, void* out, int ldo, int dtype, int rows, int cols, int act,
                           float p0, float p1, hipStream_t stream);

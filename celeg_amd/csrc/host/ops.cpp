@@ -1001,6 +1001,44 @@ void Ops::delta_gated_norm(const Tensor& o, const Tensor& weight, const Tensor& 
                                         static_cast<int>(T), heads, vdim, act, stream), "delta_gated_norm");
 }
 
+bool Ops::delta_step_ok(const DeltaShape& s, const StepBatch& batch) const {
+    return use_delta_step && !delta_general && batch.decode_only && batch.n_seqs == batch.n_tokens &&
+           celeg_delta_step_ok(s.kv_heads, s.heads, s.dim, s.vdim, s.taps);
+}
+
+void Ops::delta_step(const Tensor& proj, int col_b, int col_a, const DeltaShape& s, const Tensor& conv_w, const Tensor& a_log,
+                     const Tensor& dt_bias, const Tensor& conv_state, const Tensor& state, const Tensor& weight, const Tensor& gate, float eps,
+                     int act, const Tensor& out, const StepBatch& batch) {
+    need(delta_step_ok(s, batch), "delta_step: sizes or steps that the kernel was not written for");
+    need(act == 0 || act == 1, "delta_step: act is 0 (silu) or 1 (sigmoid)");
+    dev(proj, "proj");
+    const long long T = proj.shape[0], vw = static_cast<long long>(s.heads) * s.vdim, C = 2LL * s.kv_heads * s.dim + vw;
+    need(proj.ndim == 2 && T == batch.n_tokens && col_b >= C && col_a >= C && col_b + s.heads <= proj.shape[1] &&
+             col_a + s.heads <= proj.shape[1], "delta_step: the projections' columns do not fit");
+    dev(conv_w, "conv_w", DType::F32);
+    dev(a_log, "a_log", DType::F32);
+    dev(dt_bias, "dt_bias", DType::F32);
+    dev(weight, "weight", DType::F32);
+    need(conv_w.numel() == C * s.taps && a_log.numel() == s.heads && dt_bias.numel() == s.heads && weight.numel() == s.vdim,
+         "delta_step: one row of taps per channel, one decay constant and bias per head, one weight per value");
+    dev(conv_state, "conv_state", DType::F32, false);
+    need(conv_state.ndim == 3 && conv_state.shape[1] == std::max(s.taps - 1, 1) && conv_state.shape[2] == C &&
+             conv_state.stride[2] == 1 && conv_state.stride[1] == C, "delta_step: saved inputs must be [slots, taps - 1, channels]");
+    dev(state, "state", DType::F32, false);
+    need(state.ndim >= 2 && state.numel() / state.shape[0] == vw * s.dim && state.stride[state.ndim - 1] == 1,
+         "delta_step: state must be [slots, heads, dim, vdim]");
+    dev(gate, "gate", proj.dtype, false);
+    dev(out, "out", proj.dtype);
+    need(gate.ndim == 2 && gate.shape[0] == T && gate.shape[1] == vw && out.ndim == 2 && out.shape[0] == T && out.shape[1] == vw &&
+             out.contiguous(), "delta_step: gate and out must be [rows, heads * vdim]");
+    took(Path::DeltaRule);
+    kernel_check(celeg_delta_step(proj.data, rows_of(proj, "proj"), dt(proj, "proj"), col_b, col_a, conv_w.as<float>(), a_log.as<float>(),
+                                  dt_bias.as<float>(), conv_state.as<float>(), static_cast<size_t>(conv_state.stride[0]), state.as<float>(),
+                                  static_cast<size_t>(state.stride[0]), batch.seq_slot, weight.as<float>(), gate.data,
+                                  rows_of(gate, "gate"), eps, act, out.data, static_cast<int>(T), s.kv_heads, s.heads, s.dim, s.vdim,
+                                  s.taps, stream), "delta_step");
+}
+
 // ---------------------------------------------------------------------------- states with a decay per key channel
 void Ops::channel_decay(const Tensor& z, const Tensor& a_log, const Tensor& dt_bias, const Tensor& decay, int heads, int dim) {
     dev(z, "z");

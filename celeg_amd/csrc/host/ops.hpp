@@ -126,6 +126,7 @@ public:
     bool attention_general = false;      // always the general attention kernel
     bool delta_general = false;          // the delta rule's recurrence always by the kernel for any dim
     bool delta_pairs = true;             // the recurrence in registers takes whole blocks of rows two tokens at a time
+    bool use_delta_step = true;          // steps of one token a request: the delta rule in one kernel
     bool use_sigmoid_mfma = true;        // bfloat16 attention with sigmoid weights on the matrix cores
     bool use_biased_mfma = true;         // bfloat16 attention with a distance bias on the matrix cores
     int biased_rows_form = -1;           // likewise for the attention with a distance bias
@@ -220,6 +221,12 @@ public:
     // (act: what the gate passes through, 0 silu, 1 sigmoid)
     void delta_gated_norm(const Tensor& o, const Tensor& weight, const Tensor& gate, float eps, const Tensor& out, int heads, int vdim,
                           int act = 0);
+    // The three above in one kernel, for steps of one token a request (delta_step_ok says whether it takes the step):
+    // gate [rows, heads * vdim] (a view with dense rows), out [rows, heads * vdim] in the dtype of proj.
+    bool delta_step_ok(const DeltaShape& shape, const StepBatch& batch) const;
+    void delta_step(const Tensor& proj, int col_b, int col_a, const DeltaShape& shape, const Tensor& conv_w, const Tensor& a_log,
+                    const Tensor& dt_bias, const Tensor& conv_state, const Tensor& state, const Tensor& weight, const Tensor& gate, float eps,
+                    int act, const Tensor& out, const StepBatch& batch);
     // Matrix states with a decay per key channel, S [dim, vdim] per value head: S <- diag(decay) S;
     // u = beta (v - S^T k), or u = v where beta is null; S <- S + k u^T; o = S^T q.
     // decay = exp(-exp(a_log[head]) softplus(z + dt_bias)); z [rows, heads * dim] with dense rows, decay 32-bit

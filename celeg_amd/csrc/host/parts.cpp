@@ -1633,33 +1633,38 @@ public:
         const long long T = x.shape[0];
         Tensor proj = rt.ws.buf("delta_proj", rt.dtype, {T, w_in_->view.shape[0]});
         rt.ops.linear(x, w_in_->view, proj, nullptr, rt.ws);
-        Tensor qk = rt.ws.buf("delta_qk", DType::F32, {T, 2 * qk_width()});
-        Tensor v = rt.ws.buf("delta_v", DType::F32, {T, v_width()});
-        Tensor beta_decay = rt.ws.buf("delta_beta_decay", DType::F32, {T, 2LL * shape_.heads});
-        Tensor o = rt.ws.buf("delta_o", DType::F32, {T, v_width()});
-        if (!per_channel_) {
-            rt.ops.delta_prepare(proj, static_cast<int>(col_b_), static_cast<int>(col_a_), shape_, conv_w_->view, a_log_->view,
-                                 dt_bias_->view, cache.states.at("conv"), qk, v, beta_decay, batch);
-            rt.ops.delta_scan(qk, v, beta_decay, cache.states.at("S"), o, shape_, batch, rt.ws);
-        } else {
-            Tensor z = proj.cols(col_a_, decay_width());
-            if (decay_rank_ > 0) {
-                z = rt.ws.buf("delta_decay_in", rt.dtype, {T, decay_width()});
-                rt.ops.linear(proj.cols(col_a_, decay_rank_), a2_->view, z, nullptr, rt.ws);
-            }
-            Tensor decay = rt.ws.buf("delta_decay", DType::F32, {T, decay_width()});
-            rt.ops.channel_decay(z, a_log_->view, dt_bias_->view, decay, shape_.heads, shape_.dim);
-            rt.ops.delta_prepare(proj, static_cast<int>(col_b_), static_cast<int>(col_b_), shape_, conv_w_->view, Tensor(), Tensor(),
-                                 cache.states.at("conv"), qk, v, beta_decay, batch);
-            rt.ops.channel_scan(qk, v, decay, beta_decay.as<float>(), 2 * shape_.heads, cache.states.at("S"), o, shape_, batch);
-        }
         Tensor gate = proj.cols(col_gate_, v_width());
         if (gate_rank_ > 0) {
             gate = rt.ws.buf("delta_gate", rt.dtype, {T, v_width()});
             rt.ops.linear(proj.cols(col_gate_, gate_rank_), g2_->view, gate, nullptr, rt.ws);
         }
         Tensor gated = rt.ws.buf("delta_gated", rt.dtype, {T, v_width()});
-        rt.ops.delta_gated_norm(o, norm_->view, gate, eps_, gated, shape_.heads, shape_.vdim, gate_act_);
+        if (!per_channel_ && rt.ops.delta_step_ok(shape_, batch)) {
+            rt.ops.delta_step(proj, static_cast<int>(col_b_), static_cast<int>(col_a_), shape_, conv_w_->view, a_log_->view, dt_bias_->view,
+                              cache.states.at("conv"), cache.states.at("S"), norm_->view, gate, eps_, gate_act_, gated, batch);
+        } else {
+            Tensor qk = rt.ws.buf("delta_qk", DType::F32, {T, 2 * qk_width()});
+            Tensor v = rt.ws.buf("delta_v", DType::F32, {T, v_width()});
+            Tensor beta_decay = rt.ws.buf("delta_beta_decay", DType::F32, {T, 2LL * shape_.heads});
+            Tensor o = rt.ws.buf("delta_o", DType::F32, {T, v_width()});
+            if (!per_channel_) {
+                rt.ops.delta_prepare(proj, static_cast<int>(col_b_), static_cast<int>(col_a_), shape_, conv_w_->view, a_log_->view,
+                                     dt_bias_->view, cache.states.at("conv"), qk, v, beta_decay, batch);
+                rt.ops.delta_scan(qk, v, beta_decay, cache.states.at("S"), o, shape_, batch, rt.ws);
+            } else {
+                Tensor z = proj.cols(col_a_, decay_width());
+                if (decay_rank_ > 0) {
+                    z = rt.ws.buf("delta_decay_in", rt.dtype, {T, decay_width()});
+                    rt.ops.linear(proj.cols(col_a_, decay_rank_), a2_->view, z, nullptr, rt.ws);
+                }
+                Tensor decay = rt.ws.buf("delta_decay", DType::F32, {T, decay_width()});
+                rt.ops.channel_decay(z, a_log_->view, dt_bias_->view, decay, shape_.heads, shape_.dim);
+                rt.ops.delta_prepare(proj, static_cast<int>(col_b_), static_cast<int>(col_b_), shape_, conv_w_->view, Tensor(), Tensor(),
+                                     cache.states.at("conv"), qk, v, beta_decay, batch);
+                rt.ops.channel_scan(qk, v, decay, beta_decay.as<float>(), 2 * shape_.heads, cache.states.at("S"), o, shape_, batch);
+            }
+            rt.ops.delta_gated_norm(o, norm_->view, gate, eps_, gated, shape_.heads, shape_.vdim, gate_act_);
+        }
         Tensor out = rt.ws.buf("mixer_out", rt.dtype, {T, width_});
         rt.ops.linear(gated, w_o_->view, out, nullptr, rt.ws);
         return out;

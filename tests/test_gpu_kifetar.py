@@ -273,6 +273,28 @@ def test_delta_rule_in_registers_equals_the_general_kernel(folders):
         assert_close_f32(got[0][rid], got[1][rid], rid)
 
 
+# (one and two rows of S a wavefront beyond what it holds, one to eight value heads a key head, columns and taps at
+# the kernel's limits; the last three are left to the kernels for any size)
+@pytest.mark.parametrize("H,G,D,V,taps", [(1, 1, 8, 1, 1), (4, 2, 64, 64, 4), (2, 2, 65, 33, 2), (2, 1, 128, 63, 3), (3, 1, 64, 20, 4),
+                                          (4, 1, 33, 64, 1), (8, 1, 32, 64, 4), (5, 1, 17, 7, 2), (8, 1, 33, 16, 2), (1, 1, 16, 65, 2),
+                                          (1, 1, 16, 16, 5)])
+def test_delta_rule_one_token_a_request(tmp_path, H, G, D, V, taps):
+    """Two requests decoded together, token by token, with the whole mixer of a step in one kernel and in four: the
+    states that each step leaves are what the next one reads."""
+    cfg = {"architecture": "Kifetar", "vocab": 140, "width": 48, "norm": {"eps": 1e-5},
+           "layers": [delta(H, G, D, V, taps, ff=None), delta(G, G, 8, 8, 2, ff=32)]}
+    folder = write_model(tmp_path / "step", cfg, 11, torch.float32, std=0.2)
+    reqs = {"a": random_tokens(140, 23, seed=1), "b": random_tokens(140, 20, seed=2)}
+    steps = tail_decode_schedule(reqs, tail=17)
+    c, W = plain.load_model_folder(folder)
+    for one_kernel in (1, 0):
+        lm, _ = load(folder, "float32", steps)
+        lm.set_knob("use_delta_step", one_kernel)
+        got = EngineDriver(lm).run(steps)
+        for rid in reqs:
+            assert_close_f32(got[rid], plain.forward(c, W, reqs[rid]), f"one kernel {one_kernel}, {rid}")
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_state_that_remembers_hundreds_of_tokens(tmp_path, dtype):
     """Decays close to one: what the first tokens wrote into the state still shows 300 tokens
