@@ -212,9 +212,18 @@ Tensor Model::forward(const StepBatch& batch, Runtime& rt) {
         history = rt.ws.buf("depth_history", DType::F32, {history_entries_, T, width});
         rt.ops.cast(h, history_entry(0));
     }
+    // A block's last addition can wait for the norm of the block behind it, or for the final norm, where nothing
+    // else looks at the stream in between.
+    rt.pending_sum = PendingSum{};
+    auto norm_follows = [&](size_t i, size_t layer) {
+        if (S > 1 || rt.after_layer || token_inputs_[layer] || depth_mixes_[layer] || history.defined()) return false;
+        if (i + 1 == spec.order.size()) return final_norm_->params() && !final_norm_->foldable();
+        return !spec.order[i + 1].reinject && blocks_[static_cast<size_t>(spec.order[i + 1].layer)]->takes_pending_sum();
+    };
     for (size_t i = 0; i < spec.order.size(); ++i) {
         const size_t layer = static_cast<size_t>(spec.order[i].layer);
         rt.stream_copy = Tensor();
+        rt.leave_sum = norm_follows(i, layer);
         if (spec.order[i].reinject) {
             if (delta.defined()) rt.ops.norm_step(h, &delta, nullptr, nullptr, nullptr);     // the pending sum first
             delta = Tensor();
@@ -263,7 +272,9 @@ Tensor Model::forward(const StepBatch& batch, Runtime& rt) {
         return logits;
     }
     Tensor normed = rt.ws.buf("final_normed", rt.dtype, {R, width});
-    final_norm_->forward(h, normed, rt, delta.defined() ? &delta : nullptr, batch.logit_rows);
+    const PendingSum last = rt.take_pending_sum();
+    if (last.post) rt.ops.norm_step(h, &last.y, last.post, final_norm_->params(), &normed, batch.logit_rows, last.gain);
+    else final_norm_->forward(h, normed, rt, delta.defined() ? &delta : nullptr, batch.logit_rows);
     head_->forward(normed, logits, rt, embedding_.get());
     rt.mark("head");
     return logits;

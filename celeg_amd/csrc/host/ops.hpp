@@ -12,6 +12,7 @@
 #include <map>
 #include <memory>
 #include <string>
+#include <utility>
 
 #include "batch.hpp"
 #include "blaslt.hpp"
@@ -433,6 +434,13 @@ private:
     void library_product(const Tensor& x, const Tensor& w, const Tensor& out, Workspace& ws);
 };
 
+// An addition h += gain * post(y) that a block has left to the norm behind it, which reads h and writes it anyway.
+struct PendingSum {
+    Tensor y;
+    const Ops::NormParams* post = nullptr;     // null: nothing is pending
+    float gain = 1.f;
+};
+
 // What every part computes with: the stream, the activation dtype, the kernels, a workspace of
 // reusable buffers, and what the parts of the fused path tell each other about the residual
 // stream between kernels.
@@ -458,6 +466,11 @@ struct Runtime {
     bool stream_has_bf16 = false;
     // the stream's rows in the run's dtype, where whoever wrote the stream last left them (undefined: nobody did)
     Tensor stream_copy;
+    // leave_sum: the norm behind the block that runs now takes the block's last addition along (set by the model for every
+    // block; whoever leaves one in pending_sum has seen it set)
+    bool leave_sum = false;
+    PendingSum pending_sum;
+    PendingSum take_pending_sum() { return std::exchange(pending_sum, PendingSum{}); }
     // the step's prologue, left by the runner for the embedding's kernel to take along
     // (defer_prologue); whoever cannot take it along calls flush_prologue() before its own work
     bool defer_prologue = true;

@@ -1764,19 +1764,22 @@ public:
         rt.stream_stat_blocks = 0;
         rt.stream_has_bf16 = false;
         Tensor normed = rt.ws.buf("normed", rt.dtype, {T, width});
-        rt.ops.norm_step(h, delta.defined() ? &delta : nullptr, nullptr, &of(*mixer_norm_), &normed);
+        const PendingSum before = rt.take_pending_sum();
+        if (before.post) rt.ops.norm_step(h, &before.y, before.post, &of(*mixer_norm_), &normed, nullptr, before.gain);
+        else rt.ops.norm_step(h, delta.defined() ? &delta : nullptr, nullptr, &of(*mixer_norm_), &normed);
         Tensor y = mixer_->forward(normed, batch, cache, rt);
         rt.mark("mixer " + mixer_->spec.kind);
-        if (!has_ffn_) {
-            rt.ops.norm_step(h, &y, &of(*mixer_post_), nullptr, nullptr, nullptr, gain_);
-            return Tensor();
+        if (has_ffn_) {
+            rt.ops.norm_step(h, &y, &of(*mixer_post_), &of(*ffn_norm_), &normed, nullptr, gain_);
+            y = ffn_->forward(normed, batch, rt);
         }
-        rt.ops.norm_step(h, &y, &of(*mixer_post_), &of(*ffn_norm_), &normed, nullptr, gain_);
-        y = ffn_->forward(normed, batch, rt);
-        rt.ops.norm_step(h, &y, &of(*ffn_post_), nullptr, nullptr, nullptr, gain_);
-        rt.mark("ffn " + ffn_->spec.kind);
+        const Ops::NormParams& post = of(has_ffn_ ? *ffn_post_ : *mixer_post_);
+        if (rt.leave_sum) rt.pending_sum = PendingSum{y, &post, gain_};
+        else rt.ops.norm_step(h, &y, &post, nullptr, nullptr, nullptr, gain_);
+        if (has_ffn_) rt.mark("ffn " + ffn_->spec.kind);
         return Tensor();
     }
+    bool takes_pending_sum() const override { return true; }
 
 private:
     static const Ops::NormParams& of(const Norm& norm) {

@@ -161,6 +161,8 @@ public:
     // residual streams a row of h holds for this block: h is [T, streams * width]
     virtual int streams() const { return 1; }
     virtual Tensor forward(const Tensor& h, const Tensor& delta, const StepBatch& batch, const LayerCache& cache, Runtime& rt) = 0;
+    // whether forward() makes the addition that the block before it left in rt.pending_sum
+    virtual bool takes_pending_sum() const { return false; }
 };
 
 // ---------------------------------------------------------------------------- registries
