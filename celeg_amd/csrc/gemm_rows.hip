@@ -5,7 +5,7 @@
 // A is bfloat16; behind an RMSNorm it is the bfloat16 copy of the residual stream, W has
 // the norm's weight folded in and scale[m] = rsqrt(mean(x_m^2) + eps) comes from the
 // partial sums of squares that the producer of the stream left.
-// Epilogues: store | 32-bit store | add into the 32-bit residual stream, refresh its
+// Epilogues: store | store of an activation | 32-bit store | add into the 32-bit residual stream, refresh its
 // bfloat16 copy and leave partial sums of squares | SwiGLU of a gate and an up stream |
 // the double-gated short convolution of a B, a C and an x stream for one new token per
 // request, with its state update.
@@ -39,13 +39,14 @@
 // addition into its products with beta = 1 (src/backend/cuda/model/prefill_batched/non_attention.cpp:175-201).
 #include <algorithm>
 
+#include "activations.h"
 #include "common.h"
 #include "gemv_params.h"
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float floatx4_t __attribute__((ext_vector_type(4)));
 
-enum { E_STORE = 0, E_STORE_F32 = 1, E_RESIDUAL = 2, E_SWIGLU = 3, E_CONV = 4 };
+enum { E_STORE = 0, E_STORE_F32 = 1, E_RESIDUAL = 2, E_SWIGLU = 3, E_CONV = 4, E_ACT = 5 };
 #define ROWS_MAX_TAPS 8
 #define ROWS_MAX_STAT_BLOCKS 512
 #define ROWS_MAX_LDS (128 * 1024)
@@ -102,11 +103,14 @@ __device__ __forceinline__ float finish_output(const GemvParams& p, int r, int n
                                                const Early<EPI>& early) {
     float sum[Streams<EPI>::n];
 #pragma unroll
-    for (int s = 0; s < Streams<EPI>::n; ++s) sum[s] = scaled[s] + early.bias[s];
+    for (int s = 0; s < Streams<EPI>::n; ++s) sum[s] = (EPI == E_ACT ? round_bf16(scaled[s]) : scaled[s]) + early.bias[s];
     const size_t o = static_cast<size_t>(r) * p.ldo + n;      // 32-bit outputs: rows one after the other
     const size_t ob = static_cast<size_t>(r) * p.ldo + static_cast<size_t>(n >> 3) * p.out_k8_stride + (n & 7);
     if (EPI == E_STORE) {
         static_cast<bf16*>(p.out)[ob] = from_float<bf16>(sum[0]);
+    } else if (EPI == E_ACT) {
+        // (bias and activation of the product rounded to bfloat16, as where it is a tensor of its own)
+        static_cast<bf16*>(p.out)[ob] = from_float<bf16>(activated(sum[0], p.act, p.act_p[0], p.act_p[1]));
     } else if (EPI == E_STORE_F32) {
         static_cast<float*>(p.out)[o] = sum[0];
         return sum[0];
@@ -461,6 +465,7 @@ extern "C" int celeg_gemm_rows(const GemvParams* params, int epi, hipStream_t st
         case E_RESIDUAL: return launch_epilogue<E_RESIDUAL>(p, stream);
         case E_SWIGLU: return launch_epilogue<E_SWIGLU>(p, stream);
         case E_CONV: return launch_epilogue<E_CONV>(p, stream);
+        case E_ACT: return launch_epilogue<E_ACT>(p, stream);
         default: return static_cast<int>(hipErrorInvalidValue);
     }
 }

@@ -39,13 +39,16 @@ struct GemvParams {
     long long w_row_stride, w_kb_stride;
     // ---- bytes 128..191
     // E_CONV
-    const float* conv_w;    // [N, taps]
+    union {
+        const float* conv_w;    // [N, taps]
+        float act_p[2];         // E_ACT: the activation's numbers
+    };
     const float* conv_b;    // optional [N]
     float* state;           // [slots, taps, N]
     size_t state_slot_stride;
     const int* seq_slot;    // [M]
     int taps;
-    int reserved_;
+    int act;                // E_ACT: which activation (CelegActivation)
     const float* norm_w;    // A_NORM: [K]
     // 32-bit store of an output head: beside the logits, the best (logit, index) of every
     // workgroup's (or wavefront's) columns, packed as packed_logit packs them: [rows, row_best_ld >=

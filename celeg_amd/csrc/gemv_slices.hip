@@ -5,7 +5,7 @@
 // stream, W has the norm's weight folded into its columns by the caller, and scale[m] =
 // rsqrt(mean(x_m^2) + eps) is taken from the partial sums of squares that the producer of
 // the stream left; the scaling is applied to the 32-bit sums at the end.
-// Epilogues: store | 32-bit store | add into the 32-bit residual stream, refresh its
+// Epilogues: store | store of an activation | 32-bit store | add into the 32-bit residual stream, refresh its
 // bfloat16 copy and leave partial sums of squares | SwiGLU of a gate and an up stream |
 // the double-gated short convolution of a B, a C and an x stream for one new token per
 // request, with its state update.
@@ -27,6 +27,7 @@
 // projections y = x W^T src/model/weight_plan.cpp:82-130; the reference fuses the residual
 // addition into its products with beta = 1 (src/backend/cuda/model/prefill_batched/non_attention.cpp:175-201).
 #include "common.h"
+#include "activations.h"
 #include "gemv_params.h"
 
 typedef short bf16x4_t __attribute__((ext_vector_type(4)));
@@ -35,7 +36,7 @@ struct __attribute__((aligned(16))) Frag2 {   // 16 bytes = 8 bfloat16 = two MFM
     bf16x4_t lo, hi;
 };
 
-enum { E_STORE = 0, E_STORE_F32 = 1, E_RESIDUAL = 2, E_SWIGLU = 3, E_CONV = 4 };
+enum { E_STORE = 0, E_STORE_F32 = 1, E_RESIDUAL = 2, E_SWIGLU = 3, E_CONV = 4, E_ACT = 5 };
 #define SLICES_MAX_TAPS 8
 #define SLICES_MAX_STAT_BLOCKS 512   // partial sums of squares a row may come with
 
@@ -259,11 +260,14 @@ void gemv_slices_kernel(const void* const a_, const bf16* const w_, const int* c
 #pragma unroll
             for (int w = 0; w < KW; ++w) sum[s] += red[s][tile_ct][w][src][reg];
         }
-        sum[s] = sum[s] * scale + bias[s];
+        sum[s] = (EPI == E_ACT ? round_bf16(sum[s] * scale) : sum[s] * scale) + bias[s];
     }
     const size_t o = static_cast<size_t>(emc) * p.ldo + en;
     if (EPI == E_STORE) {
         if (e_ok) static_cast<bf16*>(p.out)[o] = from_float<bf16>(sum[0]);
+    } else if (EPI == E_ACT) {
+        // (bias and activation of the product rounded to bfloat16, as where it is a tensor of its own)
+        if (e_ok) static_cast<bf16*>(p.out)[o] = from_float<bf16>(activated(sum[0], p.act, p.act_p[0], p.act_p[1]));
     } else if (EPI == E_STORE_F32) {
         if (e_ok) static_cast<float*>(p.out)[o] = sum[0];
         if (p.row_best) {
@@ -437,6 +441,7 @@ extern "C" int celeg_gemv_slices(const GemvParams* params, int epi, hipStream_t 
         case E_RESIDUAL: return launch_epilogue<E_RESIDUAL>(p, stream);
         case E_SWIGLU: return launch_epilogue<E_SWIGLU>(p, stream);
         case E_CONV: return launch_epilogue<E_CONV>(p, stream);
+        case E_ACT: return launch_epilogue<E_ACT>(p, stream);
         default: return static_cast<int>(hipErrorInvalidValue);
     }
 }

@@ -100,6 +100,12 @@ std::shared_ptr<DeviceTensor> packed_weight(Runtime& rt, const Tensor& w) {
 
 bool qkv_tail_ok(const Runtime& rt, int rows, long long width) { return tiled_step(rt, rows, width); }
 
+// (the two kernels that take the stream's bfloat16 copy; not the older form for very many columns)
+bool activation_ok(const Runtime& rt, int rows, long long width, long long columns) {
+    return rows <= FUSED_MAX_ROWS && !tiled_step(rt, rows, width) && sliced(rt, rows, width) &&
+           (rt.ops.rows_kernel_ok(rows, {width}) || columns <= SLICED_MAX_COLUMNS);
+}
+
 void norm_linear(Runtime& rt, const Tensor& h, const Norm::Foldable& norm, const Tensor& w, const Tensor& out,
                  Epilogue epilogue, const LinearExtras& extras) {
     int blocks = rt.stream_stat_blocks;
@@ -130,6 +136,7 @@ void norm_linear(Runtime& rt, const Tensor& h, const Norm::Foldable& norm, const
     args.n_rows = extras.n_rows;
     args.bias = extras.bias;
     args.conv = extras.conv;
+    args.activation = extras.activation;
     args.row_best = extras.row_best;
     args.row_best_ld = extras.row_best_ld;
     args.row_best_rows = extras.row_best_rows;

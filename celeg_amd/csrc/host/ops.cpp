@@ -632,17 +632,37 @@ bool Ops::few_rows_faster(long long M, long long N, long long K) {
     return false;
 }
 
-bool Ops::few_rows_product(const Tensor& x, const Tensor& w, const Tensor& out) {
+// (args: the epilogue and its operands)
+bool Ops::few_rows_product(const Tensor& x, const Tensor& w, const Tensor& out, FusedArgs args) {
     const long long M = x.shape[0], K = x.shape[1], N = w.shape[0];
     const auto aligned = [](const Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data) & 15) == 0; };
-    if (M > 64 || K <= 0 || K % 8 || !few_rows_faster(M, N, K)) return false;
+    if (M <= 0 || M > 64 || K <= 0 || K % 8 || !few_rows_faster(M, N, K)) return false;
     if (!((M <= 16 && use_sliced) || rows_kernel_ok(static_cast<int>(M), {K}))) return false;
     if (rows_of(x, "x") % 8 || rows_of(x, "x") > 0xfffff || !aligned(x) || !aligned(w)) return false;
-    FusedArgs args;
-    args.epilogue = Epilogue::Store;
     args.plain = true;
     fused_linear(x, w, out, args);
     return true;
+}
+
+static bool bf16_matrices(const Tensor& x, const Tensor& w, const Tensor& out) {
+    return x.dtype == DType::BF16 && w.dtype == DType::BF16 && out.dtype == DType::BF16 && x.ndim == 2 && w.ndim == 2 && out.ndim == 2 &&
+           w.contiguous() && w.shape[1] == x.shape[1] && out.shape[0] == x.shape[0];
+}
+
+bool Ops::linear_swiglu(const Tensor& x, const Tensor& w, const Tensor& out) {
+    if (!bf16_matrices(x, w, out) || w.shape[0] != 2 * out.shape[1]) return false;
+    FusedArgs args;
+    args.epilogue = Epilogue::Swiglu;
+    return few_rows_product(x, w, out, args);
+}
+
+bool Ops::linear_activation(const Tensor& x, const Tensor& w, const Tensor& out, const Tensor* bias, const Activation& activation) {
+    if (!bf16_matrices(x, w, out) || w.shape[0] != out.shape[1]) return false;
+    FusedArgs args;
+    args.epilogue = Epilogue::Activation;
+    if (bias) args.bias = *bias;
+    args.activation = activation;
+    return few_rows_product(x, w, out, args);
 }
 
 // out = x w^T (+ bias).  x [M,K] (rows may be strided), w [N,K], out [M,N] in the dtype of x or
@@ -693,11 +713,12 @@ void Ops::linear(const Tensor& x, const Tensor& w, const Tensor& out, const Tens
     need(x.dtype == DType::BF16 && w.dtype == DType::BF16,
          std::string("linear: unsupported dtypes ") + dtype_name(x.dtype) + " x " + dtype_name(w.dtype));
     if (out.dtype == DType::BF16) {
-        if (!few_rows_product(x, w, out)) library_product(x, w, out, ws);
+        if (bias && linear_activation(x, w, out, bias, Activation{Activation::None})) return;
+        if (bias || !few_rows_product(x, w, out, FusedArgs{})) library_product(x, w, out, ws);
         if (bias) add_bias(out, *bias);
     } else if (out.dtype == DType::F32) {
         Tensor tmp = ws.buf("linear_bf16_out", DType::BF16, {M, N});
-        if (!few_rows_product(x, w, tmp)) library_product(x, w, tmp, ws);
+        if (!few_rows_product(x, w, tmp, FusedArgs{})) library_product(x, w, tmp, ws);
         cast(tmp, out);
         if (bias) add_bias(out, *bias);
     } else {
@@ -1816,6 +1837,12 @@ void Ops::fused_linear(const Tensor& a, const Tensor& w, const Tensor& out, cons
         prm.state_slot_stride = static_cast<size_t>(c.state.stride[0]);
         prm.seq_slot = c.seq_slot;
         prm.taps = static_cast<int>(L);
+    }
+    if (epi == Epilogue::Activation) {
+        need(sliced || streamed, "fused_linear: the activation goes with the kernels for bfloat16 rows");
+        prm.act = args.activation.act;
+        prm.act_p[0] = args.activation.p0;
+        prm.act_p[1] = args.activation.p1;
     }
     last_best_parts = 0;
     last_best_cols = 0;

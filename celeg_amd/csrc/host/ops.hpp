@@ -22,7 +22,14 @@
 
 namespace celeg {
 
-enum class Epilogue : int { Store = 0, StoreF32 = 1, Residual = 2, Swiglu = 3, Conv = 4 };
+enum class Epilogue : int { Store = 0, StoreF32 = 1, Residual = 2, Swiglu = 3, Conv = 4, Activation = 5 };
+
+// An activation behind a product (see Ops::activation_bias)
+struct Activation {
+    enum : int { GeluTanh = 0, Relu2 = 1, None = 2, Bent = 3 };      // (CelegActivation of the kernels)
+    int act = GeluTanh;
+    float p0 = 0.f, p1 = 0.f;
+};
 
 // What follows a q/k/v product of many rows inside its kernel (heads of 64 columns): the norm of
 // query and key heads, their rotation by the rows' positions, and the write of keys and values
@@ -67,6 +74,7 @@ struct FusedArgs {
     Tensor bias;
     Tensor stats_out;             // residual: partial sums of squares of the new rows
     const ConvOperands* conv = nullptr;
+    Activation activation;
     Tensor out_bf16;              // residual: the bfloat16 copy of the stream
     bool packed = false;          // w is [K/32, rows, 32] (pack_weight)
     bool plain = false;           // nothing is fused: counted as a plain product
@@ -192,6 +200,10 @@ public:
                        const int* token_slot, const int* last_tokens, int n);
     void resolve_tokens(int* token_ids, const int* token_slot, const int* last_tokens, int n);
     // products
+    // the whole first half of a feed-forward for few bfloat16 rows, in the product's kernel: silu(gate) * up of x w^T (w: gate
+    // rows, then up rows), and act(x w^T + bias); false (and nothing done) where the separate kernels are to be used
+    bool linear_swiglu(const Tensor& x, const Tensor& w, const Tensor& out);
+    bool linear_activation(const Tensor& x, const Tensor& w, const Tensor& out, const Tensor* bias, const Activation& activation);
     void linear(const Tensor& x, const Tensor& w, const Tensor& out, const Tensor* bias, Workspace& ws);
     // cache-backed
     void short_conv(const Tensor& bcx, const Tensor& weight, const Tensor* bias, const Tensor& state, const Tensor& out,
@@ -430,7 +442,7 @@ private:
     void attention_decode(const Tensor& q, const Tensor& out, int heads, int kv_heads, int head_dim, float scale,
                           int window, const StepBatch& batch, const KVView& kv, int T, Workspace& ws, const FreshKV* fresh = nullptr);
     static bool few_rows_faster(long long M, long long N, long long K);
-    bool few_rows_product(const Tensor& x, const Tensor& w, const Tensor& out);
+    bool few_rows_product(const Tensor& x, const Tensor& w, const Tensor& out, FusedArgs args);
     void library_product(const Tensor& x, const Tensor& w, const Tensor& out, Workspace& ws);
 };
 

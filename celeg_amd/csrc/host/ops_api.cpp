@@ -131,6 +131,7 @@ Epilogue epilogue_of(const std::string& name) {
     if (name == "residual") return Epilogue::Residual;
     if (name == "swiglu") return Epilogue::Swiglu;
     if (name == "conv") return Epilogue::Conv;
+    if (name == "activation") return Epilogue::Activation;
     throw KernelError("unknown epilogue '" + name + "'");
 }
 
@@ -301,6 +302,8 @@ Json call(celeg_ops& h, const std::string& op, const Json& a) {
         args.stats_out = maybe(a, "stats_out").t;
         args.out_bf16 = maybe(a, "out_bf16").t;
         args.packed = a.get_bool("packed", false);
+        args.activation = Activation{static_cast<int>(a.get_int("act", 0)), static_cast<float>(a.get_double("p0", 0.0)),
+                                     static_cast<float>(a.get_double("p1", 0.0))};
         ConvOperands conv;
         if (a.contains("conv") && !a["conv"].is_null()) {
             const Json& c = a["conv"];

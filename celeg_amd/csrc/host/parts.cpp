@@ -810,10 +810,12 @@ public:
     }
     Tensor forward(const Tensor& x, const StepBatch&, Runtime& rt) override {
         const long long T = x.shape[0];
-        Tensor gate_up = rt.ws.buf("ffn_gate_up", rt.dtype, {T, 2 * ff_});
-        rt.ops.linear(x, w_gate_up_->view, gate_up, nullptr, rt.ws);
         Tensor act = rt.ws.buf("ffn_act", rt.dtype, {T, ff_});
-        rt.ops.swiglu(gate_up, act, limit_, alpha_);
+        if (limit_ > 0.f || !rt.ops.linear_swiglu(x, w_gate_up_->view, act)) {
+            Tensor gate_up = rt.ws.buf("ffn_gate_up", rt.dtype, {T, 2 * ff_});
+            rt.ops.linear(x, w_gate_up_->view, gate_up, nullptr, rt.ws);
+            rt.ops.swiglu(gate_up, act, limit_, alpha_);
+        }
         Tensor out = rt.ws.buf("ffn_out", rt.dtype, {T, width_});
         rt.ops.linear(act, w_down_->view, out, nullptr, rt.ws);
         return out;
@@ -2524,7 +2526,7 @@ public:
         const std::string act = s.params.get_string("activation", "gelu_tanh");
         if (act != "gelu_tanh" && act != "relu2" && act != "xielu")
             throw SpecError("mlp: activation is 'gelu_tanh', 'relu2' or 'xielu', not '" + act + "'");
-        act_ = act == "relu2" ? 1 : act == "xielu" ? 3 : 0;
+        act_.act = act == "relu2" ? Activation::Relu2 : act == "xielu" ? Activation::Bent : Activation::GeluTanh;
         bias_ = s.params.get_bool("bias", true);
     }
     bool graph_safe() const override { return true; }
@@ -2534,15 +2536,15 @@ public:
             specs.push_back({"up_bias", vec(ff_)});
             specs.push_back({"down_bias", vec(width_)});
         }
-        if (act_ == 3) specs.push_back({"act", vec(2)});
+        if (act_.act == Activation::Bent) specs.push_back({"act", vec(2)});
         return specs;
     }
     void load(const PartTensors& t, Runtime&) override {
-        if (act_ == 3) {
+        if (act_.act == Activation::Bent) {
             const std::vector<float> a = to_host_floats(get(t, "act")->view);
             auto softplus = [](double z) { return std::max(z, 0.0) + std::log1p(std::exp(-std::fabs(z))); };
-            p0_ = static_cast<float>(softplus(a.at(0)));
-            p1_ = static_cast<float>(0.5 + softplus(a.at(1)));
+            act_.p0 = static_cast<float>(softplus(a.at(0)));
+            act_.p1 = static_cast<float>(0.5 + softplus(a.at(1)));
         }
         w_up_ = get(t, "up");
         w_down_ = get(t, "down");
@@ -2552,8 +2554,11 @@ public:
     Tensor forward(const Tensor& x, const StepBatch&, Runtime& rt) override {
         const long long T = x.shape[0];
         Tensor up = rt.ws.buf("mlp_up", rt.dtype, {T, ff_});
-        rt.ops.linear(x, w_up_->view, up, nullptr, rt.ws);
-        rt.ops.activation_bias(up, b_up_ ? &b_up_->view : nullptr, up, act_, p0_, p1_);
+        const Tensor* bias = b_up_ ? &b_up_->view : nullptr;
+        if (!rt.ops.linear_activation(x, w_up_->view, up, bias, act_)) {
+            rt.ops.linear(x, w_up_->view, up, nullptr, rt.ws);
+            rt.ops.activation_bias(up, bias, up, act_.act, act_.p0, act_.p1);
+        }
         Tensor out = rt.ws.buf("ffn_out", rt.dtype, {T, width_});
         rt.ops.linear(up, w_down_->view, out, b_down_ ? &b_down_->view : nullptr, rt.ws);
         return out;
@@ -2561,17 +2566,24 @@ public:
     // h += ffn(norm(h)) with the norm folded into the first product and the sum into the second
     bool forward_fused(const Tensor& h, const Norm::Foldable& norm, const StepBatch& batch, Runtime& rt) override {
         if (!fused::fused_rows_ok(rt, batch, {width_, ff_}) || w_up_->view.dtype != rt.dtype || w_down_->view.dtype != rt.dtype) return false;
-        Tensor up = rt.ws.buf("mlp_up", rt.dtype, {h.shape[0], ff_});
-        fused::norm_linear(rt, h, norm, w_up_->view, up, Epilogue::Store);
-        rt.ops.activation_bias(up, b_up_ ? &b_up_->view : nullptr, up, act_, p0_, p1_);
+        // few rows: the activation too, in the same kernel
+        const int rows = batch.n_tokens;
+        const bool in_product = fused::activation_ok(rt, rows, width_, ff_);
+        Tensor up = in_product ? fused::operand_rows(rt, "mlp_up_fused", rows, ff_, {width_}) : rt.ws.buf("mlp_up", rt.dtype, {rows, ff_});
+        fused::LinearExtras extras;
+        if (in_product) {
+            extras.activation = act_;
+            if (b_up_) extras.bias = b_up_->view;
+        }
+        fused::norm_linear(rt, h, norm, w_up_->view, up, in_product ? Epilogue::Activation : Epilogue::Store, extras);
+        if (!in_product) rt.ops.activation_bias(up, b_up_ ? &b_up_->view : nullptr, up, act_.act, act_.p0, act_.p1);
         fused::linear_into_stream(rt, up, w_down_->view, h, b_down_ ? &b_down_->view : nullptr);
         return true;
     }
 
 private:
     long long width_, ff_;
-    int act_ = 0;
-    float p0_ = 0.f, p1_ = 0.f;
+    Activation act_;
     bool bias_ = true;
     std::shared_ptr<DeviceTensor> w_up_, w_down_, b_up_, b_down_;
 };

@@ -212,12 +212,15 @@ struct LinearExtras {
     int n_rows = -1;
     Tensor bias;
     const ConvOperands* conv = nullptr;
+    Activation activation;
     const QkvTail* qkv = nullptr;          // steps of many rows: what follows a q/k/v product, inside its kernel
     unsigned long long* row_best = nullptr;   // an output head's 32-bit store: see FusedArgs
     int row_best_ld = 0, row_best_rows = 0;
 };
 // whether norm_linear would take a q/k/v tail for a step of this many rows
 bool qkv_tail_ok(const Runtime& rt, int rows, long long width);
+// whether norm_linear takes an activation along (Epilogue::Activation) for these rows and columns
+bool activation_ok(const Runtime& rt, int rows, long long width, long long columns);
 // out = epilogue(norm(h) w^T), the norm applied while the rows of h are read
 void norm_linear(Runtime& rt, const Tensor& h, const Norm::Foldable& norm, const Tensor& w, const Tensor& out,
                  Epilogue epilogue, const LinearExtras& extras = {});

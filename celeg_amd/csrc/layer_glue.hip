@@ -3,24 +3,10 @@
 // weighted sum over the results of all earlier layers, what a stream takes in before a run of a looped
 // range, and logits bent by a tanh.  All arithmetic is 32-bit; T is the
 // run's dtype of the branch rows.
+#include "activations.h"
 #include "common.h"
 
 namespace {
-
-__device__ __forceinline__ float lg_gelu_tanh(float z) {
-    // 0.5 z (1 + tanh(sqrt(2/pi) (z + 0.044715 z^3)))
-    const float inner = 0.7978845608028654f * (z + 0.044715f * z * z * z);
-    return 0.5f * z * (1.0f + tanhf(inner));
-}
-__device__ __forceinline__ float lg_relu2(float z) {
-    const float r = fmaxf(z, 0.f);
-    return r * r;
-}
-
-// z > 0: right z^2 + z / 2;  z <= 0: left (exp(z) - 1 - z) + z / 2 (both pieces and their slopes meet at 0)
-__device__ __forceinline__ float lg_bent(float z, float right, float left) {
-    return (z > 0.f ? right * z * z : left * (expm1f(z) - z)) + 0.5f * z;
-}
 
 // out = act(x + bias); act 0: gelu (tanh form), 1: square of relu, 2: none, 3: lg_bent with (p0, p1)
 template <typename T>
@@ -31,8 +17,7 @@ __global__ void activation_bias_kernel(const T* __restrict__ x, int ldx, const f
     if (c >= cols) return;
     float z = to_float(x[static_cast<size_t>(t) * ldx + c]);
     if (bias) z += bias[c];
-    const float y = act == 0 ? lg_gelu_tanh(z) : act == 1 ? lg_relu2(z) : act == 3 ? lg_bent(z, p0, p1) : z;
-    out[static_cast<size_t>(t) * ldo + c] = from_float<T>(y);
+    out[static_cast<size_t>(t) * ldo + c] = from_float<T>(activated(z, act, p0, p1));
 }
 
 // The same without a bias on dense rows of the run's dtype that lie one after the other: eight values a thread.
@@ -46,7 +31,7 @@ __global__ __launch_bounds__(256) void activation_dense_kernel(const T* __restri
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         const float z = to_float(in.v[e]);
-        in.v[e] = from_float<T>(act == 0 ? lg_gelu_tanh(z) : act == 1 ? lg_relu2(z) : act == 3 ? lg_bent(z, p0, p1) : z);
+        in.v[e] = from_float<T>(activated(z, act, p0, p1));
     }
     reinterpret_cast<Eight*>(out)[i] = in;
 }

@@ -344,7 +344,7 @@ class HipOps:
 
     def fused_linear(self, a, w, out, *, epilogue="store", norm_weight=None, eps=0.0, stats=None,
                      stat_blocks=0, rows=None, bias=None, stats_out=None, conv=None, n_rows=None,
-                     out_bf16=None, row_best=None):
+                     out_bf16=None, row_best=None, act=(0, 0.0, 0.0)):
         """out = epilogue(prologue(a) w^T) for up to 64 rows, bfloat16 weights (``Ops::fused_linear``).
         ``row_best`` (int64 [>= rows, >= parts], with "store_f32"): receives the best (logit, index) of every
         share of a row's columns; ``last_best_parts`` says how many parts were written.
@@ -357,7 +357,7 @@ class HipOps:
         sums of squares of the new rows, ``last_stat_blocks`` says how many a row), "swiglu"
         (``w`` is [2N, K]: gate rows then up rows), "conv" (``w`` is [3N, K]: B, C, x rows;
         ``conv`` = (taps [N, L], bias or None, state [slots, L, N], seq_slot [M]); one new token
-        per request).  ``w`` with three dimensions is in the layout of ``pack_weight``."""
+        per request), "activation" (``act``: which, and its two numbers).  ``w`` with three dimensions is in the layout of ``pack_weight``."""
         if n_rows is None and rows is not None:
             n_rows = rows.numel()
         conv_json = None
@@ -370,7 +370,7 @@ class HipOps:
                    stat_blocks=int(stat_blocks), rows=_address(rows, "rows"), n_rows=-1 if n_rows is None else int(n_rows),
                    bias=_tensor(bias, "bias"), stats_out=_tensor(stats_out, "stats_out"), conv=conv_json,
                    out_bf16=_tensor(out_bf16, "out_bf16"), packed=w.dim() == 3,
-                   row_best=_address(row_best, "row_best", torch.int64),
+                   act=int(act[0]), p0=float(act[1]), p1=float(act[2]), row_best=_address(row_best, "row_best", torch.int64),
                    row_best_ld=int(row_best.stride(0)) if row_best is not None else 0,
                    row_best_rows=int(row_best.shape[0]) if row_best is not None else 0)
         return out

@@ -52,6 +52,30 @@ def test_plain_rows_store_and_32bit_store_with_bias(ops, M, N, K):
     close(one[0], out32[M // 2], rel=1e-5)
 
 
+# (one to four and five to eight rows in slices of k, sixteen without, rows in tiles; columns beside a tile's)
+@pytest.mark.parametrize("M,N,K", [(1, 3, 8), (4, 1024, 1024), (5, 333, 96), (8, 3072, 1024), (16, 130, 200), (9, 50, 64), (17, 48, 4608),
+                                   (33, 1000, 352), (64, 272, 1024)])
+@pytest.mark.parametrize("act", [(0, 0.0, 0.0), (1, 0.0, 0.0), (2, 0.0, 0.0), (3, 0.7, 0.9)])
+def test_activation_epilogue(ops, M, N, K, act):
+    """The product rounded to bfloat16, the bias added and the activation made in 32-bit, rounded again: each output is
+    within half a step of bfloat16 (2^-8 of it) of the 64-bit one, beside half a step of the product's size times the
+    activation's slope, at most 1 + 2 |z| (1.5 + 2 p0 |z| for the last)."""
+    a, w, b = randn(M, K, seed=1, dtype=BF), randn(N, K, seed=2, scale=K ** -0.5, dtype=BF), randn(N, seed=3)
+    z = a.double() @ w.double().T + b.double()
+    if act[0] == 0:
+        ref = torch.nn.functional.gelu(z, approximate="tanh")
+    elif act[0] == 1:
+        ref = z.clamp_min(0) ** 2
+    elif act[0] == 2:
+        ref = z
+    else:
+        ref = torch.where(z > 0, act[1] * z * z, act[2] * (torch.expm1(z) - z)) + 0.5 * z
+    out = torch.full((M, N), float("nan"), dtype=BF, device=DEV)
+    ops.fused_linear(a, w, out, epilogue="activation", bias=b, act=act)
+    bound = ref.abs() * 2.0 ** -8 + ((z - b).abs() * 2.0 ** -8 + 1e-5) * (1.5 + 2 * z.abs()) + 1e-5
+    assert bool(((out.double() - ref).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("M,N,K", SHAPES)
 @pytest.mark.parametrize("with_stats", [False, True])
 def test_norm_prologue_with_and_without_partial_sums(ops, M, N, K, with_stats):
