@@ -60,7 +60,7 @@ void Sampler::begin(int slot, const GenerationConfig& config, std::shared_ptr<Xo
     rng_[slot] = rng ? std::move(rng) : std::make_shared<XorShift64Star>(config.seed);
     if (config.repetition_penalty > 1.0f && !seen_.ptr()) {
         seen_ = DeviceBuffer(static_cast<size_t>(cap_) * vocab_, true);
-    } else if (seen_.ptr()) {
+    } else if (config.repetition_penalty > 1.0f) {      // (a row without a penalty is never read)
         CELEG_HIP(hipMemsetAsync(seen_.as<uint8_t>() + static_cast<size_t>(slot) * vocab_, 0, static_cast<size_t>(vocab_), rt_.stream));
     }
 }
