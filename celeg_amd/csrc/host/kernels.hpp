@@ -166,6 +166,11 @@ int celeg_sigmoid_attention_fast(int form, const void* q, int ldq, const void* k
                                  int max_tiles, const float* temp, const float* bias, const void* gate, int ldg, void* out,
                                  int ldo, int q_heads, int kv_heads, int head_dim, int page_tokens, int n_layers, int layer,
                                  float scale, int window, hipStream_t stream);
+int celeg_sigmoid_attention_single_parts(int n_tokens, int kv_heads, int window, int context);
+int celeg_sigmoid_attention_single(const void* q, int ldq, const void* k_pool, const void* v_pool, const int* table, int table_stride,
+                                   const int* token_slot, const int* positions, const float* temp, const float* bias, const void* gate,
+                                   int ldg, void* out, int ldo, float* sums, int parts, int n_tokens, int q_heads, int kv_heads,
+                                   int head_dim, int page_tokens, int n_layers, int layer, float scale, int window, hipStream_t stream);
 // delta_rule.hip
 int celeg_delta_prepare(const void* proj, int ld, int dtype, int col_b, int col_a, const float* conv_w, const float* a_log,
                         const float* dt_bias, const float* conv_state, size_t state_stride, const int* positions,

@@ -50,6 +50,7 @@ Model::Model(ModelSpec s) : spec(std::move(s)) {
     graph_safe_ = true;
     std::function<void(const Part*)> visit = [&](const Part* p) {
         graph_safe_ = graph_safe_ && p->graph_safe();
+        short_context_ = std::max(short_context_, p->short_context());
         for (const Part* c : p->children()) visit(c);
     };
     for (const auto& np : named_parts()) visit(np.second);
@@ -451,7 +452,7 @@ bool ModelRunner::graph_applies(const std::vector<StepEntry>& entries) const {
 int ModelRunner::context_bound(const std::vector<StepEntry>& entries) const {
     int longest = 0;
     for (const StepEntry& e : entries) longest = std::max(longest, e.start_pos + static_cast<int>(e.tokens.size()));
-    for (int bound : {4096, 16384, 65536})
+    for (int bound : {model.short_context(), 4096, 16384, 65536})
         if (longest <= bound) return std::min(bound, cache.max_context);
     return cache.max_context;
 }

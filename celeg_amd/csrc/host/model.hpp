@@ -26,6 +26,7 @@ public:
 
     // whether a recorded step of this model may be replayed from a HIP graph
     bool graph_safe() const { return graph_safe_; }
+    int short_context() const { return short_context_; }
     std::vector<std::pair<std::string, Part*>> named_parts();
     // checkpoint tensor name -> what is expected of it
     ExpectedTensors expected_tensors();
@@ -54,6 +55,7 @@ private:
     std::vector<LayerCache> caches_;
     LayerCache embedding_cache_;
     bool bound_ = false, graph_safe_ = false;
+    int short_context_ = 0;
 };
 
 // The step function: runs one batch of (request, its next tokens) through the model, from the

@@ -901,7 +901,7 @@ void Ops::paged_attention(const Tensor& q, const Tensor& out, int heads, int kv_
 // ---------------------------------------------------------------------------- attention with sigmoid weights
 void Ops::sigmoid_attention(const Tensor& q, const Tensor& out, int heads, int kv_heads, int head_dim, float scale, int window,
                             const Tensor* temp, const Tensor* bias, const Tensor* gate, const StepBatch& batch, const KVView& kv,
-                            Workspace&) {
+                            Workspace& ws) {
     dev(q, "q");
     dev(out, "out", q.dtype);
     const long long T = q.shape[0], qw = static_cast<long long>(heads) * head_dim;
@@ -926,17 +926,30 @@ void Ops::sigmoid_attention(const Tensor& q, const Tensor& out, int heads, int k
     if (q.dtype == DType::BF16 && use_sigmoid_mfma && !attention_general && celeg_sigmoid_attention_fast_ok(head_dim) &&
         kv.page_tokens >= 8 && (kv.page_tokens & (kv.page_tokens - 1)) == 0 && ldq % 8 == 0 && head_dim % 8 == 0 &&
         (reinterpret_cast<uintptr_t>(q.data) & 15) == 0) {
-        // portions of prompts: tiles of 64 rows that share their staged keys; single tokens and short
-        // portions: tiles of 16 rows whose key blocks the wavefronts take in turn.  At most one
-        // partly filled tile per request.
-        const int form = sigmoid_rows_form >= 0 ? sigmoid_rows_form : (batch.max_seg_len > 16 ? 1 : 0);
-        const int max_tiles = static_cast<int>(T) / (form == 1 ? 64 : 16) + batch.n_seqs;
+        // single tokens (first in a step): a workgroup per key/value head or part of its keys.  Portions of prompts: tiles of
+        // 64 rows that share their staged keys; short portions: tiles of 16 rows whose key blocks the wavefronts take
+        // in turn (4 requests' single tokens, 16 heads over 8, at 1,100 keys: 9.5 us as such tiles, 6.8 by themselves; 32
+        // requests' 26 and 14).  At most one partly filled tile per request.
         took(batch.decode_only ? Path::AttentionSigmoidDecode : Path::AttentionSigmoidRows);
-        kernel_check(celeg_sigmoid_attention_fast(form, q.data, ldq, kv.k, kv.v, kv.table, kv.table_stride, batch.cu_seqlens, batch.seq_slot,
-                                                  batch.seq_start, batch.n_seqs, max_tiles, temp ? temp->as<float>() : nullptr,
-                                                  bias ? bias->as<float>() : nullptr, gate ? gate->data : nullptr, ldg, out.data,
-                                                  static_cast<int>(qw), heads, kv_heads, head_dim, kv.page_tokens, kv.n_layers, kv.layer,
-                                                  scale, window, stream), "sigmoid attention (bfloat16, matrix cores)");
+        const int single = sigmoid_rows_form < 0 && heads / kv_heads <= 16 ? std::min(batch.single_rows, static_cast<int>(T)) : 0;
+        if (single > 0) {
+            const int parts = celeg_sigmoid_attention_single_parts(single, kv_heads, window, batch.context_hint());
+            float* sums = parts > 1 ? ws.buf("sigmoid_parts", DType::F32, {single, qw, parts}).as<float>() : nullptr;
+            kernel_check(celeg_sigmoid_attention_single(q.data, ldq, kv.k, kv.v, kv.table, kv.table_stride, batch.token_slot, batch.positions,
+                                                        temp ? temp->as<float>() : nullptr, bias ? bias->as<float>() : nullptr,
+                                                        gate ? gate->data : nullptr, ldg, out.data, static_cast<int>(qw), sums, parts, single,
+                                                        heads, kv_heads, head_dim, kv.page_tokens, kv.n_layers, kv.layer, scale, window, stream),
+                         "sigmoid attention (bfloat16, single tokens)");
+        }
+        if (single == T) return;
+        const int form = sigmoid_rows_form >= 0 ? sigmoid_rows_form : (batch.max_seg_len > 16 ? 1 : 0);
+        const int max_tiles = (static_cast<int>(T) - single) / (form == 1 ? 64 : 16) + batch.n_seqs - single;
+        kernel_check(celeg_sigmoid_attention_fast(form, q.data, ldq, kv.k, kv.v, kv.table, kv.table_stride, batch.cu_seqlens + single,
+                                                  batch.seq_slot + single, batch.seq_start + single, batch.n_seqs - single, max_tiles,
+                                                  temp ? temp->as<float>() : nullptr, bias ? bias->as<float>() : nullptr,
+                                                  gate ? gate->data : nullptr, ldg, out.data, static_cast<int>(qw), heads, kv_heads, head_dim,
+                                                  kv.page_tokens, kv.n_layers, kv.layer, scale, window, stream),
+                     "sigmoid attention (bfloat16, matrix cores)");
         return;
     }
     kernel_check(celeg_sigmoid_attention(q.data, rows_of(q, "q"), kv.k, kv.v, dt(q, "q"), kv.table, kv.table_stride, batch.token_slot,

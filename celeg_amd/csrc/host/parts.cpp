@@ -1459,6 +1459,7 @@ public:
             "position", PartSpec::is_part(p["position"]) ? PartSpec::from_json(p["position"], "sigmoid_attention.position") : none);
     }
     bool graph_safe() const override { return true; }
+    int short_context() const override { return 640; }      // (without parts of the keys at or below: 2 us a layer at 128 keys, 0.7 more at 768)
     std::vector<const Part*> children() const override { return {position_.get()}; }
     std::optional<KVNeed> kv_need() const override { return KVNeed{kv_heads_, head_dim_, window_}; }
     WeightSpecs weight_specs() const override {

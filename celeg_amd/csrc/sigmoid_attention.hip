@@ -12,6 +12,8 @@
 // key, all sums in 32-bit in an order that depends on the row's own position only.
 #include "common.h"
 
+#include <algorithm>
+
 namespace {
 
 __device__ __forceinline__ size_t sa_cache_offset(int page, int n_layers, int layer, int kv_heads, int head, int page_tokens,
@@ -410,6 +412,154 @@ __global__ __launch_bounds__(SA_WAVES * CELEG_WAVE) void sigmoid_attention_rows_
     }
 }
 
+// The form for single tokens: a workgroup per (row, key/value head, part of the keys), the query heads that share the head
+// as the rows of the matrix instruction (up to 16), eight wavefronts that take units of 32 keys in turn, over all parts.
+// What bounds such a call is not its bytes in all but what one compute unit draws from them (some 50 GB/s: a window of
+// 1,024 keys of 64, 256 KB, takes 5 us behind 3 of launch and chain) and the chain position -> page -> keys -> weights -> sum.
+// So the keys are dealt to several workgroups, whose sums a second kernel adds (weights are not normalised: the parts just
+// add up), and nothing on the chain goes through LDS: a unit's keys and values travel from the pages straight into
+// the registers of the matrix instruction that takes them.  Row 4 quad + i of score tile kt stands for key
+// 8 quad + 4 kt + i of the unit, so that a lane ends up with the weights of eight keys that lie side by side, the eight that
+// its 16 bytes of a page's values hold.
+struct SaSingle {
+    int n_layers, layer, page_tokens, q_heads, kv_heads, ldg, ldo, window, parts;
+    float scale;
+    const float* temp;
+    const float* bias;
+    const bf16* gate;
+    bf16* out;
+    float* sums;              // [rows, kv_heads, parts, group * D], or null with one part
+};
+
+#define SA_SINGLE_WAVES 8
+template <int D>
+__global__ __launch_bounds__(SA_SINGLE_WAVES * CELEG_WAVE, D <= 64 ? 4 : 2) void sigmoid_attention_single_kernel(
+    const int* __restrict__ positions, const int* __restrict__ token_slot, const int* __restrict__ table, const bf16* __restrict__ q,
+    const bf16* __restrict__ k_pool, const bf16* __restrict__ v_pool, const int table_stride, const int ldq, const SaSingle p) {
+    constexpr int WAVES = SA_SINGLE_WAVES, KS = D / 32, DT = D / 16, UNIT = 32;
+    extern __shared__ __attribute__((aligned(16))) unsigned char sa_lds[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / CELEG_WAVE), lane = threadIdx.x % CELEG_WAVE;
+    const int t = blockIdx.x, kvh = blockIdx.y, group = p.q_heads / p.kv_heads, window = p.window;
+    const int r = lane & 15, quad = lane >> 4;
+    const int pos = positions[t];
+    const int* const pages = table + static_cast<size_t>(token_slot[t]) * table_stride;
+    const int h = kvh * group + min(r, group - 1);             // rows past the last head repeat it (not stored)
+    const int page_shift = 31 - __builtin_clz(p.page_tokens), page_mask = p.page_tokens - 1;
+    const size_t head_stride = static_cast<size_t>(p.page_tokens) * D;
+    const int kb0 = window > 0 ? max(0, pos - window + 1) & ~7 : 0;
+    const int n_units = (pos - kb0) / UNIT + 1, stride = WAVES * p.parts, first = blockIdx.z * WAVES + wave;
+    struct Unit {
+        sa_u32x4 k[2][KS], v[DT];
+    };
+    auto head_of = [&](int page) { return ((static_cast<size_t>(page) * p.n_layers + p.layer) * p.kv_heads + kvh) * head_stride; };
+    auto page_of = [&](int u, int eighth) { return pages[min(kb0 + UNIT * min(u, n_units - 1) + 8 * eighth, pos) >> page_shift]; };
+    auto fetch = [&](int u, int k_page, int v_page, Unit& unit) __attribute__((always_inline)) {
+        const int ub = kb0 + UNIT * u;
+        const size_t k_head = head_of(k_page), v_head = head_of(v_page);
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt) {
+            const int key = min(ub + 8 * (r >> 2) + 4 * kt + (r & 3), pos);
+#pragma unroll
+            for (int st = 0; st < KS; ++st)
+                unit.k[kt][st] = *reinterpret_cast<const sa_u32x4*>(k_pool + k_head + static_cast<size_t>(key & page_mask) * D + 32 * st + 8 * quad);
+        }
+        const int v_from = min(ub + 8 * quad, pos & ~7);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+            unit.v[dt] = *reinterpret_cast<const sa_u32x4*>(v_pool + v_head + static_cast<size_t>(16 * dt + r) * p.page_tokens + (v_from & page_mask));
+    };
+    Unit units[2];
+    const int k_page0 = page_of(first, r >> 2), v_page0 = page_of(first, quad);
+    int k_page = page_of(first + stride, r >> 2), v_page = page_of(first + stride, quad);
+    const bf16* const qrow = q + static_cast<size_t>(t) * ldq + static_cast<size_t>(h) * D;
+    sa_bf16x8 qreg[KS];
+#pragma unroll
+    for (int st = 0; st < KS; ++st) qreg[st] = __builtin_bit_cast(sa_bf16x8, *reinterpret_cast<const sa_u32x4*>(qrow + 32 * st + 8 * quad));
+    const float tau2 = -1.44269504089f * p.scale * (p.temp ? p.temp[h] : 1.0f), beta2 = p.bias ? -1.44269504089f * p.bias[h] : 0.0f;
+    if (first < n_units) fetch(first, k_page0, v_page0, units[0]);
+    sa_f32x4 oacc[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) oacc[dt] = sa_f32x4{0.f, 0.f, 0.f, 0.f};
+    auto take = [&](int u, Unit& unit) __attribute__((always_inline)) {
+        const int ub = kb0 + UNIT * u;
+        if (ub + UNIT - 1 > pos) {           // the last unit: what lies behind the last key may be anything
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) unit.v[dt] = sa_live_values(unit.v[dt], pos - (ub + 8 * quad) + 1);
+        }
+        sa_f32x4 sacc[2];
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt) {
+            sacc[kt] = sa_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int st = 0; st < KS; ++st)
+                sacc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(sa_bf16x8, unit.k[kt][st]), qreg[st], sacc[kt], 0, 0, 0);
+        }
+        sa_bf16x8 w;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int key = ub + 8 * quad + e;
+            const bool seen = key <= pos && (window <= 0 || key > pos - window);
+            w[e] = static_cast<__bf16>(seen ? sa_sigmoid2(fmaf(sacc[e >> 2][e & 3], tau2, beta2)) : 0.0f);
+        }
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+            oacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(sa_bf16x8, unit.v[dt]), w, oacc[dt], 0, 0, 0);
+    };
+    if (first + stride < n_units) fetch(first + stride, k_page, v_page, units[1]);
+    for (int u = first; u < n_units; u += 2 * stride) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int mine = u + e * stride;
+            if (mine >= n_units) break;
+            const bool more = mine + 2 * stride < n_units;
+            if (more) {
+                k_page = page_of(mine + 2 * stride, r >> 2);
+                v_page = page_of(mine + 2 * stride, quad);
+            }
+            take(mine, units[e]);
+            if (more) fetch(mine + 2 * stride, k_page, v_page, units[e]);
+        }
+    }
+    // the wavefronts' sums meet in LDS as [wavefront][head][D] and are added in the order of the wavefronts
+    float* const sums = reinterpret_cast<float*>(sa_lds);
+    if (r < group) {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<sa_f32x4*>(sums + (static_cast<size_t>(wave) * group + r) * D + 16 * dt + 4 * quad) = oacc[dt];
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < group * D; e += WAVES * CELEG_WAVE) {
+        float sum = sums[e];
+#pragma unroll
+        for (int w = 1; w < WAVES; ++w) sum += sums[static_cast<size_t>(w) * group * D + e];
+        if (p.sums) {
+            p.sums[((static_cast<size_t>(t) * p.kv_heads + kvh) * p.parts + blockIdx.z) * group * D + e] = sum;
+            continue;
+        }
+        const int head = kvh * group + e / D;
+        const float g = p.gate ? sa_sigmoid(to_float(p.gate[static_cast<size_t>(t) * p.ldg + head])) : 1.0f;
+        p.out[static_cast<size_t>(t) * p.ldo + static_cast<size_t>(head) * D + e % D] = from_float<bf16>(sum * g);
+    }
+}
+
+// The parts of the kernel above added up, in their order, and gated: a thread a value, all parts asked for at once.
+#define SA_MAX_PARTS 8
+__global__ __launch_bounds__(256) void sigmoid_attention_join_kernel(const float* __restrict__ sums, const bf16* __restrict__ gate,
+                                                                     bf16* __restrict__ out, const int parts, const int ldg, const int ldo,
+                                                                     const int head_dim, const int group, const int q_heads) {
+    const int t = blockIdx.y, e = blockIdx.x * 256 + threadIdx.x, width = q_heads * head_dim;
+    if (e >= width) return;
+    const int gw = group * head_dim, kvh = e / gw, head = e / head_dim;
+    const float* const mine = sums + (static_cast<size_t>(t) * width + static_cast<size_t>(kvh) * gw) * parts + (e - kvh * gw);
+    const float g = gate ? to_float(gate[static_cast<size_t>(t) * ldg + head]) : 0.f;
+    float part[SA_MAX_PARTS];
+#pragma unroll
+    for (int i = 0; i < SA_MAX_PARTS; ++i) part[i] = mine[static_cast<size_t>(min(i, parts - 1)) * gw];
+    float sum = part[0];
+#pragma unroll
+    for (int i = 1; i < SA_MAX_PARTS; ++i) sum += i < parts ? part[i] : 0.f;
+    out[static_cast<size_t>(t) * ldo + e] = from_float<bf16>(gate ? sum * sa_sigmoid(g) : sum);
+}
+
 }  // namespace
 
 extern "C" int celeg_sigmoid_attention(const void* q, int ldq, const void* k_pool, const void* v_pool, int dtype,
@@ -464,5 +614,65 @@ extern "C" int celeg_sigmoid_attention_fast(int form, const void* q, int ldq, co
     else if (head_dim == 96) CELEG_SA_FAST(96);
     else CELEG_SA_FAST(128);
 #undef CELEG_SA_FAST
+    return CELEG_LAUNCH_RESULT();
+}
+
+// ---- single tokens: rows [0, n_tokens), each a request's only row of the step; up to 16 query heads a key/value head, pages
+// of a power of two of at least 8 tokens
+
+// How many workgroups share a key/value head's keys; context: the longest there may be.  With the second kernel a call of
+// 4 or 8 requests over 8 heads takes 6.8 or 8.0 us at 1,100 keys in five parts and 8.2 or 8.9 in three, 8.8 without parts;
+// of 10 requests 9.1 and 9.0; at 768 keys 4 requests 6.3 and 7.0, at 512 keys 6.4 and 5.9, at 128 5.4 and 3.4.  So, beyond 640
+// keys: parts of eight wavefronts with a unit of 32 keys each, up to eight of them, where 320 workgroups hold four at least.
+extern "C" int celeg_sigmoid_attention_single_parts(int n_tokens, int kv_heads, int window, int context) {
+    const int keys = window > 0 ? std::min(window + 7, context) : context;
+    const int useful = (keys + 32 * SA_SINGLE_WAVES - 1) / (32 * SA_SINGLE_WAVES);
+    if (keys <= 640) return 1;
+    const int parts = std::min({useful, SA_MAX_PARTS, 320 / std::max(n_tokens * kv_heads, 1)});
+    return parts < 4 ? 1 : parts;
+}
+
+// sums: parts > 1: 32-bit [n_tokens, q_heads * head_dim, parts]
+extern "C" int celeg_sigmoid_attention_single(const void* q, int ldq, const void* k_pool, const void* v_pool, const int* table,
+                                              int table_stride, const int* token_slot, const int* positions, const float* temp,
+                                              const float* bias, const void* gate, int ldg, void* out, int ldo, float* sums, int parts,
+                                              int n_tokens, int q_heads, int kv_heads, int head_dim, int page_tokens, int n_layers,
+                                              int layer, float scale, int window, hipStream_t stream) {
+    if (n_tokens <= 0) return 0;
+    if (!celeg_sigmoid_attention_fast_ok(head_dim) || q_heads % kv_heads || q_heads / kv_heads > 16 || page_tokens < 8 ||
+        (page_tokens & (page_tokens - 1)) || ldq % 8 || (reinterpret_cast<uintptr_t>(q) & 15) || parts < 1 || parts > SA_MAX_PARTS ||
+        (parts > 1 && !sums))
+        return static_cast<int>(hipErrorInvalidValue);
+    SaSingle p;
+    p.n_layers = n_layers;
+    p.layer = layer;
+    p.page_tokens = page_tokens;
+    p.q_heads = q_heads;
+    p.kv_heads = kv_heads;
+    p.ldg = ldg;
+    p.ldo = ldo;
+    p.window = window;
+    p.parts = parts;
+    p.scale = scale;
+    p.temp = temp;
+    p.bias = bias;
+    p.gate = static_cast<const bf16*>(gate);
+    p.out = static_cast<bf16*>(out);
+    p.sums = parts > 1 ? sums : nullptr;
+    const int group = q_heads / kv_heads;
+    dim3 grid(n_tokens, kv_heads, parts);
+    const size_t lds = static_cast<size_t>(SA_SINGLE_WAVES) * group * head_dim * sizeof(float);
+#define CELEG_SA_SINGLE(D_)                                                                                                          \
+    hipLaunchKernelGGL(sigmoid_attention_single_kernel<D_>, grid, dim3(SA_SINGLE_WAVES * CELEG_WAVE), lds, stream, positions, token_slot, \
+                       table, static_cast<const bf16*>(q), static_cast<const bf16*>(k_pool), static_cast<const bf16*>(v_pool),        \
+                       table_stride, ldq, p)
+    if (head_dim == 32) CELEG_SA_SINGLE(32);
+    else if (head_dim == 64) CELEG_SA_SINGLE(64);
+    else if (head_dim == 96) CELEG_SA_SINGLE(96);
+    else CELEG_SA_SINGLE(128);
+#undef CELEG_SA_SINGLE
+    if (parts > 1)
+        hipLaunchKernelGGL(sigmoid_attention_join_kernel, dim3((q_heads * head_dim + 255) / 256, n_tokens), dim3(256), 0, stream, sums,
+                           static_cast<const bf16*>(gate), static_cast<bf16*>(out), parts, ldg, ldo, head_dim, group, q_heads);
     return CELEG_LAUNCH_RESULT();
 }

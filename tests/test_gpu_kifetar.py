@@ -259,6 +259,28 @@ def test_matrix_core_attention_equals_the_general_kernel(tmp_path, dim):
                 assert rel <= 1.5e-2, f"head size {dim}, form {form}, {rid}: rel rms {rel:.3e}"
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim", [(6, 2, 64), (16, 1, 32), (4, 4, 128), (4, 2, 96)])
+def test_single_tokens_whose_keys_are_dealt_to_several_workgroups(tmp_path, heads, kv_heads, dim):
+    """bfloat16, single tokens on both sides of 640 keys (where the keys of a head go to several workgroups) and of the
+    borders of units of 32 keys and of the windows, beside portions too, against the kernel that scores key by key: the
+    rounding of the weights to bfloat16 apart, the same."""
+    cfg = {"architecture": "Kifetar", "vocab": 150, "width": 64, "norm": {"eps": 1e-5}, "max_context": 4096,
+           "layers": [attention(heads, kv_heads, dim, window=w, rot=rot(dim // 2, 500.0), ff=None) for w in (None, 700, 33, 929)]}
+    folder = write_model(tmp_path / "single", cfg, 37, torch.bfloat16, std=0.1, change=sharp(cfg, 2.0))
+    reqs = {"a": random_tokens(cfg["vocab"], 655, seed=12), "b": random_tokens(cfg["vocab"], 961, seed=13), "c": random_tokens(cfg["vocab"], 40, seed=14)}
+    for steps in (tail_decode_schedule(reqs, tail=30), mixed_schedule(reqs, seed=4, decode_tail=5)):
+        got = {}
+        for form in ("general", -1):
+            lm, _ = load(folder, "bfloat16", steps)
+            if form == "general":
+                lm.set_knob("use_sigmoid_mfma", 0)
+            got[form] = EngineDriver(lm).run(steps)
+        for rid in reqs:
+            a, b = got[-1][rid].double()[-30:], got["general"][rid].double()[-30:]
+            rel = float((a - b).pow(2).mean().sqrt() / b.pow(2).mean().sqrt())
+            assert rel <= 1.5e-2, f"{heads} heads of {dim}, {rid}: rel rms {rel:.3e}"
+
+
 def test_delta_rule_in_registers_equals_the_general_kernel(folders):
     """32-bit: the recurrence with the state in registers against the kernel for any size, same schedule."""
     folder = folders("K4", "float32")
