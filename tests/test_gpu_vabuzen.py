@@ -554,6 +554,39 @@ def test_keys_at_the_windows_edge_and_kept_first_keys(tmp_path, dtype):
         assert lm.paths()["attention_biased_rows"] > 0 and lm.paths()["attention_biased_decode"] > 0
 
 
+@pytest.mark.parametrize("H,G,D,V,mask", [(4, 2, 64, 64, None), (16, 1, 32, 128, (900, 70)), (6, 2, 96, 40, (513, 0)), (3, 3, 128, 96, (700, 3))])
+def test_single_tokens_whose_keys_are_dealt_to_several_workgroups(tmp_path, H, G, D, V, mask):
+    """bfloat16: single tokens at contexts on both sides of 512 keys (where a head's keys go to several workgroups), with
+    windows and kept first keys, behind a long portion and beside none, against the kernel that scores key by key."""
+    from celeg_amd.config import LayerSpec, ModelSpec, PartSpec, RunStep, register_architecture, registered_architectures
+    from celeg_amd.engine import load_model
+    from celeg_amd.weights.safetensors_io import write_safetensors
+    if "VabuzenLongAlone" not in registered_architectures():
+        def build(cfg, shapes):
+            W, rows = cfg["width"], cfg["rows"]
+            block = LayerSpec(PartSpec.from_json(cfg["mixer"]), PartSpec("identity"), PartSpec("none"), PartSpec("identity"), "parallel")
+            return ModelSpec("VabuzenLongAlone", rows, W, 2048, PartSpec("embedding", {"vocab": rows, "width": W}, {"table": "table"}),
+                             (block,), (RunStep(0, None, False),), PartSpec("identity"), PartSpec("hidden", {"width": W}))
+        register_architecture("VabuzenLongAlone", build)
+    T, W_ = 1100, 64
+    t, m, part = attention_case(T, W_, H, G, D, V, D ** -0.5, 0, None, mask, seed=D + V, x_std=1.5)
+    with open(tmp_path / "config.json", "w") as fh:
+        json.dump({"architectures": ["VabuzenLongAlone"], "width": W_, "rows": T, "mixer": part}, fh)
+    write_safetensors(str(tmp_path / "model.safetensors"), {k: v.bfloat16().contiguous() for k, v in t.items()})
+    got = {}
+    cut = (500,) + (1,) * 30 + (541,) + (1,) * 29
+    for general in (True, False):
+        steps = portions_schedule({"x": list(range(T))}, sizes=cut)
+        lm = load_model(str(tmp_path), dtype="bfloat16", device=DEV, page_tokens=16, n_pages=72, max_requests=2, max_context=16 * 72, max_batched_tokens=600)
+        if general:
+            lm.set_knob("use_biased_mfma", 0)
+        got[general] = EngineDriver(lm).run(steps)["x"].double()
+    for first in (500, T - 29):
+        a, b = got[False][first:first + 29], got[True][first:first + 29]
+        rel = float((a - b).pow(2).mean().sqrt() / b.pow(2).mean().sqrt())
+        assert rel <= 1e-2, f"{H} heads of {D} and {V}, mask {mask}, from {first}: rel rms {rel:.3e}"
+
+
 @pytest.mark.parametrize("D,V", [(32, 32), (64, 128), (96, 64), (128, 96)])
 def test_matrix_core_attention_equals_the_general_kernel(tmp_path, D, V):
     """bfloat16: the kernels on the matrix cores against the kernel that scores key by key, on the same
