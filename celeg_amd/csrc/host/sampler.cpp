@@ -117,11 +117,13 @@ void Sampler::launch(const Tensor& logits, const std::vector<int>& slots) {
     std::vector<uint32_t> used(static_cast<size_t>(7 * R));
     std::memcpy(used.data(), f, static_cast<size_t>(4 * R) * 4);
     std::memcpy(used.data() + 4 * R, iv, static_cast<size_t>(3 * R) * 4);
-    if (used != uploaded_) {
+    if (all_greedy && used != uploaded_) {
         CELEG_HIP(hipMemcpyAsync(params_dev_.ptr(), params_[turn].ptr(), cap * 7 * 4, hipMemcpyHostToDevice, rt_.stream));
         uploaded_ = used;
     }
-    const float* fdev = params_dev_.as<float>();
+    // Sampled rows bring a new draw with every step: their kernel reads it from the turn's pinned buffer itself (28
+    // bytes a row, one trip over the bus), where a copy ahead of it is 4 us of the stream's time a step.
+    const float* fdev = all_greedy ? params_dev_.as<float>() : f;
     const int* idev = reinterpret_cast<const int*>(fdev + cap * 4);
     // the kernels write the tokens straight into the turn's pinned buffer (memory of the host that
     // the device can address): no copy behind them, the event tells when they are there

@@ -62,45 +62,18 @@ __device__ __forceinline__ float key_score(uint32_t key) {      // the inverse o
 
 // The top_k scores of a row (score = penalised logit / temperature) by (score desc, id
 // asc), left unordered in cand_score / cand_id [0, top_k).  All threads of the workgroup
-// call it.  KPT > 0: the row's keys are held in registers, KPT a thread, element
-// tid + SAMPLE_THREADS * j in place j (vocab <= SAMPLE_THREADS * KPT); KPT == 0: every pass
-// walks the row in memory.
-template <int KPT>
+// call it.  Every pass walks the row in memory: this is the way for rows that the two below cannot take (more
+// than 131,072 logits, thousands of equal ones).  (Forms of it with the row's keys in registers made the kernel 387 KB of code, for
+// whose sake the other ways' scalar registers were spilled.)
 __device__ __forceinline__ void top_k_candidates(
     const float* __restrict__ row, const uint8_t* __restrict__ seen, float penalty, float temperature,
     int vocab, int top_k, unsigned int* hist, unsigned int* sel, int* running, float* cand_score,
     int* cand_id) {
     const int tid = threadIdx.x;
     const int lane = tid & (CELEG_WAVE - 1);
-    constexpr int NK = KPT > 0 ? KPT : 1;
-    uint32_t keys[NK];
-    if (KPT > 0) {
-        const bool pen = seen && penalty > 1.0f;
-        float v[NK];
-        unsigned char sn[NK];
-#pragma unroll
-        for (int j = 0; j < NK; ++j) {
-            const int i = min(tid + SAMPLE_THREADS * j, vocab - 1);      // clamped, masked below
-            v[j] = row[i];
-            sn[j] = pen ? seen[i] : 0;
-        }
-#pragma unroll
-        for (int j = 0; j < NK; ++j) {
-            float x = v[j];
-            if (sn[j]) x = x >= 0.0f ? x / penalty : x * penalty;
-            keys[j] = tid + SAMPLE_THREADS * j < vocab ? order_key(x / temperature) : 0u;
-        }
-    }
     // f(key, index) for this thread's share of the row
     auto walk = [&](auto f) {
-        if (KPT > 0) {
-#pragma unroll
-            for (int j = 0; j < NK; ++j)
-                if (tid + SAMPLE_THREADS * j < vocab) f(keys[j], tid + SAMPLE_THREADS * j);
-        } else {
-            for_each_logit(row, seen, penalty, vocab, tid,
-                           [&](float x, int i) { f(order_key(x / temperature), i); });
-        }
+        for_each_logit(row, seen, penalty, vocab, tid, [&](float x, int i) { f(order_key(x / temperature), i); });
     };
     // One counting pass: bins of bin_of(key, index) >= 0.  The counts go to
     // SAMPLE_HIST_COPIES copies of the 256 bins, a lane using copy lane % copies: scores
@@ -254,13 +227,17 @@ __device__ __forceinline__ void top_k_candidates(
 // Five workgroup barriers instead of about forty, and two divisions per gathered logit
 // instead of per logit.
 #define SAMPLE_RANK_CAP 2048
-__device__ __forceinline__ void rank_gathered(const float* __restrict__ row, const uint8_t* __restrict__ seen, bool pen,
-                                              float penalty, float temperature, int top_k, int n, uint2* gathered,
-                                              float* cand_score, int* cand_id);
+__device__ __forceinline__ void rank_gathered(int top_k, int n, const unsigned long long* gathered, unsigned int* counts, float* cand_score,
+                                              int* cand_id);
+// a logit's score as the reference computes it
+__device__ __forceinline__ float exact_score(float x, bool marked, float penalty, float temperature) {
+    if (marked) x = x >= 0.0f ? x / penalty : x * penalty;
+    return x / temperature;
+}
 template <int KPT>
 __device__ __forceinline__ bool top_k_ranked(
     const float* __restrict__ row, const uint8_t* __restrict__ seen, float penalty, float temperature,
-    int vocab, int top_k, uint32_t* wave_bound, uint2* gathered, unsigned int* sel, float* cand_score,
+    int vocab, int top_k, uint32_t* wave_bound, unsigned long long* gathered, unsigned int* sel, unsigned int* counts, float* cand_score,
     int* cand_id) {
     const int tid = threadIdx.x;
     const int lane = tid & (CELEG_WAVE - 1), wave = tid / CELEG_WAVE;
@@ -330,45 +307,67 @@ __device__ __forceinline__ bool top_k_ranked(
     for (int j = 0; j < KPT; ++j)
         if (index_of(j) < vocab && keys[j] >= lower) {
             const unsigned int p = atomicAdd(&sel[1], 1u);
-            if (p < SAMPLE_RANK_CAP) gathered[p].y = static_cast<unsigned>(index_of(j));
+            if (p < SAMPLE_RANK_CAP) gathered[p] = static_cast<unsigned>(index_of(j));
         }
     __syncthreads();
     const int n = static_cast<int>(sel[1]);
     if (n > SAMPLE_RANK_CAP) return false;       // the same for every thread
-    rank_gathered(row, seen, pen, penalty, temperature, top_k, n, gathered, cand_score, cand_id);
+    for (int e = tid; e < n; e += SAMPLE_THREADS) {
+        const int id = static_cast<int>(gathered[e]);
+        gathered[e] = packed_logit(exact_score(row[id], pen && seen[id], penalty, temperature), id);
+    }
+    __syncthreads();
+    rank_gathered(top_k, n, gathered, counts, cand_score, cand_id);
     return true;
 }
 
-// The last steps of the ranking: the exact scores of the n gathered logits (gathered[e].y: their
-// indices), as the reference computes them, and every one's place among them; the first top_k places
-// go to cand_score / cand_id.  All threads call it; n is the same for all.
-__device__ __forceinline__ void rank_gathered(const float* __restrict__ row, const uint8_t* __restrict__ seen, bool pen,
-                                              float penalty, float temperature, int top_k, int n, uint2* gathered,
-                                              float* cand_score, int* cand_id) {
-    const int tid = threadIdx.x;
-    for (int e = tid; e < n; e += SAMPLE_THREADS) {
-        const int id = static_cast<int>(gathered[e].y);
-        float x = row[id];
-        if (pen && seen[id]) x = x >= 0.0f ? x / penalty : x * penalty;
-        gathered[e].x = __float_as_uint(x / temperature);
-    }
-    __syncthreads();
-    for (int e = tid; e < n; e += SAMPLE_THREADS) {
-        const uint2 mine = gathered[e];
-        const float score = __uint_as_float(mine.x);
-        const int id = static_cast<int>(mine.y);
-        int place = 0;
-        for (int u0 = 0; u0 < n; u0 += 16) {            // sixteen reads from LDS under way at a time
-            uint2 other[16];
+// The last step of the ranking: the place of every gathered (score, index), packed as packed_logit packs them, among the
+// others; the first top_k places go to cand_score / cand_id.  All threads call it; n is the same for all.  A
+// hundred are gathered as a rule.  A wavefront takes 64 of them, one a lane, and counts which of a share of
+// all n come before its own: the others travel from a lane to all by a scalar register, four instructions each and
+// no trip to LDS.  counts [SAMPLE_THREADS] holds the shares' counts.  (A thread for each of them, a
+// comparison of scores and one of indices behind a branch: 7 of the 14 us of a row of 65,536 logits and top_k 50; eight
+// lanes for each, the others read from LDS: 1.4 us there and 6.6 at top_k 128, what LDS takes to hand 16 wavefronts all of them.)
+__device__ __forceinline__ void rank_gathered(int top_k, int n, const unsigned long long* gathered, unsigned int* counts, float* cand_score,
+                                              int* cand_id) {
+    constexpr int WAVES = SAMPLE_THREADS / CELEG_WAVE;
+    const int lane = threadIdx.x % CELEG_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / CELEG_WAVE);
+    for (int first = 0; first < n; first += SAMPLE_THREADS) {          // (once, up to 1,024 gathered)
+        const int here = min(n - first, SAMPLE_THREADS);
+        const int log_groups = here > CELEG_WAVE ? 32 - __builtin_clz((here - 1) / CELEG_WAVE) : 0;      // groups of 64: a power of two
+        const int groups = 1 << log_groups, shares = WAVES >> log_groups;
+        const int group = wave & (groups - 1), share = wave >> log_groups;
+        const unsigned long long mine = gathered[first + min(group * CELEG_WAVE + lane, here - 1)];
+        // (shares are of 8 at least, so that the loop below can count 8 at a time: what lies behind the last one comes as 0)
+        const int per = (((n + shares - 1) >> (__builtin_ctz(WAVES) - log_groups)) + 7) & ~7, lo = share * per, hi = min(lo + per, n);
+        unsigned int before = 0u;
+        for (int u0 = lo; u0 < hi; u0 += CELEG_WAVE) {
+            const int at = u0 + lane;
+            const unsigned long long other = at < hi ? gathered[at] : 0ull;
+            const int low = static_cast<int>(other), high = static_cast<int>(other >> 32);
+            for (int j = 0; j < min(hi - u0, CELEG_WAVE); j += 8) {
 #pragma unroll
-            for (int j = 0; j < 16; ++j) other[j] = gathered[min(u0 + j, n - 1)];
-#pragma unroll
-            for (int j = 0; j < 16; ++j)
-                place += (u0 + j < n && better(__uint_as_float(other[j].x), static_cast<int>(other[j].y), score, id)) ? 1 : 0;
+                for (int i = 0; i < 8; ++i) {
+                    const unsigned long long o = (static_cast<unsigned long long>(static_cast<unsigned>(__builtin_amdgcn_readlane(high, j + i))) << 32) |
+                                                 static_cast<unsigned>(__builtin_amdgcn_readlane(low, j + i));
+                    before += o > mine ? 1u : 0u;
+                }
+            }
         }
-        if (place < top_k) { cand_score[place] = score; cand_id[place] = id; }
+        counts[threadIdx.x] = before;
+        __syncthreads();
+        if (static_cast<int>(threadIdx.x) < here) {
+            const int g = threadIdx.x / CELEG_WAVE;
+            unsigned int place = 0u;
+            for (int sh = 0; sh < shares; ++sh) place += counts[(sh * groups + g) * CELEG_WAVE + lane];
+            if (place < static_cast<unsigned>(top_k)) {
+                const unsigned long long own = gathered[first + threadIdx.x];
+                cand_score[place] = key_score(static_cast<uint32_t>(own >> 32));
+                cand_id[place] = packed_logit_index(own);
+            }
+        }
+        __syncthreads();
     }
-    __syncthreads();
 }
 
 // The same candidates without reading the row: an output head left, beside the logits, the best
@@ -388,7 +387,7 @@ __device__ __forceinline__ void rank_gathered(const float* __restrict__ row, con
 #define SAMPLE_PART_LIST 1024
 __device__ __forceinline__ bool top_k_from_parts(
     const float* __restrict__ row, const uint8_t* __restrict__ seen, float penalty, float temperature, int vocab, int top_k,
-    const unsigned long long* __restrict__ best, int n_parts, int cols, uint32_t* wave_bound, uint2* gathered,
+    const unsigned long long* __restrict__ best, int n_parts, int cols, uint32_t* wave_bound, unsigned long long* gathered,
     unsigned int* sel, unsigned int* part_list, float* cand_score, int* cand_id) {
     const int tid = threadIdx.x;
     const int lane = tid & (CELEG_WAVE - 1), wave = tid / CELEG_WAVE;
@@ -426,12 +425,12 @@ __device__ __forceinline__ bool top_k_from_parts(
 #pragma unroll
     for (int w = 1; w < SAMPLE_THREADS / CELEG_WAVE; ++w) lower_max = min(lower_max, wave_bound[w]);
     if (lower_max == 0u) return false;           // (some wavefront has fewer than c parts: nothing is bounded)
-    if (my_max >= lower_max) {
-        // this thread's best logit is one of top_k different logits at least: its penalised value
-        const int index = packed_logit_index(my_best);
-        const float x = stand_in(key_score(my_max), pen ? seen[index] : 0u);
-        atomicMin(&sel[2], order_key(x));
-    }
+    // a thread whose best reaches the bound holds one of top_k different logits at least: the penalised value, its
+    // wavefront's smallest by one atomic
+    uint32_t penalised = 0xffffffffu;
+    if (my_max >= lower_max) penalised = order_key(stand_in(key_score(my_max), pen ? seen[packed_logit_index(my_best)] : 0u));
+    penalised = ~group_max_u32<CELEG_WAVE>(~penalised);
+    if (lane == 0 && penalised != 0xffffffffu) atomicMin(&sel[2], penalised);
     __syncthreads();
     const uint32_t lowest = sel[2];
     const uint32_t lower = lowest > 8u ? lowest - 8u : 0u;
@@ -447,17 +446,18 @@ __device__ __forceinline__ bool top_k_from_parts(
     for (int e = tid; e < n_listed * cols; e += SAMPLE_THREADS) {
         const int i = static_cast<int>(part_list[e / cols]) * cols + e % cols;
         if (i < vocab) {
-            const float x = stand_in(row[i], pen ? seen[i] : 0u);
-            if (order_key(x) >= lower) {
+            const float x = row[i];
+            const bool marked = pen && seen[i];
+            if (order_key(stand_in(x, marked)) >= lower) {
                 const unsigned int p = atomicAdd(&sel[1], 1u);
-                if (p < SAMPLE_RANK_CAP) gathered[p].y = static_cast<unsigned>(i);
+                if (p < SAMPLE_RANK_CAP) gathered[p] = packed_logit(exact_score(x, marked, penalty, temperature), i);
             }
         }
     }
     __syncthreads();
     const int n = static_cast<int>(sel[1]);
     if (n > SAMPLE_RANK_CAP || n < top_k) return false;
-    rank_gathered(row, seen, pen, penalty, temperature, top_k, n, gathered, cand_score, cand_id);
+    rank_gathered(top_k, n, gathered, part_list, cand_score, cand_id);
     return true;
 }
 
@@ -487,10 +487,11 @@ __device__ __forceinline__ int choose_among(float* cand_score, int* cand_id, int
         }
     }
 
-    // ---- softmax, top-p prefix and the walk.  The sums run over the candidates one after
-    // the other, in the reference's order: every lane runs the same loops over the values in
-    // LDS (reads of one address by all lanes, asked for ahead of the additions that need them;
-    // a value handed from lane to lane for every addition cost ten times the addition).
+    // ---- softmax, top-p prefix and the walk.  The sums run over the candidates one after the other, in the
+    // reference's order: every lane runs the same additions over the values in LDS (reads of one address by all
+    // lanes), sixteen of them asked for together ahead of the additions, with no branch between these (a loop
+    // that ends where its sum does waits for LDS once a candidate).  (A value handed from lane to lane for every
+    // addition cost ten times the addition.)
     const float maximum = cand_score[0];
     const int id0 = cand_id[lane], id1 = cand_id[lane + 64];
     const float e0 = expf(cand_score[lane] - maximum), e1 = expf(cand_score[lane + 64] - maximum);
@@ -504,30 +505,54 @@ __device__ __forceinline__ int choose_among(float* cand_score, int* cand_id, int
     prob[lane] = e0;
     prob[lane + 64] = e1;
     wave_sync();
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    // f(value) for the first `count` places in turn, and for those behind them, which hold zeros, up to a multiple of
+    // sixteen; until done() after sixteen of them (the same in every lane)
+    auto in_order = [&](int count, auto f, auto done) {
+        for (int i0 = 0; i0 < count; i0 += 16) {
+            f4 v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = *reinterpret_cast<const f4*>(prob + i0 + 4 * j);
+#pragma unroll
+            for (int j = 0; j < 16; ++j) f(v[j >> 2][j & 3]);
+            if (__builtin_amdgcn_readfirstlane(done() ? 1 : 0)) break;
+        }
+    };
+    const auto never = [] { return false; };
     float total = 0.f;
-    for (int i = 0; i < top_k; ++i) total += prob[i];
+    in_order(top_k, [&](float x) { total += x; }, never);       // (behind top_k: exp(-inf))
     wave_sync();
     prob[lane] = e0 / total;
     prob[lane + 64] = e1 / total;
     wave_sync();
+    // (No probability is negative, or all of them are NaN, so the running sums only rise: how many are below a
+    // bound says where the first one is that is not.)
     int active = top_k;
     if (top_p < 1.0f) {
+        // the shortest prefix whose sum is not below top_p; the probabilities behind it become zeros
         float cumulative = 0.f;
-        active = 0;
-        do {
-            cumulative += prob[active++];
-        } while (active < top_k && cumulative < top_p);
+        int below = 0;
+        in_order(top_k, [&](float x) {
+            cumulative += x;
+            below += cumulative < top_p ? 1 : 0;
+        }, [&] { return !(cumulative < top_p); });
+        active = __builtin_amdgcn_readfirstlane(min(below + 1, top_k));
+        wave_sync();
+        if (lane >= active) prob[lane] = 0.f;
+        if (lane + 64 >= active) prob[lane + 64] = 0.f;
+        wave_sync();
         total = 0.f;
-        for (int i = 0; i < active; ++i) total += prob[i];
+        in_order(active, [&](float x) { total += x; }, never);
     } else {
         total = 1.0f;
     }
     float target = u * total;
-    int chosen_at = active - 1;
-    for (int i = 0; i < active; ++i) {
-        target -= prob[i];
-        if (target <= 0.0f) { chosen_at = i; break; }
-    }
+    int left_over = 0;
+    in_order(active, [&](float x) {
+        target -= x;
+        left_over += target <= 0.0f ? 0 : 1;
+    }, [&] { return target <= 0.0f; });
+    const int chosen_at = min(left_over, active - 1);
     return __shfl(chosen_at < 64 ? id0 : id1, chosen_at & 63, CELEG_WAVE);
 }
 
@@ -535,19 +560,23 @@ __device__ __forceinline__ int choose_among(float* cand_score, int* cand_id, int
 // token is given out, nothing is chosen), seen_row or -1, slot or -1}; the token also goes to last_tokens[slot] (if given and slot >= 0), where the
 // next step can take it from without the host in between, and is marked as seen in the row's
 // seen_row (if any): the step that feeds it back need not mark it.
+// PARTS: the head left the best of every part of the columns (else best is null).  Two kernels, because the one that holds
+// a row in registers is large (its scalar registers spill) and slows the other down where both are one.
+template <bool PARTS>
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     const float* __restrict__ logits, int ld, int vocab, const float* __restrict__ fparams,
     const int* __restrict__ iparams, uint8_t* __restrict__ seen_all, size_t seen_stride,
     int* __restrict__ out_tokens, int* __restrict__ last_tokens, const unsigned long long* __restrict__ best, int best_ld,
     int best_parts, int best_cols) {
-    __shared__ unsigned int part_list[SAMPLE_PART_LIST];
+    __shared__ unsigned int part_list[SAMPLE_PART_LIST];          // or the ranking's counts
+    static_assert(SAMPLE_PART_LIST >= SAMPLE_THREADS, "a count a thread");
     __shared__ float s_val[SAMPLE_THREADS / CELEG_WAVE];
     __shared__ int s_idx[SAMPLE_THREADS / CELEG_WAVE];
     __shared__ __attribute__((aligned(16))) unsigned int hist[256 * SAMPLE_HIST_COPIES];   // or SAMPLE_RANK_CAP gathered (key, id)
     __shared__ uint32_t maxes[SAMPLE_THREADS / CELEG_WAVE];       // per wavefront: the bound it offers
     __shared__ unsigned int sel[3];       // prefix, remaining, size of the last bin
     __shared__ int running[2];
-    __shared__ float cand_score[SAMPLE_MAX_K];
+    __shared__ __attribute__((aligned(16))) float cand_score[SAMPLE_MAX_K];
     __shared__ int cand_id[SAMPLE_MAX_K];
 
     const int r = blockIdx.x;
@@ -604,30 +633,20 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     }
 
     top_k = min(min(top_k, vocab), SAMPLE_MAX_K);
-    // the scores of the row are turned into keys once and kept in registers (up to 128 a
-    // thread); larger vocabularies walk the row again for every pass
-    static_assert(sizeof(hist) >= SAMPLE_RANK_CAP * sizeof(uint2), "the gathered scores share the histograms' room");
-    uint2* gathered = reinterpret_cast<uint2*>(hist);
+    static_assert(sizeof(hist) >= SAMPLE_RANK_CAP * sizeof(unsigned long long), "the gathered scores share the histograms' room");
+    unsigned long long* gathered = reinterpret_cast<unsigned long long*>(hist);
     bool sorted = false;
-    if (best) {
-        // what the output head left beside the logits: the candidates without reading the row
+    if constexpr (PARTS) {
+        // the candidates without reading the row
         sorted = top_k_from_parts(row, seen, penalty, temperature, vocab, top_k, best + static_cast<size_t>(r) * best_ld, best_parts, best_cols, maxes,
                                   gathered, sel, part_list, cand_score, cand_id);
         __syncthreads();        // (before what follows reuses the counters)
+    } else if (vocab <= SAMPLE_THREADS * 64) {
+        sorted = top_k_ranked<64>(row, seen, penalty, temperature, vocab, top_k, maxes, gathered, sel, part_list, cand_score, cand_id);
+    } else if (vocab <= SAMPLE_THREADS * 128) {
+        sorted = top_k_ranked<128>(row, seen, penalty, temperature, vocab, top_k, maxes, gathered, sel, part_list, cand_score, cand_id);
     }
-    if (sorted) {
-    } else if (vocab <= SAMPLE_THREADS * 64)
-        sorted = top_k_ranked<64>(row, seen, penalty, temperature, vocab, top_k, maxes, gathered, sel, cand_score, cand_id);
-    else if (vocab <= SAMPLE_THREADS * 128)
-        sorted = top_k_ranked<128>(row, seen, penalty, temperature, vocab, top_k, maxes, gathered, sel, cand_score, cand_id);
-    if (!sorted) {
-        if (vocab <= SAMPLE_THREADS * 64)
-            top_k_candidates<64>(row, seen, penalty, temperature, vocab, top_k, hist, sel, running, cand_score, cand_id);
-        else if (vocab <= SAMPLE_THREADS * 128)
-            top_k_candidates<128>(row, seen, penalty, temperature, vocab, top_k, hist, sel, running, cand_score, cand_id);
-        else
-            top_k_candidates<0>(row, seen, penalty, temperature, vocab, top_k, hist, sel, running, cand_score, cand_id);
-    }
+    if (!sorted) top_k_candidates(row, seen, penalty, temperature, vocab, top_k, hist, sel, running, cand_score, cand_id);
     if (tid >= top_k && tid < SAMPLE_MAX_K) { cand_score[tid] = -INFINITY; cand_id[tid] = 0x7fffffff; }
     __syncthreads();
     if (wave != 0) return;         // one wavefront does the rest: no workgroup barriers from here
@@ -767,7 +786,7 @@ extern "C" int celeg_sample(const float* logits, int ld, int rows, int vocab,
     if (best && (best_ld < best_parts || best_parts <= 0 || best_cols <= 0 ||
                  static_cast<long long>(best_parts) * best_cols < vocab))
         return static_cast<int>(hipErrorInvalidValue);
-    hipLaunchKernelGGL(sample_kernel, dim3(rows), dim3(SAMPLE_THREADS), 0, stream, logits, ld,
+    hipLaunchKernelGGL((best ? sample_kernel<true> : sample_kernel<false>), dim3(rows), dim3(SAMPLE_THREADS), 0, stream, logits, ld,
                        vocab, fparams, iparams, seen, seen_stride, out_tokens, last_tokens, best, best_ld, best_parts,
                        best_cols);
     return CELEG_LAUNCH_RESULT();
