@@ -158,10 +158,10 @@ __global__ __launch_bounds__(CELEG_WAVE) void delta_scan_kernel(
 // k1.k2, k1.q1, k1.q2, k2.q2 (1: the row, 2: the next one).  One wavefront per (row, head).
 __global__ __launch_bounds__(CELEG_WAVE) void delta_pairs_kernel(const float* __restrict__ qk, const int* __restrict__ token_seq,
                                                                  const int* __restrict__ cu_seqlens, float* __restrict__ pairs, int G,
-                                                                 int D) {
+                                                                 int D, int below) {
     const int t = blockIdx.x, g = blockIdx.y, lane = threadIdx.x;
     const int seq = token_seq[t], row0 = cu_seqlens[seq], end = cu_seqlens[seq + 1];
-    if (((t - row0) & 1) || t + 1 >= end) return;
+    if (((t - row0) & 1) || t + 1 >= end || end - row0 >= below) return;
     const float* q1 = qk + static_cast<size_t>(t) * 2 * G * D + static_cast<size_t>(g) * D;
     const float* k1 = q1 + static_cast<size_t>(G) * D;
     const float* q2 = q1 + static_cast<size_t>(2) * G * D;
@@ -197,7 +197,7 @@ template <int DL, int DPL>
 __global__ __launch_bounds__(CELEG_WAVE) void delta_scan_reg_kernel(
     const float* __restrict__ qk, const float* __restrict__ v, const float* __restrict__ beta_decay, float* __restrict__ state,
     size_t state_stride, const int* __restrict__ cu_seqlens, const int* __restrict__ seq_slot, float* __restrict__ out,
-    const float* __restrict__ pairs, int G, int H, int V) {
+    const float* __restrict__ pairs, int G, int H, int V, int below) {
     constexpr int D = DPL * DL, NC = DPL / 4, CPW = CELEG_WAVE / DL, TB = D <= 64 ? 16 : 8, ROW = 2 * D, PER_LANE = TB * ROW / CELEG_WAVE;
     typedef float f4 __attribute__((ext_vector_type(4)));
     __shared__ __attribute__((aligned(16))) float qk_s[TB * ROW];
@@ -209,7 +209,7 @@ __global__ __launch_bounds__(CELEG_WAVE) void delta_scan_reg_kernel(
     const int jj = live ? j : V - 1;          // idle lanes repeat the last column and store nothing
     const int g = h / (H / G);
     const int row0 = cu_seqlens[s], n = cu_seqlens[s + 1] - row0;
-    if (n <= 0) return;
+    if (n <= 0 || n >= below) return;         // (longer portions: delta_chunks.hip)
     float* mine = state + static_cast<size_t>(seq_slot[s]) * state_stride + static_cast<size_t>(h) * D * V;
     float S[DPL];
 #pragma unroll
@@ -570,9 +570,10 @@ extern "C" int celeg_delta_conv_state(const void* proj, int ld, int dtype, float
     return CELEG_LAUNCH_RESULT();
 }
 
+// below: requests of that many rows of the step and more are left out (the chunked form's); the kernel for any size takes all
 extern "C" int celeg_delta_scan(const float* qk, const float* v, const float* beta_decay, float* state, size_t state_stride,
                                 const int* cu_seqlens, const int* seq_slot, float* out, int n_seqs, int G, int H, int D, int V,
-                                int general, const int* token_seq, float* pairs, int n_tokens, hipStream_t stream) {
+                                int general, const int* token_seq, float* pairs, int n_tokens, int below, hipStream_t stream) {
     if (n_seqs <= 0) return 0;
     if (H % G) return static_cast<int>(hipErrorInvalidValue);
     if (!general && (D == 16 || D == 32 || D == 64 || D == 128 || D == 256)) {
@@ -580,13 +581,13 @@ extern "C" int celeg_delta_scan(const float* qk, const float* v, const float* be
         dim3 grid(n_seqs, H, (V + cpw - 1) / cpw), block(CELEG_WAVE);
         // pairs (room for n_tokens * G * 4 floats, or null): steps with rows to pair take two tokens together
         if (pairs && n_tokens > n_seqs) {
-            hipLaunchKernelGGL(delta_pairs_kernel, dim3(n_tokens, G), dim3(CELEG_WAVE), 0, stream, qk, token_seq, cu_seqlens, pairs, G, D);
+            hipLaunchKernelGGL(delta_pairs_kernel, dim3(n_tokens, G), dim3(CELEG_WAVE), 0, stream, qk, token_seq, cu_seqlens, pairs, G, D, below);
         } else {
             pairs = nullptr;
         }
 #define CELEG_DELTA_REG(DL_, DPL_)                                                                                                  \
     hipLaunchKernelGGL((delta_scan_reg_kernel<DL_, DPL_>), grid, block, 0, stream, qk, v, beta_decay, state, state_stride, cu_seqlens, \
-                       seq_slot, out, pairs, G, H, V)
+                       seq_slot, out, pairs, G, H, V, below)
         if (D == 16) CELEG_DELTA_REG(4, 4);
         else if (D == 32) CELEG_DELTA_REG(8, 4);
         else if (D == 64) CELEG_DELTA_REG(16, 4);

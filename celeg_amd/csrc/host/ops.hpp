@@ -135,6 +135,7 @@ public:
     bool attention_general = false;      // always the general attention kernel
     bool delta_general = false;          // the delta rule's recurrence always by the kernel for any dim
     bool delta_pairs = true;             // the recurrence in registers takes whole blocks of rows two tokens at a time
+    int delta_chunk_rows = -1;           // portions of as many rows go by chunks of 64 (-1: the rule by type and rows; 0: none)
     bool use_delta_step = true;          // steps of one token a request: the delta rule in one kernel
     bool use_sigmoid_mfma = true;        // bfloat16 attention with sigmoid weights on the matrix cores
     bool use_biased_mfma = true;         // bfloat16 attention with a distance bias on the matrix cores
@@ -228,8 +229,9 @@ public:
                        const Tensor& dt_bias, const Tensor& conv_state, const Tensor& qk, const Tensor& v, const Tensor& beta_decay,
                        const StepBatch& batch);
     // the recurrence over the step's rows of every request, from and into state [slots, heads, dim, vdim]
+    // (rows: what the model keeps its rows in; long portions go by chunks where that is bfloat16)
     void delta_scan(const Tensor& qk, const Tensor& v, const Tensor& beta_decay, const Tensor& state, const Tensor& out,
-                    const DeltaShape& shape, const StepBatch& batch, Workspace& ws);
+                    const DeltaShape& shape, const StepBatch& batch, Workspace& ws, DType rows = DType::F32);
     // out = o / rms(o) * weight * silu(gate) per head; o [rows, heads * vdim] 32-bit, gate a view with dense rows
     // (act: what the gate passes through, 0 silu, 1 sigmoid)
     void delta_gated_norm(const Tensor& o, const Tensor& weight, const Tensor& gate, float eps, const Tensor& out, int heads, int vdim,

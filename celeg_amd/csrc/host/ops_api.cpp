@@ -161,6 +161,7 @@ void set_knobs(Ops& ops, const Json& knobs) {
         else if (name == "use_rope_table") ops.use_rope_table = v != 0;
         else if (name == "delta_general") ops.delta_general = v != 0;
         else if (name == "delta_pairs") ops.delta_pairs = v != 0;
+        else if (name == "delta_chunk_rows") ops.delta_chunk_rows = static_cast<int>(v);
         else if (name == "use_delta_step") ops.use_delta_step = v != 0;
         else if (name == "sigmoid_rows_form") ops.sigmoid_rows_form = static_cast<int>(v);
         else if (name == "use_sigmoid_mfma") ops.use_sigmoid_mfma = v != 0;

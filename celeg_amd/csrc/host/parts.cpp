@@ -1653,7 +1653,7 @@ public:
             if (!per_channel_) {
                 rt.ops.delta_prepare(proj, static_cast<int>(col_b_), static_cast<int>(col_a_), shape_, conv_w_->view, a_log_->view,
                                      dt_bias_->view, cache.states.at("conv"), qk, v, beta_decay, batch);
-                rt.ops.delta_scan(qk, v, beta_decay, cache.states.at("S"), o, shape_, batch, rt.ws);
+                rt.ops.delta_scan(qk, v, beta_decay, cache.states.at("S"), o, shape_, batch, rt.ws, rt.dtype);
             } else {
                 Tensor z = proj.cols(col_a_, decay_width());
                 if (decay_rank_ > 0) {

@@ -281,6 +281,25 @@ def test_single_tokens_whose_keys_are_dealt_to_several_workgroups(tmp_path, head
             assert rel <= 1.5e-2, f"{heads} heads of {dim}, {rid}: rel rms {rel:.3e}"
 
 
+@pytest.mark.parametrize("heads,kv_heads,vdim", [(4, 2, 64), (3, 3, 16), (2, 1, 128)])
+def test_delta_rule_by_chunks_equals_token_by_token(tmp_path, heads, kv_heads, vdim):
+    """32-bit: portions taken 64 tokens at a time (from one row on, so with chunks of every remainder: 1, 63, 64, 65 and
+    more rows) beside single tokens and from a state that is not empty, against the recurrence token by token."""
+    cfg = {"architecture": "Kifetar", "vocab": 150, "width": 64, "norm": {"eps": 1e-5}, "max_context": 1024,
+           "layers": [delta(heads, kv_heads, 64, vdim, 4), delta(heads, kv_heads, 64, vdim, 2)]}
+    folder = write_model(tmp_path / "chunks", cfg, 43, torch.float32, std=0.2)
+    reqs = {"a": random_tokens(cfg["vocab"], 300, seed=15), "b": random_tokens(cfg["vocab"], 129, seed=16), "c": random_tokens(cfg["vocab"], 64, seed=17)}
+    for steps in (whole_schedule(reqs), portions_schedule(reqs, sizes=(63, 1, 65, 17, 128, 3)), mixed_schedule(reqs, seed=7, decode_tail=5)):
+        got = {}
+        for rows in (0, 1, 33):
+            lm, _ = load(folder, "float32", steps)
+            lm.set_knob("delta_chunk_rows", rows)
+            got[rows] = EngineDriver(lm).run(steps)
+        for rid in reqs:
+            assert_close_f32(got[1][rid], got[0][rid], rid)
+            assert_close_f32(got[33][rid], got[0][rid], rid)
+
+
 def test_delta_rule_in_registers_equals_the_general_kernel(folders):
     """32-bit: the recurrence with the state in registers against the kernel for any size, same schedule."""
     folder = folders("K4", "float32")
