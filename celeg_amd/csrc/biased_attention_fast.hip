@@ -26,8 +26,6 @@
 // Single tokens: below.
 #include "common.h"
 
-#include <algorithm>
-
 namespace {
 
 typedef __bf16 bf_bf16x8 __attribute__((ext_vector_type(8)));
@@ -113,20 +111,21 @@ struct BfFetch {
     }
 };
 
-// one staged block of 64 keys for the 16 rows of a wavefront
-template <int D, int V>
-__device__ __forceinline__ void bf_block(const __bf16* ks, const __bf16* vs, const bf_bf16x8 (&qreg)[D / 32], BfRow<V / 16>& row, int kb,
-                                         int my_pos, int window, int keep_first, bool kept_only, int r, int quad, float s2, float b1, float b2,
-                                         bool biased, float cap2) {
-    constexpr int KROW = D + 8, VROW = BF_KEYS + 8, KS = D / 32, DT = V / 16;
+// one block of 64 keys for the 16 rows of a wavefront: key_piece(kt, st), the lane's first operand of the scores (key 16 kt +
+// r, numbers 32 st + 8 quad ..), and value_piece(pair, dt), that of the output (value 16 dt + r of the keys 32 pair + 4 quad
+// .. + 3 and those 16 behind them)
+template <int D, int V, class KeyPiece, class ValuePiece>
+__device__ __forceinline__ void bf_block(const KeyPiece key_piece, const ValuePiece value_piece, const bf_bf16x8 (&qreg)[D / 32], BfRow<V / 16>& row,
+                                         int kb, int my_pos, int window, int keep_first, bool kept_only, int quad, float s2, float b1,
+                                         float b2, bool biased, float cap2) {
+    constexpr int KS = D / 32, DT = V / 16;
     bf_f32x4 sacc[4];
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt) {
         sacc[kt] = bf_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int st = 0; st < KS; ++st) {
-            const bf_bf16x8 kf = __builtin_bit_cast(bf_bf16x8, *reinterpret_cast<const bf_u32x4*>(ks + (16 * kt + r) * KROW + 32 * st + 8 * quad));
-            sacc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qreg[st], sacc[kt], 0, 0, 0);
+            sacc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(key_piece(kt, st), qreg[st], sacc[kt], 0, 0, 0);
         }
     }
     float top = -INFINITY;
@@ -180,14 +179,30 @@ __device__ __forceinline__ void bf_block(const __bf16* ks, const __bf16* vs, con
         bf_bf16x8 vf[DT];
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
-            const __bf16* vrow = vs + (16 * dt + r) * VROW + 32 * pair + 4 * quad;
-            const bf_u32x2 lo = *reinterpret_cast<const bf_u32x2*>(vrow), hi = *reinterpret_cast<const bf_u32x2*>(vrow + 16);
-            vf[dt] = __builtin_bit_cast(bf_bf16x8, bf_u32x4{lo[0], lo[1], hi[0], hi[1]});
+            vf[dt] = value_piece(pair, dt);
             row.acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[dt], pw, row.acc[dt], 0, 0, 0);
         }
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) row.acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[dt], pr, row.acc[dt], 0, 0, 0);
     }
+}
+
+// the same of a block staged in LDS
+template <int D, int V>
+__device__ __forceinline__ void bf_staged_block(const __bf16* ks, const __bf16* vs, const bf_bf16x8 (&qreg)[D / 32], BfRow<V / 16>& row, int kb,
+                                                int my_pos, int window, int keep_first, bool kept_only, int r, int quad, float s2, float b1,
+                                                float b2, bool biased, float cap2) {
+    constexpr int KROW = D + 8, VROW = BF_KEYS + 8;
+    bf_block<D, V>(
+        [&](int kt, int st) __attribute__((always_inline)) {
+            return __builtin_bit_cast(bf_bf16x8, *reinterpret_cast<const bf_u32x4*>(ks + (16 * kt + r) * KROW + 32 * st + 8 * quad));
+        },
+        [&](int pair, int dt) __attribute__((always_inline)) {
+            const __bf16* vrow = vs + (16 * dt + r) * VROW + 32 * pair + 4 * quad;
+            const bf_u32x2 lo = *reinterpret_cast<const bf_u32x2*>(vrow), hi = *reinterpret_cast<const bf_u32x2*>(vrow + 16);
+            return __builtin_bit_cast(bf_bf16x8, bf_u32x4{lo[0], lo[1], hi[0], hi[1]});
+        },
+        qreg, row, kb, my_pos, window, keep_first, kept_only, quad, s2, b1, b2, biased, cap2);
 }
 
 // a finished row: divided by its normaliser, times sigmoid(gate), stored
@@ -229,7 +244,6 @@ struct BfArgs {
 
 // The key blocks of a tile whose lowest position is pos0: first the blocks that hold the kept first keys
 // where the window has passed them (only those keys count there), then the blocks from the window's start on.
-template <int KEYS>
 struct BfBlocks {
     int n_kept, kb0;
     __device__ __forceinline__ BfBlocks(int pos0, int window, int keep) {
@@ -237,13 +251,13 @@ struct BfBlocks {
         kb0 = key_first & ~7;
         n_kept = 0;
         if (keep > 0 && kb0 > 0) {
-            if (kb0 >= keep) n_kept = (keep + KEYS - 1) / KEYS;
+            if (kb0 >= keep) n_kept = (keep + BF_KEYS - 1) / BF_KEYS;
             else kb0 = 0;                 // the window begins among the kept keys: one run from the start
         }
     }
-    __device__ __forceinline__ int count(int pos_last) const { return n_kept + (pos_last >= kb0 ? (pos_last - kb0) / KEYS + 1 : 0); }
+    __device__ __forceinline__ int count(int pos_last) const { return n_kept + (pos_last >= kb0 ? (pos_last - kb0) / BF_KEYS + 1 : 0); }
     __device__ __forceinline__ bool kept(int i) const { return i < n_kept; }
-    __device__ __forceinline__ int start(int i) const { return i < n_kept ? i * KEYS : kb0 + (i - n_kept) * KEYS; }
+    __device__ __forceinline__ int start(int i) const { return i < n_kept ? i * BF_KEYS : kb0 + (i - n_kept) * BF_KEYS; }
     // the last key a block may touch: pages between the kept keys and the window may be gone
     __device__ __forceinline__ int last(int i, int pos_last, int keep) const { return i < n_kept ? keep - 1 : pos_last; }
 };
@@ -309,7 +323,7 @@ __global__ __launch_bounds__(BF_WAVES * CELEG_WAVE) void biased_attention_rows_k
     const int page_shift = 31 - __builtin_clz(a.page_tokens), page_mask = a.page_tokens - 1;
     const size_t head_index_stride = static_cast<size_t>(a.n_layers) * a.kv_heads, layer_index = static_cast<size_t>(a.layer) * a.kv_heads;
     BfFetch<D, V, THREADS, FULL> pre;
-    const BfBlocks<BF_KEYS> blocks(tile_pos0, a.window, a.keep_first);
+    const BfBlocks blocks(tile_pos0, a.window, a.keep_first);
     const int n_blocks = blocks.count(pos_last);
     pre.load(tid, blocks.start(0), blocks.last(0, pos_last, a.keep_first), a.k_pool, a.v_pool, pages, page_shift, page_mask, a.page_tokens,
              head_index_stride, kvh, layer_index, kd, vd);
@@ -326,7 +340,7 @@ __global__ __launch_bounds__(BF_WAVES * CELEG_WAVE) void biased_attention_rows_k
         // blocks none of this wavefront's rows can see
         if (rows_here <= 0) continue;
         if (!blocks.kept(i) && (kb > wave_last || (a.window > 0 && kb >= a.keep_first && kb + BF_KEYS - 1 < wave_pos0 - a.window + 1))) continue;
-        bf_block<D, V>(ks, vs, qreg, row, kb, my_pos, a.window, a.keep_first, blocks.kept(i), r, quad, s2, b1, b2, biased, cap2);
+        bf_staged_block<D, V>(ks, vs, qreg, row, kb, my_pos, a.window, a.keep_first, blocks.kept(i), r, quad, s2, b1, b2, biased, cap2);
     }
     float total = row.sum;
     total = sum_half32(sum_row16(total));
@@ -379,7 +393,7 @@ __global__ __launch_bounds__(WAVES * CELEG_WAVE, bf_tile_waves_a_simd(D, V, FULL
     const int page_shift = 31 - __builtin_clz(a.page_tokens), page_mask = a.page_tokens - 1;
     const size_t head_index_stride = static_cast<size_t>(a.n_layers) * a.kv_heads, layer_index = static_cast<size_t>(a.layer) * a.kv_heads;
     BfFetch<D, V, CELEG_WAVE, FULL> pre;
-    const BfBlocks<BF_KEYS> blocks(pos0, a.window, a.keep_first);
+    const BfBlocks blocks(pos0, a.window, a.keep_first);
     const int n_blocks = blocks.count(pos_last);
     if (wave < n_blocks)
         pre.load(lane, blocks.start(wave), blocks.last(wave, pos_last, a.keep_first), a.k_pool, a.v_pool, pages, page_shift, page_mask,
@@ -394,7 +408,7 @@ __global__ __launch_bounds__(WAVES * CELEG_WAVE, bf_tile_waves_a_simd(D, V, FULL
         if (i + WAVES < n_blocks)
             pre.load(lane, blocks.start(i + WAVES), blocks.last(i + WAVES, pos_last, a.keep_first), a.k_pool, a.v_pool, pages, page_shift,
                      page_mask, a.page_tokens, head_index_stride, kvh, layer_index, kd, vd);
-        bf_block<D, V>(ks, vs, qreg, row, blocks.start(i), my_pos, a.window, a.keep_first, blocks.kept(i), r, quad, s2, b1, b2, biased, cap2);
+        bf_staged_block<D, V>(ks, vs, qreg, row, blocks.start(i), my_pos, a.window, a.keep_first, blocks.kept(i), r, quad, s2, b1, b2, biased, cap2);
     }
     // the wavefronts' maxima, normalisers and sums meet in LDS (every wavefront's staging area is
     // free after the barrier); the first one joins them in the order of the wavefronts and stores
@@ -439,70 +453,118 @@ __global__ __launch_bounds__(WAVES * CELEG_WAVE, bf_tile_waves_a_simd(D, V, FULL
                 quad, vd);
 }
 
-// ---- single tokens: a workgroup per (row, key/value head, part of the keys), the query heads that share the head as
-// the rows of the matrix instruction (up to 16), eight wavefronts that take units of 32 keys in turn, over all parts.
-// What bounds such a call is what one compute unit draws of the keys and values (some 50 GB/s: 1,100 keys of 64, 282 KB, 5.5
-// us) and the chain position -> page -> keys -> weights -> sum.  So many keys are dealt to several workgroups, whose
-// maxima, normalisers and sums a second kernel joins, and keys and values go from the pages straight into the
-// registers of the matrix instruction: row 4 quad + i of score tile kt stands for key 8 quad + 4 kt + i of the
-// unit, so that a lane ends up with the weights of the eight neighbouring keys that its 16 bytes of a page's values hold.
-struct BfSingle {
-    const int* positions;
-    const int* token_slot;
-    float* parts_out;         // [rows, kv_heads, parts, group, V + 2], or null with one part
-    int parts;
-};
+template <int V> constexpr int bf_entry() { return V + 8; }
+// value d of a head from its wavefronts' entries: the sums over all of them divided by the normaliser, as the tile kernel
+// joins its wavefronts
+template <int V, int WAVES>
+__device__ __forceinline__ float bf_join(const float* entries, int d) {
+    constexpr int ENTRY = bf_entry<V>();
+    float sums[WAVES], tops[WAVES];
+    bf_f32x4 norms[WAVES];
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+        sums[w] = entries[w * ENTRY + d];
+        tops[w] = entries[w * ENTRY + V];
+        norms[w] = *reinterpret_cast<const bf_f32x4*>(entries + w * ENTRY + V + 4);
+    }
+    float top = tops[0];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) top = fmaxf(top, tops[w]);
+    // (the row's own key is visible, so the maximum over all of them is finite)
+    const float first = bf_exp2(tops[0] - top);
+    float sum = sums[0] * first;
+    bf_f32x4 norm = norms[0] * first;
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) {
+        const float f = bf_exp2(tops[w] - top);
+        sum = fmaf(sums[w], f, sum);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) norm[i] = fmaf(norms[w][i], f, norm[i]);
+    }
+    return sum * (1.0f / ((norm[0] + norm[1]) + (norm[2] + norm[3])));
+}
 
-#define BF_SINGLE_WAVES 8
-#define BF_MAX_PARTS 8
-#define BF_UNIT 32
-template <int D, int V, bool FULL>
-__global__ __launch_bounds__(BF_SINGLE_WAVES * CELEG_WAVE, (D <= 64 && V <= 64 ? 4 : 2)) void biased_attention_single_kernel(const BfArgs a, const BfSingle p) {
-    constexpr int WAVES = BF_SINGLE_WAVES, KS = D / 32, DT = V / 16, VROW = V + 4;
+// ---- single tokens: the query heads that share a key/value head are the rows of the matrix instruction (up to 16), and keys and
+// values go from the pages straight into its registers, a block ahead of the one that is multiplied.  The key blocks are
+// dealt to the workgroup's wavefronts in turn as in the tile kernel, with its sums in its order: the bits are the same.
+// What bounds such a call is a wavefront's chain of blocks (1.3 us each: 16 scores a lane, bent, weighed and rounded twice)
+// behind position -> page -> keys.  16 heads of 64 over 8, us (16-row tiles a query head | this):
+//   4 requests   300 keys  7.4 | 6.6    900  12.9 | 11.9    1,500  17.0 | 15.4
+//   32           300      19.0 | 8.5    900  31.5 | 17.8    1,500  42.1 | 24.7
+// (A workgroup of one wavefront for each chain and a second kernel that joins them: 7.1, 10.4 and 13.7 alone, and nothing in
+// a request.  Units of 32 keys over up to 64 wavefronts: 8.2 at 1,500 keys, but then a row's sums run in another order.)
+template <int D, int V, int WAVES, bool FULL>
+__global__ __launch_bounds__(WAVES * CELEG_WAVE) void biased_attention_single_kernel(const BfArgs a, const int* __restrict__ positions,
+                                                                                      const int* __restrict__ token_slot) {
+    constexpr int KS = D / 32, DT = V / 16, ENTRY = bf_entry<V>();
     const int kd = FULL ? D : a.kd, vd = FULL ? V : a.vd;
     extern __shared__ __attribute__((aligned(16))) unsigned char bf_lds[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / CELEG_WAVE), lane = threadIdx.x % CELEG_WAVE;
     const int t = blockIdx.x, kvh = blockIdx.y, group = a.q_heads / a.kv_heads;
     const int r = lane & 15, quad = lane >> 4;
-    const int pos = p.positions[t];
-    const int* const pages = a.table + static_cast<size_t>(p.token_slot[t]) * a.table_stride;
+    const int pos = positions[t];
+    const int* const pages = a.table + static_cast<size_t>(token_slot[t]) * a.table_stride;
     const int h = kvh * group + min(r, group - 1);             // rows past the last head repeat it (not stored)
     const int page_shift = 31 - __builtin_clz(a.page_tokens), page_mask = a.page_tokens - 1;
-    const BfBlocks<BF_UNIT> blocks(pos, a.window, a.keep_first);
-    const int n_units = blocks.count(pos), stride = WAVES * p.parts, first = blockIdx.z * WAVES + wave;
-    struct Unit {
-        bf_u32x4 k[2][KS], v[DT];
-    };
-    auto page_of = [&](int u, int eighth) {
-        const int i = min(u, n_units - 1);
-        return pages[min(blocks.start(i) + 8 * eighth, blocks.last(i, pos, a.keep_first)) >> page_shift];
-    };
-    auto head_of = [&](int page) { return (static_cast<size_t>(page) * a.n_layers + a.layer) * a.kv_heads + kvh; };
-    auto fetch = [&](int u, int k_page, int v_page, Unit& unit) __attribute__((always_inline)) {
-        const int ub = blocks.start(u), last = blocks.last(u, pos, a.keep_first);
-        const bf16* const k_head = a.k_pool + head_of(k_page) * a.page_tokens * kd;
-        const bf16* const v_head = a.v_pool + head_of(v_page) * a.page_tokens * vd;
+    const BfBlocks blocks(pos, a.window, a.keep_first);
+    const int n_blocks = blocks.count(pos);
+    struct Block {
+        bf_u32x4 k[4][KS];
+        bf_u32x2 v[4][DT];         // [16 keys][..]: four keys of the lane's value
+    } next;
+    auto head_of = [&](int key) { return (static_cast<size_t>(pages[key >> page_shift]) * a.n_layers + a.layer) * a.kv_heads + kvh; };
+    auto fetch = [&](int i, Block& to) __attribute__((always_inline)) {
+        const int kb = blocks.start(i), last = blocks.last(i, pos, a.keep_first);
+        size_t k_head[4], v_head[4];
+        int k_key[4], v_key[4];
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt) {
-            const int key = min(ub + 8 * (r >> 2) + 4 * kt + (r & 3), last);
+        for (int kt = 0; kt < 4; ++kt) {
+            k_key[kt] = min(kb + 16 * kt + r, last);
+            v_key[kt] = min(kb + 16 * kt + 4 * quad, last & ~3);
+            k_head[kt] = head_of(k_key[kt]);
+            v_head[kt] = head_of(v_key[kt]);
+        }
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
 #pragma unroll
             for (int st = 0; st < KS; ++st) {
                 const int d = 32 * st + 8 * quad;
-                unit.k[kt][st] = *reinterpret_cast<const bf_u32x4*>(k_head + static_cast<size_t>(key & page_mask) * kd + (FULL ? d : min(d, kd - 8)));
+                to.k[kt][st] = *reinterpret_cast<const bf_u32x4*>(a.k_pool + (k_head[kt] * a.page_tokens + (k_key[kt] & page_mask)) * kd + (FULL ? d : min(d, kd - 8)));
+            }
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) {
+                const int d = 16 * dt + r;
+                to.v[kt][dt] = *reinterpret_cast<const bf_u32x2*>(a.v_pool + v_head[kt] * vd * a.page_tokens + static_cast<size_t>(FULL ? d : min(d, vd - 1)) * a.page_tokens +
+                                                                  (v_key[kt] & page_mask));
             }
         }
-        const int v_from = min(ub + 8 * quad, last & ~7);
+    };
+    // (behind the head's last number and behind the last key: zeros)
+    auto clean = [&](int i, Block& block) __attribute__((always_inline)) {
+        const int kb = blocks.start(i), last = blocks.last(i, pos, a.keep_first);
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-            const int d = 16 * dt + r;
-            unit.v[dt] = *reinterpret_cast<const bf_u32x4*>(v_head + static_cast<size_t>(FULL ? d : min(d, vd - 1)) * a.page_tokens + (v_from & page_mask));
+        for (int kt = 0; kt < 4; ++kt) {
+            if (!FULL) {
+#pragma unroll
+                for (int st = 0; st < KS; ++st)
+                    if (32 * st + 8 * quad >= kd) block.k[kt][st] = bf_u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt)
+                    if (16 * dt + r >= vd) block.v[kt][dt] = bf_u32x2{0u, 0u};
+            }
+            if (kb + BF_KEYS - 1 > last) {
+                const int live = last - (kb + 16 * kt + 4 * quad) + 1;
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        block.v[kt][dt][j] &= (live > 2 * j ? 0x0000ffffu : 0u) | (live > 2 * j + 1 ? 0xffff0000u : 0u);
+            }
         }
     };
-    Unit units[2];
-    const int k_page0 = page_of(first, r >> 2), v_page0 = page_of(first, quad);
-    int k_page = page_of(first + stride, r >> 2), v_page = page_of(first + stride, quad);
+    if (wave < n_blocks) fetch(wave, next);
     float cap2;
-    float s2 = bf_score_factor(a, pos, cap2);
+    const float s2 = bf_score_factor(a, pos, cap2);
     const bool biased = a.r1 != nullptr;
     const float b1 = biased ? a.r1[h] : 0.f, b2 = biased ? a.r2[h] : 0.f;
     bf_bf16x8 qreg[KS];
@@ -516,178 +578,62 @@ __global__ __launch_bounds__(BF_SINGLE_WAVES * CELEG_WAVE, (D <= 64 && V <= 64 ?
     BfRow<DT> row;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) row.acc[dt] = bf_f32x4{0.f, 0.f, 0.f, 0.f};
-    if ((a.sink_one || a.sink) && first == 0) {       // (once a row: the first wavefront's share)
+    if ((a.sink_one || a.sink) && wave == 0) {        // (once a row: the first wavefront's share)
         row.top = a.sink ? a.sink[h] * BF_LOG2E : 0.f;
         row.sum = quad == 0 ? 1.f : 0.f;
     }
-    auto take = [&](int u, Unit& unit) __attribute__((always_inline)) {
-        const int ub = blocks.start(u), last = blocks.last(u, pos, a.keep_first);
-        const bool kept_only = blocks.kept(u);
-        if (!FULL) {                                  // pieces behind the head's last number are zeros
-#pragma unroll
-            for (int st = 0; st < KS; ++st)
-                if (32 * st + 8 * quad >= kd) unit.k[0][st] = unit.k[1][st] = bf_u32x4{0u, 0u, 0u, 0u};
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt)
-                if (16 * dt + r >= vd) unit.v[dt] = bf_u32x4{0u, 0u, 0u, 0u};
-        }
-        if (ub + BF_UNIT - 1 > last) {                // what lies behind the last key may be anything
-            const int live = last - (ub + 8 * quad) + 1;
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    unit.v[dt][j] &= (live > 2 * j ? 0x0000ffffu : 0u) | (live > 2 * j + 1 ? 0xffff0000u : 0u);
-        }
-        float x[8], top = -INFINITY;
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt) {
-            bf_f32x4 s = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int st = 0; st < KS; ++st)
-                s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf_bf16x8, unit.k[kt][st]), qreg[st], s, 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int key = ub + 8 * quad + 4 * kt + i;
-                const bool seen = key <= pos && (kept_only ? key < a.keep_first : (a.window <= 0 || key > pos - a.window || key < a.keep_first));
-                float y = s[i] * s2;
-                if (cap2 > 0.f) y = fmaf(-2.0f * cap2, __builtin_amdgcn_rcpf(bf_exp2(y) + 1.0f), cap2);      // (s2 holds 2 log2(e) scale f / c)
-                if (biased) y -= b1 * bf_log2(fmaf(b2, static_cast<float>(pos - key), 1.0f));
-                x[4 * kt + i] = seen ? y : -INFINITY;
-                top = fmaxf(top, x[4 * kt + i]);
-            }
-        }
-        top = max_half32(max_row16(top));
-        const float new_top = fmaxf(row.top, top), base = new_top == -INFINITY ? 0.f : new_top;
-        const float keep = bf_exp2(row.top - base);
-        row.top = new_top;
-        float sum = 0.f;
-        bf_bf16x8 w, rest;                            // a weight as two bfloat16 numbers: its rounding, and what the rounding left
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const float y = bf_exp2(x[e] - base);
-            sum += y;
-            w[e] = static_cast<__bf16>(y);
-            rest[e] = static_cast<__bf16>(y - static_cast<float>(w[e]));
-        }
-        row.sum = fmaf(row.sum, keep, sum);
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-            row.acc[dt] *= keep;
-            row.acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf_bf16x8, unit.v[dt]), w, row.acc[dt], 0, 0, 0);
-            row.acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf_bf16x8, unit.v[dt]), rest, row.acc[dt], 0, 0, 0);
-        }
-    };
-    if (first < n_units) fetch(first, k_page0, v_page0, units[0]);
-    if (first + stride < n_units) fetch(first + stride, k_page, v_page, units[1]);
-    for (int u = first; u < n_units; u += 2 * stride) {
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const int mine = u + e * stride;
-            if (mine >= n_units) break;
-            const bool more = mine + 2 * stride < n_units;
-            if (more) {
-                k_page = page_of(mine + 2 * stride, r >> 2);
-                v_page = page_of(mine + 2 * stride, quad);
-            }
-            take(mine, units[e]);
-            if (more) fetch(mine + 2 * stride, k_page, v_page, units[e]);
-        }
+    for (int i = wave; i < n_blocks; i += WAVES) {
+        Block now = next;
+        if (i + WAVES < n_blocks) fetch(i + WAVES, next);
+        clean(i, now);
+        bf_block<D, V>(
+            [&](int kt, int st) __attribute__((always_inline)) { return __builtin_bit_cast(bf_bf16x8, now.k[kt][st]); },
+            [&](int pair, int dt) __attribute__((always_inline)) {
+                const bf_u32x2 lo = now.v[2 * pair][dt], hi = now.v[2 * pair + 1][dt];
+                return __builtin_bit_cast(bf_bf16x8, bf_u32x4{lo[0], lo[1], hi[0], hi[1]});
+            },
+            qreg, row, blocks.start(i), pos, a.window, a.keep_first, blocks.kept(i), quad, s2, b1, b2, biased, cap2);
     }
-    // the wavefronts' maxima, normalisers and sums meet in LDS as [wavefront][head][sums, maximum, normaliser]
-    float* const meet = reinterpret_cast<float*>(bf_lds);
-    const float total = sum_half32(sum_row16(row.sum));
+    // the wavefronts' entries meet in LDS as [head][wavefront]: sums [V], maximum, -, -, -, the normaliser's shares of four lanes
+    float* const entries = reinterpret_cast<float*>(bf_lds);
     if (r < group) {
-        float* const mine = meet + (static_cast<size_t>(wave) * group + r) * VROW;
+        float* const mine = entries + (static_cast<size_t>(r) * WAVES + wave) * ENTRY;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<bf_f32x4*>(mine + 16 * dt + 4 * quad) = row.acc[dt];
-        if (quad == 0) {
-            mine[V] = row.top;
-            mine[V + 1] = total;
-        }
+        if (quad == 0) mine[V] = row.top;
+        mine[V + 4 + quad] = row.sum;
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < group * V; e += WAVES * CELEG_WAVE) {
-        const int head = e / V, d = e % V;
-        const float* const from = meet + static_cast<size_t>(head) * VROW;
-        float top = -INFINITY, sum = 0.f, norm = 0.f;
-#pragma unroll
-        for (int w = 0; w < WAVES; ++w) top = fmaxf(top, from[static_cast<size_t>(w) * group * VROW + V]);
-        const float base = top == -INFINITY ? 0.f : top;
-#pragma unroll
-        for (int w = 0; w < WAVES; ++w) {
-            const float* const theirs = from + static_cast<size_t>(w) * group * VROW;
-            const float f = bf_exp2(theirs[V] - base);
-            norm = fmaf(theirs[V + 1], f, norm);
-            sum = fmaf(theirs[d], f, sum);
-        }
-        if (p.parts_out) {
-            float* const to = p.parts_out + (((static_cast<size_t>(t) * a.kv_heads + kvh) * p.parts + blockIdx.z) * group + head) * (V + 2);
-            to[d] = sum;
-            if (d == 0) {
-                to[V] = top;
-                to[V + 1] = norm;
-            }
-            continue;
-        }
-        if (!FULL && d >= vd) continue;
+    for (int e = threadIdx.x; e < group * vd; e += WAVES * CELEG_WAVE) {
+        const int head = e / vd, d = e - head * vd;
         const size_t at = static_cast<size_t>(kvh * group + head) * vd + d;
         const float g = a.gate ? bf_sigmoid(to_float(a.gate[static_cast<size_t>(t) * a.ldg + at])) : 1.0f;
-        a.out[static_cast<size_t>(t) * a.ldo + at] = from_float<bf16>(sum / norm * g);
+        a.out[static_cast<size_t>(t) * a.ldo + at] = from_float<bf16>(bf_join<V, WAVES>(entries + static_cast<size_t>(head) * WAVES * ENTRY, d) * g);
     }
-}
-
-// The parts of the kernel above joined in their order, a thread a value, all parts asked for at once.
-__global__ __launch_bounds__(256) void biased_attention_join_kernel(const float* __restrict__ in, const bf16* __restrict__ gate,
-                                                                    bf16* __restrict__ out, const int parts, const int ldg, const int ldo,
-                                                                    const int vd, const int v_pad, const int group, const int q_heads) {
-    const int t = blockIdx.y, e = blockIdx.x * 256 + threadIdx.x;
-    if (e >= q_heads * vd) return;
-    const int head = e / vd, d = e - head * vd, kvh = head / group, row = v_pad + 2;
-    const float* const mine = in + ((static_cast<size_t>(t) * q_heads + static_cast<size_t>(kvh) * group) * parts + (head - kvh * group)) * row;
-    const float g = gate ? to_float(gate[static_cast<size_t>(t) * ldg + e]) : 0.f;
-    float sums[BF_MAX_PARTS], tops[BF_MAX_PARTS], norms[BF_MAX_PARTS];
-#pragma unroll
-    for (int i = 0; i < BF_MAX_PARTS; ++i) {
-        const float* const part = mine + static_cast<size_t>(min(i, parts - 1)) * group * row;
-        sums[i] = part[d];
-        tops[i] = part[v_pad];
-        norms[i] = part[v_pad + 1];
-    }
-    float top = tops[0];
-#pragma unroll
-    for (int i = 1; i < BF_MAX_PARTS; ++i) top = fmaxf(top, tops[i]);       // (finite: the row's own key is in one of them)
-    float sum = 0.f, norm = 0.f;
-#pragma unroll
-    for (int i = 0; i < BF_MAX_PARTS; ++i) {
-        const float f = i < parts ? bf_exp2(tops[i] - top) : 0.f;
-        sum = fmaf(sums[i], f, sum);
-        norm = fmaf(norms[i], f, norm);
-    }
-    out[static_cast<size_t>(t) * ldo + e] = from_float<bf16>(sum / norm * (gate ? bf_sigmoid(g) : 1.0f));
-}
-
-template <int D, int V, bool FULL>
-int bf_launch_single(int n_tokens, const BfArgs& a, const BfSingle& p, hipStream_t stream) {
-    const int group = a.q_heads / a.kv_heads;
-    const size_t lds = static_cast<size_t>(BF_SINGLE_WAVES) * group * (V + 4) * sizeof(float);
-    auto kernel = &biased_attention_single_kernel<D, V, FULL>;
-    static bool raised = false;              // (16 heads of 128: 68 KB)
-    if (lds > 48 * 1024 && !raised) {
-        hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
-        if (err != hipSuccess) return static_cast<int>(err);
-        raised = true;
-    }
-    hipLaunchKernelGGL(kernel, dim3(n_tokens, a.kv_heads, p.parts), dim3(BF_SINGLE_WAVES * CELEG_WAVE), lds, stream, a, p);
-    if (p.parts_out)
-        hipLaunchKernelGGL(biased_attention_join_kernel, dim3((a.q_heads * a.vd + 255) / 256, n_tokens), dim3(256), 0, stream, p.parts_out,
-                           a.gate, a.out, p.parts, a.ldg, a.ldo, a.vd, V, group, a.q_heads);
-    return CELEG_LAUNCH_RESULT();
 }
 
 constexpr int bf_block_bytes(int d, int v) { return (BF_KEYS * (d + 8) + v * (BF_KEYS + 8)) * 2; }
 // single tiles: eight wavefronts share out the key blocks where their staging areas fit LDS
 constexpr int bf_tile_waves(int d, int v) { return 8 * bf_block_bytes(d, v) <= 160 * 1024 ? 8 : BF_WAVES; }
+
+struct BfSingle {
+    const int* positions;
+    const int* token_slot;
+};
+template <int D, int V, bool FULL>
+int bf_launch_single(int n_tokens, const BfArgs& a, const BfSingle& p, hipStream_t stream) {
+    constexpr int WAVES = bf_tile_waves(D, V);
+    const size_t lds = static_cast<size_t>(WAVES) * (a.q_heads / a.kv_heads) * bf_entry<V>() * sizeof(float);
+    auto kernel = &biased_attention_single_kernel<D, V, WAVES, FULL>;
+    static bool raised = false;              // (16 heads of 96: 53 KB)
+    if (lds > 48 * 1024 && !raised) {
+        hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
+        if (err != hipSuccess) return static_cast<int>(err);
+        raised = true;
+    }
+    hipLaunchKernelGGL(kernel, dim3(n_tokens, a.kv_heads), dim3(WAVES * CELEG_WAVE), lds, stream, a, p.positions, p.token_slot);
+    return CELEG_LAUNCH_RESULT();
+}
 
 template <int D, int V, bool FULL>
 int bf_launch_full(int form, int max_tiles, const BfArgs& a, const BfSingle& single, hipStream_t stream) {
@@ -724,26 +670,11 @@ extern "C" int celeg_biased_attention_fast_ok(int head_dim, int v_dim) {
     return head_dim > 0 && head_dim <= 128 && head_dim % 8 == 0 && v_dim > 0 && v_dim <= 128 && v_dim % 4 == 0;
 }
 
-// How many workgroups share a key/value head's keys; keys: the most that a row may see.  With the second kernel a call
-// of 4 requests over 8 heads of 64 takes 7.2 us at 300 keys and 8.2 at 1,500, without parts 6.3 and 16.7 (16-row tiles a query
-// head: 7.4 and 16.9); of 10 requests 11.3 and 16.9 at 1,500, of 32 29 and 28 (42).  So, beyond 512 keys: parts of eight
-// wavefronts with a unit of 32 keys each, up to eight of them, where 512 workgroups hold four at least; else none.
-extern "C" int celeg_biased_attention_parts(int n_tokens, int kv_heads, int keys) {
-    if (keys <= 512) return 1;
-    const int useful = (keys + BF_UNIT * BF_SINGLE_WAVES - 1) / (BF_UNIT * BF_SINGLE_WAVES);
-    const int parts = std::min({std::max(useful, 4), BF_MAX_PARTS, 512 / std::max(n_tokens * kv_heads, 1)});
-    return parts < 4 ? 1 : parts;
-}
-extern "C" long long celeg_biased_attention_parts_floats(int q_heads, int v_dim, int parts) {
-    return static_cast<long long>(q_heads) * ((v_dim + 31) / 32 * 32 + 2) * parts;
-}
-
 // bfloat16 on the matrix cores; form 0: tiles of 16 rows whose key blocks the wavefronts share out
 // (single tokens, short portions), form 1: tiles of 64 rows that stage a key block once for four
 // wavefronts (portions of prompts); max_tiles: an upper bound on the step's tiles (sum over
 // requests of ceil(rows / 16 or 64)); form 2: single tokens, max_tiles rows of one token a request with their positions
-// and slots, up to 16 query heads a key/value head (parts > 1: parts_out 32-bit, celeg_biased_attention_parts_floats
-// of them a row); pages of a power of two of at least 8 tokens; q, gate and out
+// and slots, up to 16 query heads a key/value head; pages of a power of two of at least 8 tokens; q, gate and out
 // rows start at multiples of 16, 8 and 8 bytes
 extern "C" int celeg_biased_attention_fast(int form, const void* q, int ldq, const void* k_pool, const void* v_pool, const int* table,
                                            int table_stride, const int* cu_seqlens, const int* seq_slot, const int* seq_start, int n_seqs,
@@ -751,9 +682,9 @@ extern "C" int celeg_biased_attention_fast(int form, const void* q, int ldq, con
                                            int q_heads, int kv_heads, int head_dim, int v_dim, int page_tokens, int n_layers, int layer,
                                            float scale, float coef, int every, int window, int keep_first, int sink_one,
                                            const float* sink, float softcap, const int* positions, const int* token_slot,
-                                           float* parts_out, int parts, hipStream_t stream) {
+                                           hipStream_t stream) {
     if (max_tiles <= 0 || n_seqs <= 0) return 0;
-    if (form == 2 && (!positions || !token_slot || q_heads / kv_heads > 16 || parts < 1 || parts > BF_MAX_PARTS || (parts > 1 && !parts_out)))
+    if (form == 2 && (!positions || !token_slot || q_heads / kv_heads > 16))
         return static_cast<int>(hipErrorInvalidValue);
     if (!celeg_biased_attention_fast_ok(head_dim, v_dim) || q_heads % kv_heads || page_tokens < 8 || (page_tokens & (page_tokens - 1)) ||
         ldq % 8 || ldo % 4 || (gate && ldg % 4) || (r1 == nullptr) != (r2 == nullptr))
@@ -793,8 +724,6 @@ extern "C" int celeg_biased_attention_fast(int form, const void* q, int ldq, con
     BfSingle single;
     single.positions = positions;
     single.token_slot = token_slot;
-    single.parts = parts;
-    single.parts_out = parts > 1 ? parts_out : nullptr;
     switch ((head_dim + 31) / 32) {
         case 1: return bf_launch_v<32>(v_dim, form, max_tiles, a, single, stream);
         case 2: return bf_launch_v<64>(v_dim, form, max_tiles, a, single, stream);

@@ -227,9 +227,7 @@ int celeg_biased_attention_fast(int form, const void* q, int ldq, const void* k_
                                 const float* r1, const float* r2, const void* gate, int ldg, void* out, int ldo, int q_heads,
                                 int kv_heads, int head_dim, int v_dim, int page_tokens, int n_layers, int layer, float scale, float coef,
                                 int every, int window, int keep_first, int sink_one, const float* sink, float softcap,
-                                const int* positions, const int* token_slot, float* parts_out, int parts, hipStream_t stream);
-int celeg_biased_attention_parts(int n_tokens, int kv_heads, int keys);
-long long celeg_biased_attention_parts_floats(int q_heads, int v_dim, int parts);
+                                const int* positions, const int* token_slot, hipStream_t stream);
 // matrix_memory.hip
 int celeg_matrix_memory(const void* proj, int ld, int dtype, int col_q, int col_k, int col_v, int col_g, int col_i, int col_f,
                         const float* bias_i, const float* bias_f, const float* norm, float* S, size_t ldS, float* n, size_t ldn,

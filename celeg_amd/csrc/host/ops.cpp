@@ -1386,33 +1386,33 @@ void Ops::biased_attention(const Tensor& q, const Tensor& out, const ScoreShape&
         dev(*gate, "gate", q.dtype, false);
         need(gate->ndim == 2 && gate->shape[0] == T && gate->shape[1] == out.shape[1], "biased_attention: gate [rows, heads * v_dim]");
     }
+    (void)ws;
     took(Path::AttentionBiased);
     const int ldq = rows_of(q, "q"), ldo = rows_of(out, "out"), ldg = gate ? rows_of(*gate, "gate") : 0;
     auto aligned = [](const void* p, uintptr_t bytes) { return (reinterpret_cast<uintptr_t>(p) & (bytes - 1)) == 0; };
     if (q.dtype == DType::BF16 && use_biased_mfma && !attention_general && celeg_biased_attention_fast_ok(s.head_dim, s.v_dim) &&
         kv.page_tokens >= 8 && (kv.page_tokens & (kv.page_tokens - 1)) == 0 && ldq % 8 == 0 && ldo % 4 == 0 && ldg % 4 == 0 &&
         aligned(q.data, 16) && aligned(out.data, 8) && (!gate || aligned(gate->data, 8))) {
-        // single tokens (first in a step): a workgroup per key/value head or part of its keys.  Portions of prompts: tiles of
-        // 64 rows that share their staged keys; short portions: tiles of 16 rows whose key blocks the wavefronts take
-        // in turn.  At most one partly filled tile per request.
+        // Single tokens (first in a step), where a tile of 16 rows a query head would be more than a workgroup a compute unit:
+        // a workgroup per key/value head (16 heads over 8, 300 keys: 32 requests 19.0 -> 8.5 us; with 4 requests the kernels'
+        // times are 7.4 and 6.6, but a whole request of 700 to 1,500 keys was 1 % slower).  Portions of prompts: tiles of
+        // 64 rows that share their staged keys; short portions and few single tokens: tiles of 16 rows whose key blocks
+        // the wavefronts take in turn.  At most one partly filled tile per request.
         took(batch.decode_only ? Path::AttentionBiasedDecode : Path::AttentionBiasedRows);
-        const int single = biased_rows_form < 0 && s.heads / s.kv_heads <= 16 ? std::min(batch.single_rows, static_cast<int>(T)) : 0;
-        const int keys = s.window > 0 ? std::min(s.window + 7 + keep_first, batch.context_hint()) : batch.context_hint();
-        const int parts = single > 0 ? celeg_biased_attention_parts(single, s.kv_heads, keys) : 1;
-        float* parts_out = parts > 1 ? ws.buf("biased_parts", DType::F32, {single, celeg_biased_attention_parts_floats(s.heads, s.v_dim, parts)}).as<float>()
-                                     : nullptr;
+        const int tokens = std::min(batch.single_rows, static_cast<int>(T));
+        const int single = biased_rows_form == 2 || (biased_rows_form < 0 && tokens * s.heads > 256) ? (s.heads / s.kv_heads <= 16 ? tokens : 0) : 0;
         auto run = [&](int form, int tiles, int from) {
             kernel_check(celeg_biased_attention_fast(form, q.data, ldq, kv.k, kv.v, kv.table, kv.table_stride, batch.cu_seqlens + from,
                                                      batch.seq_slot + from, batch.seq_start + from, batch.n_seqs - from, tiles,
                                                      r1 ? r1->as<float>() : nullptr, r2 ? r2->as<float>() : nullptr, gate ? gate->data : nullptr,
                                                      ldg, out.data, ldo, s.heads, s.kv_heads, s.head_dim, s.v_dim, kv.page_tokens, kv.n_layers,
                                                      kv.layer, s.scale, s.coef, s.every, s.window, keep_first, sink_one, sink_at, s.softcap,
-                                                     batch.positions, batch.token_slot, parts_out, parts, stream),
+                                                     batch.positions, batch.token_slot, stream),
                          "biased attention (bfloat16, matrix cores)");
         };
         if (single > 0) run(2, single, 0);
         if (single == T) return;
-        const int form = biased_rows_form >= 0 ? biased_rows_form : (batch.max_seg_len > 16 ? 1 : 0);
+        const int form = biased_rows_form == 0 || biased_rows_form == 1 ? biased_rows_form : (batch.max_seg_len > 16 ? 1 : 0);
         run(form, (static_cast<int>(T) - single) / (form == 1 ? 64 : 16) + batch.n_seqs - single, single);
         return;
     }

@@ -139,7 +139,7 @@ public:
     bool use_delta_step = true;          // steps of one token a request: the delta rule in one kernel
     bool use_sigmoid_mfma = true;        // bfloat16 attention with sigmoid weights on the matrix cores
     bool use_biased_mfma = true;         // bfloat16 attention with a distance bias on the matrix cores
-    int biased_rows_form = -1;           // likewise for the attention with a distance bias
+    int biased_rows_form = -1;           // likewise for the attention with a distance bias (2: single tokens by themselves, however few)
     int sigmoid_rows_form = -1;          // -1: single tokens by themselves, the rest by the longest portion; all as 0 tiles of 16 rows, 1 tiles of 64 rows
     bool use_router_kernel = true;       // the router's product inside the routing kernel
     bool use_moe_mfma = true;            // bfloat16 products of routed experts and per-head matrices on the matrix cores

@@ -1881,7 +1881,6 @@ public:
         gated_ = gate == "sigmoid";
     }
     bool graph_safe() const override { return true; }
-    int short_context() const override { return 512; }      // (without parts of the keys up to there: 1 to 2 us a layer)
     std::vector<const Part*> children() const override {
         return position_ ? std::vector<const Part*>{position_.get()} : std::vector<const Part*>{};
     }

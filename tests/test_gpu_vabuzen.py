@@ -555,9 +555,9 @@ def test_keys_at_the_windows_edge_and_kept_first_keys(tmp_path, dtype):
 
 
 @pytest.mark.parametrize("H,G,D,V,mask", [(4, 2, 64, 64, None), (16, 1, 32, 128, (900, 70)), (6, 2, 96, 40, (513, 0)), (3, 3, 128, 96, (700, 3))])
-def test_single_tokens_whose_keys_are_dealt_to_several_workgroups(tmp_path, H, G, D, V, mask):
-    """bfloat16: single tokens at contexts on both sides of 512 keys (where a head's keys go to several workgroups), with
-    windows and kept first keys, behind a long portion and beside none, against the kernel that scores key by key."""
+def test_single_tokens_of_long_contexts(tmp_path, H, G, D, V, mask):
+    """bfloat16: single tokens whose wavefronts have one to three blocks of 64 keys, groups of 1 to 16 query heads, with
+    windows and kept first keys, against the kernel that scores key by key."""
     from celeg_amd.config import LayerSpec, ModelSpec, PartSpec, RunStep, register_architecture, registered_architectures
     from celeg_amd.engine import load_model
     from celeg_amd.weights.safetensors_io import write_safetensors
@@ -574,14 +574,13 @@ def test_single_tokens_whose_keys_are_dealt_to_several_workgroups(tmp_path, H, G
         json.dump({"architectures": ["VabuzenLongAlone"], "width": W_, "rows": T, "mixer": part}, fh)
     write_safetensors(str(tmp_path / "model.safetensors"), {k: v.bfloat16().contiguous() for k, v in t.items()})
     got = {}
-    cut = (500,) + (1,) * 30 + (541,) + (1,) * 29
+    cut = (630,) + (1,) * 30 + (411,) + (1,) * 29
     for general in (True, False):
         steps = portions_schedule({"x": list(range(T))}, sizes=cut)
-        lm = load_model(str(tmp_path), dtype="bfloat16", device=DEV, page_tokens=16, n_pages=72, max_requests=2, max_context=16 * 72, max_batched_tokens=600)
-        if general:
-            lm.set_knob("use_biased_mfma", 0)
+        lm = load_model(str(tmp_path), dtype="bfloat16", device=DEV, page_tokens=16, n_pages=72, max_requests=2, max_context=16 * 72, max_batched_tokens=640)
+        lm.set_knob(*(("use_biased_mfma", 0) if general else ("biased_rows_form", 2)))
         got[general] = EngineDriver(lm).run(steps)["x"].double()
-    for first in (500, T - 29):
+    for first in (630, T - 29):
         a, b = got[False][first:first + 29], got[True][first:first + 29]
         rel = float((a - b).pow(2).mean().sqrt() / b.pow(2).mean().sqrt())
         assert rel <= 1e-2, f"{H} heads of {D} and {V}, mask {mask}, from {first}: rel rms {rel:.3e}"
