@@ -14,6 +14,7 @@
 //    owns a column of S, so the three sums over dim are the lane's own and no lane waits for another;
 //  * delta_gated_norm: o / rms(o) * w * silu(gate), per head;
 //  * delta_step: all four of these for steps of one token a request.
+// (The recurrence over long portions of prompts by chunks: delta_chunks.hip.)
 #include "common.h"
 
 namespace {
