@@ -1012,11 +1012,18 @@ void Ops::delta_scan(const Tensor& qk, const Tensor& v, const Tensor& beta_decay
     need(state.ndim >= 2 && state.numel() / state.shape[0] == per_slot && state.stride[state.ndim - 1] == 1,
          "delta_scan: state must be [slots, heads, dim, vdim]");
     need(s.dim <= 256 && (s.dim <= 248 || s.dim == 256), "delta_scan: dim " + std::to_string(s.dim) + " exceeds 256");
-    // Portions of 128 rows and more by chunks of 64 (16 heads of 64 x 64, token by token | by chunks: 64 rows 17 | 24 us, 130
-    // rows 30 | 27, 1,500 rows 266 | 72).  All of it is 32-bit, but its sums run in another order, against 64 bits
-    // 1.3e-7 off where token by token is 0.8e-7: it is taken where bfloat16 rows come of it, not in 32-bit models.
-    const int least = delta_chunk_rows >= 0 ? delta_chunk_rows : rows == DType::BF16 ? 128 : 0;
-    int below = std::numeric_limits<int>::max();
+    // Long portions by chunks of 64 tokens: where bfloat16 rows come of it (32-bit models keep the chain of tokens), from 192 rows
+    // on, and where the longest has 192 for every round that the chunks' first kernel, a workgroup a (chunk, head), takes on the
+    // compute units: the chain's time is the longest portion's, the chunks' that of all of them.  16 heads of 64 x 64, token by token |
+    // by chunks, us: 128 rows 28 | 31, 192 rows 39 | 35, 1,500 rows 269 | 117, three requests of 2,048 in all 207 | 126, two of 256 60 |
+    // 47, four of 192 49 | 49, six of 320 94 | 93; left to the chain: five of 400 110 | 114, eight of 256 80 | 94.
+    int least = delta_chunk_rows >= 0 ? delta_chunk_rows : rows == DType::BF16 ? 192 : 0, below = std::numeric_limits<int>::max();
+    const auto& lens = batch.host_seg_lens;
+    if (least > 0 && delta_chunk_rows < 0) {
+        int long_chunks = 0;
+        for (int n : lens) long_chunks += n >= least ? (n + 63) / 64 : 0;
+        if (batch.max_seg_len < 192 * ((long_chunks * s.heads + 255) / 256)) least = 0;
+    }
     if (least > 0 && batch.max_seg_len >= least && !delta_general && celeg_delta_chunks_ok(s.kv_heads, s.heads, s.dim, s.vdim)) {
         below = least;
         const int chunks = static_cast<int>(T) / 64 + batch.n_seqs;
@@ -1025,7 +1032,6 @@ void Ops::delta_scan(const Tensor& qk, const Tensor& v, const Tensor& beta_decay
                                         static_cast<size_t>(state.stride[0]), batch.cu_seqlens, batch.seq_slot, out.as<float>(),
                                         chunk_ws.as<float>(), batch.n_seqs, chunks, least, s.kv_heads, s.heads, s.dim, s.vdim, stream),
                      "delta_chunks");
-        const auto& lens = batch.host_seg_lens;
         const bool all = lens.size() == static_cast<size_t>(batch.n_seqs) && std::all_of(lens.begin(), lens.end(), [&](int n) { return n >= least; });
         if (all || (batch.n_seqs == 1)) return;
     }
