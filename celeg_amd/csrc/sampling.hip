@@ -62,9 +62,9 @@ __device__ __forceinline__ float key_score(uint32_t key) {      // the inverse o
 
 // The top_k scores of a row (score = penalised logit / temperature) by (score desc, id
 // asc), left unordered in cand_score / cand_id [0, top_k).  All threads of the workgroup
-// call it.  Every pass walks the row in memory: this is the way for rows that the two below cannot take (more
-// than 131,072 logits, thousands of equal ones).  (Forms of it with the row's keys in registers made the kernel 387 KB of code, for
-// whose sake the other ways' scalar registers were spilled.)
+// call it.  Every pass walks the row in memory: this is the way for rows that the two below cannot take (thousands of
+// equal logits; 270 us at 65,536 of them).  (Forms of it with the row's keys in registers made the kernel 387 KB of code, for
+// whose sake the other ways' scalar registers were spilled, and took no less.)
 __device__ __forceinline__ void top_k_candidates(
     const float* __restrict__ row, const uint8_t* __restrict__ seen, float penalty, float temperature,
     int vocab, int top_k, unsigned int* hist, unsigned int* sel, int* running, float* cand_score,
@@ -210,13 +210,13 @@ __device__ __forceinline__ void top_k_candidates(
     __syncthreads();
 }
 
-// The same candidates by ranking, for rows whose logits fit in registers, already in the
+// The same candidates by ranking, already in the
 // order (score desc, id asc); false (nothing written) if more logits than SAMPLE_RANK_CAP
 // reach the bound from below, as when very many are equal: the caller then selects by
 // counting passes as above.
-//   1. Every thread keeps its logits as ordered keys of a cheap stand-in for the score
-//      (the penalty applied by multiplication, no division by the temperature: the same
-//      order up to a unit or two in the last place) and finds its largest.
+//   1. Every thread finds the largest of its logits' keys: of a cheap stand-in for the score
+//      (no division by the temperature, with KPT > 0 the penalty applied by multiplication: the same
+//      order up to a unit or two in the last place).
 //   2. A bound from below: with c = ceil(top_k / 16), the c-th largest thread maximum of
 //      each of the 16 wavefronts; at least 16 c >= top_k logits reach the smallest of these
 //      16 values, so the top_k-th largest stand-in does too.  Eight units in the last place
@@ -226,13 +226,19 @@ __device__ __forceinline__ void top_k_candidates(
 //      a thread per such logit counts the ones that come before it: that is its place.
 // Five workgroup barriers instead of about forty, and two divisions per gathered logit
 // instead of per logit.
+// KPT > 0: the keys stay in registers, KPT a thread, between the two looks at them; KPT == 0: both walk the row in memory
+// (what the first leaves in the caches).  One row, top_k 50, us in registers | in memory: 12,001 logits 19.8 | 10.4, 18,000
+// 15.4 | 12.7, 65,536 15.5 | 20.0, 128 a thread for 100,352 53.8 | 23.8: registers from 32,769 to 65,536, and not in the
+// kernel whose first way is another one, which they would slow down.
 #define SAMPLE_RANK_CAP 2048
 __device__ __forceinline__ void rank_gathered(int top_k, int n, const unsigned long long* gathered, unsigned int* counts, float* cand_score,
                                               int* cand_id);
-// a logit's score as the reference computes it
+// a logit under its penalty, and its score, as the reference computes them
+__device__ __forceinline__ float penalised(float x, bool marked, float penalty) {
+    return !marked ? x : x >= 0.0f ? x / penalty : x * penalty;
+}
 __device__ __forceinline__ float exact_score(float x, bool marked, float penalty, float temperature) {
-    if (marked) x = x >= 0.0f ? x / penalty : x * penalty;
-    return x / temperature;
+    return penalised(x, marked, penalty) / temperature;
 }
 template <int KPT>
 __device__ __forceinline__ bool top_k_ranked(
@@ -250,8 +256,18 @@ __device__ __forceinline__ bool top_k_ranked(
     const bool by_fours = (vocab & 3) == 0 && (reinterpret_cast<uintptr_t>(row) & 15) == 0 &&
                           (!pen || (reinterpret_cast<uintptr_t>(seen) & 3) == 0);
     auto index_of = [&](int j) { return by_fours ? 4 * (tid + SAMPLE_THREADS * (j >> 2)) + (j & 3) : tid + SAMPLE_THREADS * j; };
-    uint32_t keys[KPT];
-    if (by_fours) {
+    // (KPT == 0: rows so short that groups of four would leave wavefronts without any go one by one)
+    auto walk = [&](auto f) {
+        if (vocab >= 4 * SAMPLE_THREADS) {
+            for_each_logit(row, seen, penalty, vocab, tid, f);
+            return;
+        }
+        for (int i = tid; i < vocab; i += SAMPLE_THREADS) f(penalised(row[i], pen && seen[i], penalty), i);
+    };
+    uint32_t keys[KPT > 0 ? KPT : 1], my_max = 0u;
+    if constexpr (KPT == 0) {
+        walk([&](float x, int) { my_max = max(my_max, order_key(x)); });
+    } else if (by_fours) {
         floatx4_t v[KPT / 4];
         unsigned sn[KPT / 4];
         const int n4 = vocab >> 2;
@@ -284,7 +300,6 @@ __device__ __forceinline__ bool top_k_ranked(
             keys[j] = tid + SAMPLE_THREADS * j < vocab ? order_key(x) : 0u;
         }
     }
-    uint32_t my_max = 0u;
 #pragma unroll
     for (int j = 0; j < KPT; ++j) my_max = max(my_max, keys[j]);
     // the c-th largest maximum of this wavefront: c times the largest, one lane struck out each time
@@ -303,6 +318,13 @@ __device__ __forceinline__ bool top_k_ranked(
 #pragma unroll
     for (int w = 1; w < SAMPLE_THREADS / CELEG_WAVE; ++w) lower = min(lower, wave_bound[w]);
     lower = lower > 8u ? lower - 8u : 0u;
+    if constexpr (KPT == 0)
+        walk([&](float x, int i) {
+            if (order_key(x) >= lower) {
+                const unsigned int p = atomicAdd(&sel[1], 1u);
+                if (p < SAMPLE_RANK_CAP) gathered[p] = packed_logit(x / temperature, i);
+            }
+        });
 #pragma unroll
     for (int j = 0; j < KPT; ++j)
         if (index_of(j) < vocab && keys[j] >= lower) {
@@ -312,10 +334,11 @@ __device__ __forceinline__ bool top_k_ranked(
     __syncthreads();
     const int n = static_cast<int>(sel[1]);
     if (n > SAMPLE_RANK_CAP) return false;       // the same for every thread
-    for (int e = tid; e < n; e += SAMPLE_THREADS) {
-        const int id = static_cast<int>(gathered[e]);
-        gathered[e] = packed_logit(exact_score(row[id], pen && seen[id], penalty, temperature), id);
-    }
+    if constexpr (KPT > 0)
+        for (int e = tid; e < n; e += SAMPLE_THREADS) {
+            const int id = static_cast<int>(gathered[e]);
+            gathered[e] = packed_logit(exact_score(row[id], pen && seen[id], penalty, temperature), id);
+        }
     __syncthreads();
     rank_gathered(top_k, n, gathered, counts, cand_score, cand_id);
     return true;
@@ -382,7 +405,9 @@ __device__ __forceinline__ void rank_gathered(int top_k, int n, const unsigned l
 //      (a few hundred logits instead of the row), and what reaches the bound is gathered and ranked
 //      as in top_k_ranked.
 // false (nothing written that matters) if the parts are too many for the threads, too few to bound
-// anything, or more parts or logits reach the bound than there is room for: the caller then reads the row.
+// anything, or more parts or logits reach the bound than there is room for (a penalty that throws many of the best far down): the
+// caller then ranks the row in memory (us, at the counting passes | ranked: one row of 100,352 logits in parts of 16
+// columns 119 | 24, 64 of 50,257 in parts of 57 90 | 29, one of 65,536 with its 300 best ones seen and a penalty of 1.4 97 | 25).
 #define SAMPLE_PARTS_PER_THREAD 4
 #define SAMPLE_PART_LIST 1024
 __device__ __forceinline__ bool top_k_from_parts(
@@ -427,10 +452,10 @@ __device__ __forceinline__ bool top_k_from_parts(
     if (lower_max == 0u) return false;           // (some wavefront has fewer than c parts: nothing is bounded)
     // a thread whose best reaches the bound holds one of top_k different logits at least: the penalised value, its
     // wavefront's smallest by one atomic
-    uint32_t penalised = 0xffffffffu;
-    if (my_max >= lower_max) penalised = order_key(stand_in(key_score(my_max), pen ? seen[packed_logit_index(my_best)] : 0u));
-    penalised = ~group_max_u32<CELEG_WAVE>(~penalised);
-    if (lane == 0 && penalised != 0xffffffffu) atomicMin(&sel[2], penalised);
+    uint32_t smallest = 0xffffffffu;
+    if (my_max >= lower_max) smallest = order_key(stand_in(key_score(my_max), pen ? seen[packed_logit_index(my_best)] : 0u));
+    smallest = ~group_max_u32<CELEG_WAVE>(~smallest);
+    if (lane == 0 && smallest != 0xffffffffu) atomicMin(&sel[2], smallest);
     __syncthreads();
     const uint32_t lowest = sel[2];
     const uint32_t lower = lowest > 8u ? lowest - 8u : 0u;
@@ -560,8 +585,8 @@ __device__ __forceinline__ int choose_among(float* cand_score, int* cand_id, int
 // token is given out, nothing is chosen), seen_row or -1, slot or -1}; the token also goes to last_tokens[slot] (if given and slot >= 0), where the
 // next step can take it from without the host in between, and is marked as seen in the row's
 // seen_row (if any): the step that feeds it back need not mark it.
-// PARTS: the head left the best of every part of the columns (else best is null).  Two kernels, because the one that holds
-// a row in registers is large (its scalar registers spill) and slows the other down where both are one.
+// PARTS: the head left the best of every part of the columns (else best is null).  Two kernels, because the one that may
+// hold a row in registers is large (its scalar registers spill) and slows the other down where both are one.
 template <bool PARTS>
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     const float* __restrict__ logits, int ld, int vocab, const float* __restrict__ fparams,
@@ -641,10 +666,15 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
         sorted = top_k_from_parts(row, seen, penalty, temperature, vocab, top_k, best + static_cast<size_t>(r) * best_ld, best_parts, best_cols, maxes,
                                   gathered, sel, part_list, cand_score, cand_id);
         __syncthreads();        // (before what follows reuses the counters)
-    } else if (vocab <= SAMPLE_THREADS * 64) {
+        if (!sorted) {
+            sorted = top_k_ranked<0>(row, seen, penalty, temperature, vocab, top_k, maxes, gathered, sel, part_list, cand_score, cand_id);
+            __syncthreads();
+        }
+    } else if (vocab > SAMPLE_THREADS * 32 && vocab <= SAMPLE_THREADS * 64) {
         sorted = top_k_ranked<64>(row, seen, penalty, temperature, vocab, top_k, maxes, gathered, sel, part_list, cand_score, cand_id);
-    } else if (vocab <= SAMPLE_THREADS * 128) {
-        sorted = top_k_ranked<128>(row, seen, penalty, temperature, vocab, top_k, maxes, gathered, sel, part_list, cand_score, cand_id);
+    } else {
+        sorted = top_k_ranked<0>(row, seen, penalty, temperature, vocab, top_k, maxes, gathered, sel, part_list, cand_score, cand_id);
+        __syncthreads();
     }
     if (!sorted) top_k_candidates(row, seen, penalty, temperature, vocab, top_k, hist, sel, running, cand_score, cand_id);
     if (tid >= top_k && tid < SAMPLE_MAX_K) { cand_score[tid] = -INFINITY; cand_id[tid] = 0x7fffffff; }
