@@ -1019,15 +1019,16 @@ void Ops::delta_scan(const Tensor& qk, const Tensor& v, const Tensor& beta_decay
     // 47, four of 192 49 | 49, six of 320 94 | 93; left to the chain: five of 400 110 | 114, eight of 256 80 | 94.
     int least = delta_chunk_rows >= 0 ? delta_chunk_rows : rows == DType::BF16 ? 192 : 0, below = std::numeric_limits<int>::max();
     const auto& lens = batch.host_seg_lens;
-    if (least > 0 && delta_chunk_rows < 0) {
-        int long_chunks = 0;
-        for (int n : lens) long_chunks += n >= least ? (n + 63) / 64 : 0;
-        if (batch.max_seg_len < 192 * ((long_chunks * s.heads + 255) / 256)) least = 0;
-    }
-    if (least > 0 && batch.max_seg_len >= least && !delta_general && celeg_delta_chunks_ok(s.kv_heads, s.heads, s.dim, s.vdim)) {
+    int chunks = 0;
+    if (least > 0)
+        for (int n : lens) chunks += n >= least ? (n + 63) / 64 : 0;
+    if (delta_chunk_rows < 0 && batch.max_seg_len < 192 * ((chunks * s.heads + 255) / 256)) chunks = 0;
+    if (chunks > 0 && !delta_general && celeg_delta_chunks_ok(s.kv_heads, s.heads, s.dim, s.vdim)) {
         below = least;
-        const int chunks = static_cast<int>(T) / 64 + batch.n_seqs;
-        Tensor chunk_ws = ws.buf("delta_chunks", DType::F32, {celeg_delta_chunks_floats(chunks, s.heads, s.vdim)});
+        // (room for as many chunks as T rows can have, so that it does not grow with the requests beside a portion: a chunk
+        // of 16 heads of 64 x 64 is 1.9 MB, and a workspace that grows has every recorded step recorded again)
+        const int most = static_cast<int>(T / 64 + T / least);
+        Tensor chunk_ws = ws.buf("delta_chunks", DType::F32, {celeg_delta_chunks_floats(most, s.heads, s.vdim)});
         kernel_check(celeg_delta_chunks(qk.as<float>(), v.as<float>(), beta_decay.as<float>(), state.as<float>(),
                                         static_cast<size_t>(state.stride[0]), batch.cu_seqlens, batch.seq_slot, out.as<float>(),
                                         chunk_ws.as<float>(), batch.n_seqs, chunks, least, s.kv_heads, s.heads, s.dim, s.vdim, stream),

@@ -300,6 +300,34 @@ def test_delta_rule_by_chunks_equals_token_by_token(tmp_path, heads, kv_heads, v
             assert_close_f32(got[33][rid], got[0][rid], rid)
 
 
+def test_requests_beside_a_portion_leave_recorded_steps_alone(tmp_path):
+    """bfloat16: what the chunks of a portion are kept in has room for the step's rows, however many requests these are of,
+    so steps recorded before are replayed after a step of as many rows and more requests."""
+    from celeg_amd.engine import StepEntry, load_model
+    cfg = {"architecture": "Kifetar", "vocab": 150, "width": 64, "norm": {"eps": 1e-5}, "max_context": 1024,
+           "layers": [delta(4, 2, 64, 64, 4)]}
+    folder = write_model(tmp_path / "beside", cfg, 47, torch.bfloat16, std=0.2)
+    reqs = {str(i): random_tokens(cfg["vocab"], 400, seed=20 + i) for i in range(20)}
+    lm = load_model(folder, dtype="bfloat16", device=DEV, page_tokens=16, n_pages=20 * 25, max_requests=20, max_context=400,
+                    max_batched_tokens=320)
+    slots, at = [lm.cache.open() for _ in reqs], [0] * len(reqs)
+
+    def step(*entries):
+        batch = []
+        for i, n, want in entries:
+            assert lm.cache.prepare(slots[i], at[i], n)
+            batch.append(StepEntry(slots[i], at[i], reqs[str(i)][at[i]:at[i] + n], list(range(n - want, n))))
+            at[i] += n
+        lm.runner.step(batch)
+        return lm.runner.counters()["captures"]
+    decode = [(i, 1, 1) for i in range(20)]
+    step(*decode)
+    step((0, 296, 16), (2, 4, 4))
+    before = step(*decode)
+    step((1, 281, 1), *[(i, 1, 1) for i in range(2, 20)], (0, 1, 1))
+    assert step(*decode) == before
+
+
 def test_delta_rule_in_registers_equals_the_general_kernel(folders):
     """32-bit: the recurrence with the state in registers against the kernel for any size, same schedule."""
     folder = folders("K4", "float32")
