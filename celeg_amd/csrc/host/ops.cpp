@@ -1019,7 +1019,7 @@ void Ops::delta_scan(const Tensor& qk, const Tensor& v, const Tensor& beta_decay
     // 47, four of 192 49 | 49, six of 320 94 | 93; left to the chain: five of 400 110 | 114, eight of 256 80 | 94.
     int least = delta_chunk_rows >= 0 ? delta_chunk_rows : rows == DType::BF16 ? 192 : 0, below = std::numeric_limits<int>::max();
     const auto& lens = batch.host_seg_lens;
-    int chunks = 0;
+    int chunks = 0, n_seqs = batch.n_seqs, n_tokens = batch.n_tokens;
     if (least > 0)
         for (int n : lens) chunks += n >= least ? (n + 63) / 64 : 0;
     if (delta_chunk_rows < 0 && batch.max_seg_len < 192 * ((chunks * s.heads + 255) / 256)) chunks = 0;
@@ -1033,16 +1033,17 @@ void Ops::delta_scan(const Tensor& qk, const Tensor& v, const Tensor& beta_decay
                                         static_cast<size_t>(state.stride[0]), batch.cu_seqlens, batch.seq_slot, out.as<float>(),
                                         chunk_ws.as<float>(), batch.n_seqs, chunks, least, s.kv_heads, s.heads, s.dim, s.vdim, stream),
                      "delta_chunks");
-        const bool all = lens.size() == static_cast<size_t>(batch.n_seqs) && std::all_of(lens.begin(), lens.end(), [&](int n) { return n >= least; });
-        if (all || (batch.n_seqs == 1)) return;
+        // what is left: single tokens lie first in a step, then the portions up to the last short one
+        while (n_seqs > 0 && lens[static_cast<size_t>(n_seqs - 1)] >= least) n_tokens -= lens[static_cast<size_t>(--n_seqs)];
+        if (n_seqs == 0) return;
     }
     // rows that have a neighbour in their request's step are taken two at a time
     float* pairs = nullptr;
-    if (delta_pairs && !delta_general && batch.n_tokens > batch.n_seqs)
+    if (delta_pairs && !delta_general && n_tokens > n_seqs)
         pairs = ws.buf("delta_pairs", DType::F32, {T, 4LL * s.kv_heads}).as<float>();
     kernel_check(celeg_delta_scan(qk.as<float>(), v.as<float>(), beta_decay.as<float>(), state.as<float>(),
-                                  static_cast<size_t>(state.stride[0]), batch.cu_seqlens, batch.seq_slot, out.as<float>(), batch.n_seqs,
-                                  s.kv_heads, s.heads, s.dim, s.vdim, delta_general ? 1 : 0, batch.token_seq, pairs, batch.n_tokens, below,
+                                  static_cast<size_t>(state.stride[0]), batch.cu_seqlens, batch.seq_slot, out.as<float>(), n_seqs,
+                                  s.kv_heads, s.heads, s.dim, s.vdim, delta_general ? 1 : 0, batch.token_seq, pairs, n_tokens, below,
                                   stream), "delta_scan");
 }
 

@@ -300,6 +300,30 @@ def test_delta_rule_by_chunks_equals_token_by_token(tmp_path, heads, kv_heads, v
             assert_close_f32(got[33][rid], got[0][rid], rid)
 
 
+def test_long_and_short_portions_and_single_tokens_in_one_step(tmp_path):
+    """32-bit: portions by chunks (from 33 rows on) before, between and behind shorter ones and single tokens of the same step,
+    against the recurrence token by token."""
+    cfg = {"architecture": "Kifetar", "vocab": 150, "width": 64, "norm": {"eps": 1e-5}, "max_context": 1024,
+           "layers": [delta(4, 2, 64, 64, 4), delta(2, 2, 64, 32, 2)]}
+    folder = write_model(tmp_path / "mixed", cfg, 53, torch.float32, std=0.2)
+    cuts = [(1, 50, 5, 70, 20), (1, 1, 64, 3, 40), (1, 1, 1, 90, 33), (130, 1, 7, 1, 1), (2, 40, 32, 35, 1), (1, 1, 1, 1, 34)]
+    reqs = {name: random_tokens(cfg["vocab"], sum(c[i] for c in cuts), seed=60 + i) for i, name in enumerate("abcde")}
+    steps, at = [], {name: 0 for name in reqs}
+    for n, cut in enumerate(cuts):
+        entries = []
+        for name, m in zip(reqs, cut):
+            entries.append({"id": name, "tokens": reqs[name][at[name]:at[name] + m], "want": list(range(m))})
+            at[name] += m
+        steps.append({"step": n, "entries": entries, "end": list(reqs) if n + 1 == len(cuts) else []})
+    got = {}
+    for rows in (0, 33):
+        lm, _ = load(folder, "float32", steps, max_requests=5)
+        lm.set_knob("delta_chunk_rows", rows)
+        got[rows] = EngineDriver(lm).run(steps)
+    for name in reqs:
+        assert_close_f32(got[33][name], got[0][name], name)
+
+
 def test_requests_beside_a_portion_leave_recorded_steps_alone(tmp_path):
     """bfloat16: what the chunks of a portion are kept in has room for the step's rows, however many requests these are of,
     so steps recorded before are replayed after a step of as many rows and more requests."""
