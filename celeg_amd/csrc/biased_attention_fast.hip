@@ -623,14 +623,9 @@ struct BfSingle {
 template <int D, int V, bool FULL>
 int bf_launch_single(int n_tokens, const BfArgs& a, const BfSingle& p, hipStream_t stream) {
     constexpr int WAVES = bf_tile_waves(D, V);
+    static_assert(WAVES * 16 * bf_entry<V>() * sizeof(float) <= 64 * 1024, "within what a launch may ask for by itself");      // (16 heads of 96: 53 KB)
     const size_t lds = static_cast<size_t>(WAVES) * (a.q_heads / a.kv_heads) * bf_entry<V>() * sizeof(float);
     auto kernel = &biased_attention_single_kernel<D, V, WAVES, FULL>;
-    static bool raised = false;              // (16 heads of 96: 53 KB)
-    if (lds > 48 * 1024 && !raised) {
-        hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
-        if (err != hipSuccess) return static_cast<int>(err);
-        raised = true;
-    }
     hipLaunchKernelGGL(kernel, dim3(n_tokens, a.kv_heads), dim3(WAVES * CELEG_WAVE), lds, stream, a, p.positions, p.token_slot);
     return CELEG_LAUNCH_RESULT();
 }

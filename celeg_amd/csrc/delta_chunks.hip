@@ -385,14 +385,11 @@ extern "C" int celeg_delta_chunks(const float* qk, const float* v, const float* 
                                   int G, int H, int D, int V, hipStream_t stream) {
     if (n_seqs <= 0 || max_chunks <= 0) return 0;
     if (!celeg_delta_chunks_ok(G, H, D, V) || least < 1) return static_cast<int>(hipErrorInvalidValue);
-    // (V = 64: 119 KB, 128: 153 KB)
+    // (V = 64: 119 KB, 128: 153 KB; asked for with every call, since the limit is the current device's)
     const size_t lds = DC_ROWS * DC_PITCH * sizeof(float) + static_cast<size_t>(2 * DC_ROWS + V) * DC_PITCH64 * sizeof(double);
-    static bool raised = false;
-    if (!raised) {
-        hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_chunk_prepare_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 156 * 1024);
-        if (err != hipSuccess) return static_cast<int>(err);
-        raised = true;
-    }
+    const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_chunk_prepare_kernel),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+    if (err != hipSuccess) return static_cast<int>(err);
     hipLaunchKernelGGL(delta_chunk_prepare_kernel, dim3(max_chunks, H), dim3(DC_PREPARE_THREADS), lds, stream, qk, v, beta_decay, cu_seqlens, ws,
                        n_seqs, least, G, H, V);
     hipLaunchKernelGGL(delta_chunk_scan_kernel, dim3(n_seqs, H, V / 16), dim3(256), 0, stream, state, state_stride, cu_seqlens, seq_slot, ws,
