@@ -115,11 +115,13 @@ def test_chunks_are_no_further_from_the_exact_result_than_the_chain(lens, G, H, 
 
 
 # (sizes with two, four and eight wavefronts a head and with 8 and 16 rows of S each)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("G,H,D,V,mean,pace", [(8, 16, 64, 64, 0.0, 0.0), (4, 8, 64, 64, 1.0, -3.0), (2, 8, 64, 32, 0.5, -1.0),
                                                (2, 16, 32, 64, 0.5, -3.0), (4, 4, 128, 64, 1.0, -2.0)])
-def test_a_step_in_one_kernel_is_no_further_from_the_exact_result_than_in_four(G, H, D, V, mean, pace):
-    """32-bit: 60 steps of three requests, in one kernel and in four, each from the state that it left itself; the exact
-    ones from the convolved, normed inputs that both make alike."""
+def test_a_step_in_one_kernel_is_no_further_from_the_exact_result_than_in_four(G, H, D, V, mean, pace, dtype):
+    """60 steps of three requests, in one kernel and in four, each from the state that it left itself; the exact
+    ones from the convolved, normed inputs that both make alike.  (bfloat16: the rounding of the result is nearly all of
+    the distance in both.)"""
     n, taps, steps, eps = 3, 4, 60, 1e-6
     C = 2 * G * D + H * V
     ld, col_b, col_a = C + H * V + 2 * H, C + H * V, C + H * V + H
@@ -132,19 +134,19 @@ def test_a_step_in_one_kernel_is_no_further_from_the_exact_result_than_in_four(G
     exact = states[0].double()
     slots, cu, seq, zero = ints([2, 0, 1]), ints([0, 1, 2, 3]), ints([0, 1, 2]), ints([0, 0, 0])
     conv_stride, stride = ctypes.c_size_t((taps - 1) * C), ctypes.c_size_t(H * D * V)
-    lib = native.lib()
+    lib, code = native.lib(), int(dtype == torch.bfloat16)
     qk, v, gates, o = (torch.empty(n, w, device=DEV) for w in (2 * G * D, H * V, 2 * H, H * V))
     off, size = [0.0, 0.0], 0.0
     for _ in range(steps):
-        proj, outs = rand(n, ld) + mean, [torch.empty(n, H * V, device=DEV) for _ in range(2)]
-        gate = ctypes.c_void_p(proj.data_ptr() + 4 * C)
-        check(lib.celeg_delta_prepare(ptr(proj), ld, 0, col_b, col_a, ptr(conv_w), ptr(a_log), ptr(dt_bias), ptr(saved[0]), conv_stride,
+        proj, outs = (rand(n, ld) + mean).to(dtype), [torch.empty(n, H * V, dtype=dtype, device=DEV) for _ in range(2)]
+        gate = ctypes.c_void_p(proj.data_ptr() + proj.element_size() * C)
+        check(lib.celeg_delta_prepare(ptr(proj), ld, code, col_b, col_a, ptr(conv_w), ptr(a_log), ptr(dt_bias), ptr(saved[0]), conv_stride,
                                       ptr(zero), ptr(seq), ptr(zero), ptr(slots), ptr(qk), ptr(v), ptr(gates), n, G, H, D, V, taps, None))
-        check(lib.celeg_delta_conv_state(ptr(proj), ld, 0, ptr(saved[0]), conv_stride, ptr(cu), ptr(slots), n, C, taps, None))
+        check(lib.celeg_delta_conv_state(ptr(proj), ld, code, ptr(saved[0]), conv_stride, ptr(cu), ptr(slots), n, C, taps, None))
         check(lib.celeg_delta_scan(ptr(qk), ptr(v), ptr(gates), ptr(states[0]), stride, ptr(cu), ptr(slots), ptr(o), n, G, H, D, V, 0, ptr(seq),
                                    None, n, NO_LIMIT, None))
-        check(lib.celeg_delta_gated_norm(ptr(o), ptr(norm_w), gate, ld, 0, ctypes.c_float(eps), ptr(outs[0]), n, H, V, 0, None))
-        check(lib.celeg_delta_step(ptr(proj), ld, 0, col_b, col_a, ptr(conv_w), ptr(a_log), ptr(dt_bias), ptr(saved[1]), conv_stride,
+        check(lib.celeg_delta_gated_norm(ptr(o), ptr(norm_w), gate, ld, code, ctypes.c_float(eps), ptr(outs[0]), n, H, V, 0, None))
+        check(lib.celeg_delta_step(ptr(proj), ld, code, col_b, col_a, ptr(conv_w), ptr(a_log), ptr(dt_bias), ptr(saved[1]), conv_stride,
                                    ptr(states[1]), stride, ptr(slots), ptr(norm_w), gate, ld, ctypes.c_float(eps), 0, ptr(outs[1]), n, G, H, D,
                                    V, taps, None))
         heads = qk.double().view(n, 2, G, D).repeat_interleave(H // G, 2)
@@ -158,6 +160,6 @@ def test_a_step_in_one_kernel_is_no_further_from_the_exact_result_than_in_four(G
             for i in range(2):
                 off[i] += float(((outs[i][t].double().view(H, V) - y) ** 2).sum())
         assert torch.equal(saved[0], saved[1])
-    assert math.sqrt(off[1] / size) <= math.sqrt(off[0] / size)
+    assert math.sqrt(off[1] / size) <= (1.0 if dtype == torch.float32 else 1.01) * math.sqrt(off[0] / size)
     # (both round the state once a step in the same way; what differs, the sums that go into it, is the smaller part)
     assert distance(states[1], exact) <= 1.02 * distance(states[0], exact)
