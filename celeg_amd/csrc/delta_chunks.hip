@@ -9,7 +9,7 @@
 //  * delta_chunk_prepare, a workgroup a (chunk, head), all at once: L, then W and U' with (I + L) W = b A K and
 //    (I + L) U' = b V by blocks of 16 rows, P_ij = R_ij q_i.k_j, A_i and R_Cj;
 //  * delta_chunk_scan, a workgroup per (request, head, 16 columns of S), the chain: U = U' - W S, then the state;
-//    four wavefronts share a chunk's rows and meet twice, the next chunk's operands on their way meanwhile;
+//    four wavefronts share a chunk's rows and meet twice, the next two chunks' operands on their way meanwhile;
 //  * delta_chunk_out, a workgroup a (chunk, head, 16 columns), all at once: O = A q S + P U.
 //
 // U' - W S and A q S + P U are differences of large numbers where keys are alike, so in 32-bit this form is 1.2 to 3.5 times
@@ -19,6 +19,8 @@
 // 0.8e-7 | 1.3e-7 | 0.25e-7, alike and no decay 2.0e-7 | 3.4e-7 | 0.43e-7, of four dimensions 0.9e-7 | 3.1e-7 | 0.29e-7.
 // 16 heads of 64 x 64: 1,500 tokens 269 us token by token, 117 as these three (37 + 60 + 19; all 32-bit they were 72), three
 // requests of 2,048 in all 207 and 126.  (Operands two chunks ahead and four chains of sums in the scan: 127 -> 117.)
+//
+// Keys of 64 only: at 128 a chunk's keys, triangle and right sides do not fit LDS.
 //
 // v_mfma_f64_16x16x4_f64: lane l gives row l % 16 of the first operand and column l % 16 of the second at value l / 16 of k,
 // and holds rows l / 16 + 4 e of column l % 16 of the sums.  The first operand's rows are dealt to the lanes so that these
@@ -360,8 +362,22 @@ __global__ __launch_bounds__(256) void delta_chunk_out_kernel(const float* __res
     for (int p = 0; p < 4; ++p) sum = dc_piece(dc_wide(q4[p]), dc_wide(s4[p]), sum);
     sum *= before;
 #pragma unroll
-    for (int p = 0; p < 4; ++p)
-        if (p <= wave) sum = dc_piece(p4[p], u4[p], sum);
+    for (int p = 0; p < 3; ++p)
+        if (p < wave) sum = dc_piece(p4[p], u4[p], sum);
+    // (the tile on the diagonal, whose operands are the last piece's whatever the wavefront; the zeros above the diagonal
+    // must not meet a later token's infinities or NaN)
+    bool odd = false;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) odd = odd || !(fabs(u4[3][e]) < static_cast<double>(INFINITY));
+    if (__ballot(odd) == 0ull) {
+        sum = dc_piece(p4[3], u4[3], sum);
+    } else {
+        const double* const p_tile = reinterpret_cast<const double*>(mine + DC_P) + static_cast<size_t>(16 * wave) * C + 16 * wave;
+        const double* const u_tile = u - 4 * q + 16 * wave;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            for (int j = 0; j <= 4 * q + e; ++j) sum[e] = fma(p_tile[(4 * q + e) * C + j], u_tile[j], sum[e]);
+    }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const int row = 16 * wave + 4 * q + e;

@@ -114,6 +114,20 @@ def test_chunks_are_no_further_from_the_exact_result_than_the_chain(lens, G, H, 
     assert distance(states, want_states) <= distance(chain_states, want_states)
 
 
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("at", [0, 15, 100, 127, 129, 199])
+def test_a_value_that_is_not_finite_reaches_no_earlier_token(value, at):
+    """One value of one token: the outputs before it are what they are without it, those from it on are not finite."""
+    case, H, V, column = Portions([200], 2, 4, 64, "apart", 0.05, 0.3), 4, 64, 70
+    clean = case.run(True)[0]
+    case.v[at, column] = value
+    out = case.run(True)[0]
+    assert torch.equal(out[:at], clean[:at])
+    assert not bool(torch.isfinite(out[at:, column]).any())
+    others = [c for c in range(H * V) if c != column]
+    assert torch.equal(out[:, others], clean[:, others])
+
+
 # (sizes with two, four and eight wavefronts a head and with 8 and 16 rows of S each)
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("G,H,D,V,mean,pace", [(8, 16, 64, 64, 0.0, 0.0), (4, 8, 64, 64, 1.0, -3.0), (2, 8, 64, 32, 0.5, -1.0),
