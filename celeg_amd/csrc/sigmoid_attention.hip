@@ -89,6 +89,7 @@ __global__ __launch_bounds__(CELEG_WAVE) void sigmoid_attention_kernel(
 }
 
 // ---------------------------------------------------------------- bfloat16 on the matrix cores
+// (Single tokens have a kernel of their own, below, where up to 16 query heads share a key/value head.)
 // One workgroup of four wavefronts (eight for heads of up to 64 values, whose staging areas fit)
 // per (16 rows of one request's step, query head).  The keys
 // the rows can see, from the first key of the first row's window (rounded down to 8, which stays
@@ -417,7 +418,8 @@ __global__ __launch_bounds__(SA_WAVES * CELEG_WAVE) void sigmoid_attention_rows_
 // What bounds such a call is not its bytes in all but what one compute unit draws from them (some 50 GB/s: a window of
 // 1,024 keys of 64, 256 KB, takes 5 us behind 3 of launch and chain) and the chain position -> page -> keys -> weights -> sum.
 // So the keys are dealt to several workgroups, whose sums a second kernel adds (weights are not normalised: the parts just
-// add up), and nothing on the chain goes through LDS: a unit's keys and values travel from the pages straight into
+// add up; a row's order of sums is therefore that of the number of parts, which the rows of the step choose too), and nothing
+// on the chain goes through LDS: a unit's keys and values travel from the pages straight into
 // the registers of the matrix instruction that takes them.  Row 4 quad + i of score tile kt stands for key
 // 8 quad + 4 kt + i of the unit, so that a lane ends up with the weights of eight keys that lie side by side, the eight that
 // its 16 bytes of a page's values hold.
