@@ -324,6 +324,25 @@ def test_long_and_short_portions_and_single_tokens_in_one_step(tmp_path):
         assert_close_f32(got[33][name], got[0][name], name)
 
 
+# (16 heads: a round is 16 chunks; one portion of 192 and of 191 rows, two of 256 in a round, eight of them in two, one of 400 beside)
+@pytest.mark.parametrize("lens,chunks", [((192,), True), ((191,), False), ((256, 256), True), ((256,) * 8, False), ((400, 1, 60), True)])
+def test_which_portions_go_by_chunks(tmp_path, lens, chunks):
+    """bfloat16: the engine's own rule takes what forcing it takes, bit for bit, and the two ways differ in some bit."""
+    cfg = {"architecture": "Kifetar", "vocab": 150, "width": 64, "norm": {"eps": 1e-5}, "max_context": 4096,
+           "layers": [delta(16, 8, 64, 64, 4)]}
+    folder = write_model(tmp_path / "rule", cfg, 59, torch.bfloat16, std=0.2)
+    reqs = {f"r{i}": random_tokens(cfg["vocab"], n, seed=70 + i) for i, n in enumerate(lens)}
+    steps = [{"step": 0, "entries": [{"id": k, "tokens": t, "want": list(range(len(t)))} for k, t in reqs.items()], "end": list(reqs)}]
+    got = {}
+    for rows in (-1, 0, 192 if chunks else 64):
+        lm, _ = load(folder, "bfloat16", steps, max_requests=8)
+        lm.set_knob("delta_chunk_rows", rows)
+        got[rows] = torch.cat(list(EngineDriver(lm).run(steps).values()))
+    forced = got[192 if chunks else 64]
+    assert torch.equal(got[-1], forced if chunks else got[0])
+    assert not torch.equal(got[0], forced)
+
+
 def test_requests_beside_a_portion_leave_recorded_steps_alone(tmp_path):
     """bfloat16: what the chunks of a portion are kept in has room for the step's rows, however many requests these are of,
     so steps recorded before are replayed after a step of as many rows and more requests."""
