@@ -45,9 +45,18 @@ enum { T_STORE = 0, T_RESIDUAL = 2, T_SWIGLU = 3, T_QKV = 5 };   // (0, 2, 3: th
 __device__ __forceinline__ float round_bf16(float x) { return to_float(from_float<bf16>(x)); }
 
 // g / (1 + e^-g) with the hardware's exponential and reciprocal (an ulp each, in 32-bit; the
-// result is rounded to bfloat16): the exact division and exponential cost the SwiGLU product
-// of 2,048 rows 3 us.
-__device__ __forceinline__ float tile_silu(float g) { return g * __frcp_rn(1.0f + __expf(-g)); }
+// result is rounded to bfloat16): the exact exponential cost the SwiGLU product of 2,048 rows
+// 3 us, the exact division (twelve instructions a value, where the epilogue is bound by them) another 1.9, and half as much at 600 rows.
+__device__ __forceinline__ float tile_silu(float g) { return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)); }
+
+// A store of 16 bytes a lane that does not stay in the die's L2 until the kernel's end.  Where a product's workgroups all
+// end together, what they wrote leaves the L2s only then, with nothing beside it: written through, w1 with w3 at 2,048 rows (19
+// MB) takes 39.3 us instead of 40.9, at 1,000 rows 26.9 instead of 27.8.  (The residual epilogue, 32-bit and bfloat16
+// values of 12 MB at 2,048 rows, gains 0.2 to 0.6 us there and loses as much at 300 rows and 3 us of 58 at 4,000: it stores plainly.)
+// `s_nop`: the data's registers may not be written right behind the instruction.
+__device__ __forceinline__ void store_through(bf16x8_t* const to, const bf16x8_t& v) {
+    asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 2" ::"v"(to), "v"(v) : "memory");
+}
 
 template <int N>
 __device__ __forceinline__ void wait_loads() {
@@ -652,7 +661,7 @@ __device__ __forceinline__ void wide_swiglu_epilogue(
         for (int i = 0; i < 8; ++i) o[i] = static_cast<__bf16>(tile_silu(static_cast<float>(g[i])) * static_cast<float>(u[i]));
         bf16* const to = static_cast<bf16*>(p.out) + static_cast<size_t>(m) * p.ldo + n;
         if (wide_stores && n + 8 <= N) {
-            *reinterpret_cast<bf16x8_t*>(to) = o;
+            store_through(reinterpret_cast<bf16x8_t*>(to), o);
         } else {
             *reinterpret_cast<bf16x4_t*>(to) = bf16x4_t{o[0], o[1], o[2], o[3]};
             if (n + 8 <= N) *reinterpret_cast<bf16x4_t*>(to + 4) = bf16x4_t{o[4], o[5], o[6], o[7]};
