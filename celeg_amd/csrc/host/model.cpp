@@ -305,7 +305,7 @@ void ModelRunner::drop_graphs() {
         if (g.second.graph) (void)hipGraphDestroy(g.second.graph);
     }
     graphs_.clear();
-    n_portion_graphs_ = 0;
+    n_portion_graphs_[0] = n_portion_graphs_[1] = 0;
 }
 
 void ModelRunner::set_token_source(int* last_tokens) {
@@ -533,15 +533,19 @@ ModelRunner::Captured& ModelRunner::record(std::pair<int, int> key, const StepBa
 // A step that is one portion of a prompt is some 150 launches with gaps between them: a size
 // that has come before (the portions that a token budget cuts have the same size again and
 // again) is recorded too, per number of rows and per context below or from 4,096 tokens (the
-// attention over rows chooses its tiles by that).
+// attention over rows chooses its tiles by that).  Short questions have few sizes and little work a launch: one
+// prompt of 24 tokens at the 350M shape takes 674 us launched one by one, 617 replayed, so they are
+// recorded from two rows on, out of a budget of their own (sizes below 32 rows do not take the places of longer portions).
 bool ModelRunner::portion_graph_applies(const std::vector<StepEntry>& entries) {
     if (!use_graphs || !model.graph_safe() || rt.after_layer || rt.phases || sync_launches() || entries.size() != 1) return false;
     const StepEntry& e = entries[0];
     const int T = static_cast<int>(e.tokens.size());
     if (T < portion_graph_min_tokens || e.want.size() != 1 || e.want[0] != T - 1) return false;
     if (graphs_.count({-T, 0}) || graphs_.count({-T, 1})) return true;
-    if (portion_sizes_seen_.size() >= 64 && !portion_sizes_seen_.count(T)) return false;     // sizes that never repeat
-    return ++portion_sizes_seen_[T] >= 2 && n_portion_graphs_ < 16;
+    const bool few = T < few_portion_rows;
+    auto& seen = portion_sizes_seen_[few];
+    if (seen.size() >= 64 && !seen.count(T)) return false;     // sizes that never repeat
+    return ++seen[T] >= 2 && n_portion_graphs_[few] < 16;
 }
 
 Tensor ModelRunner::step_from_portion_graph(const std::vector<StepEntry>& entries) {
@@ -556,7 +560,7 @@ Tensor ModelRunner::step_from_portion_graph(const std::vector<StepEntry>& entrie
     const std::pair<int, int> key{-T, far ? 1 : 0};
     auto it = graphs_.find(key);
     if (it == graphs_.end() || it->second.generation != rt.ws.generation) {
-        if (it == graphs_.end()) ++n_portion_graphs_;
+        if (it == graphs_.end()) ++n_portion_graphs_[T < few_portion_rows];
         const std::vector<std::vector<TableUpdate>> empty(static_cast<size_t>(cache.n_groups()));
         StepEntry spare;
         spare.slot = cache.null_slot;

@@ -81,7 +81,7 @@ public:
     Runtime& rt;
     const int max_batched_tokens;
     bool use_graphs = true;
-    int portion_graph_min_tokens = 32;      // portions of fewer rows are never recorded
+    int portion_graph_min_tokens = 2;       // portions of fewer rows are never recorded
     long long steps_run = 0, graph_replays = 0, captures = 0;
     double capture_seconds = 0.0;
     const StepBatch& last_batch() const { return last_batch_; }
@@ -120,8 +120,9 @@ private:
     // (batch-size bucket, bound on the context) for steps of single tokens; (-rows, context
     // from 4,096 tokens or not) for steps of one portion
     std::map<std::pair<int, int>, Captured> graphs_;
-    std::map<int, int> portion_sizes_seen_;
-    int n_portion_graphs_ = 0;
+    static constexpr int few_portion_rows = 32;
+    std::map<int, int> portion_sizes_seen_[2];     // [portions of fewer rows than that]
+    int n_portion_graphs_[2] = {0, 0};
     std::vector<int> buckets_;
     int update_room_ = 0;
     int* token_source_ = nullptr;

@@ -70,3 +70,26 @@ def test_portion_graphs_on_both_sides_of_4096_tokens(tmp_path):
     counters = lm.runner.counters()
     assert counters["captures"] == 2 and counters["graph_replays"] == 8      # 9 portions of 512: one eager
     lm.close()
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+def test_portions_of_few_rows_are_replayed_out_of_a_budget_of_their_own(model_folders, dtype):
+    """2 to 31 rows: recorded when the size has come before, at most 16 of them, and a longer portion is recorded all the same."""
+    from celeg_amd.engine import load_model
+    storage = torch.float32 if dtype == "float32" else torch.bfloat16
+    folder = model_folders("D", storage, WEIGHT_STD)
+    cfg, W = plain.load_model_folder(folder)
+    lm = load_model(folder, dtype=dtype, page_tokens=16, n_pages=40, max_requests=2, max_batched_tokens=64)
+    captures = 0
+    for size in [2, 7, 8, 9, 16, 17, 24, 31] + list(range(10, 16)) + [18, 19, 20, 21]:
+        tokens = random_tokens(cfg["vocab_size"], 3 * size, seed=size)
+        got = feed_in_portions(lm, tokens, size)
+        ref = plain.model_logits(cfg, W, tokens)[[size - 1, 2 * size - 1, 3 * size - 1]]
+        assert_close(got, ref, dtype, f"portions of {size}")
+        captures = min(captures + 1, 16)
+        assert lm.runner.counters()["captures"] == captures
+    tokens = random_tokens(cfg["vocab_size"], 80, seed=5)
+    assert_close(feed_in_portions(lm, tokens, 40), plain.model_logits(cfg, W, tokens)[[39, 79]], dtype, "portions of 40")
+    assert lm.runner.counters()["captures"] == captures + 1
+    lm.cache.check()
+    lm.close()
