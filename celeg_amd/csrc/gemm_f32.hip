@@ -142,47 +142,110 @@ __global__ __launch_bounds__(MAX_THREADS) void gemm_f32_kernel(
     }
 }
 
+// What surrounds a product of few rows, folded into it (a decode step is a chain of short kernels, each of
+// which costs 1.7 us empty): in front the RMSNorm of its rows (every workgroup normalises them for itself while its
+// weights are on their way), behind it the addition into the residual stream, SwiGLU of a gate and an up stream,
+// or the double-gated short convolution of a B, a C and an x stream for one new token per request with its state
+// update.  Streams: rows [s N, (s + 1) N) of W.  An output is computed from the same 32-bit sums by the same
+// operations as where these are kernels of their own; the sum of squares is added up by segments of k.
+// Reference semantics: RMSNorm src/backend/cpu/kernels/elementwise.cpp:56-76, SwiGLU elementwise.cpp:101-119, short
+// convolution src/backend/cpu/kernels/convolution.cpp:7-28.
+enum { F32_STORE = 0, F32_RESIDUAL = 2, F32_SWIGLU = 3, F32_CONV = 4 };      // (the numbers of the bfloat16 products)
+#define F32_MAX_TAPS 8
+struct F32Tail {
+    const float* norm_w;        // [K]
+    float eps;
+    int taps;
+    const float* conv_w;        // [N, taps]
+    const float* conv_b;        // optional [N]
+    float* state;               // [slots, taps, N]
+    size_t state_slot_stride;
+    const int* seq_slot;        // [M]
+};
+template <int EPI> constexpr int f32_streams() { return EPI == F32_SWIGLU ? 2 : EPI == F32_CONV ? 3 : 1; }
+
 // The products of up to 16 rows.  The 16 x 16 tile of the instruction is cut into G x G blocks: its rows are
 // (segment g of G, column j of 16 / G) of W, its columns (segment g', row m of 16 / G) of X, so the blocks
 // g = g' on the diagonal are G segments' sums of the same outputs and the others are dropped.  A workgroup
-// then owns 16 / G columns, and a matrix of few columns (w2: 1,024) is spread over G times as many
-// workgroups; a segment's sum is formed by the same instructions, so the outputs keep their bits.
+// then owns 16 / G columns (of all streams together), and a matrix of few columns (w2: 1,024) is spread over G times
+// as many workgroups; a segment's sum is formed by the same instructions, so the outputs keep their bits.
 // 2 rows: 1024 x 4608 7.2 us (on 16 columns a workgroup 14.8), 1024 x 1024 3.3 (4.5).
-template <int G, bool VEC>
-__global__ __launch_bounds__(1024) void gemm_f32_slices_kernel(
+// (a norm's rows are whole in one round of at most 16 / G wavefronts, K <= 2,048: the more registers are left to each)
+template <int G, bool VEC, int EPI, bool NORM>
+__global__ __launch_bounds__(NORM ? 1024 / G : 1024) void gemm_f32_slices_kernel(
     const float* __restrict__ X, int ldx, const float* __restrict__ W, int ldw,
-    const float* __restrict__ bias, float* __restrict__ Y, int ldy, int M, int N, int K, int wide_store) {
+    const float* __restrict__ bias, float* __restrict__ Y, int ldy, int M, int N, int K, int wide_store, const F32Tail f) {
     constexpr int MP = 16 / G, ITEMS = MP * MP / 4;      // sums of four neighbouring columns of a row
-    extern __shared__ f32x4_t parts[];                    // [segment of the round][item]
+    constexpr int NS = f32_streams<EPI>(), OWN = MP / NS;      // columns of a stream that the workgroup owns
+    extern __shared__ f32x4_t parts[];                    // [segment of the round][item], then [row][segment] and [row][column] floats
     const int wave = threadIdx.x / CELEG_WAVE, lane = threadIdx.x % CELEG_WAVE;
     const int n_waves = blockDim.x / CELEG_WAVE;
+    float* const row_squares = reinterpret_cast<float*>(parts + static_cast<size_t>(n_waves) * G * ITEMS);
+    float* const sums = row_squares + (NORM ? n_waves * G * MP : 0);
     const int qd = lane >> 4, r16 = lane & 15;
-    const int col0 = blockIdx.x * MP;
+    const int col0 = blockIdx.x * OWN;
     const float* const x_row = X + static_cast<size_t>(min(r16 % MP, M - 1)) * ldx;
-    const float* const w_row = W + static_cast<size_t>(min(col0 + r16 % MP, N - 1)) * ldw;
+    const int tile_col = NS == 1 || r16 % MP < NS * OWN ? r16 % MP : 0;      // (what OWN x NS columns leave of the tile repeats the first)
+    const float* const w_row = W + (static_cast<size_t>(tile_col / OWN) * N + min(col0 + tile_col % OWN, N - 1)) * ldw;
     // this lane's sums: row (lane % MP) and columns 4 (quad in its block) .. + 3, of segment `of`
     const int of = qd / (MP / 4), item = (qd % (MP / 4)) * MP + lane % MP;
     const bool on_diagonal = r16 / MP == of;
     const int segments = (K + F32_SEGMENT - 1) / F32_SEGMENT;
-    f32x4_t total = {0.f, 0.f, 0.f, 0.f};
+    f32x4_t total = {0.f, 0.f, 0.f, 0.f}, old = {0.f, 0.f, 0.f, 0.f};
+
+    // ---- what the end needs from memory, asked for ahead of the products
+    const int row = threadIdx.x % MP, col = col0 + 4 * (threadIdx.x / MP);      // of the item this thread adds up
+    if (EPI == F32_RESIDUAL && threadIdx.x < ITEMS && row < M) {
+        const float* y = Y + static_cast<size_t>(row) * ldy + col;
+        if (wide_store && col + 3 < N) old = *reinterpret_cast<const f32x4_t*>(y);
+        else
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (col + r < N) old[r] = y[r];
+    }
+    const int out_row = threadIdx.x / OWN, out_col = col0 + threadIdx.x % OWN;   // of the output this thread finishes (SwiGLU, convolution)
+    const bool finishes = NS > 1 && threadIdx.x < MP * OWN && out_row < M && out_col < N;
+    float taps[EPI == F32_CONV ? F32_MAX_TAPS : 1], state[EPI == F32_CONV ? F32_MAX_TAPS - 1 : 1], conv_b = 0.f;
+    float* state_at = nullptr;
+    const auto fetch_conv = [&]() __attribute__((always_inline)) {
+        if (!finishes) return;
+        state_at = f.state + static_cast<size_t>(f.seq_slot[out_row]) * f.state_slot_stride + out_col;
+#pragma unroll
+        for (int i = 0; i < F32_MAX_TAPS; ++i) taps[i] = f.conv_w[static_cast<size_t>(out_col) * f.taps + min(i, f.taps - 1)];
+#pragma unroll
+        for (int i = 0; i < F32_MAX_TAPS - 1; ++i) state[i] = state_at[static_cast<size_t>(min(i + 1, f.taps - 1)) * N];
+        if (f.conv_b) conv_b = f.conv_b[out_col];
+    };
+    if constexpr (EPI == F32_CONV && G > 1) fetch_conv();      // (16 wavefronts have no registers to hold them)
+
     for (int first = 0; first < segments; first += n_waves * G) {
         const int mine = first + wave * G;                // this wavefront's segments: G of them from here
         const int k0 = (mine + r16 / MP) * F32_SEGMENT + 4 * qd;
-        f32x4_t wv[F32_PIECES], xv[F32_PIECES];
-        if (VEC && (mine + G) * F32_SEGMENT <= K) {
-#pragma unroll
-            for (int s = 0; s < F32_PIECES; ++s) wv[s] = *reinterpret_cast<const f32x4_t*>(w_row + k0 + 16 * s);
+        f32x4_t wv[F32_PIECES], xv[F32_PIECES], nw[NORM ? F32_PIECES : 1];
+        const auto load_x = [&]() __attribute__((always_inline)) {
 #pragma unroll
             for (int s = 0; s < F32_PIECES; ++s) xv[s] = *reinterpret_cast<const f32x4_t*>(x_row + k0 + 16 * s);
+        };
+        if (VEC && (mine + G) * F32_SEGMENT <= K) {
+            if constexpr (NORM) {       // (the rows first: their squares are added up while the weights are on their way)
+                load_x();
+#pragma unroll
+                for (int s = 0; s < F32_PIECES; ++s) nw[s] = *reinterpret_cast<const f32x4_t*>(f.norm_w + k0 + 16 * s);
+            }
+#pragma unroll
+            for (int s = 0; s < F32_PIECES; ++s) wv[s] = *reinterpret_cast<const f32x4_t*>(w_row + k0 + 16 * s);
+            if constexpr (!NORM) load_x();
         } else {
 #pragma unroll
             for (int s = 0; s < F32_PIECES; ++s) {
                 const int k = k0 + 16 * s;
                 wv[s] = xv[s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+                if constexpr (NORM) nw[s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
                 if (VEC) {
                     if (k < K) {
                         wv[s] = *reinterpret_cast<const f32x4_t*>(w_row + k);
                         xv[s] = *reinterpret_cast<const f32x4_t*>(x_row + k);
+                        if constexpr (NORM) nw[s] = *reinterpret_cast<const f32x4_t*>(f.norm_w + k);
                     }
                 } else {
 #pragma unroll
@@ -193,6 +256,23 @@ __global__ __launch_bounds__(1024) void gemm_f32_slices_kernel(
                         }
                 }
             }
+        }
+        if constexpr (NORM) {           // (one round: the launch sees to it)
+            float squares = 0.f;
+#pragma unroll
+            for (int s = 0; s < F32_PIECES; ++s)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) squares += xv[s][i] * xv[s][i];
+            squares = sum_half32(sum_row16(squares));     // over the four lanes that share a row and a segment
+            if (qd == 0) row_squares[(r16 % MP) * (n_waves * G) + wave * G + r16 / MP] = squares;
+            __syncthreads();
+            float all = 0.f;
+            for (int g = 0; g < segments; ++g) all += row_squares[(r16 % MP) * (n_waves * G) + g];
+            const float inv = 1.0f / sqrtf(all / static_cast<float>(K) + f.eps);
+#pragma unroll
+            for (int s = 0; s < F32_PIECES; ++s)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) xv[s][i] = xv[s][i] * inv * nw[s][i];
         }
         f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -206,32 +286,76 @@ __global__ __launch_bounds__(1024) void gemm_f32_slices_kernel(
         if (threadIdx.x < ITEMS)
             for (int g = 0; g < n; ++g) total += parts[g * ITEMS + threadIdx.x];
     }
-    const int row = threadIdx.x % MP, col = col0 + 4 * (threadIdx.x / MP);
+    if constexpr (NS > 1) {
+        if constexpr (EPI == F32_CONV && G == 1) fetch_conv();
+        if (threadIdx.x < ITEMS)
+            *reinterpret_cast<f32x4_t*>(sums + row * MP + 4 * (threadIdx.x / MP)) = total;
+        __syncthreads();
+        if (!finishes) return;
+        float v[NS];
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+            v[s] = sums[out_row * MP + s * OWN + threadIdx.x % OWN] + (bias ? bias[static_cast<size_t>(s) * N + out_col] : 0.f);
+        float* const y = Y + static_cast<size_t>(out_row) * ldy + out_col;
+        if constexpr (EPI == F32_SWIGLU) {
+            *y = (v[0] / (1.0f + expf(-v[0]))) * v[1];
+        } else {
+            const float bx = v[0] * v[2];
+            float conv = 0.f, last_tap = 0.f;
+#pragma unroll
+            for (int tap = 0; tap < F32_MAX_TAPS - 1; ++tap)
+                if (tap + 1 < f.taps) {
+                    conv = fmaf(taps[tap], state[tap], conv);
+                    state_at[static_cast<size_t>(tap) * N] = state[tap];         // shift by one position
+                }
+#pragma unroll
+            for (int tap = 0; tap < F32_MAX_TAPS; ++tap)
+                if (tap == f.taps - 1) last_tap = taps[tap];
+            conv = fmaf(last_tap, bx, conv);
+            state_at[static_cast<size_t>(f.taps - 1) * N] = bx;
+            *y = v[1] * (conv + conv_b);
+        }
+        return;
+    }
     if (threadIdx.x >= ITEMS || row >= M) return;
     float* y = Y + static_cast<size_t>(row) * ldy + col;
     if (wide_store && col + 3 < N) {
         if (bias) total += f32x4_t{bias[col], bias[col + 1], bias[col + 2], bias[col + 3]};
+        if (EPI == F32_RESIDUAL) total += old;
         *reinterpret_cast<f32x4_t*>(y) = total;
         return;
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-        if (col + r < N) y[r] = total[r] + (bias ? bias[col + r] : 0.f);
+        if (col + r < N) {
+            const float v = total[r] + (bias ? bias[col + r] : 0.f);
+            y[r] = EPI == F32_RESIDUAL ? old[r] + v : v;
+        }
 }
 
-template <int G>
+template <int G, int EPI = F32_STORE, bool NORM = false>
 static int launch_f32_slices(const float* X, int ldx, const float* W, int ldw, const float* bias, float* Y, int ldy,
-                             int M, int N, int K, hipStream_t stream) {
+                             int M, int N, int K, hipStream_t stream, const F32Tail& tail = F32Tail{}) {
     const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     const bool vec = K % 4 == 0 && ldx % 4 == 0 && ldw % 4 == 0 && aligned(X) && aligned(W);
     const int wide_store = ldy % 4 == 0 && aligned(Y);
-    constexpr int MP = 16 / G;
+    constexpr int MP = 16 / G, OWN = MP / f32_streams<EPI>();
     const int groups = ((K + F32_SEGMENT - 1) / F32_SEGMENT + G - 1) / G;
     const int rounds = (groups + 15) / 16, waves = (groups + rounds - 1) / rounds;     // as even as it goes: 36 are 3 rounds of 12
-    const dim3 grid((N + MP - 1) / MP), block(waves * CELEG_WAVE);
-    const size_t lds = static_cast<size_t>(waves) * G * (MP * MP / 4) * sizeof(f32x4_t);
-    auto kernel = vec ? &gemm_f32_slices_kernel<G, true> : &gemm_f32_slices_kernel<G, false>;
-    hipLaunchKernelGGL(kernel, grid, block, lds, stream, X, ldx, W, ldw, bias, Y, ldy, M, N, K, wide_store);
+    // (all of a row is needed for its norm, and the end of a product with two or three streams takes a thread an output)
+    if ((NORM && (rounds > 1 || !vec || !aligned(tail.norm_w))) || (EPI != F32_STORE && !vec)) return static_cast<int>(hipErrorInvalidValue);
+    const int threads = max(waves * CELEG_WAVE, f32_streams<EPI>() > 1 ? (MP * OWN + CELEG_WAVE - 1) / CELEG_WAVE * CELEG_WAVE : 0);
+    const dim3 grid((N + OWN - 1) / OWN), block(threads);
+    const size_t waves_run = threads / CELEG_WAVE;
+    const size_t lds = waves_run * G * (MP * MP / 4) * sizeof(f32x4_t) + (NORM ? waves_run * G * MP * sizeof(float) : 0) +
+                       (f32_streams<EPI>() > 1 ? MP * MP * sizeof(float) : 0);
+    if constexpr (EPI == F32_STORE && !NORM) {
+        auto kernel = vec ? &gemm_f32_slices_kernel<G, true, EPI, NORM> : &gemm_f32_slices_kernel<G, false, EPI, NORM>;
+        hipLaunchKernelGGL(kernel, grid, block, lds, stream, X, ldx, W, ldw, bias, Y, ldy, M, N, K, wide_store, tail);
+    } else {
+        hipLaunchKernelGGL((gemm_f32_slices_kernel<G, true, EPI, NORM>), grid, block, lds, stream, X, ldx, W, ldw, bias, Y, ldy, M, N, K,
+                           wide_store, tail);
+    }
     return CELEG_LAUNCH_RESULT();
 }
 
@@ -353,14 +477,44 @@ static int launch_f32_short(const float* X, int ldx, const float* W, int ldw, co
     return CELEG_LAUNCH_RESULT();
 }
 
+// blocks of 4 or 8 columns while tiles of 16 would leave compute units without a second workgroup
+static int f32_slices_of(int M, int weight_rows) { return weight_rows >= 512 * 16 || M > 8 ? 1 : M > 4 ? 2 : 4; }
+
+// Up to 16 rows with what surrounds them (epi: the numbers above; N: columns of a stream; norm_w null: none).  X, W and
+// norm_w on 16 bytes, ldx, ldw and K multiples of 4; with a norm K up to 2,048.
+extern "C" int celeg_gemm_f32_fused(const float* X, int ldx, const float* W, int ldw, const float* bias, float* Y, int ldy, int M,
+                                    int N, int K, int epi, const float* norm_w, float eps, const float* conv_w, const float* conv_b,
+                                    float* state, size_t state_slot_stride, const int* seq_slot, int taps, hipStream_t stream) {
+    if (M <= 0 || N <= 0) return 0;
+    if (M > 16 || K <= 0 || (norm_w && K > 16 * F32_SEGMENT) ||
+        (epi == F32_CONV && (taps < 1 || taps > F32_MAX_TAPS || !conv_w || !state || !seq_slot)))
+        return static_cast<int>(hipErrorInvalidValue);
+    F32Tail f{norm_w, eps, taps, conv_w, conv_b, state, state_slot_stride, seq_slot};
+#define F32_FUSED(EPI, NORM)                                                                                             \
+    (g == 4 ? launch_f32_slices<4, EPI, NORM>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream, f)                           \
+     : g == 2 ? launch_f32_slices<2, EPI, NORM>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream, f)                         \
+              : launch_f32_slices<1, EPI, NORM>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream, f))
+    // (with a norm a wavefront holds its weight beside the rows: half as many wavefronts of two segments each, 2 rows by 1,024:
+    // w1 with w3 12.7 us, in_proj with the convolution 7.2, q/k/v 5.8; blocks of 16 columns 15.8, 8.4 and 7.8, of 4 12.4, 7.6 and 6.1;
+    // 4 rows 13.3, 7.5, 5.9; 15.9, 8.6, 7.9; 13.9, 8.2, 6.3)
+    const int g = norm_w ? (M > 8 ? 1 : 2) : f32_slices_of(M, N);
+    switch (epi) {
+        case F32_STORE: return norm_w ? F32_FUSED(F32_STORE, true) : static_cast<int>(hipErrorInvalidValue);
+        case F32_RESIDUAL: return norm_w ? static_cast<int>(hipErrorInvalidValue) : F32_FUSED(F32_RESIDUAL, false);
+        case F32_SWIGLU: return norm_w ? F32_FUSED(F32_SWIGLU, true) : static_cast<int>(hipErrorInvalidValue);
+        case F32_CONV: return norm_w ? F32_FUSED(F32_CONV, true) : static_cast<int>(hipErrorInvalidValue);
+        default: return static_cast<int>(hipErrorInvalidValue);
+    }
+#undef F32_FUSED
+}
+
 extern "C" int celeg_gemm_f32(const float* X, int ldx, const float* W, int ldw, const float* bias,
                               float* Y, int ldy, int M, int N, int K, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
     if (K <= 0) return static_cast<int>(hipErrorInvalidValue);
-    // (blocks of 4 or 8 columns while tiles of 16 would leave compute units without a second workgroup)
     if (M <= 16) {
-        const int g = N >= 512 * 16 || M > 8 ? 1 : M > 4 ? 2 : 4;
-        return (g == 4 ? launch_f32_slices<4> : g == 2 ? launch_f32_slices<2> : launch_f32_slices<1>)(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
+        const int g = f32_slices_of(M, N);
+        return (g == 4 ? launch_f32_slices<4> : g == 2 ? launch_f32_slices<2> : launch_f32_slices<1>)(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream, F32Tail{});
     }
     if (M <= 32) return launch_f32<2, 1, 8, 512>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
     if (M <= 64) return launch_f32<4, 1, 4, 512>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);

@@ -29,6 +29,10 @@ bool fused_rows_ok(const Runtime& rt, const StepBatch& batch, std::initializer_l
     return rows <= limit;
 }
 
+bool fused_f32_ok(const Runtime& rt, const StepBatch& batch, std::initializer_list<long long> inner) {
+    return rt.dtype == DType::F32 && rt.use_fused && Ops::fused_linear_f32_ok(batch.n_tokens, inner);
+}
+
 Tensor stream_stats(Runtime& rt, long long width, int rows) {
     if (rows > STAT_COLUMNS)     // a step of many rows: one partial sum per tile of columns
         return rt.ws.buf("stream_stats_many", DType::F32, {rows, TILED_MAX_STAT_BLOCKS});
@@ -43,6 +47,7 @@ Tensor stream_stats(Runtime& rt, long long width, int rows) {
 // (inner size producer_inner), writes it.
 Tensor operand_rows(Runtime& rt, const std::string& name, int rows, long long width,
                     std::initializer_list<long long> producer_inner) {
+    if (rt.dtype == DType::F32) return rt.ws.buf(name + "_f32", DType::F32, {rows, width});
     if (rows > STAT_COLUMNS) return rt.ws.buf(name + "_many", DType::BF16, {rows, width});
     bool side_by_side = rt.ops.rows_kernel_ok(rows, {width});
     for (long long k : producer_inner) side_by_side = side_by_side && rt.ops.rows_kernel_ok(rows, {k});
@@ -112,6 +117,17 @@ void norm_linear(Runtime& rt, const Tensor& h, const Norm::Foldable& norm, const
     const int T = static_cast<int>(h.shape[0]);
     const long long width = h.shape[1];
     const int M = extras.n_rows >= 0 ? extras.n_rows : T;
+    if (rt.dtype == DType::F32) {
+        if (extras.rows || extras.qkv || w.dtype != DType::F32) throw KernelError("norm_linear: not a 32-bit product with a norm");
+        FusedArgs args;
+        args.epilogue = epilogue;
+        args.norm_weight = norm.weight;
+        args.eps = norm.eps;
+        args.bias = extras.bias;
+        args.conv = extras.conv;
+        rt.ops.fused_linear_f32(h, w, out, args);
+        return;
+    }
     if (tiled_step(rt, T, width)) {
         if (extras.rows || (epilogue != Epilogue::Store && epilogue != Epilogue::Swiglu) || w.dtype != DType::BF16)
             throw KernelError("norm_linear: not a product of the path for many rows");
@@ -184,6 +200,15 @@ void norm_linear(Runtime& rt, const Tensor& h, const Norm::Foldable& norm, const
 void linear_into_stream(Runtime& rt, const Tensor& a, const Tensor& w, const Tensor& h, const Tensor* bias) {
     const int T = static_cast<int>(h.shape[0]);
     const long long width = h.shape[1];
+    if (rt.dtype == DType::F32) {
+        FusedArgs args;
+        args.epilogue = Epilogue::Residual;
+        if (bias) args.bias = *bias;
+        rt.ops.fused_linear_f32(a, w, h, args);
+        rt.stream_stat_blocks = 0;
+        rt.stream_has_bf16 = false;
+        return;
+    }
     if (tiled_step(rt, T, width)) {
         Tensor stats = stream_stats(rt, width, T);
         Tensor xb = stream_bf16(rt, T, width);

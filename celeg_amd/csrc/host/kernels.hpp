@@ -80,6 +80,9 @@ int celeg_moe_combine(const void* y, int dtype, const int* place_of, const float
 // gemm_f32.hip
 int celeg_gemm_f32(const float* X, int ldx, const float* W, int ldw, const float* bias, float* Y, int ldy, int M,
                    int N, int K, hipStream_t stream);
+int celeg_gemm_f32_fused(const float* X, int ldx, const float* W, int ldw, const float* bias, float* Y, int ldy, int M, int N, int K, int epi,
+                         const float* norm_w, float eps, const float* conv_w, const float* conv_b, float* state, size_t state_slot_stride,
+                         const int* seq_slot, int taps, hipStream_t stream);
 // short_conv.hip
 int celeg_short_conv(const void* bcx, int ld_bcx, int dtype, const float* w, const float* bias, float* state,
                      size_t state_slot_stride, void* out, const int* positions, const int* token_seq,

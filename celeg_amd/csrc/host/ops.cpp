@@ -1779,6 +1779,56 @@ void Ops::embed_stats(const Tensor& table, const int* token_ids, const Tensor& o
 // stats[row, :stat_blocks] its partial sums of squares, from which the rows' 1/rms (with eps)
 // scales the sums; their Residual epilogue refreshes out_bf16, the bfloat16 copy of the stream,
 // if given.  They also take w in the layout of fold_weight(packed).
+// Few 32-bit rows: the first inner size is the width of the stream, whose norm takes whole rows in one round.
+bool Ops::fused_linear_f32_ok(int rows, std::initializer_list<long long> inner) {
+    if (rows < 1 || rows > 16 || inner.size() == 0 || *inner.begin() > 2048) return false;
+    for (long long k : inner)
+        if (k <= 0 || k % 4) return false;
+    return true;
+}
+
+void Ops::fused_linear_f32(const Tensor& a, const Tensor& w, const Tensor& out, const FusedArgs& args) {
+    dev(a, "a", DType::F32);
+    dev(w, "w", DType::F32);
+    dev(out, "out", DType::F32);
+    const Epilogue epi = args.epilogue;
+    const bool norm = args.norm_weight.defined();
+    need(norm ? epi == Epilogue::Store || epi == Epilogue::Swiglu || epi == Epilogue::Conv : epi == Epilogue::Residual,
+         "fused_linear (32-bit): this combination is not built");
+    const int streams = epi == Epilogue::Swiglu ? 2 : epi == Epilogue::Conv ? 3 : 1;
+    need(a.ndim == 2 && w.ndim == 2 && out.ndim == 2 && w.contiguous() && !args.rows, "fused_linear (32-bit): a, w and out must be matrices");
+    const long long M = a.shape[0], K = a.shape[1], N = w.shape[0] / streams;
+    need(w.shape[1] == K && w.shape[0] % streams == 0 && out.shape[0] == M && out.shape[1] == N, "fused_linear (32-bit): shapes do not fit");
+    if (args.bias.defined()) {
+        dev(args.bias, "bias", DType::F32);
+        need(args.bias.numel() == streams * N, "fused_linear (32-bit): bias does not fit");
+    }
+    if (norm) {
+        dev(args.norm_weight, "norm_weight", DType::F32);
+        need(args.norm_weight.numel() == K, "fused_linear (32-bit): norm weight must have the inner size");
+    }
+    const ConvOperands* c = epi == Epilogue::Conv ? args.conv : nullptr;
+    need(epi != Epilogue::Conv || c, "fused_linear (32-bit): the convolution epilogue needs its operands");
+    if (c) {
+        dev(c->taps, "conv taps", DType::F32);
+        dev(c->state, "state", DType::F32, false);
+        need(c->taps.ndim == 2 && c->taps.shape[0] == N && c->state.ndim == 3 && c->state.shape[1] == c->taps.shape[1] &&
+                 c->state.shape[2] == N && c->state.stride[2] == 1 && c->state.stride[1] == N,
+             "fused_linear (32-bit): the convolution's operands do not fit");
+        if (c->bias.defined()) dev(c->bias, "conv bias", DType::F32);
+        need(!c->bias.defined() || c->bias.numel() == N, "fused_linear (32-bit): the convolution's bias does not fit");
+    }
+    took(Path::LinearF32);
+    kernel_check(celeg_gemm_f32_fused(a.as<float>(), rows_of(a, "a"), w.as<float>(), static_cast<int>(K),
+                                      args.bias.defined() ? args.bias.as<float>() : nullptr, out.as<float>(), rows_of(out, "out"),
+                                      static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), static_cast<int>(epi),
+                                      norm ? args.norm_weight.as<float>() : nullptr, args.eps, c ? c->taps.as<float>() : nullptr,
+                                      c && c->bias.defined() ? c->bias.as<float>() : nullptr, c ? c->state.as<float>() : nullptr,
+                                      c ? static_cast<size_t>(c->state.stride[0]) : 0, c ? c->seq_slot : nullptr,
+                                      c ? static_cast<int>(c->taps.shape[1]) : 0, stream),
+                 "fused_linear (32-bit)");
+}
+
 void Ops::fused_linear(const Tensor& a, const Tensor& w, const Tensor& out, const FusedArgs& args) {
     dev(w, "w", DType::BF16);
     const Epilogue epi = args.epilogue;

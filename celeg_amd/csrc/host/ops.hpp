@@ -418,6 +418,9 @@ public:
                       const StepPrologue* prologue = nullptr);
     void embed_stats(const Tensor& table, const int* token_ids, const Tensor& out, const Tensor& stats);
     void fused_linear(const Tensor& a, const Tensor& w, const Tensor& out, const FusedArgs& args);
+    // The same for 32-bit rows and weights, with a norm (Store, Swiglu, Conv) or into the stream (Residual).
+    static bool fused_linear_f32_ok(int rows, std::initializer_list<long long> inner);
+    void fused_linear_f32(const Tensor& a, const Tensor& w, const Tensor& out, const FusedArgs& args);
     // fused products of many rows
     bool tiled_linear_ok(int rows, int n, std::initializer_list<long long> inner) const;
     int tiled_stat_blocks(int rows, int n, int k) const;

@@ -414,7 +414,8 @@ public:
                        Runtime& rt) override {
         const long long qw = static_cast<long long>(heads_) * head_dim_;
         const Tensor& w_in = cache.writes_kv ? w_qkv_->view : w_q_->view;
-        if (!fused::fused_rows_ok(rt, batch, {width_, qw}) || w_in.dtype != rt.dtype || w_o_->view.dtype != rt.dtype)
+        if (!(fused::fused_rows_ok(rt, batch, {width_, qw}) || fused::fused_f32_ok(rt, batch, {width_, qw})) || w_in.dtype != rt.dtype ||
+            w_o_->view.dtype != rt.dtype)
             return false;
         Tensor attended = project_and_attend(h, &norm, batch, cache, rt);
         fused::linear_into_stream(rt, attended, w_o_->view, h);
@@ -727,7 +728,8 @@ public:
     // residual addition folded into the two products
     bool forward_fused(const Tensor& h, const Norm::Foldable& norm, const StepBatch& batch, const LayerCache& cache,
                        Runtime& rt) override {
-        if (!fused::fused_rows_ok(rt, batch, {width_}) || w_in_->view.dtype != rt.dtype || w_out_->view.dtype != rt.dtype)
+        if (!(fused::fused_rows_ok(rt, batch, {width_}) || fused::fused_f32_ok(rt, batch, {width_})) || w_in_->view.dtype != rt.dtype ||
+            w_out_->view.dtype != rt.dtype)
             return false;
         const int T = batch.n_tokens;
         fused::LinearExtras extras;
@@ -823,8 +825,8 @@ public:
     // h += ffn(norm(h)): the norm and the SwiGLU folded into the first product, the residual
     // addition into the second
     bool forward_fused(const Tensor& h, const Norm::Foldable& norm, const StepBatch& batch, Runtime& rt) override {
-        if (limit_ > 0.f || !fused::fused_rows_ok(rt, batch, {width_, ff_}) || w_gate_up_->view.dtype != rt.dtype ||
-            w_down_->view.dtype != rt.dtype)
+        if (limit_ > 0.f || !(fused::fused_rows_ok(rt, batch, {width_, ff_}) || fused::fused_f32_ok(rt, batch, {width_, ff_})) ||
+            w_gate_up_->view.dtype != rt.dtype || w_down_->view.dtype != rt.dtype)
             return false;
         Tensor act = fused::operand_rows(rt, "ffn_act_fused", batch.n_tokens, ff_, {width_});
         fused::norm_linear(rt, h, norm, w_gate_up_->view, act, Epilogue::Swiglu);

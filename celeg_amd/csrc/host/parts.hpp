@@ -205,6 +205,9 @@ constexpr int SLICED_MAX_ROWS = 16, SLICED_MAX_STAT_BLOCKS = 512, SLICED_MAX_COL
 
 bool tiled_step(const Runtime& rt, int rows, long long width);
 bool fused_rows_ok(const Runtime& rt, const StepBatch& batch, std::initializer_list<long long> inner);
+// The same in 32-bit: up to 16 rows, for parts that ask for products with a norm in front (stored, SwiGLU or the short
+// convolution behind) and products into the stream, and nothing else of what is below.
+bool fused_f32_ok(const Runtime& rt, const StepBatch& batch, std::initializer_list<long long> inner);
 Tensor stream_stats(Runtime& rt, long long width, int rows = 0);
 Tensor operand_rows(Runtime& rt, const std::string& name, int rows, long long width, std::initializer_list<long long> producer_inner);
 Tensor stream_bf16(Runtime& rt, int rows, long long width);

@@ -1,0 +1,111 @@
+"""The 32-bit products of few rows with what surrounds them, called as the host code calls them: every epilogue at row counts on both
+sides of a change of layout, columns and inner sizes beside a tile's, against 64 bits; and a model's logits with and without them."""
+import ctypes
+
+import pytest
+import torch
+
+import plain_lfm2 as plain
+from celeg_amd import native
+from helpers import WEIGHT_STD, random_tokens
+from test_gpu_single_tokens import check, ptr
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+EPS = 2.0 ** -24
+STORE, RESIDUAL, SWIGLU, CONV = 0, 2, 3, 4
+
+
+def call(x, w, y, N, epi, norm=None, bias=None, conv=None):
+    taps, conv_b, state, slots = conv or (None, None, None, None)
+    return native.lib().celeg_gemm_f32_fused(
+        ptr(x), x.stride(0), ptr(w), w.stride(0), ptr(bias), ptr(y), y.stride(0), x.shape[0], N, x.shape[1], epi, ptr(norm),
+        ctypes.c_float(1e-5), ptr(taps), ptr(conv_b), ptr(state), ctypes.c_size_t(0 if state is None else state.stride(0)), ptr(slots),
+        0 if taps is None else taps.shape[1], None)
+
+
+@pytest.mark.parametrize("M", [1, 2, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("N,K", [(1, 4), (5, 132), (33, 128), (20, 1000), (66, 2048), (1024, 1024)])
+def test_every_epilogue_against_64_bits(M, N, K):
+    gen = torch.Generator().manual_seed(M * 1000 + N + K)
+    r = lambda *s: torch.randn(*s, generator=gen)
+    x, norm = (2.0 * r(M, K)).to(DEV), (1.0 + 0.3 * r(K)).to(DEV)
+    xd, nd = x.double(), norm.double()
+    normed = xd / torch.sqrt((xd * xd).mean(-1, keepdim=True) + 1e-5) * nd
+
+    def product(rows, w):
+        """64-bit sums and a bound on 32-bit ones: 128 products a segment one after the other, 16 segments, the row's scale"""
+        return rows @ w.double().T, (128 + 16 + 24) * EPS * (rows.abs() @ w.double().abs().T)
+
+    # stored behind a norm
+    w, b = (0.1 * r(N, K)).to(DEV), r(N).to(DEV)
+    y = torch.full((M, N + 3), 7.0, device=DEV)[:, :N]
+    check(call(x, w, y, N, STORE, norm, b))
+    want, bound = product(normed, w)
+    want = want + b.double()
+    assert ((y.double() - want).abs() <= bound + EPS * want.abs() + 1e-30).all()
+    # into the stream: the plain product's own sum, added in 32-bit
+    h = r(M, N).to(DEV)
+    plain_out, got = torch.empty(M, N, device=DEV), h.clone()
+    check(native.lib().celeg_gemm_f32(ptr(x), K, ptr(w), K, ptr(b), ptr(plain_out), N, M, N, K, None))
+    check(call(x, w, got, N, RESIDUAL, None, b))
+    assert torch.equal(got, h + plain_out)
+    # SwiGLU
+    w2 = (0.1 * r(2 * N, K)).to(DEV)
+    y = torch.empty(M, N, device=DEV)
+    check(call(x, w2, y, N, SWIGLU, norm))
+    g, eg = product(normed, w2[:N])
+    u, eu = product(normed, w2[N:])
+    silu = g * torch.sigmoid(g)
+    assert ((y.double() - silu * u).abs() <= 1.1 * eg * u.abs() + 2 * silu.abs() * eu + 2 * eg * eu + 16 * EPS * (silu * u).abs() + 1e-30).all()
+    # the short convolution, one new token per request, with its state
+    for L in (1, 3, 8):
+        w3, taps, cb = (0.1 * r(3 * N, K)).to(DEV), r(N, L).to(DEV), r(N).to(DEV)
+        state = r(M + 2, 2, L, N).to(DEV)[:, 1]
+        before, slots = state.clone(), torch.tensor([(3 * i + 1) % (M + 2) if (M + 2) % 3 else (i + 1) % (M + 2) for i in range(M)], dtype=torch.int32, device=DEV)
+        check(call(x, w3, y, N, CONV, norm, None, (taps, cb, state, slots)))
+        (B, eB), (C, eC), (X, eX) = (product(normed, w3[i * N:(i + 1) * N]) for i in range(3))
+        old = before[slots.long()].double()
+        bx, ebx = B * X, eB * X.abs() + B.abs() * eX + eB * eX + EPS * (B * X).abs()
+        terms = torch.cat([old[:, 1:], bx[:, None]], 1) * taps.double().T[None]
+        conv = terms.sum(1) + cb.double()
+        econv = taps.double().T[-1].abs() * ebx + (L + 2) * EPS * (terms.abs().sum(1) + cb.double().abs())
+        assert ((y.double() - C * conv).abs() <= eC * conv.abs() + C.abs() * econv + eC * econv + 2 * EPS * (C * conv).abs() + 1e-30).all()
+        now = state[slots.long()]
+        assert torch.equal(now[:, :L - 1], before[slots.long()][:, 1:])
+        assert ((now[:, L - 1].double() - bx).abs() <= ebx).all()
+        others = [s for s in range(M + 2) if s not in slots.tolist()]
+        assert torch.equal(state[others], before[others])
+
+
+@pytest.mark.parametrize("K", [2304, 4608])
+def test_long_rows_go_into_the_stream_and_are_refused_behind_a_norm(K):
+    gen = torch.Generator().manual_seed(K)
+    for M in (1, 4, 5, 16):
+        x, w, h = (torch.randn(*s, generator=gen).to(DEV) for s in ((M, K), (40, K), (M, 40)))
+        plain_out, got = torch.empty(M, 40, device=DEV), h.clone()
+        check(native.lib().celeg_gemm_f32(ptr(x), K, ptr(w), K, None, ptr(plain_out), 40, M, 40, K, None))
+        check(call(x, w, got, 40, RESIDUAL))
+        assert torch.equal(got, h + plain_out)
+        assert call(x, w, got, 40, STORE, torch.ones(K, device=DEV)) != 0
+
+
+@pytest.mark.parametrize("name", ["B", "D"])
+def test_logits_with_and_without(model_folders, name):
+    from celeg_amd.engine import StepEntry, load_model
+    folder = model_folders(name, torch.float32, WEIGHT_STD)
+    cfg, W = plain.load_model_folder(folder)
+    tokens = random_tokens(cfg["vocab_size"], 40, seed=3)
+    ref = plain.model_logits(cfg, W, tokens).double()
+    errors = {}
+    for fused in (1, 0):
+        lm = load_model(folder, dtype="float32", page_tokens=16, n_pages=16, max_requests=2, max_batched_tokens=64)
+        lm.set_knob("use_fused", fused)
+        slot, rows = lm.cache.open(), []
+        for first, n in [(0, 7), (7, 16), (23, 9)] + [(i, 1) for i in range(32, 40)]:
+            assert lm.cache.prepare(slot, first, n)
+            rows.append(lm.runner.step([StepEntry(slot, first, tokens[first:first + n], [n - 1])])[0].double())
+        got, want = torch.stack(rows), ref[[6, 22] + list(range(31, 40))]
+        errors[fused] = float((got - want).norm() / want.norm())
+        lm.close()
+    assert errors[1] <= 2e-6 and errors[0] <= 2e-6, errors
