@@ -358,9 +358,11 @@ extern "C" int celeg_qk_norm_rope_store(
 // CUDA kernels/attention_paged.cuh:2-141).
 // Bound by the latency of its loads.  VEC: keys and, from a chunk that starts on a boundary, values
 // come 16 bytes a load (a dimension's keys lie side by side in a page), a chunk's values 16 keys ahead of
-// the sums; the sums run in the same order without it.  32-bit, 2 requests decoding at 350 tokens, 16
-// heads of 64: 15.3 us; their prompts (424 rows) 66.7 us; before, with one wavefront and a value a load, 91.7 and
-// 164 us.
+// the sums; the sums run in the same order without it.  No condition stands round a key's product with its values (each read
+// of a weight from LDS would be waited for by itself).  Heads of 64 and few rows (WHOLE, 122 registers): all keys and values of
+// a chunk are asked for before the first is used.  16 heads of 64, before (with that condition, divisions by the page's
+// size and values 16 keys at a time) and now: 32-bit, 2 requests decoding at 350 tokens 15.2 -> 8.8 us, one at 8,000 213 -> 110,
+// prompts of 424 rows 52.5 -> 44.0; bfloat16, 2 requests 12.3 -> 6.8, a prompt of 512 rows 86.7 -> 60.
 #define ATT_MAX_DIM_CHUNKS 4  // head_dim <= 256
 // Wavefronts a row: four, and with a window no more than it has chunks of 64 keys, so that each has a chunk and the
 // sums are those of four.  Idle wavefronts cost a prompt what live ones do: 1,024 rows, 16 heads of 64, bfloat16, a
@@ -368,10 +370,14 @@ extern "C" int celeg_qk_norm_rope_store(
 // wavefronts than chunks would be faster for prompts (96: 187 us with one, 270 with four) but slower for single
 // tokens (25 against 17 us), and a row's sums must not depend on what else is in the step.
 #define ATT_MAX_WAVES 4
+// rows x heads up to which keys and values of a chunk come whole: 2 requests at 350 tokens 8.8 us against 9.3, 8 requests 16.8
+// against 19.0, one at 8,000 110 against 134; 424 rows of prompts 47.5 against 44.0, 1,024 rows 365 against 361
+#define WHOLE_MOST 1024
 
 template <typename T> struct Wide;      // 16 bytes as 32-bit numbers
 template <> struct Wide<float> {
     static constexpr int N = 4;
+    typedef Quad<float>::raw raw;
     static __device__ __forceinline__ void load(const float* p, float (&v)[4]) { Quad<float>::load(p, v); }
 };
 template <> struct Wide<bf16> {
@@ -384,8 +390,8 @@ template <> struct Wide<bf16> {
     }
 };
 
-// DC: head_dim in pieces of 64, rounded up
-template <typename T, int DC, int WAVES, bool VEC>
+// DC: head_dim in pieces of 64, rounded up; POW2: page_tokens is a power of two; WHOLE: head_dim is 64
+template <typename T, int DC, int WAVES, bool VEC, bool POW2, bool WHOLE>
 __global__ __launch_bounds__(WAVES * CELEG_WAVE) void paged_attention_kernel(
     const T* __restrict__ q, int ldq, const T* __restrict__ k_pool, const T* __restrict__ v_pool,
     const int* __restrict__ table, int table_stride, const int* __restrict__ token_slot,
@@ -405,6 +411,10 @@ __global__ __launch_bounds__(WAVES * CELEG_WAVE) void paged_attention_kernel(
     const int pos = positions[t];
     const int* pages = table + static_cast<size_t>(token_slot[t]) * table_stride;
     const int first = window > 0 ? max(0, pos - window + 1) : 0;
+    // (a division by a number that the compiler does not know is thirty instructions, and a chunk makes one a value's page)
+    const int shift = POW2 ? __ffs(page_tokens) - 1 : 0;
+    const auto page_index = [&](int key) { return POW2 ? key >> shift : key / page_tokens; };
+    const auto in_page = [&](int key) { return POW2 ? key & (page_tokens - 1) : key % page_tokens; };
 
     const T* qrow = q + static_cast<size_t>(t) * ldq + static_cast<size_t>(h) * head_dim;
     for (int d = threadIdx.x; d < head_dim; d += WAVES * CELEG_WAVE) qs[d] = to_float(qrow[d]);
@@ -419,10 +429,35 @@ __global__ __launch_bounds__(WAVES * CELEG_WAVE) void paged_attention_kernel(
     for (int base = first + wave * CELEG_WAVE; base <= pos; base += WAVES * CELEG_WAVE) {
         const int key = base + lane;
         const bool valid = key <= pos;
-        const int page = pages[min(key, pos) / page_tokens];
+        const int page = pages[page_index(min(key, pos))];
+        const int n_keys = min(CELEG_WAVE, pos - base + 1);
+        auto values = [&](int kk) __attribute__((always_inline)) {        // dimension 0 at key base + kk of this head
+            const int page2 = __builtin_amdgcn_readlane(page, kk);
+            return v_pool + cache_offset(page2, n_layers, layer, kv_heads, kvh, page_tokens, 0, head_dim) + in_page(base + kk);
+        };
+        typename Wide<T>::raw kr[WHOLE ? CELEG_WAVE / W : 1], vr[WHOLE ? CELEG_WAVE / W : 1];
+        if constexpr (WHOLE) {
+            if (wide_values) {
+                const int k_at = min(key, pos);
+                const T* const kp = k_pool + cache_offset(page, n_layers, layer, kv_heads, kvh, page_tokens, in_page(k_at), CELEG_WAVE);
+#pragma unroll
+                for (int a = 0; a < CELEG_WAVE / W; ++a) kr[a] = *reinterpret_cast<const typename Wide<T>::raw*>(kp + a * W);
+#pragma unroll
+                for (int a = 0; a < CELEG_WAVE / W; ++a)
+                    vr[a] = *reinterpret_cast<const typename Wide<T>::raw*>(values(min(a * W, n_keys - 1) / W * W) +
+                                                                           static_cast<size_t>(lane) * page_tokens);
+            }
+        }
         float s = -INFINITY;
-        if (valid) {
-            const T* kp = k_pool + cache_offset(page, n_layers, layer, kv_heads, kvh, page_tokens, key % page_tokens, head_dim);
+        if (WHOLE && wide_values) {
+            float dot = 0.f;
+#pragma unroll
+            for (int a = 0; a < (WHOLE ? CELEG_WAVE / W : 0); ++a)
+#pragma unroll
+                for (int i = 0; i < W; ++i) dot = fmaf(qs[a * W + i], static_cast<float>(kr[a][i]), dot);
+            s = valid ? dot * scale : -INFINITY;
+        } else if (valid) {
+            const T* kp = k_pool + cache_offset(page, n_layers, layer, kv_heads, kvh, page_tokens, in_page(key), head_dim);
             float dot = 0.f;
             if (VEC) {
 #pragma unroll 8
@@ -452,12 +487,18 @@ __global__ __launch_bounds__(WAVES * CELEG_WAVE) void paged_attention_kernel(
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
         for (int j = 0; j < DC; ++j) acc[j] *= corr;
-        const int n_keys = min(CELEG_WAVE, pos - base + 1);
-        auto values = [&](int kk) __attribute__((always_inline)) {        // dimension 0 at key base + kk of this head
-            const int page2 = __builtin_amdgcn_readlane(page, kk);
-            return v_pool + cache_offset(page2, n_layers, layer, kv_heads, kvh, page_tokens, 0, head_dim) + (base + kk) % page_tokens;
-        };
-        if (wide_values) {
+        if (WHOLE && wide_values) {
+            // (behind the row's own key memory may hold anything; a condition round a key's product would have each read of its
+            // weight waited for by itself: 64 trips to LDS in a row)
+            if (n_keys == CELEG_WAVE) {
+#pragma unroll
+                for (int k2 = 0; k2 < (WHOLE ? CELEG_WAVE : 0); ++k2) acc[0] = fmaf(ps[k2], static_cast<float>(vr[k2 / W][k2 % W]), acc[0]);
+            } else {
+#pragma unroll
+                for (int k2 = 0; k2 < (WHOLE ? CELEG_WAVE : 0); ++k2)
+                    acc[0] = fmaf(ps[k2], k2 < n_keys ? static_cast<float>(vr[k2 / W][k2 % W]) : 0.f, acc[0]);
+            }
+        } else if (wide_values) {
             for (int kk = 0; kk < n_keys; kk += 16) {
                 float v[AHEAD][DC][W];
 #pragma unroll
@@ -472,11 +513,9 @@ __global__ __launch_bounds__(WAVES * CELEG_WAVE) void paged_attention_kernel(
 #pragma unroll
                     for (int i = 0; i < W; ++i) {
                         const int k2 = kk + a * W + i;
-                        if (k2 < n_keys) {                  // (behind the row's own key memory may hold anything)
-                            const float pk = ps[k2];
+                        const float pk = ps[k2];            // (0 behind the row's own key, where memory may hold anything)
 #pragma unroll
-                            for (int j = 0; j < DC; ++j) acc[j] = fmaf(pk, v[a][j][i], acc[j]);
-                        }
+                        for (int j = 0; j < DC; ++j) acc[j] = fmaf(pk, k2 < n_keys ? v[a][j][i] : 0.f, acc[j]);
                     }
             }
         } else {
@@ -541,8 +580,16 @@ static int launch_paged_attention(const void* q, int ldq, const void* k_pool, co
                            table, table_stride, token_slot, positions, static_cast<T*>(out), ldo, q_heads, kv_heads,
                            head_dim, page_tokens, n_layers, layer, scale, window);
     };
-    if (vec) launch(paged_attention_kernel<T, DC, WAVES, true>);
-    else launch(paged_attention_kernel<T, DC, WAVES, false>);
+    const bool pow2 = (page_tokens & (page_tokens - 1)) == 0;
+    if constexpr (DC == 1) {
+        if (vec && pow2 && head_dim == CELEG_WAVE && static_cast<long long>(n_tokens) * q_heads <= WHOLE_MOST) {
+            launch(paged_attention_kernel<T, DC, WAVES, true, true, true>);
+            return CELEG_LAUNCH_RESULT();
+        }
+    }
+    if (vec && pow2) launch(paged_attention_kernel<T, DC, WAVES, true, true, false>);
+    else if (vec) launch(paged_attention_kernel<T, DC, WAVES, true, false, false>);
+    else launch(paged_attention_kernel<T, DC, WAVES, false, false, false>);
     return CELEG_LAUNCH_RESULT();
 }
 
