@@ -11,11 +11,11 @@
 // leave their sums in LDS, where the workgroup adds them in order.  Few rows are bound by reading W: up to 16
 // columns a workgroup, up to 16 wavefronts that each ask for 8 KiB at once, so
 // that even a 1024 x 1024 matrix is asked for by 512 wavefronts in one trip to memory.  Many rows are bound
-// by the matrix cores: larger tiles, operands straight from the caches (16 bytes a cycle and CU of them).
+// by the matrix cores: staged tiles, further down; this kernel where those are too few for the CUs.
 // Measured in a chain over different matrices (before: 64 x 64 tiles of vector instructions, k in order,
 // 137 us for products of up to 64 rows and few columns with K = 1,024): 2 rows, 1024 x 1024 3.3 us, 3072 x 1024
 // 5.5 us, 1024 x 4608 7.2 us (before 613), 65536 x 1024 54 us (5.0 TB/s; before 247); 64 rows, 3072 x 1024
-// 13.7 us; 2,048 rows, 4608 x 1024 256 us (76 TFLOP/s).  Error against 64 bits 2.1e-7 of the result (2-norm), before 3 times that.
+// 13.7 us; 424 rows, 1024 x 4608 64 us (before the order of its loads was pinned 74).  Error against 64 bits 2.1e-7 of the result (2-norm), before 3 times that.
 #include "common.h"
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -26,7 +26,7 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 // GROUP: pieces of 16 values of k that are asked for together.  VEC: rows of X and W lie on 16 bytes
 // and K is a multiple of 4; the same sums in the same order without it.
 template <int RT, int CT, int GROUP, int MAX_THREADS, bool VEC>
-__global__ __launch_bounds__(MAX_THREADS) void gemm_f32_kernel(
+__global__ __launch_bounds__(MAX_THREADS, 2) void gemm_f32_kernel(
     const float* __restrict__ X, int ldx, const float* __restrict__ W, int ldw,
     const float* __restrict__ bias, float* __restrict__ Y, int ldy, int M, int N, int K, int wide_store) {
     constexpr int TILES = RT * CT;
@@ -89,10 +89,15 @@ __global__ __launch_bounds__(MAX_THREADS) void gemm_f32_kernel(
         f32x4_t w1[CT][GROUP], x1[RT][GROUP];
 #pragma unroll
         for (int g = 0; g < F32_PIECES / GROUP; g += 2) {
+            // (the order pinned: left alone the compiler asks for a group right ahead of the products that use it)
             load(k0 + (g + 1) * 16 * GROUP, whole, w1, x1);
+            if (CT > 1) __builtin_amdgcn_sched_barrier(0);
             multiply(w0, x0);
+            if (CT > 1) __builtin_amdgcn_sched_barrier(0);
             if (g + 2 < F32_PIECES / GROUP) load(k0 + (g + 2) * 16 * GROUP, whole, w0, x0);
+            if (CT > 1) __builtin_amdgcn_sched_barrier(0);
             multiply(w1, x1);
+            if (CT > 1) __builtin_amdgcn_sched_barrier(0);
         }
     };
 
@@ -371,18 +376,22 @@ static int launch_f32(const float* X, int ldx, const float* W, int ldw, const fl
     const int waves = max(least, (segments + rounds - 1) / rounds);
     const dim3 grid((N + 16 * CT - 1) / (16 * CT), (M + 16 * RT - 1) / (16 * RT)), block(waves * CELEG_WAVE);
     const size_t lds = static_cast<size_t>(waves) * RT * CT * CELEG_WAVE * sizeof(f32x4_t);
-    if (vec)
-        hipLaunchKernelGGL((gemm_f32_kernel<RT, CT, GROUP, MAX_THREADS, true>), grid, block, lds, stream, X, ldx, W, ldw, bias, Y, ldy, M, N, K, wide_store);
-    else
-        hipLaunchKernelGGL((gemm_f32_kernel<RT, CT, GROUP, MAX_THREADS, false>), grid, block, lds, stream, X, ldx, W, ldw, bias, Y, ldy, M, N, K, wide_store);
+    // (64 x 64 tiles are for rows that cannot be read 16 bytes at a time)
+    if constexpr (RT * CT <= 8) {
+        if (vec) {
+            hipLaunchKernelGGL((gemm_f32_kernel<RT, CT, GROUP, MAX_THREADS, true>), grid, block, lds, stream, X, ldx, W, ldw, bias, Y, ldy, M, N, K, wide_store);
+            return CELEG_LAUNCH_RESULT();
+        }
+    }
+    hipLaunchKernelGGL((gemm_f32_kernel<RT, CT, GROUP, MAX_THREADS, false>), grid, block, lds, stream, X, ldx, W, ldw, bias, Y, ldy, M, N, K, wide_store);
     return CELEG_LAUNCH_RESULT();
 }
 
-// The products of many rows over a short K.  A wavefront has a tile of 16 RT x 16 CT outputs to itself and goes
-// through the segments one after the other, each summed and added as above, so the outputs have the same bits; there
-// is nothing to join, and a last segment that is not whole costs what it has.  2,048 x 4,096: K = 32 18 us (on the
-// kernel above, most of whose wavefronts then wait, 86; before that 26), K = 128 50 (95), K = 160 60 (100; 75).
-template <int RT, int CT, bool VEC>
+// The products of many rows over a short K whose rows cannot be read 16 bytes at a time.  A wavefront has a tile of
+// 16 RT x 16 CT outputs to itself and goes through the segments one after the other, each summed and added as above, so
+// the outputs have the same bits; there is nothing to join, and a last segment that is not whole costs what it has.
+// 2,048 x 4,096, K = 33 28 us (on the kernel above, most of whose wavefronts then wait, 128).
+template <int RT, int CT>
 __global__ __launch_bounds__(256) void gemm_f32_short_kernel(
     const float* __restrict__ X, int ldx, const float* __restrict__ W, int ldw,
     const float* __restrict__ bias, float* __restrict__ Y, int ldy, int M, int N, int K, int wide_store) {
@@ -399,13 +408,9 @@ __global__ __launch_bounds__(256) void gemm_f32_short_kernel(
     for (int ct = 0; ct < CT; ++ct) w_row[ct] = W + static_cast<size_t>(min(col0 + ct * 16 + r16, N - 1)) * ldw;
     auto four = [&](const float* row, int k) __attribute__((always_inline)) {
         f32x4_t v = {0.f, 0.f, 0.f, 0.f};
-        if (VEC) {
-            if (k < K) v = *reinterpret_cast<const f32x4_t*>(row + k);
-        } else {
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (k + i < K) v[i] = row[k + i];
-        }
+        for (int i = 0; i < 4; ++i)
+            if (k + i < K) v[i] = row[k + i];
         return v;
     };
     f32x4_t acc[CT][RT], total[CT][RT];
@@ -468,12 +473,9 @@ __global__ __launch_bounds__(256) void gemm_f32_short_kernel(
 template <int RT, int CT>
 static int launch_f32_short(const float* X, int ldx, const float* W, int ldw, const float* bias, float* Y, int ldy,
                             int M, int N, int K, hipStream_t stream) {
-    const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-    const bool vec = K % 4 == 0 && ldx % 4 == 0 && ldw % 4 == 0 && aligned(X) && aligned(W);
-    const int wide_store = ldy % 4 == 0 && aligned(Y);
+    const int wide_store = ldy % 4 == 0 && (reinterpret_cast<uintptr_t>(Y) & 15) == 0;
     const dim3 grid((N + 64 * CT - 1) / (64 * CT), (M + 16 * RT - 1) / (16 * RT)), block(4 * CELEG_WAVE);
-    auto kernel = vec ? &gemm_f32_short_kernel<RT, CT, true> : &gemm_f32_short_kernel<RT, CT, false>;
-    hipLaunchKernelGGL(kernel, grid, block, 0, stream, X, ldx, W, ldw, bias, Y, ldy, M, N, K, wide_store);
+    hipLaunchKernelGGL((gemm_f32_short_kernel<RT, CT>), grid, block, 0, stream, X, ldx, W, ldw, bias, Y, ldy, M, N, K, wide_store);
     return CELEG_LAUNCH_RESULT();
 }
 
@@ -508,6 +510,142 @@ extern "C" int celeg_gemm_f32_fused(const float* X, int ldx, const float* W, int
 #undef F32_FUSED
 }
 
+// Products of many rows: a workgroup of four wavefronts (two by two) has all of k for a tile of BM x BN, the same sums in
+// the same order.  The operands go through LDS, 32 values of k (a line of 128 bytes a row) at a time and three such steps deep: two
+// are on their way while one is multiplied, so a wavefront waits once a step, for loads that it asked for two steps before,
+// and an operand is read from the L2 once a tile instead of once a wavefront.  Straight from the caches (the kernel
+// above, and one that kept all of k and read a piece ahead) the loads of rows 4 KiB apart met in the same channels:
+// 55 to 82 TFLOP/s as soon as a SIMD had more than one wavefront.  Here the matrix cores are the bound: 2,048 rows, N = 9,216, K =
+// 1,024 317 us (122 TFLOP/s of 153; before 564), N = 2,048 73 (117); 1,024 rows, N = 9,216 166 (286), N = 3,072 59
+// (92); 424 rows, N = 9,216 75 (129), N = 3,072 34 (48); 200 rows, N = 9,216 46 (90); 2,048 rows, K = 256, N = 1,024 13.6 (23).
+#define F32_STEP 32
+#define F32_STEP_CHUNKS (F32_STEP / 4)
+
+template <int N>
+__device__ __forceinline__ void f32_wait_loads() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+template <int BM, int BN>
+__global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(
+    const float* __restrict__ X, int ldx, const float* __restrict__ W, int ldw,
+    const float* __restrict__ bias, float* __restrict__ Y, int ldy, int M, int N, int K, int wide_store) {
+    constexpr int RT = BM / 32, CT = BN / 32, ROWS = BM + BN, LOADS = ROWS * F32_STEP_CHUNKS / 256, STAGES = 3;
+    constexpr int STEPS_A_SEGMENT = F32_SEGMENT / F32_STEP;
+    __shared__ __attribute__((aligned(128))) float stage[STAGES][ROWS * F32_STEP];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / CELEG_WAVE), lane = threadIdx.x % CELEG_WAVE;
+    const int qd = lane >> 4, r16 = lane & 15;
+    const int row0 = blockIdx.y * BM, col0 = blockIdx.x * BN;
+    // chunk c of 16 bytes of a staged row lies at c ^ (row / 2 % 8): 16 lanes that read one chunk of 16 rows meet every bank once
+    // (a thread's loads are of rows 32 apart: the same chunk; a chunk past the end of the row is the row's last one)
+    const int my_chunk = (static_cast<int>(threadIdx.x) % F32_STEP_CHUNKS) ^ ((static_cast<int>(threadIdx.x) / (2 * F32_STEP_CHUNKS)) & 7);
+    const float* src[LOADS];
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+        const int row = (i * 256 + static_cast<int>(threadIdx.x)) / F32_STEP_CHUNKS;
+        src[i] = row < BM ? X + static_cast<size_t>(min(row0 + row, M - 1)) * ldx : W + static_cast<size_t>(min(col0 + row - BM, N - 1)) * ldw;
+    }
+    auto issue = [&](int step) __attribute__((always_inline)) {
+        float* to = stage[step % STAGES];
+        const int k = min(step * F32_STEP + 4 * my_chunk, K - 4);
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i)
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[i] + k),
+                                             (__attribute__((address_space(3))) void*)(to + (i * 256 + wave * CELEG_WAVE) * 4), 16, 0, 0);
+    };
+    const int wr = (wave & 1) * (BM / 2), wc = (wave >> 1) * (BN / 2);
+    f32x4_t acc[CT][RT], total[CT][RT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) total[ct][rt] = acc[ct][rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const int steps = (K + F32_STEP - 1) / F32_STEP;
+    auto multiply = [&](int step, bool whole) __attribute__((always_inline)) {
+        const float* st = stage[step % STAGES];
+#pragma unroll
+        for (int s = 0; s < F32_STEP / 16; ++s) {
+            const int chunk = 4 * s + qd, at = 4 * (chunk ^ ((r16 >> 1) & 7));
+            f32x4_t x[RT], w[CT];
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) x[rt] = *reinterpret_cast<const f32x4_t*>(st + (wr + rt * 16 + r16) * F32_STEP + at);
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) w[ct] = *reinterpret_cast<const f32x4_t*>(st + (BM + wc + ct * 16 + r16) * F32_STEP + at);
+            if (!whole) {
+                const bool in = step * F32_STEP + 4 * chunk < K;
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) x[rt][i] = in ? x[rt][i] : 0.f;
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) w[ct][i] = in ? w[ct][i] : 0.f;
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                    for (int rt = 0; rt < RT; ++rt)
+                        acc[ct][rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[ct][i], x[rt][i], acc[ct][rt], 0, 0, 0);
+        }
+    };
+    auto add_segment = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                total[ct][rt] += acc[ct][rt];
+                acc[ct][rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            }
+    };
+    issue(0);
+    if (steps > 1) issue(1);
+    const int whole = K / F32_STEP;
+    for (int step = 0; step < whole; ++step) {
+        if (step + 1 < steps) f32_wait_loads<LOADS>();
+        else f32_wait_loads<0>();
+        __syncthreads();                                  // the step is here, and everyone has read the one before it
+        if (step + 2 < steps) issue(step + 2);
+        multiply(step, true);
+        if ((step + 1) % STEPS_A_SEGMENT == 0) add_segment();
+    }
+    if (whole < steps) {
+        f32_wait_loads<0>();
+        __syncthreads();
+        multiply(whole, false);
+    }
+    if (steps % STEPS_A_SEGMENT || whole < steps) add_segment();
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        const int row = row0 + wr + rt * 16 + r16;
+        if (row >= M) continue;
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            const int col = col0 + wc + ct * 16 + 4 * qd;
+            float* y = Y + static_cast<size_t>(row) * ldy + col;
+            f32x4_t v = total[ct][rt];
+            if (wide_store && col + 3 < N) {
+                if (bias) v += f32x4_t{bias[col], bias[col + 1], bias[col + 2], bias[col + 3]};
+                *reinterpret_cast<f32x4_t*>(y) = v;
+                continue;
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (col + r < N) y[r] = v[r] + (bias ? bias[col + r] : 0.f);
+        }
+    }
+}
+
+template <int BM, int BN>
+static int launch_f32_tile(const float* X, int ldx, const float* W, int ldw, const float* bias, float* Y, int ldy,
+                           int M, int N, int K, hipStream_t stream) {
+    const int wide_store = ldy % 4 == 0 && (reinterpret_cast<uintptr_t>(Y) & 15) == 0;
+    const dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
+    hipLaunchKernelGGL((gemm_f32_tile_kernel<BM, BN>), grid, dim3(256), 0, stream, X, ldx, W, ldw, bias, Y, ldy, M, N, K, wide_store);
+    return CELEG_LAUNCH_RESULT();
+}
+
 extern "C" int celeg_gemm_f32(const float* X, int ldx, const float* W, int ldw, const float* bias,
                               float* Y, int ldy, int M, int N, int K, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
@@ -516,17 +654,36 @@ extern "C" int celeg_gemm_f32(const float* X, int ldx, const float* W, int ldw, 
         const int g = f32_slices_of(M, N);
         return (g == 4 ? launch_f32_slices<4> : g == 2 ? launch_f32_slices<2> : launch_f32_slices<1>)(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream, F32Tail{});
     }
+    const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    const bool vec = K % 4 == 0 && ldx % 4 == 0 && ldw % 4 == 0 && aligned(X) && aligned(W);
+    // Staged tiles once the smallest of them give every CU more than one, and below that where k is too short to be cut
+    // over eight wavefronts (200 rows, K = 1,024: N = 1,024 16.1 us against 15.9 cut, N = 3,072 24.4 against 30.3; N = 1,024,
+    // K = 4,608 89 against 64; K = 384, N = 2,048 7.9 against 8.5; 40 rows, K = 256 5.7 against 5.8, K = 384 7.6 against 6.8).
+    // (A grid has 65,535 rows of tiles.)
+    const long long small = static_cast<long long>((M + 31) / 32) * ((N + 63) / 64);
+    if (vec && (small > 256 || (M > 32 && K <= 2 * F32_SEGMENT) || (M > 64 && K < 8 * F32_SEGMENT))) {
+        // The tile by what a round of them over 256 CUs takes (in 0.1 us at K = 1,024, all in proportion to K: 64 x 128 tiles
+        // go two at a time through a CU): 424 rows, N = 9,216 75 us with 64 x 128, 78 with 64 x 64, 84 with 32 x 64;
+        // 424 rows, N = 3,072 42, 40 and 34; 1,024 rows, N = 9,216 179, 166 and 183.
+        const auto rounds = [](long long m, long long n) { return (m * n + 255) / 256; };
+        const long long c32 = 20 + 101 * rounds((M + 31) / 32, (N + 63) / 64), c64 = 40 + 185 * rounds((M + 63) / 64, (N + 63) / 64),
+                        c128 = 70 + 350 * rounds((M + 63) / 64, (N + 127) / 128);
+        if (c128 < c64 && c128 < c32) return launch_f32_tile<64, 128>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
+        if (c64 < c32 || M > 32 * 65535) return launch_f32_tile<64, 64>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
+        return launch_f32_tile<32, 64>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
+    }
     if (M <= 32) return launch_f32<2, 1, 8, 512>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
     if (M <= 64) return launch_f32<4, 1, 4, 512>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
-    // One segment of k is one wavefront's work in the kernel above and the others of its workgroup wait; with two, the
-    // wavefront to itself is the faster one once there are tiles enough for every CU (K = 256: 1,024 x 1,024
-    // 14.7 us against 16.9, 424 x 1,024 13.4 against 9.4; K = 384: 2,048 x 1,024 36 against 32).
-    const long long tiles = static_cast<long long>((M + 63) / 64) * ((N + 63) / 64);
-    if (M <= 32 * 65535 && (K <= F32_SEGMENT || (K <= 2 * F32_SEGMENT && tiles >= 256)))      // (a grid has 65,535 rows of tiles)
-        return launch_f32_short<2, 2>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
-    // 64 x 64 tiles (an operand from the caches serves four products) once there are two for every CU; below
-    // that (350 rows: 96 of them at N = 1,024) half the tile and twice the wavefronts
-    if (tiles >= 512)
-        return launch_f32<4, 4, 2, 256>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
+    if (!vec) {
+        // Rows that cannot be read 16 bytes at a time.  One segment of k is one wavefront's work in the kernel above and the
+        // others of its workgroup wait: a tile a wavefront (1,024 x 4,096, K = 33 16 us; 64 x 64 tiles 30, 32 x 64 66), with a little
+        // more than one too once every CU has tiles (1,024 x 1,024, K = 129 13.9 against 15.0).  64 x 64 tiles from one a CU
+        // on (1,024 x 1,024, K = 255 17.8 us, 32 x 64 21.4, a tile a wavefront 25.8; K = 1,023 34 and 40; 424 rows, 112
+        // tiles, 32 and 21).
+        const long long tiles = static_cast<long long>((M + 63) / 64) * ((N + 63) / 64);
+        if (M <= 32 * 65535 && (K <= F32_SEGMENT || (K <= F32_SEGMENT + 16 && tiles >= 256)))
+            return launch_f32_short<2, 2>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
+        if (tiles >= 256) return launch_f32<4, 4, 2, 256>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
+    }
     return launch_f32<2, 4, 2, 512>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
 }

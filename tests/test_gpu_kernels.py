@@ -276,6 +276,22 @@ def test_gemm_f32_many_rows(ops, M, N, K):
     assert torch.equal(one[0], out[M - 1])
 
 
+@pytest.mark.parametrize("M,N,K", [(33, 65, 36), (65, 129, 32), (63, 8257, 100), (130, 8257, 132), (257, 4161, 68), (1057, 1100, 260),
+                                   (513, 6465, 4), (2049, 2049, 96), (31, 16449, 160)])
+def test_gemm_f32_staged_tiles(ops, M, N, K):
+    """Each size of the staged tiles with rows, columns and a step of 32 that do not fill it, one step and many: the bits of rows that
+    cannot be read 16 bytes at a time (another kernel, the same order of sums) and the bound of such sums."""
+    wide, out, same = randn(M, K + 3, seed=27), torch.zeros(M + 1, N, device=DEV), torch.empty(M, N + 3, device=DEV)
+    w, b = randn(N, K, seed=28), randn(N, seed=29)
+    ops.linear(wide[:, 1:K + 1], w, same[:, :N], bias=b)
+    ops.linear(wide[:, 1:K + 1].contiguous(), w, out[:M], bias=b)
+    assert torch.equal(out[:M], same[:, :N]) and float(out[M].abs().max()) == 0
+    x = wide[:, 1:K + 1].double()
+    # a chain of at most 128 products, the segments' sums, the bias: each within 2^-24 of the magnitudes summed
+    bound = (min(K, 128) + K // 128 + 3) * 2.0 ** -24 * (x.abs() @ w.double().abs().T + b.double().abs())
+    assert bool(((out[:M].double() - x @ w.double().T - b.double()).abs() <= bound).all())
+
+
 def test_linear_bf16_and_stored_f32_matrix(ops):
     M, N, K = 9, 200, 96
     x = randn(M, K, seed=10, dtype=torch.bfloat16)
