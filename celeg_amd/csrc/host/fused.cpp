@@ -47,7 +47,6 @@ Tensor stream_stats(Runtime& rt, long long width, int rows) {
 // (inner size producer_inner), writes it.
 Tensor operand_rows(Runtime& rt, const std::string& name, int rows, long long width,
                     std::initializer_list<long long> producer_inner) {
-    if (rt.dtype == DType::F32) return rt.ws.buf(name + "_f32", DType::F32, {rows, width});
     if (rows > STAT_COLUMNS) return rt.ws.buf(name + "_many", DType::BF16, {rows, width});
     bool side_by_side = rt.ops.rows_kernel_ok(rows, {width});
     for (long long k : producer_inner) side_by_side = side_by_side && rt.ops.rows_kernel_ok(rows, {k});

@@ -736,7 +736,7 @@ public:
         if (b_in_) extras.bias = b_in_->view;
         Tensor y;
         if (batch.decode_only && batch.n_seqs == T && taps_ <= 8 && !fused::tiled_step(rt, T, width_)) {   // the fused form holds 8 taps
-            y = fused::operand_rows(rt, "conv_y_fused", T, width_, {width_});
+            y = rt.dtype == DType::F32 ? rt.ws.buf("conv_y", rt.dtype, {T, width_}) : fused::operand_rows(rt, "conv_y_fused", T, width_, {width_});
             ConvOperands conv;
             conv.taps = taps_view_;
             if (b_conv_) conv.bias = b_conv_->view;
@@ -828,7 +828,10 @@ public:
         if (limit_ > 0.f || !(fused::fused_rows_ok(rt, batch, {width_, ff_}) || fused::fused_f32_ok(rt, batch, {width_, ff_})) ||
             w_gate_up_->view.dtype != rt.dtype || w_down_->view.dtype != rt.dtype)
             return false;
-        Tensor act = fused::operand_rows(rt, "ffn_act_fused", batch.n_tokens, ff_, {width_});
+        // (32-bit rows have one layout: the buffer of longer steps, so that a step of few rows makes none of its own, upon which
+        // recorded steps would be recorded again)
+        Tensor act = rt.dtype == DType::F32 ? rt.ws.buf("ffn_act", rt.dtype, {batch.n_tokens, ff_})
+                                            : fused::operand_rows(rt, "ffn_act_fused", batch.n_tokens, ff_, {width_});
         fused::norm_linear(rt, h, norm, w_gate_up_->view, act, Epilogue::Swiglu);
         fused::linear_into_stream(rt, act, w_down_->view, h);
         return true;
