@@ -44,10 +44,25 @@ enum { T_STORE = 0, T_RESIDUAL = 2, T_SWIGLU = 3, T_QKV = 5 };   // (0, 2, 3: th
 
 __device__ __forceinline__ float round_bf16(float x) { return to_float(from_float<bf16>(x)); }
 
-// g / (1 + e^-g) with the hardware's exponential and reciprocal (an ulp each, in 32-bit; the
-// result is rounded to bfloat16): the exact exponential cost the SwiGLU product of 2,048 rows
-// 3 us, the exact division (twelve instructions a value, where the epilogue is bound by them) another 1.9, and half as much at 600 rows.
-__device__ __forceinline__ float tile_silu(float g) { return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)); }
+// o = g / (1 + e^-g) * u with the hardware's exponential (an ulp, in 32-bit: the exact one cost the SwiGLU product
+// of 2,048 rows 3 us) and a correctly rounded reciprocal.  One Newton step behind v_rcp_f32 rounds correctly wherever the
+// reciprocal is a normal number (tried: every 24-bit divisor), for a third of the instructions of the exact division, which
+// stays for the gates whose 1 + e^-g is 2^126 or more (below -87.3; v_rcp_f32 makes 0 of their reciprocals).  w1 with w3,
+// exact division | this | v_rcp_f32 alone: 2,048 rows 42.9 | 40.5 | 39.7 us, 1,000 rows 25.5 | 24.3 | 23.9, 600 rows 19.5 | 19.2 | 18.9.
+template <int N>
+__device__ __forceinline__ void tile_swiglu(const float (&g)[N], const float (&u)[N], float (&o)[N]) {
+    float x[N], largest = 1.0f;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        x[i] = 1.0f + __expf(-g[i]);
+        largest = fmaxf(largest, x[i]);
+        const float r = __builtin_amdgcn_rcpf(x[i]);
+        o[i] = g[i] * fmaf(fmaf(-x[i], r, 1.0f), r, r) * u[i];
+    }
+    if (largest >= 0x1p126f)
+#pragma unroll
+        for (int i = 0; i < N; ++i) o[i] = g[i] * __frcp_rn(x[i]) * u[i];
+}
 
 // A store of 16 bytes a lane that does not stay in the die's L2 until the kernel's end.  Where a product's workgroups all
 // end together, what they wrote leaves the L2s only then, with nothing beside it: written through, w1 with w3 at 2,048 rows (19
@@ -177,14 +192,17 @@ __device__ __forceinline__ void tile_epilogue(
                                  static_cast<__bf16>(old[2]), static_cast<__bf16>(old[3])};
             } else {
                 float o[4];
+                if constexpr (EPI == T_SWIGLU) {
+                    float g[4], u[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    if (EPI == T_SWIGLU) {
-                        const float g = round_bf16(v[0][i]), u = round_bf16(v[NS - 1][i]);
-                        o[i] = tile_silu(g) * u;
-                    } else {
-                        o[i] = v[0][i];
+                    for (int i = 0; i < 4; ++i) {
+                        g[i] = round_bf16(v[0][i]);
+                        u[i] = round_bf16(v[NS - 1][i]);
                     }
+                    tile_swiglu(g, u, o);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) o[i] = v[0][i];
                 }
                 const bf16x4_t piece = bf16x4_t{static_cast<__bf16>(o[0]), static_cast<__bf16>(o[1]),
                                                 static_cast<__bf16>(o[2]), static_cast<__bf16>(o[3])};
@@ -656,9 +674,16 @@ __device__ __forceinline__ void wide_swiglu_epilogue(
         if (m >= M || n >= N) continue;
         const bf16x8_t g = *reinterpret_cast<const bf16x8_t*>(lds + row * PITCH + ch * 16);
         const bf16x8_t u = *reinterpret_cast<const bf16x8_t*>(lds + static_cast<size_t>(BM) * PITCH + row * PITCH + ch * 16);
+        float gate[8], up[8], y[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            gate[i] = static_cast<float>(g[i]);
+            up[i] = static_cast<float>(u[i]);
+        }
+        tile_swiglu(gate, up, y);
         bf16x8_t o;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) o[i] = static_cast<__bf16>(tile_silu(static_cast<float>(g[i])) * static_cast<float>(u[i]));
+        for (int i = 0; i < 8; ++i) o[i] = static_cast<__bf16>(y[i]);
         bf16* const to = static_cast<bf16*>(p.out) + static_cast<size_t>(m) * p.ldo + n;
         if (wide_stores && n + 8 <= N) {
             store_through(reinterpret_cast<bf16x8_t*>(to), o);

@@ -82,6 +82,49 @@ def test_swiglu(ops, shape, M, ff, K):
     assert float((out.double() - ref).abs().max()) <= bound
 
 
+def swiglu_of(ops, gates, ups):
+    """What the SwiGLU epilogue makes of every pair of a gate and an up value: each is one product with 1."""
+    M, N, K = len(gates), len(ups), 64
+    a, w = torch.zeros(M, K, dtype=BF), torch.zeros(2 * N, K, dtype=BF)
+    a[:, 0], a[:, 1], w[:N, 0], w[N:, 1] = gates, 1.0, 1.0, ups
+    out = torch.empty(M, N, dtype=BF, device=DEV)
+    ops.tiled_linear(a.to(DEV), w.to(DEV), out, epilogue="swiglu")
+    return out.cpu()
+
+
+@pytest.mark.parametrize("shape", [0, 9, 10])
+def test_swiglu_of_every_gate(ops, shape):
+    """Every normal gate, those whose 1 + e^-g has a reciprocal below the normal numbers among them."""
+    ops._lib("gemm_tiles").celeg_gemm_tiles_force(shape)
+    gates = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(BF)
+    gates = gates[torch.isfinite(gates) & ((gates.abs() >= 2.0 ** -126) | (gates == 0))]
+    ups = torch.tensor([1.0, -1.4453125, 0.75, 1.9921875] + [2.0 ** k for k in range(-10, 10)], dtype=BF)
+    got, g = swiglu_of(ops, gates, ups).double(), gates.double()
+    want = torch.where(g < -700, torch.zeros_like(g), g / (1 + torch.exp(-g.clamp(min=-700))))[:, None] * ups.double()
+    # the rounding to bfloat16, the exponential's error (|g| 2^-24 from its argument, an ulp of its own) and three roundings; where
+    # e^-g is beyond 32-bit (below -88.7) the result is 0, what it should be then is below 2^-110 with these ups
+    bound = want.abs() * (2.0 ** -8 + (g.abs().clamp(max=100.0)[:, None] + 8) * 2.0 ** -23) + 2.0 ** -126
+    holds = ((got - want).abs() <= bound) | (want.abs() >= 2.0 ** 127)           # (there the product overflows)
+    assert bool(holds[g >= -88.5].all())
+    assert float(got[g < -88.75].abs().max()) == 0
+
+
+@pytest.mark.parametrize("shape", [0, 9, 10])
+def test_swiglu_divides_as_32_bit_division_does(ops, shape):
+    """The quotient is rounded correctly: where no error of the exponential within its bound can change 1 + e^-g, the result's
+    bits follow from it (among them 5.9375, whose quotient lies beside the middle of two bfloat16 numbers)."""
+    ops._lib("gemm_tiles").celeg_gemm_tiles_force(shape)
+    gates = torch.arange(0x3E00, 0x4190, dtype=torch.int32).to(torch.int16).view(BF)       # 0.125 .. 17.9
+    ups = torch.arange(0x3F80, 0x4000, dtype=torch.int32).to(torch.int16).view(BF)         # every mantissa
+    e = torch.exp(-gates.double())
+    error = e * (gates.double() + 4) * 2.0 ** -23
+    x = (1 + e).float()
+    sure = ((1 + e - error).float() == x) & ((1 + e + error).float() == x)
+    assert int(sure.sum()) > 200 and bool(sure[gates == 5.9375].all())
+    want = ((gates.float() * (torch.ones_like(x) / x))[:, None] * ups.float()).to(BF)
+    assert torch.equal(swiglu_of(ops, gates, ups)[sure], want[sure])
+
+
 @pytest.mark.parametrize("shape", list(range(N_SHAPES)) + [-1])
 @pytest.mark.parametrize("M,N,K", SIZES)
 def test_residual_adds_in_place_refreshes_the_copy_and_leaves_partial_sums(ops, shape, M, N, K):
