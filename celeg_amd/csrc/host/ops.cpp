@@ -72,6 +72,7 @@ const char* path_name(Path p) {
         case Path::DecayScanStep: return "decay_scan_step";
         case Path::RoutedExperts: return "routed_experts";
         case Path::LinearF32: return "linear_f32";
+        case Path::LinearF32Fused: return "linear_f32_fused";
         case Path::LinearLibrary: return "linear_library";
         case Path::LinearFewRows: return "linear_few_rows";
         case Path::LinearStandIn: return "linear_stand_in";
@@ -1779,9 +1780,13 @@ void Ops::embed_stats(const Tensor& table, const int* token_ids, const Tensor& o
 // stats[row, :stat_blocks] its partial sums of squares, from which the rows' 1/rms (with eps)
 // scales the sums; their Residual epilogue refreshes out_bf16, the bfloat16 copy of the stream,
 // if given.  They also take w in the layout of fold_weight(packed).
-// Few 32-bit rows: the first inner size is the width of the stream, whose norm takes whole rows in one round.
+// Few 32-bit rows: the first inner size is the width of the stream.  Streams of up to 1,024: a sub-layer's norm, product, end
+// and product into the stream at 2 and 16 rows, kernels of their own | folded, us: width 1,024, q/k/v 10.9 | 9.7, 15.2 | 14.7, SwiGLU of
+// 4,608 23.3 | 19.3, 39.0 | 37.5, convolution 16.6 | 11.2, 19.7 | 16.2; width 1,152 14.9 | 17.8, 16.7 | 16.7, of 3,072 22.6 | 23.2, 31.3 | 32.1,
+// 20.7 | 22.9, 20.9 | 18.0; width 2,048 16.4 | 19.7, 23.2 | 25.0, of 8,192 52.4 | 57.5, 79.4 | 94.6, 26.9 | 31.6, 36.3 | 40.2: a workgroup of
+// eight or sixteen wavefronts that all wait for the norm has nobody beside it on its compute unit.
 bool Ops::fused_linear_f32_ok(int rows, std::initializer_list<long long> inner) {
-    if (rows < 1 || rows > 16 || inner.size() == 0 || *inner.begin() > 2048) return false;
+    if (rows < 1 || rows > 16 || inner.size() == 0 || *inner.begin() > 1024) return false;
     for (long long k : inner)
         if (k <= 0 || k % 4) return false;
     return true;
@@ -1818,7 +1823,7 @@ void Ops::fused_linear_f32(const Tensor& a, const Tensor& w, const Tensor& out, 
         if (c->bias.defined()) dev(c->bias, "conv bias", DType::F32);
         need(!c->bias.defined() || c->bias.numel() == N, "fused_linear (32-bit): the convolution's bias does not fit");
     }
-    took(Path::LinearF32);
+    took(Path::LinearF32Fused);
     kernel_check(celeg_gemm_f32_fused(a.as<float>(), rows_of(a, "a"), w.as<float>(), static_cast<int>(K),
                                       args.bias.defined() ? args.bias.as<float>() : nullptr, out.as<float>(), rows_of(out, "out"),
                                       static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), static_cast<int>(epi),

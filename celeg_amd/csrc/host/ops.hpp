@@ -112,7 +112,7 @@ struct StepPrologue {
 // graph records; a replay counts nothing): what tests and tools ask to see that a size took the
 // path it was meant to take.
 enum class Path : int {
-    AttentionDecode = 0, AttentionDecodeFresh, AttentionRows, AttentionGeneral, AttentionSigmoid, AttentionSigmoidRows, AttentionSigmoidDecode, DeltaRule, AttentionLatent, AttentionLatentRows, AttentionLatentDecode, AttentionBiased, AttentionBiasedRows, AttentionBiasedDecode, ChannelScan, MatrixMemory, MatrixMemoryRows, MatrixMemoryStep, DecayScan, DecayScanRows, DecayScanStep, LinearRecurrentUnit, RoutedExperts, LinearF32, LinearLibrary, LinearFewRows, LinearStandIn,
+    AttentionDecode = 0, AttentionDecodeFresh, AttentionRows, AttentionGeneral, AttentionSigmoid, AttentionSigmoidRows, AttentionSigmoidDecode, DeltaRule, AttentionLatent, AttentionLatentRows, AttentionLatentDecode, AttentionBiased, AttentionBiasedRows, AttentionBiasedDecode, ChannelScan, MatrixMemory, MatrixMemoryRows, MatrixMemoryStep, DecayScan, DecayScanRows, DecayScanStep, LinearRecurrentUnit, RoutedExperts, LinearF32, LinearF32Fused, LinearLibrary, LinearFewRows, LinearStandIn,
     FusedSliced, FusedRows, FusedStaged, Tiled, TiledQkv, ArgmaxMerged, Count
 };
 const char* path_name(Path p);

@@ -175,8 +175,8 @@ class LoadedModel:
 
     def paths(self) -> Dict[str, int]:
         """How many launches each kernel family has taken so far (attention_decode,
-        attention_decode_fresh, attention_rows, attention_general, linear_f32, linear_library, linear_few_rows,
-        fused_sliced, fused_rows, fused_staged, tiled, tiled_qkv ...), counted when the host
+        attention_decode_fresh, attention_rows, attention_general, linear_f32, linear_f32_fused, linear_library,
+        linear_few_rows, fused_sliced, fused_rows, fused_staged, tiled, tiled_qkv ...), counted when the host
         launches (also while a graph records; a replay counts nothing)."""
         return dict(self.native.knobs()["paths"])
 

@@ -109,3 +109,34 @@ def test_logits_with_and_without(model_folders, name):
         errors[fused] = float((got - want).norm() / want.norm())
         lm.close()
     assert errors[1] <= 2e-6 and errors[0] <= 2e-6, errors
+
+
+def one_layer_of_each(folder, width):
+    """A model of a short convolution's and an attention's layer, float32."""
+    from celeg_amd.weights import write_random_model
+    config = {"architectures": ["Lfm2ForCausalLM"], "vocab_size": 256, "hidden_size": width, "num_hidden_layers": 2,
+              "layer_types": ["conv", "full_attention"], "num_attention_heads": width // 32, "num_key_value_heads": width // 64,
+              "head_dim": 32, "intermediate_size": 320, "block_auto_adjust_ff_dim": False, "rope_theta": 10000.0, "conv_L_cache": 3,
+              "conv_bias": False, "tie_word_embeddings": True, "norm_eps": 1e-5, "max_position_embeddings": 128, "eos_token_id": 7}
+    return write_random_model(config, str(folder), seed=width, dtype=torch.float32, std=0.03)
+
+
+@pytest.mark.parametrize("width,folded", [(1024, True), (1088, False), (2048, False)])
+def test_which_streams_are_folded(tmp_path, width, folded):
+    """Up to 16 rows of streams up to 1,024 wide: four products of each layer; wider streams and more rows none."""
+    from celeg_amd.engine import StepEntry, load_model
+    folder = one_layer_of_each(tmp_path, width)
+    cfg, W = plain.load_model_folder(folder)
+    tokens = random_tokens(cfg["vocab_size"], 34, seed=4)
+    ref = plain.model_logits(cfg, W, tokens).double()
+    lm = load_model(folder, dtype="float32", page_tokens=16, n_pages=16, max_requests=2, max_batched_tokens=64)
+    lm.set_knob("use_graphs", 0)
+    slot, rows = lm.cache.open(), []
+    for first, n in ((0, 16), (16, 17), (33, 1)):
+        before = lm.paths()["linear_f32_fused"]
+        assert lm.cache.prepare(slot, first, n)
+        rows.append(lm.runner.step([StepEntry(slot, first, tokens[first:first + n], [n - 1])])[0].double())
+        assert lm.paths()["linear_f32_fused"] - before == (8 if folded and n <= 16 else 0)
+    got, want = torch.stack(rows), ref[[15, 32, 33]]
+    assert float((got - want).norm() / want.norm()) <= 2e-6
+    lm.close()
