@@ -492,21 +492,23 @@ extern "C" int celeg_gemm_f32_fused(const float* X, int ldx, const float* W, int
         (epi == F32_CONV && (taps < 1 || taps > F32_MAX_TAPS || !conv_w || !state || !seq_slot)))
         return static_cast<int>(hipErrorInvalidValue);
     F32Tail f{norm_w, eps, taps, conv_w, conv_b, state, state_slot_stride, seq_slot};
-#define F32_FUSED(EPI, NORM)                                                                                             \
-    (g == 4 ? launch_f32_slices<4, EPI, NORM>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream, f)                           \
-     : g == 2 ? launch_f32_slices<2, EPI, NORM>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream, f)                         \
-              : launch_f32_slices<1, EPI, NORM>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream, f))
+#define F32_FUSED(G, EPI, NORM) launch_f32_slices<G, EPI, NORM>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream, f)
+#define F32_NORMED(EPI) (!norm_w ? static_cast<int>(hipErrorInvalidValue) : M > 8 ? F32_FUSED(1, EPI, true) : F32_FUSED(2, EPI, true))
     // (with a norm a wavefront holds its weight beside the rows: half as many wavefronts of two segments each, 2 rows by 1,024:
     // w1 with w3 12.7 us, in_proj with the convolution 7.2, q/k/v 5.8; blocks of 16 columns 15.8, 8.4 and 7.8, of 4 12.4, 7.6 and 6.1;
     // 4 rows 13.3, 7.5, 5.9; 15.9, 8.6, 7.9; 13.9, 8.2, 6.3)
-    const int g = norm_w ? (M > 8 ? 1 : 2) : f32_slices_of(M, N);
     switch (epi) {
-        case F32_STORE: return norm_w ? F32_FUSED(F32_STORE, true) : static_cast<int>(hipErrorInvalidValue);
-        case F32_RESIDUAL: return norm_w ? static_cast<int>(hipErrorInvalidValue) : F32_FUSED(F32_RESIDUAL, false);
-        case F32_SWIGLU: return norm_w ? F32_FUSED(F32_SWIGLU, true) : static_cast<int>(hipErrorInvalidValue);
-        case F32_CONV: return norm_w ? F32_FUSED(F32_CONV, true) : static_cast<int>(hipErrorInvalidValue);
+        case F32_STORE: return F32_NORMED(F32_STORE);
+        case F32_SWIGLU: return F32_NORMED(F32_SWIGLU);
+        case F32_CONV: return F32_NORMED(F32_CONV);
+        case F32_RESIDUAL: {
+            if (norm_w) return static_cast<int>(hipErrorInvalidValue);
+            const int g = f32_slices_of(M, N);
+            return g == 4 ? F32_FUSED(4, F32_RESIDUAL, false) : g == 2 ? F32_FUSED(2, F32_RESIDUAL, false) : F32_FUSED(1, F32_RESIDUAL, false);
+        }
         default: return static_cast<int>(hipErrorInvalidValue);
     }
+#undef F32_NORMED
 #undef F32_FUSED
 }
 
