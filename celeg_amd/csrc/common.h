@@ -106,6 +106,15 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
     return total;
 }
 
+// The squares of four neighbouring values of a row, the first link of its norm's chain, and a chain with four more.  Which
+// products are fused is said here and not left to the compiler: kernels that form a norm in one order give the same bits.
+__device__ __forceinline__ float squares_of_four(float a, float b, float c, float d) {
+    return fmaf(d, d, fmaf(c, c, fmaf(a, a, __fmul_rn(b, b))));
+}
+__device__ __forceinline__ float add_four_squares(float sum, float a, float b, float c, float d) {
+    return fmaf(d, d, fmaf(c, c, fmaf(b, b, fmaf(a, a, sum))));
+}
+
 // larger float <-> larger key
 __device__ __forceinline__ uint32_t order_key(float f) {
     const uint32_t u = __float_as_uint(f);

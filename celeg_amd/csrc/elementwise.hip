@@ -162,10 +162,9 @@ __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(
     for (int j = 0; j < NV; ++j) {
         const bool in = static_cast<int>(threadIdx.x) + j * 256 < groups;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
+        for (int e = 0; e < 4; ++e)
             if (delta) v[j][e] += d[j][e];
-            if (in) sum += v[j][e] * v[j][e];
-        }
+        if (in) sum = j == 0 ? squares_of_four(v[j][0], v[j][1], v[j][2], v[j][3]) : add_four_squares(sum, v[j][0], v[j][1], v[j][2], v[j][3]);
         if (in && delta && write_back) Vec4<TX>::store(x + src + 4 * (threadIdx.x + j * 256), v[j]);
     }
     sum = block_sum(sum, scratch);

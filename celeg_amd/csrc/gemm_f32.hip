@@ -1,7 +1,8 @@
 // True 32-bit matrix product for the 32-bit path: Y[M,N] = X[M,K] W[N,K]^T (+ bias).
 // No reduced-precision matrix mode: the matrix cores' 32-bit instruction (16x16x4).  Every output
-// element is summed in the same order whatever M, the tile or the batch is, so the logits of a row do
-// not depend on how rows were batched: k in segments of 128, a segment as a chain of 32 instructions
+// element is summed in the same order whatever M, the tile or the batch is, so a row's products do
+// not depend on how rows were batched (nor does a norm folded into them, below; of the norm's own kernels the one for 64 and
+// more rows of up to 1,024 values adds its squares in another order): k in segments of 128, a segment as a chain of 32 instructions
 // (instruction i of a piece of 16 takes the values i, 4 + i, 8 + i and 12 + i), then the segments'
 // sums in order.
 // The reference's projections: y = x W^T, weights [out, in] row-major
@@ -152,7 +153,7 @@ __global__ __launch_bounds__(MAX_THREADS, 2) void gemm_f32_kernel(
 // weights are on their way), behind it the addition into the residual stream, SwiGLU of a gate and an up stream,
 // or the double-gated short convolution of a B, a C and an x stream for one new token per request with its state
 // update.  Streams: rows [s N, (s + 1) N) of W.  An output is computed from the same 32-bit sums by the same
-// operations as where these are kernels of their own; the sum of squares is added up by segments of k.
+// operations as where these are kernels of their own, the squares of a row in the order of its norm's kernel.
 // Reference semantics: RMSNorm src/backend/cpu/kernels/elementwise.cpp:56-76, SwiGLU elementwise.cpp:101-119, short
 // convolution src/backend/cpu/kernels/convolution.cpp:7-28.
 enum { F32_STORE = 0, F32_RESIDUAL = 2, F32_SWIGLU = 3, F32_CONV = 4 };      // (the numbers of the bfloat16 products)
@@ -182,11 +183,13 @@ __global__ __launch_bounds__(NORM ? 1024 / G : 1024) void gemm_f32_slices_kernel
     const float* __restrict__ bias, float* __restrict__ Y, int ldy, int M, int N, int K, int wide_store, const F32Tail f) {
     constexpr int MP = 16 / G, ITEMS = MP * MP / 4;      // sums of four neighbouring columns of a row
     constexpr int NS = f32_streams<EPI>(), OWN = MP / NS;      // columns of a stream that the workgroup owns
-    extern __shared__ f32x4_t parts[];                    // [segment of the round][item], then [row][segment] and [row][column] floats
+    extern __shared__ f32x4_t parts[];                    // [segment of the round][item], then the norm's weight, [row][256 values], [wavefront][piece][lane] and [row][column] floats
     const int wave = threadIdx.x / CELEG_WAVE, lane = threadIdx.x % CELEG_WAVE;
     const int n_waves = blockDim.x / CELEG_WAVE;
-    float* const row_squares = reinterpret_cast<float*>(parts + static_cast<size_t>(n_waves) * G * ITEMS);
-    float* const sums = row_squares + (NORM ? n_waves * G * MP : 0);
+    f32x4_t* const norm_w = parts + static_cast<size_t>(n_waves) * G * ITEMS;
+    float* const row_squares = reinterpret_cast<float*>(norm_w + (NORM ? blockDim.x : 0));
+    float* const chains = row_squares + (NORM ? 8 * MP : 0);
+    float* const sums = chains + (NORM && G == 1 ? 8 * F32_PIECES * CELEG_WAVE : 0);
     const int qd = lane >> 4, r16 = lane & 15;
     const int col0 = blockIdx.x * OWN;
     const float* const x_row = X + static_cast<size_t>(min(r16 % MP, M - 1)) * ldx;
@@ -226,31 +229,33 @@ __global__ __launch_bounds__(NORM ? 1024 / G : 1024) void gemm_f32_slices_kernel
     for (int first = 0; first < segments; first += n_waves * G) {
         const int mine = first + wave * G;                // this wavefront's segments: G of them from here
         const int k0 = (mine + r16 / MP) * F32_SEGMENT + 4 * qd;
-        f32x4_t wv[F32_PIECES], xv[F32_PIECES], nw[NORM ? F32_PIECES : 1];
+        f32x4_t wv[F32_PIECES], xv[F32_PIECES], nw = {0.f, 0.f, 0.f, 0.f};
         const auto load_x = [&]() __attribute__((always_inline)) {
 #pragma unroll
             for (int s = 0; s < F32_PIECES; ++s) xv[s] = *reinterpret_cast<const f32x4_t*>(x_row + k0 + 16 * s);
         };
+        // (the norm's weight goes by way of LDS, four values a thread, 256 a wavefront; held beside the operands, 32 registers)
+        const auto load_norm = [&]() __attribute__((always_inline)) {
+            if (4 * static_cast<int>(threadIdx.x) < K) nw = *reinterpret_cast<const f32x4_t*>(f.norm_w + 4 * threadIdx.x);
+        };
         if (VEC && (mine + G) * F32_SEGMENT <= K) {
             if constexpr (NORM) {       // (the rows first: their squares are added up while the weights are on their way)
                 load_x();
-#pragma unroll
-                for (int s = 0; s < F32_PIECES; ++s) nw[s] = *reinterpret_cast<const f32x4_t*>(f.norm_w + k0 + 16 * s);
+                load_norm();
             }
 #pragma unroll
             for (int s = 0; s < F32_PIECES; ++s) wv[s] = *reinterpret_cast<const f32x4_t*>(w_row + k0 + 16 * s);
             if constexpr (!NORM) load_x();
         } else {
+            if constexpr (NORM) load_norm();
 #pragma unroll
             for (int s = 0; s < F32_PIECES; ++s) {
                 const int k = k0 + 16 * s;
                 wv[s] = xv[s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-                if constexpr (NORM) nw[s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
                 if (VEC) {
                     if (k < K) {
                         wv[s] = *reinterpret_cast<const f32x4_t*>(w_row + k);
                         xv[s] = *reinterpret_cast<const f32x4_t*>(x_row + k);
-                        if constexpr (NORM) nw[s] = *reinterpret_cast<const f32x4_t*>(f.norm_w + k);
                     }
                 } else {
 #pragma unroll
@@ -263,21 +268,43 @@ __global__ __launch_bounds__(NORM ? 1024 / G : 1024) void gemm_f32_slices_kernel
             }
         }
         if constexpr (NORM) {           // (one round: the launch sees to it)
+            norm_w[threadIdx.x] = nw;
+            // The squares in the order of rmsnorm_vec_kernel (up to 1,024 values its own bits): chains over four neighbouring values,
+            // the 64 chains of 256 values as a tree (128 values apart, 64, .. down to 4), these sums one after the other.
+            const auto chain = [&](int s) __attribute__((always_inline)) { return squares_of_four(xv[s][0], xv[s][1], xv[s][2], xv[s][3]); };
+            const auto tree = [&](auto&& of) __attribute__((always_inline)) {
+                const float even = (of(0) + of(4)) + (of(2) + of(6));
+                return sum_row16(sum_half32(even + ((of(1) + of(5)) + (of(3) + of(7)))));
+            };
+            static_assert(G <= 2 && F32_PIECES == 8, "256 values are a wavefront's two segments or those of two neighbouring wavefronts");
             float squares = 0.f;
+            if constexpr (G == 2) {
+                squares = tree([&](int s) __attribute__((always_inline)) { const float v = chain(s); return v + lane_move<LANES_ROTATE_8>(v); });
+            } else {
+                float* const theirs = chains + (wave / 2) * F32_PIECES * CELEG_WAVE + lane;
+                if (wave % 2)
 #pragma unroll
-            for (int s = 0; s < F32_PIECES; ++s)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) squares += xv[s][i] * xv[s][i];
-            squares = sum_half32(sum_row16(squares));     // over the four lanes that share a row and a segment
-            if (qd == 0) row_squares[(r16 % MP) * (n_waves * G) + wave * G + r16 / MP] = squares;
+                    for (int s = 0; s < F32_PIECES; ++s) theirs[s * CELEG_WAVE] = chain(s);
+                __syncthreads();
+                if (wave % 2 == 0) {
+                    const bool there = wave + 1 < n_waves;
+                    squares = tree([&](int s) __attribute__((always_inline)) { return chain(s) + (there ? theirs[s * CELEG_WAVE] : 0.f); });
+                }
+            }
+            constexpr int SUMS = 16 * F32_SEGMENT / 256;
+            if (qd == 0 && (G == 2 ? r16 < MP : wave % 2 == 0)) row_squares[(r16 % MP) * SUMS + wave * G / 2] = squares;
             __syncthreads();
             float all = 0.f;
-            for (int g = 0; g < segments; ++g) all += row_squares[(r16 % MP) * (n_waves * G) + g];
+#pragma unroll
+            for (int g = 0; g < SUMS; ++g)
+                if (g * 256 < K) all += row_squares[(r16 % MP) * SUMS + g];
             const float inv = 1.0f / sqrtf(all / static_cast<float>(K) + f.eps);
 #pragma unroll
-            for (int s = 0; s < F32_PIECES; ++s)
+            for (int s = 0; s < F32_PIECES; ++s) {
+                const f32x4_t w4 = norm_w[k0 / 4 + 4 * s];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) xv[s][i] = xv[s][i] * inv * nw[s][i];
+                for (int i = 0; i < 4; ++i) xv[s][i] = xv[s][i] * inv * w4[i];
+            }
         }
         f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -352,7 +379,7 @@ static int launch_f32_slices(const float* X, int ldx, const float* W, int ldw, c
     const int threads = max(waves * CELEG_WAVE, f32_streams<EPI>() > 1 ? (MP * OWN + CELEG_WAVE - 1) / CELEG_WAVE * CELEG_WAVE : 0);
     const dim3 grid((N + OWN - 1) / OWN), block(threads);
     const size_t waves_run = threads / CELEG_WAVE;
-    const size_t lds = waves_run * G * (MP * MP / 4) * sizeof(f32x4_t) + (NORM ? waves_run * G * MP * sizeof(float) : 0) +
+    const size_t lds = waves_run * G * (MP * MP / 4) * sizeof(f32x4_t) + (NORM ? (4 * threads + 8 * MP + (G == 1 ? 8 * F32_PIECES * CELEG_WAVE : 0)) * sizeof(float) : 0) +
                        (f32_streams<EPI>() > 1 ? MP * MP * sizeof(float) : 0);
     if constexpr (EPI == F32_STORE && !NORM) {
         auto kernel = vec ? &gemm_f32_slices_kernel<G, true, EPI, NORM> : &gemm_f32_slices_kernel<G, false, EPI, NORM>;
@@ -494,9 +521,9 @@ extern "C" int celeg_gemm_f32_fused(const float* X, int ldx, const float* W, int
     F32Tail f{norm_w, eps, taps, conv_w, conv_b, state, state_slot_stride, seq_slot};
 #define F32_FUSED(G, EPI, NORM) launch_f32_slices<G, EPI, NORM>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream, f)
 #define F32_NORMED(EPI) (!norm_w ? static_cast<int>(hipErrorInvalidValue) : M > 8 ? F32_FUSED(1, EPI, true) : F32_FUSED(2, EPI, true))
-    // (with a norm a wavefront holds its weight beside the rows: half as many wavefronts of two segments each, 2 rows by 1,024:
-    // w1 with w3 12.7 us, in_proj with the convolution 7.2, q/k/v 5.8; blocks of 16 columns 15.8, 8.4 and 7.8, of 4 12.4, 7.6 and 6.1;
-    // 4 rows 13.3, 7.5, 5.9; 15.9, 8.6, 7.9; 13.9, 8.2, 6.3)
+    // (behind a norm blocks of 8 columns up to 8 rows, a wavefront two segments, the halves of 256 values: with the norm's weight still
+    // in registers 2 rows by 1,024 took, w1 with w3 12.7 us, in_proj with the convolution 7.2, q/k/v 5.8; blocks of 16 columns 15.8, 8.4
+    // and 7.8, of 4 12.4, 7.6 and 6.1; 4 rows 13.3, 7.5, 5.9; 15.9, 8.6, 7.9; 13.9, 8.2, 6.3.  By way of LDS w1 with w3 11.7.)
     switch (epi) {
         case F32_STORE: return F32_NORMED(F32_STORE);
         case F32_SWIGLU: return F32_NORMED(F32_SWIGLU);

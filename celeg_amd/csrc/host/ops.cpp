@@ -1785,8 +1785,10 @@ void Ops::embed_stats(const Tensor& table, const int* token_ids, const Tensor& o
 // 4,608 23.3 | 19.3, 39.0 | 37.5, convolution 16.6 | 11.2, 19.7 | 16.2; width 1,152 14.9 | 17.8, 16.7 | 16.7, of 3,072 22.6 | 23.2, 31.3 | 32.1,
 // 20.7 | 22.9, 20.9 | 18.0; width 2,048 16.4 | 19.7, 23.2 | 25.0, of 8,192 52.4 | 57.5, 79.4 | 94.6, 26.9 | 31.6, 36.3 | 40.2: a workgroup of
 // eight or sixteen wavefronts that all wait for the norm has nobody beside it on its compute unit.
+// From 256 on, where the norm's own kernel adds the squares in the order of these products, so that a row has the same bits
+// in steps of up to 16 rows and in longer ones.
 bool Ops::fused_linear_f32_ok(int rows, std::initializer_list<long long> inner) {
-    if (rows < 1 || rows > 16 || inner.size() == 0 || *inner.begin() > 1024) return false;
+    if (rows < 1 || rows > 16 || inner.size() == 0 || *inner.begin() < 256 || *inner.begin() > 1024) return false;
     for (long long k : inner)
         if (k <= 0 || k % 4) return false;
     return true;

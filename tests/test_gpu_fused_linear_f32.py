@@ -90,6 +90,30 @@ def test_long_rows_go_into_the_stream_and_are_refused_behind_a_norm(K):
         assert call(x, w, got, 40, STORE, torch.ones(K, device=DEV)) != 0
 
 
+@pytest.mark.parametrize("M", [1, 3, 8, 9, 16])
+@pytest.mark.parametrize("K", [256, 260, 380, 384, 388, 516, 640, 768, 896, 1000, 1020, 1024])
+def test_the_norm_has_the_bits_of_its_own_kernel(M, K):
+    """A row's result is the same whether its norm is folded in (steps of up to 16 rows) or a kernel of its own (longer steps)."""
+    gen = torch.Generator().manual_seed(K + M)
+    x = (torch.randn(M, K, generator=gen) * torch.exp(2.0 * torch.randn(M, K, generator=gen))).to(DEV)
+    norm, w = (1.0 + 0.3 * torch.randn(K, generator=gen)).to(DEV), torch.randn(24, K, generator=gen).to(DEV)
+    normed, got, want = torch.empty_like(x), torch.empty(M, 24, device=DEV), torch.empty(M, 24, device=DEV)
+    check(native.lib().celeg_rmsnorm(ptr(x), 0, None, 0, ptr(norm), ptr(normed), 0, None, M, K, ctypes.c_float(1e-5), 0, None))
+    check(native.lib().celeg_gemm_f32(ptr(normed), K, ptr(w), K, None, ptr(want), 24, M, 24, K, None))
+    check(call(x, w, got, 24, STORE, norm))
+    assert torch.equal(got, want)
+    # the other ends: the convolution of one tap of 1 multiplies the streams, SwiGLU is a row's own
+    out, one = torch.empty(M, 8, device=DEV), torch.empty(1, 12, device=DEV)
+    conv = (torch.ones(8, 1, device=DEV), None, torch.zeros(M, 1, 8, device=DEV), torch.arange(M, dtype=torch.int32, device=DEV))
+    check(call(x, w, out, 8, CONV, norm, None, conv))
+    streams = want.view(M, 3, 8)
+    assert torch.equal(out, streams[:, 1] * (streams[:, 0] * streams[:, 2]))
+    out = torch.empty(M, 12, device=DEV)
+    check(call(x, w, out, 12, SWIGLU, norm))
+    check(call(x[M - 1:], w, one, 12, SWIGLU, norm))
+    assert torch.equal(one[0], out[M - 1])
+
+
 @pytest.mark.parametrize("name", ["B", "D"])
 def test_logits_with_and_without(model_folders, name):
     from celeg_amd.engine import StepEntry, load_model
@@ -121,9 +145,10 @@ def one_layer_of_each(folder, width):
     return write_random_model(config, str(folder), seed=width, dtype=torch.float32, std=0.03)
 
 
-@pytest.mark.parametrize("width,folded", [(1024, True), (1088, False), (2048, False)])
+@pytest.mark.parametrize("width,folded", [(192, False), (256, True), (1024, True), (1088, False), (2048, False)])
 def test_which_streams_are_folded(tmp_path, width, folded):
-    """Up to 16 rows of streams up to 1,024 wide: four products of each layer; wider streams and more rows none."""
+    """Up to 16 rows of streams 256 to 1,024 wide: four products of each layer; other streams and more rows none.  A row's logits are the
+    same beside 0, 15 and 16 other tokens."""
     from celeg_amd.engine import StepEntry, load_model
     folder = one_layer_of_each(tmp_path, width)
     cfg, W = plain.load_model_folder(folder)
@@ -139,4 +164,14 @@ def test_which_streams_are_folded(tmp_path, width, folded):
         assert lm.paths()["linear_f32_fused"] - before == (8 if folded and n <= 16 else 0)
     got, want = torch.stack(rows), ref[[15, 32, 33]]
     assert float((got - want).norm() / want.norm()) <= 2e-6
+    last = []
+    for sizes in ((16, 17), (16, 16, 1), (17, 16), (1, 15, 17)):         # position 32 ends a portion of 17, 1, 16 and 17
+        slot, at = lm.cache.open(), 0
+        for n in sizes:
+            assert lm.cache.prepare(slot, at, n)
+            out = lm.runner.step([StepEntry(slot, at, tokens[at:at + n], [n - 1])])[0].clone()
+            at += n
+        last.append(out)
+        lm.cache.close(slot)
+    assert all(torch.equal(x, last[0]) for x in last)
     lm.close()
