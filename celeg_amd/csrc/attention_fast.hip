@@ -54,8 +54,24 @@ __device__ __forceinline__ size_t kv_block(int page, int n_layers, int layer, in
 // The running maximum of a row follows the scores only when some row's grows by more than
 // 8 (a factor 2^8): until then probabilities are taken against the older value, stay below
 // 2^8, and numerator and denominator carry the same factor.
-template <int HD, int RT, int NH, bool SHARE>
-__global__ __launch_bounds__(256 * NH) void attention_rows_kernel(
+// AHEAD: of how many of a round's four tiles of 16 keys the operands are read before the first product that uses one (0: left
+// to the compiler, which waits for every second read; 2,001 rows behind 18,000 tokens, 16 heads of 64: 252 us, four tiles ahead 233).
+// As many as leave a SIMD the wavefronts that it holds without, else the reads cost more than they save.  Before all this | four
+// tiles ahead everywhere | as here, us (32 heads on 8; 8,192 rows of one prompt; 64 prompts of 128; 4 x 2,048 behind 6,000 tokens):
+// heads sharing keys, 64 342 | 365 | 334, 54 | 78 | 54, 567 | 607 | 549; of 128 575 | 565 | 569, 106 | 105 | 105, 969 | 943 | 949; of 96
+// 539 | 481 | 478, 92 | 99 | 92, 895 | 799 | 786 (as for short prompts, where three wavefronts fit, 524, 92, 876); of 32 (left 400 | 404 | 395).
+// Tiles of 128 rows, heads of 128, not shared, 16 heads, 2,048 rows 50.8 | 50.4 (9 registers to memory) | 48.8.
+constexpr int rows_ahead(int head_dim, int row_tiles, int sets, bool share) {
+    if (sets == 1) return 0;
+    if (share) return head_dim == 32 ? 1 : head_dim == 128 && row_tiles == 1 ? 0 : 2;
+    return head_dim * row_tiles < 256 ? 4 : 0;
+}
+// wavefronts that a SIMD is to hold where the compiler would take a few registers too many for them
+constexpr int rows_waves(int head_dim, int row_tiles, int sets, int ahead) {
+    return head_dim == 96 && ((row_tiles == 1 && sets == 1) || (row_tiles == 2 && ahead == 1)) ? 3 : 1;
+}
+template <int HD, int RT, int NH, bool SHARE, int AHEAD>
+__global__ __launch_bounds__(256 * NH, rows_waves(HD, RT, NH, AHEAD)) void attention_rows_kernel(
     const bf16* __restrict__ q, int ldq, const bf16* __restrict__ k_pool,
     const bf16* __restrict__ v_pool, const int* __restrict__ table, int table_stride,
     const int* __restrict__ cu_seqlens, const int* __restrict__ seq_slot,
@@ -198,7 +214,13 @@ __global__ __launch_bounds__(256 * NH) void attention_rows_kernel(
         // (the pages by a branch round all of them: a choice between two addresses for each would be loads that wait for
         // LDS and for memory alike)
         unsigned kpage[CH], vpage[CH];
-        if (pages_in_lds) {
+        if (SHARE && HD == 32) {        // (one piece a thread: the choice costs less than the branch, 400 us against 408)
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                kpage[j] = pages_in_lds ? spages[pg + k_pg[j]] : pages[min(max(page0 + pg + k_pg[j], live_page), last_page)];
+                vpage[j] = pages_in_lds ? spages[pg + v_pg[j]] : pages[min(max(page0 + pg + v_pg[j], live_page), last_page)];
+            }
+        } else if (pages_in_lds) {
 #pragma unroll
             for (int j = 0; j < CH; ++j) {
                 kpage[j] = spages[pg + k_pg[j]];
@@ -238,23 +260,34 @@ __global__ __launch_bounds__(256 * NH) void attention_rows_kernel(
         for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
             for (int kt = 0; kt < 4; ++kt) sacc[rt][kt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
-        // (all keys' operands of a round ahead of its products: left to the compiler every second one was waited for. 2,001 rows
-        // behind 18,000 tokens, 16 heads of 64: 252 -> 233 us with the pages' ways and the queries' wait as they are, 2,048 rows 28.2 -> 27.3.  The values' operands
-        // ahead of the exponentials likewise 252 to 257, the next round's scores beside this one's exponentials 312)
-        bf16x8_t kf[4][KS];
+        const auto keys_of = [&](int kt, int st) __attribute__((always_inline)) {
+            return *reinterpret_cast<const bf16x8_t*>(sK + (buf * 64 + 16 * kt + c) * KROW + qd * DQ + st * 8);
+        };
+        const auto multiply = [&](const bf16x8_t kf, int kt, int st) __attribute__((always_inline)) {
 #pragma unroll
-        for (int st = 0; st < KS; ++st)
+            for (int rt = 0; rt < RT; ++rt)
+                sacc[rt][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qreg[rt][st], sacc[rt][kt], 0, 0, 0);
+        };
+        if constexpr (AHEAD > 0) {
+#pragma unroll
+            for (int k0 = 0; k0 < 4; k0 += AHEAD) {
+                bf16x8_t kf[AHEAD > 0 ? AHEAD : 1][KS];
+#pragma unroll
+                for (int st = 0; st < KS; ++st)
+#pragma unroll
+                    for (int kt = 0; kt < AHEAD; ++kt) kf[kt][st] = keys_of(k0 + kt, st);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int st = 0; st < KS; ++st)
+#pragma unroll
+                    for (int kt = 0; kt < AHEAD; ++kt) multiply(kf[kt][st], k0 + kt, st);
+            }
+        } else {
 #pragma unroll
             for (int kt = 0; kt < 4; ++kt)
-                kf[kt][st] = *reinterpret_cast<const bf16x8_t*>(sK + (buf * 64 + 16 * kt + c) * KROW + qd * DQ + st * 8);
-        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int st = 0; st < KS; ++st)
-#pragma unroll
-            for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-                for (int rt = 0; rt < RT; ++rt)
-                    sacc[rt][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[kt][st], qreg[rt][st], sacc[rt][kt], 0, 0, 0);
+                for (int st = 0; st < KS; ++st) multiply(keys_of(kt, st), kt, st);
+        }
         bf16x8_t pb[RT][2];
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
@@ -409,19 +442,75 @@ extern "C" long long celeg_attention_rows_lds_bytes(int head_dim, int sets, int 
     return staging + min(static_cast<long long>(min(table_stride + 8, ROWS_MAX_PAGES_IN_LDS)), room) * 4;
 }
 
-template <int HD, int RT, int NH, bool SHARE>
+// LDS of a launch: staging buffers, and a tile's pages with room for a round's worth behind the last: the whole of a request's
+// block-table row where that is at most ROWS_MAX_PAGES_IN_LDS entries (16 KB; with the largest staging buffers, 143,360 bytes, still
+// inside 160 KB)
+template <int HD, int NH, bool SHARE>
+static size_t rows_lds(int table_stride, int& pages_room) {
+    const size_t staging = static_cast<size_t>(SHARE ? 1 : NH) * 2 * (64 * (HD + 8) + HD * (64 + 8)) * sizeof(bf16);
+    pages_room = min(min(table_stride + 8, ROWS_MAX_PAGES_IN_LDS),
+                     staging < 160 * 1024 ? static_cast<int>((160 * 1024 - staging) / sizeof(int)) : 0);
+    return staging + static_cast<size_t>(pages_room) * sizeof(int);
+}
+
+// An instantiation of the kernel, as a type, and the choice of one: use(RowsKernel<..>{}) for these sizes.
+template <int HD_, int RT_, int NH_, bool SHARE_, int AHEAD_ = rows_ahead(HD_, RT_, NH_, SHARE_)>
+struct RowsKernel {
+    static constexpr int HD = HD_, RT = RT_, NH = NH_, AHEAD = AHEAD_;
+    static constexpr bool SHARE = SHARE_;
+};
+template <int HD, typename F>
+static int use_rows_form(int rows_per_tile, int form, F use) {
+    if (rows_per_tile == 64)
+        return form == 1 ? use(RowsKernel<HD, 1, 1, false>{}) : form == 2 ? use(RowsKernel<HD, 1, 2, false>{}) : use(RowsKernel<HD, 1, 2, true>{});
+    return form == 1 ? use(RowsKernel<HD, 2, 1, false>{}) : form == 2 ? use(RowsKernel<HD, 2, 2, false>{}) : use(RowsKernel<HD, 2, 2, true>{});
+}
+template <typename F>
+static int use_rows_kernel(int head_dim, int rows_per_tile, int form, int keys, F use) {
+    if (rows_per_tile != 64 && rows_per_tile != 128) return static_cast<int>(hipErrorInvalidValue);
+    if (form < 1 || form > 4) return static_cast<int>(hipErrorInvalidValue);
+    if (form == 4) {
+        if (rows_per_tile != 64 || (head_dim != 32 && head_dim != 64)) return static_cast<int>(hipErrorInvalidValue);
+        return head_dim == 32 ? use(RowsKernel<32, 1, 4, false>{}) : use(RowsKernel<64, 1, 4, false>{});
+    }
+    // heads of 96 that share keys, few rounds a tile: a third wavefront a SIMD gains more than reads further ahead (64 prompts of
+    // 128 92 us against 99, 32 of 256 81.0 against 83.9; 16 of 512 89.8 against 87.8)
+    if (head_dim == 96 && form == 3 && rows_per_tile == 128 && keys < 512) return use(RowsKernel<96, 2, 2, true, 1>{});
+    switch (head_dim) {
+        case 32: return use_rows_form<32>(rows_per_tile, form, use);
+        case 64: return use_rows_form<64>(rows_per_tile, form, use);
+        case 96: return use_rows_form<96>(rows_per_tile, form, use);
+        case 128: return use_rows_form<128>(rows_per_tile, form, use);
+        default: return static_cast<int>(hipErrorInvalidValue);
+    }
+}
+
+// What a compute unit holds of the kernel chosen for these sizes: its workgroups, and the bytes of registers that a lane keeps in memory.
+extern "C" int celeg_attention_rows_residency(int head_dim, int rows_per_tile, int form, int keys, int table_stride, int* workgroups,
+                                              int* spilled) {
+    return use_rows_kernel(head_dim, rows_per_tile, form, keys, [&](auto k) {
+        using K = decltype(k);
+        auto kernel = attention_rows_kernel<K::HD, K::RT, K::NH, K::SHARE, K::AHEAD>;
+        int pages_room = 0;
+        const size_t lds = rows_lds<K::HD, K::NH, K::SHARE>(table_stride, pages_room);
+        hipFuncAttributes attributes;
+        hipError_t e = hipFuncGetAttributes(&attributes, reinterpret_cast<const void*>(kernel));
+        if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(workgroups, kernel, 256 * K::NH, lds);
+        *spilled = static_cast<int>(attributes.localSizeBytes);
+        return static_cast<int>(e);
+    });
+}
+
+template <typename K>
 static int launch_attention_rows(
     const void* q, int ldq, const void* k_pool, const void* v_pool, const int* table,
     int table_stride, const int* cu_seqlens, const int* seq_slot, const int* seq_start,
     int n_seqs, int n_tokens, void* out, int ldo, int q_heads, int kv_heads, int page_tokens,
     int n_layers, int layer, float scale, int window, hipStream_t stream) {
-    // staging buffers, and a tile's pages with room for a round's worth behind the last: the
-    // whole of a request's block-table row where that is at most ROWS_MAX_PAGES_IN_LDS entries
-    // (16 KB; with the largest staging buffers, 143,360 bytes, still inside 160 KB)
-    const size_t staging = static_cast<size_t>(SHARE ? 1 : NH) * 2 * (64 * (HD + 8) + HD * (64 + 8)) * sizeof(bf16);
-    const int pages_room = min(min(table_stride + 8, ROWS_MAX_PAGES_IN_LDS),
-                               staging < 160 * 1024 ? static_cast<int>((160 * 1024 - staging) / sizeof(int)) : 0);
-    const size_t lds = staging + static_cast<size_t>(pages_room) * sizeof(int);
+    constexpr int HD = K::HD, RT = K::RT, NH = K::NH;
+    constexpr bool SHARE = K::SHARE;
+    int pages_room = 0;
+    const size_t lds = rows_lds<HD, NH, SHARE>(table_stride, pages_room);
     static_assert(SHARE || static_cast<size_t>(NH - 1) * 4 * RT * (4 * (HD / 16) + 2) * 64 * sizeof(float) <=
                                static_cast<size_t>(NH) * 2 * (64 * (HD + 8) + HD * (64 + 8)) * sizeof(bf16),
                   "what the sets hand over fits the staging buffers");
@@ -429,7 +518,7 @@ static int launch_attention_rows(
     // the kernel multiplies page numbers by the elements of a page in 32 x 32 -> 64 bits
     if (static_cast<size_t>(n_layers) * kv_heads * page_tokens * HD >= (size_t{1} << 31))
         return static_cast<int>(hipErrorInvalidValue);
-    auto kernel = attention_rows_kernel<HD, RT, NH, SHARE>;
+    auto kernel = attention_rows_kernel<HD, RT, NH, SHARE, K::AHEAD>;
     if (lds > 48 * 1024) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -472,13 +561,13 @@ extern "C" int celeg_attention_rows_bf16(
     if (page_tokens < 16 || (page_tokens & (page_tokens - 1)) || q_heads % kv_heads || (ldq % 8) ||
         (ldo % 4))
         return static_cast<int>(hipErrorInvalidValue);
+    int keys = context_hint > 0 ? context_hint : n_tokens;
+    if (window > 0 && window < keys) keys = window;
     if (rows_per_tile == 0) {
         // tiles of 128 rows read the staged keys for twice the rows, tiles of 64 rows put twice
         // the workgroups on the chip: the larger ones once there are enough, sooner if each
         // has many keys to go through
         const long long small_tiles = static_cast<long long>(n_tokens / 64 + n_seqs) * q_heads;
-        int keys = context_hint > 0 ? context_hint : n_tokens;
-        if (window > 0 && window < keys) keys = window;
         rows_per_tile = small_tiles >= 1024 || (small_tiles >= 512 && keys >= 4096) ? 128 : 64;
     }
     if (rows_per_tile != 64 && rows_per_tile != 128) return static_cast<int>(hipErrorInvalidValue);
@@ -487,29 +576,10 @@ extern "C" int celeg_attention_rows_bf16(
         const long long shared = static_cast<long long>(n_tokens / rows_per_tile + n_seqs) * kv_heads * ((group + 1) / 2);
         form = group >= 2 && shared >= 1024 ? 3 : 2;
     }
-    if (form < 1 || form > 4) return static_cast<int>(hipErrorInvalidValue);
-    if (form == 4 && (rows_per_tile != 64 || head_dim > 64)) return static_cast<int>(hipErrorInvalidValue);
-#define CELEG_ROWS_ARGS                                                                            \
-    q, ldq, k_pool, v_pool, table, table_stride, cu_seqlens, seq_slot, seq_start, n_seqs, n_tokens, \
-        out, ldo, q_heads, kv_heads, page_tokens, n_layers, layer, scale, window, stream
-#define CELEG_ROWS_RT(HD_, RT_)                                                              \
-    (form == 1 ? launch_attention_rows<HD_, RT_, 1, false>(CELEG_ROWS_ARGS)                   \
-     : form == 2 ? launch_attention_rows<HD_, RT_, 2, false>(CELEG_ROWS_ARGS)                 \
-                 : launch_attention_rows<HD_, RT_, 2, true>(CELEG_ROWS_ARGS))
-#define CELEG_ROWS(HD_) return rows_per_tile == 64 ? CELEG_ROWS_RT(HD_, 1) : CELEG_ROWS_RT(HD_, 2)
-    if (form == 4)
-        return head_dim == 32 ? launch_attention_rows<32, 1, 4, false>(CELEG_ROWS_ARGS)
-                              : launch_attention_rows<64, 1, 4, false>(CELEG_ROWS_ARGS);
-    switch (head_dim) {
-        case 32: CELEG_ROWS(32);
-        case 64: CELEG_ROWS(64);
-        case 96: CELEG_ROWS(96);
-        case 128: CELEG_ROWS(128);
-        default: return static_cast<int>(hipErrorInvalidValue);
-    }
-#undef CELEG_ROWS
-#undef CELEG_ROWS_RT
-#undef CELEG_ROWS_ARGS
+    return use_rows_kernel(head_dim, rows_per_tile, form, keys, [&](auto k) {
+        return launch_attention_rows<decltype(k)>(q, ldq, k_pool, v_pool, table, table_stride, cu_seqlens, seq_slot, seq_start, n_seqs, n_tokens,
+                                                  out, ldo, q_heads, kv_heads, page_tokens, n_layers, layer, scale, window, stream);
+    });
 }
 
 // ================================================================ one row per request

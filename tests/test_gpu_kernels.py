@@ -963,6 +963,31 @@ def test_attention_rows_with_the_block_table_looked_up_in_memory(ops):
         lib.celeg_attention_rows_pages_in_lds(0)
 
 
+@pytest.mark.parametrize("heads,kv_heads,head_dim", [(4, 1, 32), (4, 2, 64), (3, 1, 96)])
+def test_shared_attention_rows_with_the_block_table_looked_up_in_memory(ops, heads, kv_heads, head_dim):
+    lib = ops._lib("attention_fast")
+    lib.celeg_attention_rows_pages_in_lds(8)
+    ops.attention_rows_per_tile, ops.attention_rows_form = 128, 3
+    try:
+        attention_case(ops, torch.bfloat16, heads, kv_heads, head_dim, lengths=[717, 150, 390], cuts=[330, 61, 200], boost=(2, 700))
+    finally:
+        lib.celeg_attention_rows_pages_in_lds(0)
+        ops.attention_rows_per_tile = ops.attention_rows_form = 0
+
+
+@pytest.mark.parametrize("head_dim,rows_per_tile,form,keys,least", [
+    (32, 64, 2, 4096, 3), (32, 128, 2, 4096, 2), (32, 64, 3, 4096, 3), (32, 128, 3, 4096, 2), (64, 64, 2, 4096, 1), (64, 128, 2, 4096, 1),
+    (64, 64, 3, 4096, 2), (64, 128, 3, 4096, 2), (96, 64, 2, 4096, 1), (96, 128, 2, 4096, 1), (96, 64, 3, 4096, 2), (96, 128, 3, 4096, 1),
+    (96, 128, 3, 256, 1), (128, 64, 2, 4096, 1), (128, 128, 2, 4096, 1), (128, 64, 3, 4096, 2), (128, 128, 3, 4096, 1),
+    (32, 64, 1, 4096, 4), (64, 64, 1, 4096, 3), (96, 64, 1, 4096, 2), (96, 128, 1, 4096, 2), (128, 64, 1, 4096, 2), (128, 128, 1, 4096, 1)])
+def test_attention_rows_keeps_its_workgroups_on_a_compute_unit(ops, head_dim, rows_per_tile, form, keys, least):
+    """Reading a round's keys ahead takes registers: no kernel may keep some of them in memory, and where LDS lets a compute unit
+    hold several workgroups, the registers must too (with one of two, 64 prompts of 128 tokens took 78 us instead of 54)."""
+    workgroups, spilled = ctypes.c_int(0), ctypes.c_int(-1)
+    code = ops._lib("attention_fast").celeg_attention_rows_residency(head_dim, rows_per_tile, form, keys, 2048, ctypes.byref(workgroups), ctypes.byref(spilled))
+    assert code == 0 and spilled.value == 0 and workgroups.value >= least, (workgroups.value, spilled.value)
+
+
 @pytest.mark.parametrize("head_dim,page_tokens", [(64, 16), (128, 16), (32, 32)])
 def test_window_attention_never_reads_pages_it_has_given_back(ops, head_dim, page_tokens):
     """A window group hands back the pages that the window has passed; the device's block
