@@ -359,10 +359,12 @@ extern "C" int celeg_qk_norm_rope_store(
 // Bound by the latency of its loads.  VEC: keys and, from a chunk that starts on a boundary, values
 // come 16 bytes a load (a dimension's keys lie side by side in a page), a chunk's values 16 keys ahead of
 // the sums; the sums run in the same order without it.  No condition stands round a key's product with its values (each read
-// of a weight from LDS would be waited for by itself).  Heads of 64 and few rows (WHOLE, 122 registers): all keys and values of
-// a chunk are asked for before the first is used.  16 heads of 64, before (with that condition, divisions by the page's
-// size and values 16 keys at a time) and now: 32-bit, 2 requests decoding at 350 tokens 15.2 -> 8.8 us, one at 8,000 213 -> 110,
-// prompts of 424 rows 52.5 -> 44.0; bfloat16, 2 requests 12.3 -> 6.8, a prompt of 512 rows 86.7 -> 60.
+// of a weight from LDS would be waited for by itself).  Heads of 64 and few rows (WHOLE): a chunk of more than 16 keys is asked
+// for as a whole, its values, in 32-bit, while the keys' products are made (keys and values together are more registers than
+// four wavefronts a SIMD have); of a shorter one the 16 at a time that there are (3 keys 3.4 us against 4.3, 60 requests at 8 4.1
+// against 5.2, 17 keys 4.7 against 4.05).  16 heads of 64, before (with that condition, divisions by the page's size and values
+// 16 keys at a time) and now: 32-bit, 2 requests decoding at 350 tokens 14.9 -> 8.0 us, one at 8,000 214 -> 109, prompts of 424
+// rows 52.5 -> 44.0; bfloat16, 2 requests 12.2 -> 6.2, a prompt of 512 rows 86.7 -> 60.
 #define ATT_MAX_DIM_CHUNKS 4  // head_dim <= 256
 // Wavefronts a row: four, and with a window no more than it has chunks of 64 keys, so that each has a chunk and the
 // sums are those of four.  Idle wavefronts cost a prompt what live ones do: 1,024 rows, 16 heads of 64, bfloat16, a
@@ -436,8 +438,9 @@ __global__ __launch_bounds__(WAVES * CELEG_WAVE) void paged_attention_kernel(
             return v_pool + cache_offset(page2, n_layers, layer, kv_heads, kvh, page_tokens, 0, head_dim) + in_page(base + kk);
         };
         typename Wide<T>::raw kr[WHOLE ? CELEG_WAVE / W : 1], vr[WHOLE ? CELEG_WAVE / W : 1];
+        const bool whole = WHOLE && wide_values && n_keys > 16;
         if constexpr (WHOLE) {
-            if (wide_values) {
+            if (whole) {
                 const int k_at = min(key, pos);
                 const T* const kp = k_pool + cache_offset(page, n_layers, layer, kv_heads, kvh, page_tokens, in_page(k_at), CELEG_WAVE);
 #pragma unroll
@@ -449,7 +452,7 @@ __global__ __launch_bounds__(WAVES * CELEG_WAVE) void paged_attention_kernel(
             }
         }
         float s = -INFINITY;
-        if (WHOLE && wide_values) {
+        if (whole) {
             float dot = 0.f;
 #pragma unroll
             for (int a = 0; a < (WHOLE ? CELEG_WAVE / W : 0); ++a)
@@ -487,7 +490,7 @@ __global__ __launch_bounds__(WAVES * CELEG_WAVE) void paged_attention_kernel(
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
         for (int j = 0; j < DC; ++j) acc[j] *= corr;
-        if (WHOLE && wide_values) {
+        if (whole) {
             // (behind the row's own key memory may hold anything; a condition round a key's product would have each read of its
             // weight waited for by itself: 64 trips to LDS in a row)
             if (n_keys == CELEG_WAVE) {

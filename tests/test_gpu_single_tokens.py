@@ -166,3 +166,33 @@ def test_sigmoid_attention_of_single_tokens_is_no_further_from_the_exact_result(
         torch.cuda.synchronize()
         off[parts] = float((out.double() - want).norm() / want.norm())
     assert max(off[parts] for parts in (1, 5, 8)) <= 1.01 * off[0] <= 4e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, BF])
+@pytest.mark.parametrize("window", [0, 24])
+def test_general_attention_of_few_rows_has_the_bits_of_many(dtype, window):
+    """Heads of 64: few rows ask for a chunk of more than 16 keys as a whole, shorter ones and many rows for 16 at a time. The same bits, and
+    64 bits' results, with contexts at the edges of both and anything behind a request's last key."""
+    contexts, H, G, D = [1, 2, 15, 16, 17, 18, 31, 32, 33, 64, 65, 79, 80, 81, 129, 300], 16, 8, 64
+    d = Decoding(contexts, H, G, D, D)
+    q, k, v = d.q.to(dtype), d.k.to(dtype), d.v.to(dtype)
+    times = 5                                     # 80 rows of 16 heads are more than what counts as few
+
+    def run(n):
+        # (all of them named: an address keeps no tensor alive)
+        out, rows, slots, positions = torch.empty(n * d.n, H * D, dtype=dtype, device=DEV), q.repeat(n, 1), d.slots.repeat(n), d.positions.repeat(n)
+        check(native.lib().celeg_paged_attention(
+            ptr(rows), H * D, ptr(k), ptr(v), 0 if dtype == torch.float32 else 1, ptr(d.table), d.per, ptr(slots), ptr(positions), ptr(out),
+            H * D, n * d.n, H, G, D, PAGE, d.layers, d.layer, ctypes.c_float(0.125), window, None))
+        torch.cuda.synchronize()
+        return out
+
+    few = run(1)
+    assert torch.equal(run(times), few.repeat(times, 1))
+    for i, c in enumerate(contexts):
+        keys, values = (t[-window:].cpu().repeat_interleave(H // G, 1) for t in d.keys_and_values(i))
+        w = torch.softmax((d.q[i].double().cpu().view(H, D) * keys).sum(-1).T * 0.125, -1)
+        want = (w.T[..., None] * values).sum(0).reshape(-1)
+        # 32-bit scores, weights and sums of up to 300 keys, each step within 2^-24 of the magnitudes; a bfloat16 result is rounded
+        bound = 2.0 ** -24 * 400 * float(values.abs().max()) + (0.0 if dtype == torch.float32 else 2.0 ** -8) * want.abs()
+        assert bool(((few[i].double().cpu() - want).abs() <= bound).all()), c
