@@ -374,7 +374,7 @@ extern "C" int celeg_qk_norm_rope_store(
 #define ATT_MAX_WAVES 4
 // rows x heads up to which keys and values of a chunk come whole: 2 requests at 350 tokens 8.8 us against 9.3, 8 requests 16.8
 // against 19.0, one at 8,000 110 against 134; 424 rows of prompts 47.5 against 44.0, 1,024 rows 365 against 361
-#define WHOLE_MOST 1024
+#define FEW_MOST 1024
 
 template <typename T> struct Wide;      // 16 bytes as 32-bit numbers
 template <> struct Wide<float> {
@@ -392,14 +392,20 @@ template <> struct Wide<bf16> {
     }
 };
 
-// DC: head_dim in pieces of 64, rounded up; POW2: page_tokens is a power of two; WHOLE: head_dim is 64
-template <typename T, int DC, int WAVES, bool VEC, bool POW2, bool WHOLE>
+// DC: head_dim in pieces of 64, rounded up; POW2: page_tokens is a power of two; FEW: few rows, where they have a form of their own
+// (and head_dim is 64 if DC is 1)
+template <typename T, int DC, int WAVES> constexpr bool att_few() { return DC == 1 || (sizeof(T) == 2 && DC == ATT_MAX_DIM_CHUNKS && WAVES == 2); }
+template <typename T, int DC, int WAVES, bool VEC, bool POW2, bool FEW>
 __global__ __launch_bounds__(WAVES * CELEG_WAVE) void paged_attention_kernel(
     const T* __restrict__ q, int ldq, const T* __restrict__ k_pool, const T* __restrict__ v_pool,
     const int* __restrict__ table, int table_stride, const int* __restrict__ token_slot,
     const int* __restrict__ positions, T* __restrict__ out, int ldo, int q_heads, int kv_heads,
     int head_dim, int page_tokens, int n_layers, int layer, float scale, int window) {
     constexpr int W = Wide<T>::N;
+    constexpr bool WHOLE = FEW && DC == 1;
+    // (of two wavefronts a row, bfloat16 heads beyond 128 take five registers too many without the condition for a fifth wavefront a
+    // SIMD: 400 rows of heads of 256, a window of 96, 345 us with it and 372 without; 4 single tokens 38.6 and 34.8)
+    constexpr bool CONDITION = att_few<T, DC, WAVES>() && DC > 1 && !FEW;
     constexpr int AHEAD = 16 / W;                   // loads of values in flight: 16 keys
     __shared__ float qs[DC * CELEG_WAVE];
     __shared__ float ps_all[WAVES][CELEG_WAVE];
@@ -516,6 +522,7 @@ __global__ __launch_bounds__(WAVES * CELEG_WAVE) void paged_attention_kernel(
 #pragma unroll
                     for (int i = 0; i < W; ++i) {
                         const int k2 = kk + a * W + i;
+                        if (CONDITION && k2 >= n_keys) continue;
                         const float pk = ps[k2];            // (0 behind the row's own key, where memory may hold anything)
 #pragma unroll
                         for (int j = 0; j < DC; ++j) acc[j] = fmaf(pk, k2 < n_keys ? v[a][j][i] : 0.f, acc[j]);
@@ -584,14 +591,19 @@ static int launch_paged_attention(const void* q, int ldq, const void* k_pool, co
                            head_dim, page_tokens, n_layers, layer, scale, window);
     };
     const bool pow2 = (page_tokens & (page_tokens - 1)) == 0;
-    if constexpr (DC == 1) {
-        if (vec && pow2 && head_dim == CELEG_WAVE && static_cast<long long>(n_tokens) * q_heads <= WHOLE_MOST) {
+    if constexpr (att_few<T, DC, WAVES>()) {
+        if (vec && pow2 && (DC > 1 || head_dim == CELEG_WAVE) && static_cast<long long>(n_tokens) * q_heads <= FEW_MOST) {
             launch(paged_attention_kernel<T, DC, WAVES, true, true, true>);
             return CELEG_LAUNCH_RESULT();
         }
     }
-    if (vec && pow2) launch(paged_attention_kernel<T, DC, WAVES, true, true, false>);
-    else if (vec) launch(paged_attention_kernel<T, DC, WAVES, true, false, false>);
+    if constexpr (!att_few<T, DC, WAVES>() || DC == 1) {        // (the others' many rows keep the divisions too: 96 registers, with shifts 147)
+        if (vec && pow2) {
+            launch(paged_attention_kernel<T, DC, WAVES, true, true, false>);
+            return CELEG_LAUNCH_RESULT();
+        }
+    }
+    if (vec) launch(paged_attention_kernel<T, DC, WAVES, true, false, false>);
     else launch(paged_attention_kernel<T, DC, WAVES, false, false, false>);
     return CELEG_LAUNCH_RESULT();
 }

@@ -169,11 +169,12 @@ def test_sigmoid_attention_of_single_tokens_is_no_further_from_the_exact_result(
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, BF])
-@pytest.mark.parametrize("window", [0, 24])
-def test_general_attention_of_few_rows_has_the_bits_of_many(dtype, window):
-    """Heads of 64: few rows ask for a chunk of more than 16 keys as a whole, shorter ones and many rows for 16 at a time. The same bits, and
-    64 bits' results, with contexts at the edges of both and anything behind a request's last key."""
-    contexts, H, G, D = [1, 2, 15, 16, 17, 18, 31, 32, 33, 64, 65, 79, 80, 81, 129, 300], 16, 8, 64
+@pytest.mark.parametrize("D,window", [(64, 0), (64, 24), (160, 96), (256, 65), (256, 128)])
+def test_general_attention_of_few_rows_has_the_bits_of_many(dtype, D, window):
+    """Heads of 64: few rows ask for a chunk of more than 16 keys as a whole, shorter ones and many rows for 16 at a time; heads beyond 128
+    with windows of 65 to 128 keys: few rows have no condition round a key's product. The same bits, and 64 bits' results, with contexts
+    at the edges and anything behind a request's last key."""
+    contexts, H, G = [1, 2, 15, 16, 17, 18, 31, 32, 33, 64, 65, 79, 80, 81, 129, 300], 16, 8
     d = Decoding(contexts, H, G, D, D)
     q, k, v = d.q.to(dtype), d.k.to(dtype), d.v.to(dtype)
     times = 5                                     # 80 rows of 16 heads are more than what counts as few
