@@ -26,8 +26,9 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 // GROUP: pieces of 16 values of k that are asked for together.  VEC: rows of X and W lie on 16 bytes
 // and K is a multiple of 4; the same sums in the same order without it.
-template <int RT, int CT, int GROUP, int MAX_THREADS, bool VEC>
-__global__ __launch_bounds__(MAX_THREADS, 2) void gemm_f32_kernel(
+// WAVES: wavefronts that a SIMD is to hold.
+template <int RT, int CT, int GROUP, int MAX_THREADS, bool VEC, int WAVES>
+__global__ __launch_bounds__(MAX_THREADS, WAVES) void gemm_f32_kernel(
     const float* __restrict__ X, int ldx, const float* __restrict__ W, int ldw,
     const float* __restrict__ bias, float* __restrict__ Y, int ldy, int M, int N, int K, int wide_store) {
     constexpr int TILES = RT * CT;
@@ -90,15 +91,16 @@ __global__ __launch_bounds__(MAX_THREADS, 2) void gemm_f32_kernel(
         f32x4_t w1[CT][GROUP], x1[RT][GROUP];
 #pragma unroll
         for (int g = 0; g < F32_PIECES / GROUP; g += 2) {
-            // (the order pinned: left alone the compiler asks for a group right ahead of the products that use it)
+            // (the order pinned: left alone the compiler asks for a group right ahead of the products that use it.  A value at a
+            // time that is the better order: 424 x 1,024, K = 1,023 19.0 us, pinned 20.6; 200 x 3,072 34.7, 38.7)
             load(k0 + (g + 1) * 16 * GROUP, whole, w1, x1);
-            if (CT > 1) __builtin_amdgcn_sched_barrier(0);
+            if (VEC && CT > 1) __builtin_amdgcn_sched_barrier(0);
             multiply(w0, x0);
-            if (CT > 1) __builtin_amdgcn_sched_barrier(0);
+            if (VEC && CT > 1) __builtin_amdgcn_sched_barrier(0);
             if (g + 2 < F32_PIECES / GROUP) load(k0 + (g + 2) * 16 * GROUP, whole, w0, x0);
-            if (CT > 1) __builtin_amdgcn_sched_barrier(0);
+            if (VEC && CT > 1) __builtin_amdgcn_sched_barrier(0);
             multiply(w1, x1);
-            if (CT > 1) __builtin_amdgcn_sched_barrier(0);
+            if (VEC && CT > 1) __builtin_amdgcn_sched_barrier(0);
         }
     };
 
@@ -391,7 +393,7 @@ static int launch_f32_slices(const float* X, int ldx, const float* W, int ldw, c
     return CELEG_LAUNCH_RESULT();
 }
 
-template <int RT, int CT, int GROUP, int MAX_THREADS>
+template <int RT, int CT, int GROUP, int MAX_THREADS, int WAVES = 2>
 static int launch_f32(const float* X, int ldx, const float* W, int ldw, const float* bias, float* Y, int ldy,
                       int M, int N, int K, hipStream_t stream) {
     const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
@@ -406,11 +408,11 @@ static int launch_f32(const float* X, int ldx, const float* W, int ldw, const fl
     // (64 x 64 tiles are for rows that cannot be read 16 bytes at a time)
     if constexpr (RT * CT <= 8) {
         if (vec) {
-            hipLaunchKernelGGL((gemm_f32_kernel<RT, CT, GROUP, MAX_THREADS, true>), grid, block, lds, stream, X, ldx, W, ldw, bias, Y, ldy, M, N, K, wide_store);
+            hipLaunchKernelGGL((gemm_f32_kernel<RT, CT, GROUP, MAX_THREADS, true, WAVES>), grid, block, lds, stream, X, ldx, W, ldw, bias, Y, ldy, M, N, K, wide_store);
             return CELEG_LAUNCH_RESULT();
         }
     }
-    hipLaunchKernelGGL((gemm_f32_kernel<RT, CT, GROUP, MAX_THREADS, false>), grid, block, lds, stream, X, ldx, W, ldw, bias, Y, ldy, M, N, K, wide_store);
+    hipLaunchKernelGGL((gemm_f32_kernel<RT, CT, GROUP, MAX_THREADS, false, WAVES>), grid, block, lds, stream, X, ldx, W, ldw, bias, Y, ldy, M, N, K, wide_store);
     return CELEG_LAUNCH_RESULT();
 }
 
@@ -712,7 +714,12 @@ extern "C" int celeg_gemm_f32(const float* X, int ldx, const float* W, int ldw, 
         const long long tiles = static_cast<long long>((M + 63) / 64) * ((N + 63) / 64);
         if (M <= 32 * 65535 && (K <= F32_SEGMENT || (K <= F32_SEGMENT + 16 && tiles >= 256)))
             return launch_f32_short<2, 2>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
-        if (tiles >= 256) return launch_f32<4, 4, 2, 256>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
+        // Of these a CU holds two in 256 registers each, or one in what the compiler likes: the two take 1.5 to 1.9 times as
+        // long (K = 1,023, 64 x 64 tiles in a round: 512 54 us, 256 30; K = 255 25 and 16), so it goes by the rounds: 600 x 4,096 90 us by
+        // ones, 108 by twos, 2,048 x 3,072, K = 1,025 227 and 180.
+        if (tiles >= 256)
+            return 7 * ((tiles + 511) / 512) <= 4 * ((tiles + 255) / 256) ? launch_f32<4, 4, 2, 256, 2>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream)
+                                                                         : launch_f32<4, 4, 2, 256, 1>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
     }
     return launch_f32<2, 4, 2, 512>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
 }
