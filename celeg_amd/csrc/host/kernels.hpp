@@ -52,7 +52,7 @@ int celeg_latent_attention(const void* q, int ldq, const void* pool, int dtype, 
                            int n_tokens, int heads, int rank, int rot, int page_tokens, int n_layers, int layer,
                            float scale, int window, hipStream_t stream);
 // latent_fast.hip
-int celeg_latent_attention_fast_ok(int rank, int rot);
+int celeg_latent_attention_fast_ok(int rank, int rot, int n_layers, int page_tokens);
 int celeg_latent_attention_tile_rows(int rank, int rot);
 int celeg_latent_attention_fast(int form, const void* q, int ldq, const void* pool, const int* table, int table_stride,
                                 const int* cu_seqlens, const int* seq_slot, const int* seq_start, int n_seqs, int max_tiles,

@@ -288,7 +288,7 @@ void Ops::latent_attention(const Tensor& q_lat, const Tensor& out, const LatentS
     latent_cache_fits(s, kv, q_lat.dtype, "latent_attention");
     took(Path::AttentionLatent);
     if (q_lat.dtype == DType::BF16 && use_latent_mfma && !attention_general && scale > 0.f && out.contiguous() &&
-        celeg_latent_attention_fast_ok(s.rank, s.rot) && (kv.page_tokens & (kv.page_tokens - 1)) == 0) {
+        celeg_latent_attention_fast_ok(s.rank, s.rot, kv.n_layers, kv.page_tokens)) {
         const int T = batch.n_tokens, n_single = std::min(batch.single_rows, T);
         const float* sink_p = sink ? sink->as<float>() : nullptr;
         if (n_single > 0) {

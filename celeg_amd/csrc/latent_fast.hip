@@ -126,7 +126,8 @@ __global__ __launch_bounds__(256, (KS <= 9 ? 2 : 1)) void latent_attention_mfma_
         wave_computes = true;
     }
     const int* pages = table + static_cast<size_t>(slot) * table_stride;
-    const unsigned page_stride = static_cast<unsigned>(n_layers) * page_tokens * D;
+    // (in pieces of 8 values, so that 32 bits hold pages of up to 64 GiB; the host has checked that they do)
+    const unsigned row_pieces = static_cast<unsigned>(D) / 8, page_stride = static_cast<unsigned>(n_layers) * page_tokens * row_pieces;
     const __bf16* layer_base = pool + static_cast<size_t>(layer) * page_tokens * D;
     const int page_shift = 31 - __clz(page_tokens);     // page_tokens is a power of two
 
@@ -149,9 +150,9 @@ __global__ __launch_bounds__(256, (KS <= 9 ? 2 : 1)) void latent_attention_mfma_
             const int i = tid + 256 * j, key = i / CHUNKS, ch = i - key * CHUNKS;
             there |= (page[j] >= 0 && ch * 8 < D ? 1u : 0u) << j;
             // (no branch round a load: a piece that is not there asks for one of page 0 or for its row's last)
-            const unsigned in_page = static_cast<unsigned>(((blk * LATF_KEYS + key) & (page_tokens - 1)) * D + min(ch * 8, D - 8));
-            staged[j] = *reinterpret_cast<const lat_u32x4*>(
-                layer_base + (static_cast<unsigned long long>(static_cast<unsigned>(max(page[j], 0))) * page_stride + in_page));
+            const unsigned in_page = static_cast<unsigned>((blk * LATF_KEYS + key) & (page_tokens - 1)) * row_pieces + min(static_cast<unsigned>(ch), row_pieces - 1);
+            staged[j] = reinterpret_cast<const lat_u32x4*>(
+                layer_base)[static_cast<unsigned long long>(static_cast<unsigned>(max(page[j], 0))) * page_stride + in_page];
         }
     };
     // key 32 h + 8 a + 4 b + r of a block lies at row 32 h + 16 b + 4 a + r: the 16 keys of a tile of scores in 16 rows
@@ -416,8 +417,10 @@ extern "C" int celeg_latent_attention_tile_rows(int rank, int rot) {
     return 64;        // one tile of 16 columns a wavefront (two were measured slower: half the workgroups, and no more overlap)
 }
 
-extern "C" int celeg_latent_attention_fast_ok(int rank, int rot) {
-    return rank > 0 && rank % 16 == 0 && rank <= 512 && rot >= 0 && (rank + rot) % 8 == 0 && rank + rot <= 576;
+extern "C" int celeg_latent_attention_fast_ok(int rank, int rot, int n_layers, int page_tokens) {
+    return rank > 0 && rank % 16 == 0 && rank <= 512 && rot >= 0 && (rank + rot) % 8 == 0 && rank + rot <= 576 && n_layers > 0 &&
+           page_tokens > 0 && (page_tokens & (page_tokens - 1)) == 0 &&
+           static_cast<unsigned long long>(n_layers) * page_tokens * ((rank + rot) / 8) < (1ull << 32);
 }
 
 // form 0: rows of the sequences of more than one token (max_tiles: a bound on their tiles of 64 rows);
@@ -430,8 +433,7 @@ extern "C" int celeg_latent_attention_fast(int form, const void* q, int ldq, con
                                            float* ws_o, float* ws_ml, int n_splits, int blocks_per_split, int heads,
                                            int rank, int rot, int page_tokens, int n_layers, int layer, float scale,
                                            int window, int exact, hipStream_t stream) {
-    if (!celeg_latent_attention_fast_ok(rank, rot) || (form == 1 && n_splits > LATF_MAX_SPLITS) || page_tokens <= 0 ||
-        (page_tokens & (page_tokens - 1)))
+    if (!celeg_latent_attention_fast_ok(rank, rot, n_layers, page_tokens) || (form == 1 && n_splits > LATF_MAX_SPLITS))
         return static_cast<int>(hipErrorInvalidValue);
     const int D = rank + rot, KS = (D + 31) / 32, DT = rank / 16;
     const float scale_log2e = scale * LOG2E;

@@ -65,3 +65,45 @@ def test_rows_and_single_tokens_against_64_bits(rank, rot, window, exact):
         error = (got[cu[i]:cu[i + 1]] - want).abs()
         assert (error <= 1.05 * bound).all(), (i, (error / bound).max())
 
+
+
+@pytest.mark.parametrize("single", [True, False])
+def test_pages_of_more_values_than_32_bits_count(single):
+    """A page of 4,096 tokens and 1,822 layers of 576 values is 4.3 G values (8.6 GB): the rows of the last of three pages and the
+    last layer are read where they lie.  The same bits as from a pool of small pages."""
+    rank, rot, H, page, layers = 512, 64, 3, 4096, 1822
+    D = rank + rot
+    if torch.cuda.mem_get_info()[0] < (40 << 30):
+        pytest.skip("no room for three pages of 8.6 GB")
+    context, rows_new = page + 64, 1 if single else 70
+    big = torch.empty(3 * layers * page * D, dtype=BF, device=DEV)
+    gen = torch.Generator().manual_seed(5)
+    rows = torch.randn(context, D, generator=gen).to(BF).to(DEV)
+    table_big = ints([2, 1])
+    for i, p in enumerate((2, 1)):
+        part = rows[i * page:(i + 1) * page]
+        start = (p * layers + layers - 1) * page * D
+        big[start:start + part.numel()] = part.reshape(-1)
+    small_page = 16
+    per = (context + small_page - 1) // small_page
+    small = torch.zeros(per, small_page, D, dtype=BF, device=DEV)
+    small.view(-1, D)[:context] = rows
+    table_small = ints(list(range(per)))
+    q = torch.randn(rows_new, H * D, generator=gen).to(BF).to(DEV)
+    cu, slot, start, token_slot = ints([0, rows_new]), ints([0]), ints([context - rows_new]), ints([0] * rows_new)
+    positions = ints(list(range(context - rows_new, context)))
+    splits, per_split, scale = 4, 17, 1.5 / math.sqrt(D)
+    parts_o, parts_ml = torch.empty(H * splits * rank, device=DEV), torch.empty(H * splits * 2, device=DEV)
+
+    def run(pool, table, table_stride, page_tokens, n_layers):
+        out = torch.full((rows_new, H * rank), 7.0, dtype=BF, device=DEV)
+        check(native.lib().celeg_latent_attention_fast(
+            1 if single else 0, ptr(q), H * D, ptr(pool), ptr(table), table_stride, ptr(cu), ptr(slot), ptr(start), 1, 0 if single else 2,
+            ptr(token_slot), ptr(positions), 1 if single else 0, None, ptr(out), H * rank, ptr(parts_o), ptr(parts_ml), splits, per_split, H,
+            rank, rot, page_tokens, n_layers, n_layers - 1, ctypes.c_float(scale), 0, 1, None))
+        torch.cuda.synchronize()
+        return out
+
+    assert torch.equal(run(big, table_big, 2, page, layers), run(small, table_small, per, small_page, 1))
+    assert native.lib().celeg_latent_attention_fast_ok(rank, rot, layers, page) == 1
+    assert native.lib().celeg_latent_attention_fast_ok(rank, rot, layers * 8, page) == 0        # what the kernel's 32 bits do not hold
