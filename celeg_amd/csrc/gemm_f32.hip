@@ -678,6 +678,22 @@ static int launch_f32_tile(const float* X, int ldx, const float* W, int ldw, con
     return CELEG_LAUNCH_RESULT();
 }
 
+// The staged tile of a product whose rows lie on 16 bytes: 1 32 x 64, 2 64 x 64, 3 64 x 128, 0 none of them.
+// Staged tiles once the smallest of them give every CU more than one, and below that where k is too short to be cut
+// over eight wavefronts (200 rows, K = 1,024: N = 1,024 16.1 us against 15.9 cut, N = 3,072 24.4 against 30.3; N = 1,024,
+// K = 4,608 89 against 64; K = 384, N = 2,048 7.9 against 8.5; 40 rows, K = 256 5.7 against 5.8, K = 384 7.6 against 6.8).
+// The tile by what a round of them over 256 CUs takes (in 0.1 us at K = 1,024, all in proportion to K: 64 x 128 tiles
+// go two at a time through a CU): 424 rows, N = 9,216 75 us with 64 x 128, 78 with 64 x 64, 84 with 32 x 64;
+// 424 rows, N = 3,072 42, 40 and 34; 1,024 rows, N = 9,216 179, 166 and 183.  (A grid has 65,535 rows of tiles.)
+extern "C" int celeg_gemm_f32_staged_tile(int M, int N, int K) {
+    const long long small = static_cast<long long>((M + 31) / 32) * ((N + 63) / 64);
+    if (M <= 16 || !(small > 256 || (M > 32 && K <= 2 * F32_SEGMENT) || (M > 64 && K < 8 * F32_SEGMENT))) return 0;
+    const auto rounds = [](long long m, long long n) { return (m * n + 255) / 256; };
+    const long long c32 = 20 + 101 * rounds((M + 31) / 32, (N + 63) / 64), c64 = 40 + 185 * rounds((M + 63) / 64, (N + 63) / 64),
+                    c128 = 70 + 350 * rounds((M + 63) / 64, (N + 127) / 128);
+    return c128 < c64 && c128 < c32 ? 3 : c64 < c32 || M > 32 * 65535 ? 2 : 1;
+}
+
 extern "C" int celeg_gemm_f32(const float* X, int ldx, const float* W, int ldw, const float* bias,
                               float* Y, int ldy, int M, int N, int K, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
@@ -688,21 +704,10 @@ extern "C" int celeg_gemm_f32(const float* X, int ldx, const float* W, int ldw, 
     }
     const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     const bool vec = K % 4 == 0 && ldx % 4 == 0 && ldw % 4 == 0 && aligned(X) && aligned(W);
-    // Staged tiles once the smallest of them give every CU more than one, and below that where k is too short to be cut
-    // over eight wavefronts (200 rows, K = 1,024: N = 1,024 16.1 us against 15.9 cut, N = 3,072 24.4 against 30.3; N = 1,024,
-    // K = 4,608 89 against 64; K = 384, N = 2,048 7.9 against 8.5; 40 rows, K = 256 5.7 against 5.8, K = 384 7.6 against 6.8).
-    // (A grid has 65,535 rows of tiles.)
-    const long long small = static_cast<long long>((M + 31) / 32) * ((N + 63) / 64);
-    if (vec && (small > 256 || (M > 32 && K <= 2 * F32_SEGMENT) || (M > 64 && K < 8 * F32_SEGMENT))) {
-        // The tile by what a round of them over 256 CUs takes (in 0.1 us at K = 1,024, all in proportion to K: 64 x 128 tiles
-        // go two at a time through a CU): 424 rows, N = 9,216 75 us with 64 x 128, 78 with 64 x 64, 84 with 32 x 64;
-        // 424 rows, N = 3,072 42, 40 and 34; 1,024 rows, N = 9,216 179, 166 and 183.
-        const auto rounds = [](long long m, long long n) { return (m * n + 255) / 256; };
-        const long long c32 = 20 + 101 * rounds((M + 31) / 32, (N + 63) / 64), c64 = 40 + 185 * rounds((M + 63) / 64, (N + 63) / 64),
-                        c128 = 70 + 350 * rounds((M + 63) / 64, (N + 127) / 128);
-        if (c128 < c64 && c128 < c32) return launch_f32_tile<64, 128>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
-        if (c64 < c32 || M > 32 * 65535) return launch_f32_tile<64, 64>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
-        return launch_f32_tile<32, 64>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
+    switch (vec ? celeg_gemm_f32_staged_tile(M, N, K) : 0) {
+        case 1: return launch_f32_tile<32, 64>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
+        case 2: return launch_f32_tile<64, 64>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
+        case 3: return launch_f32_tile<64, 128>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
     }
     if (M <= 32) return launch_f32<2, 1, 8, 512>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
     if (M <= 64) return launch_f32<4, 1, 4, 512>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);

@@ -279,7 +279,7 @@ def test_gemm_f32_many_rows(ops, M, N, K):
 @pytest.mark.parametrize("M,N,K", [(33, 65, 36), (65, 129, 32), (63, 8257, 100), (130, 8257, 132), (257, 4161, 68), (1057, 1100, 260),
                                    (513, 6465, 4), (2049, 2049, 96), (31, 16449, 160)])
 def test_gemm_f32_staged_tiles(ops, M, N, K):
-    """Each size of the staged tiles with rows, columns and a step of 32 that do not fill it, one step and many: the bits of rows that
+    """The smallest of the staged tiles with rows, columns and a step of 32 that do not fill it, one step and many: the bits of rows that
     cannot be read 16 bytes at a time (another kernel, the same order of sums) and the bound of such sums."""
     wide, out, same = randn(M, K + 3, seed=27), torch.zeros(M + 1, N, device=DEV), torch.empty(M, N + 3, device=DEV)
     w, b = randn(N, K, seed=28), randn(N, seed=29)
@@ -290,6 +290,15 @@ def test_gemm_f32_staged_tiles(ops, M, N, K):
     # a chain of at most 128 products, the segments' sums, the bias: each within 2^-24 of the magnitudes summed
     bound = (min(K, 128) + K // 128 + 3) * 2.0 ** -24 * (x.abs() @ w.double().abs().T + b.double().abs())
     assert bool(((out[:M].double() - x @ w.double().T - b.double()).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("tile,M,N", [(1, 63, 8257), (1, 2049, 2049), (2, 1023, 2045), (2, 1001, 2001), (3, 2047, 2045), (3, 425, 9201)])
+@pytest.mark.parametrize("K", [4, 36, 132, 260, 416])
+def test_gemm_f32_every_staged_tile(ops, tile, M, N, K):
+    """Each of the three staged tiles, chosen as the dispatch chooses it, with rows and columns that do not fill it and K below a step of
+    32, a step that is not whole, several segments: the bits of rows that cannot be read 16 bytes at a time, and 64 bits' sums."""
+    assert ops._lib("gemm_f32").celeg_gemm_f32_staged_tile(M, N, K) == tile
+    test_gemm_f32_staged_tiles(ops, M, N, K)
 
 
 def test_linear_bf16_and_stored_f32_matrix(ops):
