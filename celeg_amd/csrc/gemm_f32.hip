@@ -720,12 +720,16 @@ extern "C" int celeg_gemm_f32(const float* X, int ldx, const float* W, int ldw, 
         const long long tiles = static_cast<long long>((M + 63) / 64) * ((N + 63) / 64);
         if (M <= 32 * 65535 && (K <= F32_SEGMENT || (K <= F32_SEGMENT + 16 && tiles >= 256)))
             return launch_f32_short<2, 2>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
-        // Of these a CU holds two in 256 registers each, or one in what the compiler likes: the two take 1.5 to 1.9 times as
-        // long (K = 1,023, 64 x 64 tiles in a round: 512 54 us, 256 30; K = 255 25 and 16), so it goes by the rounds: 600 x 4,096 90 us by
-        // ones, 108 by twos, 2,048 x 3,072, K = 1,025 227 and 180.
-        if (tiles >= 256)
-            return 7 * ((tiles + 511) / 512) <= 4 * ((tiles + 255) / 256) ? launch_f32<4, 4, 2, 256, 2>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream)
-                                                                         : launch_f32<4, 4, 2, 256, 1>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
+        // Of these a CU holds two in 256 registers each, or one in what the compiler likes.  Two take 1.75 times as long as one, and a
+        // rest of few tiles as long as one if K is long: by the rounds, then (600 x 4,096, K = 1,023 93 us by ones, 109 by twos; K = 4,095 321
+        // and 297; 768 x 4,096, K = 2,047 175 and 198; 2,048 x 3,072, K = 1,025 227 and 180), and two up to 256 values of k, where
+        // half of a tile's wavefronts wait (600 x 4,096, K = 255 51 and 39).
+        if (tiles >= 256) {
+            const long long rest = tiles % 512, ones = 100 * ((tiles + 255) / 256),
+                            twos = 175 * (tiles / 512) + (rest == 0 ? 0 : rest <= 192 && K > 8 * F32_SEGMENT ? 100 : 175);
+            return K <= 2 * F32_SEGMENT || twos <= ones ? launch_f32<4, 4, 2, 256, 2>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream)
+                                                        : launch_f32<4, 4, 2, 256, 1>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
+        }
     }
     return launch_f32<2, 4, 2, 512>(X, ldx, W, ldw, bias, Y, ldy, M, N, K, stream);
 }
