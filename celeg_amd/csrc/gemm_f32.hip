@@ -681,13 +681,20 @@ static int launch_f32_tile(const float* X, int ldx, const float* W, int ldw, con
 // The staged tile of a product whose rows lie on 16 bytes: 1 32 x 64, 2 64 x 64, 3 64 x 128, 0 none of them.
 // Staged tiles once the smallest of them give every CU more than one, and below that where k is too short to be cut
 // over eight wavefronts (200 rows, K = 1,024: N = 1,024 16.1 us against 15.9 cut, N = 3,072 24.4 against 30.3; N = 1,024,
-// K = 4,608 89 against 64; K = 384, N = 2,048 7.9 against 8.5; 40 rows, K = 256 5.7 against 5.8, K = 384 7.6 against 6.8).
+// K = 4,608 89 against 64; K = 384, N = 2,048 7.9 against 8.5; 40 rows, K = 256 5.7 against 5.8, K = 384 7.6 against 6.8).  Cut
+// products gain where rows are not whole lines apart (K % 32: other channels), staged ones pay a step for what is left of k, and
+// columns that are stored one at a time: 33 to 64 rows, K = 160 4.1 against 4.9, K = 188 4.6 against 4.8, K = 196 5.0 against 4.75, K = 224
+// 4.9 against 5.2, K = 252 5.4 against 4.8, N = 1,091, K = 160 5.1 against 5.5, K = 188 5.55 against 5.3, K = 256 6.35 against 5.85; 65 rows and more,
+// K = 480 8.7 against 9.8, K = 496 9.2 against 8.3, K = 512 9.2 against 9.6.
 // The tile by what a round of them over 256 CUs takes (in 0.1 us at K = 1,024, all in proportion to K: 64 x 128 tiles
 // go two at a time through a CU): 424 rows, N = 9,216 75 us with 64 x 128, 78 with 64 x 64, 84 with 32 x 64;
 // 424 rows, N = 3,072 42, 40 and 34; 1,024 rows, N = 9,216 179, 166 and 183.  (A grid has 65,535 rows of tiles.)
 extern "C" int celeg_gemm_f32_staged_tile(int M, int N, int K) {
     const long long small = static_cast<long long>((M + 31) / 32) * ((N + 63) / 64);
-    if (M <= 16 || !(small > 256 || (M > 32 && K <= 2 * F32_SEGMENT) || (M > 64 && K < 8 * F32_SEGMENT))) return 0;
+    const bool lines = K % F32_STEP == 0, wide = N % 4 == 0;
+    const bool few = M > 32 && (K <= 160 || (wide && (K <= 192 || (lines && K <= 2 * F32_SEGMENT))));
+    const bool more = M > 64 && K < 8 * F32_SEGMENT && !(!lines && K > 15 * F32_STEP && K < 16 * F32_STEP);
+    if (M <= 16 || !(small > 256 || few || more)) return 0;
     const auto rounds = [](long long m, long long n) { return (m * n + 255) / 256; };
     const long long c32 = 20 + 101 * rounds((M + 31) / 32, (N + 63) / 64), c64 = 40 + 185 * rounds((M + 63) / 64, (N + 63) / 64),
                     c128 = 70 + 350 * rounds((M + 63) / 64, (N + 127) / 128);
