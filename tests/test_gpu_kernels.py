@@ -301,6 +301,14 @@ def test_gemm_f32_every_staged_tile(ops, tile, M, N, K):
     test_gemm_f32_staged_tiles(ops, M, N, K)
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (33, 100, 160), (33, 100, 164), (64, 99, 160), (64, 99, 164), (40, 260, 192), (40, 260, 196), (63, 260, 224), (63, 260, 256), (63, 261, 256),
+    (65, 100, 480), (65, 100, 484), (65, 100, 508), (65, 100, 512), (70, 130, 1020), (70, 130, 1024),      # cut along k or staged
+    (1025, 1025, 260), (1025, 1090, 1028), (700, 3000, 516), (700, 3000, 1028)])                           # 64 x 64 tiles by ones or twos
+def test_gemm_f32_where_the_choice_changes(ops, M, N, K):
+    test_gemm_f32_staged_tiles(ops, M, N, K)
+
+
 def test_linear_bf16_and_stored_f32_matrix(ops):
     M, N, K = 9, 200, 96
     x = randn(M, K, seed=10, dtype=torch.bfloat16)
