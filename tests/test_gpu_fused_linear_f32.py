@@ -7,7 +7,7 @@ import torch
 
 import plain_lfm2 as plain
 from celeg_amd import native
-from helpers import WEIGHT_STD, random_tokens
+from helpers import random_tokens
 from test_gpu_single_tokens import check, ptr
 
 pytestmark = pytest.mark.gpu
@@ -114,14 +114,25 @@ def test_the_norm_has_the_bits_of_its_own_kernel(M, K):
     assert torch.equal(one[0], out[M - 1])
 
 
-@pytest.mark.parametrize("name", ["B", "D"])
-def test_logits_with_and_without(model_folders, name):
+def one_layer_of_each(folder, width, bias=False):
+    """A model of a short convolution's and an attention's layer, float32."""
+    from celeg_amd.weights import write_random_model
+    config = {"architectures": ["Lfm2ForCausalLM"], "vocab_size": 256, "hidden_size": width, "num_hidden_layers": 2,
+              "layer_types": ["conv", "full_attention"], "num_attention_heads": width // 32, "num_key_value_heads": width // 64,
+              "head_dim": 32, "intermediate_size": 320, "block_auto_adjust_ff_dim": False, "rope_theta": 10000.0, "conv_L_cache": 3,
+              "conv_bias": bias, "tie_word_embeddings": True, "norm_eps": 1e-5, "max_position_embeddings": 128, "eos_token_id": 7}
+    return write_random_model(config, str(folder), seed=width, dtype=torch.float32, std=0.03)
+
+
+@pytest.mark.parametrize("width,bias", [(256, True), (640, False), (1024, True)])
+def test_logits_with_and_without(tmp_path, width, bias):
+    """Steps of 7, 16, 9 and 1 rows with the folded products (their path counts them) and without (it does not): the same bits, near 64 bits."""
     from celeg_amd.engine import StepEntry, load_model
-    folder = model_folders(name, torch.float32, WEIGHT_STD)
+    folder = one_layer_of_each(tmp_path, width, bias)
     cfg, W = plain.load_model_folder(folder)
     tokens = random_tokens(cfg["vocab_size"], 40, seed=3)
     ref = plain.model_logits(cfg, W, tokens).double()
-    errors = {}
+    got = {}
     for fused in (1, 0):
         lm = load_model(folder, dtype="float32", page_tokens=16, n_pages=16, max_requests=2, max_batched_tokens=64)
         lm.set_knob("use_fused", fused)
@@ -129,20 +140,11 @@ def test_logits_with_and_without(model_folders, name):
         for first, n in [(0, 7), (7, 16), (23, 9)] + [(i, 1) for i in range(32, 40)]:
             assert lm.cache.prepare(slot, first, n)
             rows.append(lm.runner.step([StepEntry(slot, first, tokens[first:first + n], [n - 1])])[0].double())
-        got, want = torch.stack(rows), ref[[6, 22] + list(range(31, 40))]
-        errors[fused] = float((got - want).norm() / want.norm())
+        assert (lm.paths()["linear_f32_fused"] > 0) == bool(fused)
+        got[fused], want = torch.stack(rows), ref[[6, 22] + list(range(31, 40))]
+        assert float((got[fused] - want).norm() / want.norm()) <= 2e-6
         lm.close()
-    assert errors[1] <= 2e-6 and errors[0] <= 2e-6, errors
-
-
-def one_layer_of_each(folder, width):
-    """A model of a short convolution's and an attention's layer, float32."""
-    from celeg_amd.weights import write_random_model
-    config = {"architectures": ["Lfm2ForCausalLM"], "vocab_size": 256, "hidden_size": width, "num_hidden_layers": 2,
-              "layer_types": ["conv", "full_attention"], "num_attention_heads": width // 32, "num_key_value_heads": width // 64,
-              "head_dim": 32, "intermediate_size": 320, "block_auto_adjust_ff_dim": False, "rope_theta": 10000.0, "conv_L_cache": 3,
-              "conv_bias": False, "tie_word_embeddings": True, "norm_eps": 1e-5, "max_position_embeddings": 128, "eos_token_id": 7}
-    return write_random_model(config, str(folder), seed=width, dtype=torch.float32, std=0.03)
+    assert torch.equal(got[1], got[0])
 
 
 @pytest.mark.parametrize("width,folded", [(192, False), (256, True), (1024, True), (1088, False), (2048, False)])
