@@ -1765,28 +1765,12 @@ void Ops::embed_stats(const Tensor& table, const int* token_ids, const Tensor& o
                  "embed_stats");
 }
 
-// out = epilogue(prologue(a) w^T) for up to 64 rows, bfloat16 weights.
-//
-// a: bfloat16 rows [M, K], or, with norm_weight, the 32-bit residual stream, normalised on the
-// fly (stats[row, :stat_blocks] holding partial sums of squares of its rows if stat_blocks > 0).
-// rows picks rows of a.  Epilogues: Store (bfloat16 [M, N]), StoreF32, Residual (out is the
-// stream, [M, N] 32-bit, added to in place; stats_out [>= M, residual_stat_blocks] receives
-// partial sums of squares of the new rows, last_stat_blocks says how many a row), Swiglu (w is
-// [2N, K]: gate rows then up rows), Conv (w is [3N, K]: B, C, x rows; one new token per request).
-//
-// Up to 16 bfloat16 rows go to the k-sliced kernels, and 9 to 64 rows with an inner size that
-// is a multiple of 32 to the kernel that streams the weights.  Both also take the form behind a
-// norm whose weight the caller has folded into w: a is then the bfloat16 copy of the stream and
-// stats[row, :stat_blocks] its partial sums of squares, from which the rows' 1/rms (with eps)
-// scales the sums; their Residual epilogue refreshes out_bf16, the bfloat16 copy of the stream,
-// if given.  They also take w in the layout of fold_weight(packed).
-// Few 32-bit rows: the first inner size is the width of the stream.  Streams of up to 1,024: a sub-layer's norm, product, end
-// and product into the stream at 2 and 16 rows, kernels of their own | folded, us: width 1,024, q/k/v 10.9 | 9.7, 15.2 | 14.7, SwiGLU of
-// 4,608 23.3 | 19.3, 39.0 | 37.5, convolution 16.6 | 11.2, 19.7 | 16.2; width 1,152 14.9 | 17.8, 16.7 | 16.7, of 3,072 22.6 | 23.2, 31.3 | 32.1,
-// 20.7 | 22.9, 20.9 | 18.0; width 2,048 16.4 | 19.7, 23.2 | 25.0, of 8,192 52.4 | 57.5, 79.4 | 94.6, 26.9 | 31.6, 36.3 | 40.2: a workgroup of
-// eight or sixteen wavefronts that all wait for the norm has nobody beside it on its compute unit.
-// From 256 on, where the norm's own kernel adds the squares in the order of these products, so that a row has the same bits
-// in steps of up to 16 rows and in longer ones.
+// Few 32-bit rows: the first inner size is the width of the stream.  Streams of 256 to 1,024, where the norm's own kernel adds the
+// squares in the order of these products, so that a row has the same bits in steps of up to 16 rows and in longer ones.  A
+// sub-layer's norm, product, end and product into the stream at 2 and 16 rows, kernels of their own | folded, us: width 1,024, q/k/v 11.1 |
+// 9.4, 15.5 | 14.6, SwiGLU of 4,608 23.4 | 18.5, 39.2 | 36.2, convolution 16.7 | 11.0, 19.7 | 15.8; width 2,048 (not folded) 16.6 | 16.2,
+// 23.1 | 23.4, of 8,192 53.3 | 54.1, 79.4 | 90.5, 27.0 | 24.4, 36.6 | 37.9: a workgroup of eight or sixteen wavefronts that all wait
+// for the norm has nobody beside it on its compute unit.
 bool Ops::fused_linear_f32_ok(int rows, std::initializer_list<long long> inner) {
     if (rows < 1 || rows > 16 || inner.size() == 0 || *inner.begin() < 256 || *inner.begin() > 1024) return false;
     for (long long k : inner)
@@ -1836,6 +1820,21 @@ void Ops::fused_linear_f32(const Tensor& a, const Tensor& w, const Tensor& out, 
                  "fused_linear (32-bit)");
 }
 
+// out = epilogue(prologue(a) w^T) for up to 64 rows, bfloat16 weights.
+//
+// a: bfloat16 rows [M, K], or, with norm_weight, the 32-bit residual stream, normalised on the
+// fly (stats[row, :stat_blocks] holding partial sums of squares of its rows if stat_blocks > 0).
+// rows picks rows of a.  Epilogues: Store (bfloat16 [M, N]), StoreF32, Residual (out is the
+// stream, [M, N] 32-bit, added to in place; stats_out [>= M, residual_stat_blocks] receives
+// partial sums of squares of the new rows, last_stat_blocks says how many a row), Swiglu (w is
+// [2N, K]: gate rows then up rows), Conv (w is [3N, K]: B, C, x rows; one new token per request).
+//
+// Up to 16 bfloat16 rows go to the k-sliced kernels, and 9 to 64 rows with an inner size that
+// is a multiple of 32 to the kernel that streams the weights.  Both also take the form behind a
+// norm whose weight the caller has folded into w: a is then the bfloat16 copy of the stream and
+// stats[row, :stat_blocks] its partial sums of squares, from which the rows' 1/rms (with eps)
+// scales the sums; their Residual epilogue refreshes out_bf16, the bfloat16 copy of the stream,
+// if given.  They also take w in the layout of fold_weight(packed).
 void Ops::fused_linear(const Tensor& a, const Tensor& w, const Tensor& out, const FusedArgs& args) {
     dev(w, "w", DType::BF16);
     const Epilogue epi = args.epilogue;

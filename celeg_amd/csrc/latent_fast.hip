@@ -27,7 +27,10 @@
 // Measured in a recorded chain, 16 heads, rank 256 with 32 rotated, weights as two numbers, a window of 1,024, the same bits
 // (before: conditions as above, rows copied transposed within LDS, four barriers a block, one wavefront of four at
 // work in form 1): 2,048 rows of a prompt 152 -> 72 us, 77 rows behind 1,100 keys 127 -> 46, four single tokens with the
-// join 14.3 -> 8.8; rank 512 with 64 rotated, no window, 1,024 rows 277 -> 96.
+// join 14.3 -> 8.8; rank 512 with 64 rotated, no window, 1,024 rows 277 -> 96.  Sizes between the three gain less but gain (every
+// key; 2,048 rows, 77 behind 1,100 keys, four single tokens at 400): rank 16 with 8 rotated 61.5 -> 61.9, 36.3 -> 31.9, 8.5 -> 7.8, 128 with 32
+// 138 -> 65, 77 -> 32, 10.7 -> 8.2, 128 with 64 171 -> 96, 97 -> 48, 12.4 -> 9.1, 256 with 64, which runs as 576 with 512, 691 -> 309,
+// 204 -> 94, 20.7 -> 11.1.
 //
 // With a window the blocks begin at the first key that any column of the workgroup sees, and keys a column
 // no longer sees are masked; pages wholly before the window may be another request's by then and are not read.
