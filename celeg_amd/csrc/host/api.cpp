@@ -332,10 +332,9 @@ celeg_status celeg_engine_last_logits(celeg_engine* engine, float* out, size_t c
     if (!engine) return CELEG_INVALID_ARGUMENT;
     return guarded([&] {
         int r = 0, v = 0;
-        const std::vector<float> host = engine->engine->last_logits(r, v);
+        engine->engine->last_logits(out, capacity, r, v);
         if (rows) *rows = r;
         if (vocab) *vocab = v;
-        if (out) std::memcpy(out, host.data(), std::min(capacity, host.size()) * sizeof(float));
     }, &engine->last_error);
 }
 

@@ -229,18 +229,19 @@ Json Engine::request_metrics(long long id) {
         .set("preemptions", req.preemptions).set("error", req.error);
 }
 
-std::vector<float> Engine::last_logits(int& rows, int& vocab) {
+void Engine::last_logits(float* out, size_t capacity, int& rows, int& vocab) {
     rows = vocab = 0;
-    if (!last_logits_.defined()) return {};
+    if (!last_logits_.defined()) return;
     rows = static_cast<int>(last_logits_.shape[0]);
     vocab = static_cast<int>(last_logits_.shape[1]);
-    std::vector<float> host(static_cast<size_t>(rows) * vocab);
-    if (host.empty()) return host;
+    const size_t width = static_cast<size_t>(vocab), wanted = out ? std::min(capacity, static_cast<size_t>(rows) * width) : 0;
+    if (wanted == 0) return;
     CELEG_HIP(hipStreamSynchronize(loaded_->stream));
-    CELEG_HIP(hipMemcpy2D(host.data(), static_cast<size_t>(vocab) * 4, last_logits_.data,
-                          static_cast<size_t>(last_logits_.row_stride()) * 4, static_cast<size_t>(vocab) * 4,
-                          static_cast<size_t>(rows), hipMemcpyDeviceToHost));
-    return host;
+    const float* const from = last_logits_.as<float>();
+    const size_t stride = static_cast<size_t>(last_logits_.row_stride());
+    const size_t whole = stride == width ? wanted : width;     // floats that lie one after the other
+    for (size_t at = 0; at < wanted; at += whole)
+        CELEG_HIP(hipMemcpy(out + at, from + at / width * stride, std::min(whole, wanted - at) * sizeof(float), hipMemcpyDeviceToHost));
 }
 
 }  // namespace celeg

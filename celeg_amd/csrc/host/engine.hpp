@@ -48,8 +48,9 @@ public:
     void run() { run_steps(-1); }
     Json metrics() const;
     Json request_metrics(long long id);
-    // 32-bit logits of the last step on the host, [rows, vocab] (for --dump-logits)
-    std::vector<float> last_logits(int& rows, int& vocab);
+    // 32-bit logits of the last step, [rows, vocab]: their sizes, and up to `capacity` floats of them copied to `out` (null:
+    // the sizes alone), straight from the device: one row of 65,536 29 us, with a buffer between and a copy for the sizes 68
+    void last_logits(float* out, size_t capacity, int& rows, int& vocab);
 
     LoadedModel& loaded() { return *loaded_; }
     Scheduler& scheduler() { return *scheduler_; }
