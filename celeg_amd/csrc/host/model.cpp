@@ -50,10 +50,19 @@ Model::Model(ModelSpec s) : spec(std::move(s)) {
     graph_safe_ = true;
     std::function<void(const Part*)> visit = [&](const Part* p) {
         graph_safe_ = graph_safe_ && p->graph_safe();
-        short_context_ = std::max(short_context_, p->short_context());
         for (const Part* c : p->children()) visit(c);
     };
     for (const auto& np : named_parts()) visit(np.second);
+}
+
+int Model::short_context(int requests, DType dtype) const {
+    int longest = 0;
+    std::function<void(const Part*)> visit = [&](const Part* p) {
+        longest = std::max(longest, p->short_context(requests, dtype));
+        for (const Part* c : p->children()) visit(c);
+    };
+    for (const auto& np : const_cast<Model*>(this)->named_parts()) visit(np.second);
+    return longest;
 }
 
 void Model::resolve_cache_sharing() {
@@ -295,6 +304,7 @@ ModelRunner::ModelRunner(Model& m, CacheManager& c, Runtime& r, int max_tokens)
     std::set<int> buckets;
     for (int i = 0; i < 12; ++i) buckets.insert(std::min(1 << i, S));
     buckets_.assign(buckets.begin(), buckets.end());
+    for (int bucket : buckets_) short_contexts_[bucket] = model.short_context(bucket, rt.dtype);
 }
 
 ModelRunner::~ModelRunner() { drop_graphs(); }
@@ -449,10 +459,10 @@ bool ModelRunner::graph_applies(const std::vector<StepEntry>& entries) const {
 // A recorded step's launches are fixed, and the attention over few requests sizes its grid by
 // the context: a graph is therefore good up to a bound on the context, and there is one per
 // (batch-size bucket, bound).
-int ModelRunner::context_bound(const std::vector<StepEntry>& entries) const {
+int ModelRunner::context_bound(const std::vector<StepEntry>& entries, int bucket) const {
     int longest = 0;
     for (const StepEntry& e : entries) longest = std::max(longest, e.start_pos + static_cast<int>(e.tokens.size()));
-    for (int bound : {model.short_context(), 4096, 16384, 65536})
+    for (int bound : {short_contexts_.at(bucket), 4096, 16384, 65536})
         if (longest <= bound) return std::min(bound, cache.max_context);
     return cache.max_context;
 }
@@ -460,7 +470,7 @@ int ModelRunner::context_bound(const std::vector<StepEntry>& entries) const {
 Tensor ModelRunner::step_from_graph(const std::vector<StepEntry>& entries) {
     const int S = static_cast<int>(entries.size());
     const int bucket = *std::lower_bound(buckets_.begin(), buckets_.end(), S);
-    const int bound = context_bound(entries);
+    const int bound = context_bound(entries, bucket);
     const std::vector<int> caps(static_cast<size_t>(cache.n_groups()), bucket + 8);
     auto it = graphs_.find({bucket, bound});
     if (it == graphs_.end() || it->second.generation != rt.ws.generation) capture(bucket, caps, bound);

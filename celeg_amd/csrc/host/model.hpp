@@ -26,7 +26,7 @@ public:
 
     // whether a recorded step of this model may be replayed from a HIP graph
     bool graph_safe() const { return graph_safe_; }
-    int short_context() const { return short_context_; }
+    int short_context(int requests, DType dtype) const;
     std::vector<std::pair<std::string, Part*>> named_parts();
     // checkpoint tensor name -> what is expected of it
     ExpectedTensors expected_tensors();
@@ -55,7 +55,6 @@ private:
     std::vector<LayerCache> caches_;
     LayerCache embedding_cache_;
     bool bound_ = false, graph_safe_ = false;
-    int short_context_ = 0;
 };
 
 // The step function: runs one batch of (request, its next tokens) through the model, from the
@@ -103,7 +102,8 @@ private:
     };
     void validate(const std::vector<StepEntry>& entries) const;
     bool graph_applies(const std::vector<StepEntry>& entries) const;
-    int context_bound(const std::vector<StepEntry>& entries) const;
+    int context_bound(const std::vector<StepEntry>& entries, int bucket) const;
+    std::map<int, int> short_contexts_;      // by the bucket of a recorded step: Model::short_context
     Tensor step_from_graph(const std::vector<StepEntry>& entries);
     Captured& capture(int bucket, const std::vector<int>& caps, int bound);
     Captured& record(std::pair<int, int> key, const StepBatch& batch);

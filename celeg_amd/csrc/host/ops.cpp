@@ -844,7 +844,7 @@ bool Ops::attention_fresh_ok(int heads, int head_dim, const Tensor* inv_freq, in
     const int chunks = (heads / kv.kv_heads + 15) / 16;
     const long long groups = static_cast<long long>(kv.kv_heads) * chunks * batch.n_tokens;
     const int rounds = (hint_of(batch, kv) + 63) / 64;
-    const bool whole = decode_whole(groups, rounds);
+    const bool whole = decode_whole(groups, rounds, head_dim);
     if (whole) {
         // the kernel's loop over the rounds runs 1.7 % slower in this form, which outweighs the
         // kernel saved from about 8,192 tokens for each of 64 requests on (at 32,768: 4.94 against
@@ -1590,9 +1590,19 @@ void Ops::depth_mix(const Tensor& history, const Tensor& h, const Tensor& w, int
 // kernel, once there are enough of them: 192 (24 requests of 8 key/value heads) at any length, 96 at
 // contexts up to 4,096 tokens (12 and 16 requests at 2,048 tokens: 1 and 3 % of a decode step
 // faster than in parts; 16 requests at 8,192: 3 % slower).
-bool Ops::decode_whole(long long groups, int rounds) const {
+// Up to how many rounds of 64 keys one workgroup a (request, key/value head) is faster than parts and the kernel that joins
+// them, however few they are: its 16 wavefronts have a round each, and what a compute unit pulls alone (16 KB a round) stays
+// below what the second kernel costs.  16 heads over 8, in a recorded chain, us (one workgroup | parts):
+//   keys             60          250         400         510         640         760         890        1,020
+//   1 request     5.0 | 7.5   5.9 | 7.5   6.4 | 7.5   7.2 | 7.5   7.7 | 7.5   8.6 | 7.6   9.3 | 7.6  10.1 | 7.6
+//   4 requests    5.1 | 7.7   6.0 | 7.8   6.6 | 7.8   7.3 | 7.8   8.0 | 8.6   9.2 | 9.0   9.8 | 9.1  10.5 | 8.9
+//   8 requests    5.1 | 9.7   6.0 |10.1   7.0 |10.3   7.5 |10.2   8.0 |10.3   9.0 |10.3   9.7 |10.3  10.7 |10.7
+// (groups of 4 heads the same within 0.2; heads of 128 have not been measured.)
+int Ops::decode_short_rounds(long long groups, int head_dim) { return head_dim != 64 ? 0 : groups >= 64 ? 16 : 10; }
+
+bool Ops::decode_whole(long long groups, int rounds, int head_dim) const {
     if (attention_decode_whole >= 0) return attention_decode_whole > 0;
-    return groups >= 192 || (groups >= 96 && rounds <= 64);
+    return groups >= 192 || (groups >= 96 && rounds <= 64) || rounds <= decode_short_rounds(groups, head_dim);
 }
 
 int Ops::decode_split_rounds(long long groups, int rounds) const {
@@ -1613,7 +1623,7 @@ void Ops::attention_decode(const Tensor& q, const Tensor& out, int heads, int kv
     const int bound = hint ? std::min(hint, max_context) : max_context;
     const int rounds = (bound + 63) / 64;
     const int chunks = (heads / kv_heads + 15) / 16;
-    const int whole = decode_whole(static_cast<long long>(kv_heads) * chunks * T, rounds) ? 1 : 0;
+    const int whole = decode_whole(static_cast<long long>(kv_heads) * chunks * T, rounds, head_dim) ? 1 : 0;
     const int split_rounds = decode_split_rounds(static_cast<long long>(kv_heads) * chunks * T, rounds);
     const int n_parts = (rounds + split_rounds - 1) / split_rounds;
     const size_t parts = static_cast<size_t>(T) * heads * n_parts;

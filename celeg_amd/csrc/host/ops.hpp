@@ -131,7 +131,8 @@ public:
     int decode_part_thresholds[2] = {64, 256};
     bool decode_parts_fill = true;       // parts of 16 rounds where they are one workgroup a compute unit
     int decode_split_rounds(long long groups, int rounds) const;
-    bool decode_whole(long long groups, int rounds) const;
+    bool decode_whole(long long groups, int rounds, int head_dim) const;
+    static int decode_short_rounds(long long groups, int head_dim);
     bool attention_general = false;      // always the general attention kernel
     bool delta_general = false;          // the delta rule's recurrence always by the kernel for any dim
     bool delta_pairs = true;             // the recurrence in registers takes whole blocks of rows two tokens at a time

@@ -46,9 +46,9 @@ public:
     // recorded step can be replayed from a HIP graph.  A part that plans on the host must leave
     // this false; a model with such a part is never replayed from a graph.
     virtual bool graph_safe() const { return false; }
-    // up to which context a recorded step of single tokens is better recorded for itself (0: no such border): the
+    // up to which context a recorded step of so many single tokens is better recorded for itself (0: no such border): the
     // grid that pays for a window of keys costs a step of few keys time
-    virtual int short_context() const { return 0; }
+    virtual int short_context(int requests, DType dtype) const { return 0; }
     virtual WeightSpecs weight_specs() const { return {}; }
     virtual void load(const PartTensors& tensors, Runtime& rt) {}
     // parts nested inside this one (an attention's position encoding), for graph safety
