@@ -9,6 +9,11 @@
 // refresh its bfloat16 copy and leave partial sums of squares | SwiGLU of a gate and an
 // up stream.
 //
+// The weights lie as they are ([rows, K]) or, for the residual epilogue, packed in blocks of 32 values of k ([K/32, rows, 32],
+// the copy that the products of few rows read): a load then asks for 1 KB in a row where it otherwise asks for 128 bytes of
+// eight rows.  With weights from memory (2,048 rows: 75 MB cross the fabric behind the L2s) w2 of 1,024 x 4,608 takes 32.1 us
+// packed and 35.0 as they are, out_proj of 1,024 x 1,024 12.1 and 12.5; celeg_gemm_tiles_packed says where it is worth it.
+//
 // Layout.  A workgroup owns a tile of BM rows x BN weight rows (for SwiGLU: BN/2 gate rows
 // and the BN/2 up rows of the same columns) over the whole of K.  Blocks of 64 values of k
 // of both operands travel from memory straight into LDS (16 bytes a lane,
@@ -19,6 +24,8 @@
 // c ^ (r & 7) of its row, which spreads the rows that neighbouring lanes read at the same
 // chunk over the banks (measured: as fast as reading 1 KB in a row; rows padded to 144 bytes
 // or a swap of neighbouring rows on top were 1.6 times slower).
+// (A row of packed weights is 64 bytes a half of the block, its chunk c at c ^ ((r / 2) & 3): read by lane % 16 as the row and
+// lane / 16 as the chunk, both lie over all banks, 4 cycles a KB; at c ^ ((r / 4) & 3) 8 cycles.)
 // The loads place the chunks: a load instruction writes 1 KB = 8 rows, lane l at row l / 8,
 // chunk l % 8, so lane l asks memory for the chunk that belongs there.
 // WGM x WGN wavefronts share the tile; a wavefront keeps (BN/WGN/16) x (BM/WGM/16) tiles of
@@ -421,7 +428,55 @@ __device__ __forceinline__ void qkv_epilogue(const TileParams& p, floatx4_t (&ac
     }
 }
 
-template <int BM, int BN, int WGM, int WGN, int STAGES, int EPI>
+// A tile whose K is cut over several workgroups: each leaves its sums in memory and counts itself in; the last one to arrive
+// adds them all up, in the order of the slices, and goes on (true), the others are done.  Nobody waits for anybody.
+// The sums are written and read past the dies' caches (accesses of device scope), and they have arrived where a wavefront's
+// count of accesses in flight is down to none: no cache is written back or invalidated in between.
+// [tile][slice][wavefront][piece][lane] of four sums.
+template <int NW, int FN, int FM>
+__device__ __forceinline__ bool tile_join(const TileParams& p, floatx4_t (&acc)[FN][FM], const int tile, const int slice,
+                                          const int wave, const int lane, char* const lds) {
+    typedef unsigned long long u64;
+    constexpr int PIECES = FN * FM;
+    const int slices = p.k_slices;
+    const auto part = [&](int s, int piece) {
+        return reinterpret_cast<u64*>(p.parts) + (((static_cast<size_t>(tile) * slices + s) * NW + wave) * PIECES + piece) * 128 + 2 * lane;
+    };
+    floatx4_t own[PIECES];
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+        own[i] = acc[i / FM][i % FM];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const float pair[2] = {own[i][2 * h], own[i][2 * h + 1]};
+            __hip_atomic_store(part(slice, i) + h, __builtin_bit_cast(u64, pair), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();                              // (the stages are no longer read)
+    if (threadIdx.x == 0)
+        *reinterpret_cast<int*>(lds) = __hip_atomic_fetch_add(p.arrived + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    const bool last = *reinterpret_cast<int*>(lds) == slices - 1;
+    __syncthreads();
+    if (!last) return false;
+    if (threadIdx.x == 0) __hip_atomic_store(p.arrived + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);     // (for the next launch)
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) acc[i / FM][i % FM] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < slices; ++s) {
+        u64 v[PIECES][2];
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) v[i][h] = __hip_atomic_load(part(s, i) + h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) acc[i / FM][i % FM] += s == slice ? own[i] : __builtin_bit_cast(floatx4_t, v[i]);
+    }
+    return true;
+}
+
+// PACKED: the weights are.  SPLIT: p.k_slices workgroups a tile share its K.
+template <int BM, int BN, int WGM, int WGN, int STAGES, int EPI, bool PACKED, bool SPLIT>
 __global__ __launch_bounds__(WGM * WGN * 64)
 void gemm_tiles_kernel(const TileParams p, const int tiles_m, const int tiles_n, const int dies_m) {
     constexpr int NW = WGM * WGN;
@@ -434,6 +489,7 @@ void gemm_tiles_kernel(const TileParams p, const int tiles_m, const int tiles_n,
                                                    // not divide, the last ones ask for the last group again)
     static_assert(FN % NS == 0 && WTM % 16 == 0 && WTN % 16 == 0, "tile shape");
     static_assert(GPW * STAGES < 64, "more loads in flight than the counter holds");
+    static_assert(!PACKED || (BM / 8 % NW == 0 && EPI == T_RESIDUAL), "a wavefront's load i is of A or of packed weights");
     extern __shared__ __attribute__((aligned(1024))) char lds[];
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -449,12 +505,16 @@ void gemm_tiles_kernel(const TileParams p, const int tiles_m, const int tiles_n,
     const int di = die / dies_n, dj = die % dies_n;
     const int r0 = di * tiles_m / dies_m, rows = (di + 1) * tiles_m / dies_m - r0;
     const int c0 = dj * tiles_n / dies_n, cols = (dj + 1) * tiles_n / dies_n - c0;
-    if (local >= rows * cols) return;
-    const int tile_n = c0 + local / rows;
-    const int m0 = (r0 + local % rows) * BM;
+    const int slices = SPLIT ? p.k_slices : 1;
+    if (local >= rows * cols * slices) return;
+    const int slice = SPLIT ? local % slices : 0, place = SPLIT ? local / slices : local;
+    const int tile_n = c0 + place / rows;
+    const int tile_m = r0 + place % rows, m0 = tile_m * BM;
     const int n0 = tile_n * (BN / NS);
 
     // ---- what this lane asks memory for: group g = wave + i * NW, rows 8g .. 8g+7 of the stage
+    const int first_kb = SPLIT ? slice * (K >> 6) / slices : 0;
+    const size_t w_next = PACKED ? static_cast<size_t>(p.w_block) * 4 : 128;      // bytes from a block of weights to the next
     const char* src[GPW];
 #pragma unroll
     for (int i = 0; i < GPW; ++i) {
@@ -464,18 +524,25 @@ void gemm_tiles_kernel(const TileParams p, const int tiles_m, const int tiles_n,
         if (g < BM / 8) {
             const int m = min(m0 + row, M - 1);
             src[i] = reinterpret_cast<const char*>(p.a + static_cast<size_t>(m) * p.lda) + chunk * 16;
+        } else if (PACKED) {
+            // 16 rows of half a block of k: the first half's groups, then the second's
+            const int half = (g - BM / 8) / (BN / 16), b = (g - BM / 8) % (BN / 16) * 16 + (lane >> 2);
+            const int s = b / (BN / NS), n = min(n0 + b % (BN / NS), N - 1);
+            src[i] = reinterpret_cast<const char*>(p.w + half * p.w_block + (static_cast<size_t>(s) * p.stream_rows + n) * 32) +
+                     ((lane & 3) ^ ((b >> 1) & 3)) * 16;
         } else {
             const int b = row - BM;
             const int s = b / (BN / NS), j = b % (BN / NS);
             const int n = min(n0 + j, N - 1);
             src[i] = reinterpret_cast<const char*>(p.w + (static_cast<size_t>(s) * p.stream_rows + n) * p.ldw) + chunk * 16;
         }
+        if (SPLIT) src[i] += static_cast<size_t>(first_kb) * (g < BM / 8 ? 128 : w_next);
     }
     auto issue = [&](int stage, int kb) {
         char* const base = lds + stage * STAGE_BYTES;
 #pragma unroll
         for (int i = 0; i < GPW; ++i)
-            __builtin_amdgcn_global_load_lds(GPTR(src[i] + static_cast<size_t>(kb) * 128),
+            __builtin_amdgcn_global_load_lds(GPTR(src[i] + static_cast<size_t>(kb) * (i < BM / 8 / NW ? 128 : w_next)),
                                              LPTR(base + min(wave + i * NW, GROUPS - 1) * 1024), 16, 0, 0);
     };
 
@@ -485,6 +552,7 @@ void gemm_tiles_kernel(const TileParams p, const int tiles_m, const int tiles_n,
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
         lane_off[ks] = r16 * 128 + (((ks * 4 + q) ^ (r16 & 7)) * 16);
+    const int packed_off = r16 * 64 + ((q ^ ((r16 >> 1) & 3)) * 16);
 
     floatx4_t acc[FN][FM];
 #pragma unroll
@@ -498,7 +566,7 @@ void gemm_tiles_kernel(const TileParams p, const int tiles_m, const int tiles_n,
     QkvEarly<EPI == T_QKV ? FM : 1> qkv_early;
     if constexpr (EPI == T_QKV) qkv_early_rows<BM, WGM, WGN>(p, qkv_early, m0, n0 + wn * WTN, wm, lane);
 
-    const int nkb = K >> 6;                       // K % 64 == 0 (checked by the host)
+    const int nkb = (SPLIT ? (slice + 1) * (K >> 6) / slices : K >> 6) - first_kb;      // K % 64 == 0 (checked by the host)
 #pragma unroll
     for (int s = 0; s < STAGES; ++s)
         if (s < nkb) issue(s, s);
@@ -512,13 +580,13 @@ void gemm_tiles_kernel(const TileParams p, const int tiles_m, const int tiles_n,
     bf16x8_t af[2][FM], wf[2][FN];
     auto fetch = [&](int stage, int ks, bf16x8_t (&a)[FM], bf16x8_t (&w)[FN]) {
         const char* const sa = lds + stage * STAGE_BYTES + (wm * WTM) * 128 + lane_off[ks];
-        const char* const sw = lds + stage * STAGE_BYTES + BM * 128 + lane_off[ks];
+        const char* const sw = lds + stage * STAGE_BYTES + BM * 128 + (PACKED ? ks * BN * 64 + packed_off : lane_off[ks]);
 #pragma unroll
         for (int tm = 0; tm < FM; ++tm) a[tm] = *reinterpret_cast<const bf16x8_t*>(sa + tm * 2048);
 #pragma unroll
         for (int tn = 0; tn < FN; ++tn) {
             const int brow = (tn / (FN / NS)) * (BN / NS) + wn * (WTN / NS) + (tn % (FN / NS)) * 16;
-            w[tn] = *reinterpret_cast<const bf16x8_t*>(sw + brow * 128);
+            w[tn] = *reinterpret_cast<const bf16x8_t*>(sw + brow * (PACKED ? 64 : 128));
         }
     };
     auto multiply = [&](const bf16x8_t (&a)[FM], const bf16x8_t (&w)[FN]) {
@@ -551,6 +619,9 @@ void gemm_tiles_kernel(const TileParams p, const int tiles_m, const int tiles_n,
         stage = next;
     }
 
+    if constexpr (SPLIT) {
+        if (!tile_join<NW>(p, acc, tile_m * tiles_n + tile_n, slice, wave, lane, lds)) return;
+    }
     if constexpr (EPI == T_QKV) {
         static_assert(EPI != T_QKV || (WTN == QKV_HD && FN == 4), "a wavefront holds one head of 64 columns");
         qkv_epilogue<BM, WGM, WGN>(p, acc, scale, qkv_early, m0, n0 + wn * WTN, wm, wn, lane, lds);
@@ -846,6 +917,7 @@ void gemm_tiles_wide_kernel(const TileParams p, const int tiles_m, const int til
 struct TileShape {
     int id;         // index into the table below
     int bm, bn;     // bn counts weight rows of all streams
+    int slices;     // workgroups a tile, which share its K
 };
 
 // For tests and tuning: a shape that overrides the choice below (-1: none).
@@ -902,7 +974,36 @@ static Dies dies_of(int tiles_m, int tiles_n, int M, int weight_rows) {
     return best;
 }
 
-static TileShape tile_shape(int M, int N, int K, int streams) {
+// Whether K is cut over workgroups of which the last to arrive adds the sums (packed weights, residual): where the product's
+// own tiles leave most compute units idle and K is long, so that each slice keeps 16 blocks of k, and no die gets more
+// workgroups than it has compute units.  Measured with weights from memory, us (cut | whole, both packed):
+//   rows                     65 to 70       130           200           300           450           600
+//   1,024 x 4,608            11.1 | 17.8   12.1 | 17.8   14.0 | 17.9   16.5 | 17.9   17.3 | 18.2   21.4 | 21.8
+//   2,048 x 8,192            18.1 | 28.6   24.6 | 28.8   24.7 | 28.9   29.0 | 36.5   (35.4 | 35.9)
+// (2,048 x 2,048 and less: the same or slower; tiles that fill the compute units, cut: 2 to 20 % slower; a second round of
+// workgroups on one die, 772 x 5,120 at 700 rows: 31.5 us against 26.3.)
+static TileShape tile_split(int M, int N, int K) {
+    const auto fits = [&](int id, int slices) {
+        return dies_of((M + k_shape_bm[id] - 1) / k_shape_bm[id], (N + k_shape_bn[id] - 1) / k_shape_bn[id], M, N).per_die * slices <= DIE_UNITS;
+    };
+    const auto shape = [&](int id, int slices) { return TileShape{id, k_shape_bm[id], k_shape_bn[id], slices}; };
+    if (K < 4096) return shape(0, 1);
+    if (fits(0, 4)) return shape(0, 4);
+    if (fits(0, 3)) return shape(0, 3);
+    if (fits(1, 4)) return shape(1, 4);
+    if (fits(1, 2)) return shape(1, 2);
+    if (fits(3, 3)) return shape(3, 3);
+    return shape(0, 1);
+}
+// For tests and tuning: so many slices instead of the rule's (0: the rule; 1: none).
+static int g_force_slices = 0;
+extern "C" void celeg_gemm_tiles_force_slices(int slices) { g_force_slices = slices; }
+
+static TileShape tile_shape(int M, int N, int K, int streams, bool may_split = false) {
+    if (may_split && g_force_slices != 1 && g_force_shape < 0) {
+        const TileShape cut = tile_split(M, N, K);
+        if (cut.slices > 1) return cut;
+    }
     int id = 0;
     if (g_force_shape >= 0 && g_force_shape < N_TILE_SHAPES) id = g_force_shape;
     else {
@@ -951,10 +1052,13 @@ static TileShape tile_shape(int M, int N, int K, int streams) {
             id = rounds288 * 22 < rounds128 * 10 ? 10 : 8;
         }
     }
-    return TileShape{id, k_shape_bm[id], k_shape_bn[id]};
+    return TileShape{id, k_shape_bm[id], k_shape_bn[id], 1};
 }
 
-template <int BM, int BN, int WGM, int WGN, int STAGES, int KB, int EPI>
+#define TILE_SPLITS(ID) ((ID) == 0 || (ID) == 1 || (ID) == 3)      // the shapes that tile_split names
+#define TILE_SPLIT_MOST_BYTES (256 * 64 * 128 * 4)                 // of sums: 256 workgroups of the largest of them
+
+template <int BM, int BN, int WGM, int WGN, int STAGES, int KB, int EPI, bool PACKED, bool SPLIT>
 static int launch_tiles(const TileParams& p, hipStream_t stream) {
     constexpr int NS = TileStreams<EPI>::n;
     constexpr size_t stages_lds = static_cast<size_t>(STAGES) * (BM + BN) * (KB == 32 ? 64 : 128);
@@ -963,7 +1067,7 @@ static int launch_tiles(const TileParams& p, hipStream_t stream) {
     constexpr size_t lds = stages_lds > swiglu_lds ? stages_lds : swiglu_lds;
     void (*kernel)(const TileParams, const int, const int, const int);
     if constexpr (KB != 0) kernel = &gemm_tiles_wide_kernel<BM, BN, WGM, WGN, STAGES, KB, EPI>;
-    else kernel = &gemm_tiles_kernel<BM, BN, WGM, WGN, STAGES, EPI>;
+    else kernel = &gemm_tiles_kernel<BM, BN, WGM, WGN, STAGES, EPI, PACKED, SPLIT>;
     static_assert(lds <= 160 * 1024, "more LDS than a compute unit has");
     static bool raised = false;              // once per instantiation: more LDS than the default limit
     if (lds > 48 * 1024 && !raised) {
@@ -977,7 +1081,7 @@ static int launch_tiles(const TileParams& p, hipStream_t stream) {
     if (g_force_dies_m > 0) dies_m = g_force_dies_m;
     const int dies_n = 8 / dies_m;
     const int per_die = ((tiles_m + dies_m - 1) / dies_m) * ((tiles_n + dies_n - 1) / dies_n);
-    dim3 grid(per_die * 8), block(WGM * WGN * 64);
+    dim3 grid(per_die * 8 * (SPLIT ? p.k_slices : 1)), block(WGM * WGN * 64);
     hipLaunchKernelGGL(kernel, grid, block, lds, stream, p, tiles_m, tiles_n, dies_m);
     return CELEG_LAUNCH_RESULT();
 }
@@ -986,16 +1090,54 @@ template <int EPI>
 static int launch_epilogue(const TileParams& p, hipStream_t stream) {
     const TileShape s = tile_shape(p.M, p.N, p.K, TileStreams<EPI>::n);
 #define TILE_CASE(ID, BM, BN, WGM, WGN, STAGES, KB) \
-    if (s.id == ID) return launch_tiles<BM, BN, WGM, WGN, STAGES, KB, EPI>(p, stream);
+    if (s.id == ID) return launch_tiles<BM, BN, WGM, WGN, STAGES, KB, EPI, false, false>(p, stream);
     TILE_SHAPES(TILE_CASE)
 #undef TILE_CASE
     return static_cast<int>(hipErrorInvalidValue);
 }
 
-// Number of partial sums of squares a row gets from the "residual" epilogue for these
-// sizes (one per tile column): the caller sizes stats_out [>= M, >= blocks].
-extern "C" int celeg_gemm_tiles_blocks(int M, int N, int K) {
+// The residual epilogue with packed weights, K cut where there is room for the sums.
+template <int EPI>
+static int launch_packed(const TileParams& params, hipStream_t stream) {
+    TileParams p = params;
+    TileShape s = tile_shape(p.M, p.N, p.K, 1, p.parts && p.arrived);
+    if (g_force_slices > 1 && p.parts && p.arrived && TILE_SPLITS(s.id) && g_force_slices <= p.K / 64) s.slices = g_force_slices;
+    p.k_slices = s.slices;
+    const long long tiles = static_cast<long long>((p.M + s.bm - 1) / s.bm) * ((p.N + s.bn - 1) / s.bn);
+    if (s.slices > 1 && (tiles > 256 || tiles * s.slices * s.bm * s.bn * 4 > TILE_SPLIT_MOST_BYTES)) return static_cast<int>(hipErrorInvalidValue);
+#define TILE_CASE(ID, BM, BN, WGM, WGN, STAGES, KB)                                                                     \
+    if constexpr (KB == 0) {                                                                                            \
+        if constexpr (TILE_SPLITS(ID)) {                                                                                \
+            if (s.id == ID && s.slices > 1) return launch_tiles<BM, BN, WGM, WGN, STAGES, KB, EPI, true, true>(p, stream); \
+        }                                                                                                               \
+        if (s.id == ID) return launch_tiles<BM, BN, WGM, WGN, STAGES, KB, EPI, true, false>(p, stream);          \
+    }
+    TILE_SHAPES(TILE_CASE)
+#undef TILE_CASE
+    return static_cast<int>(hipErrorInvalidValue);      // (the wide tiles read weights as they are)
+}
+
+// Whether the residual epilogue is better given packed weights for these sizes, and room for a cut K's sums (bytes, and zeros
+// ahead of them that the launch leaves as zeros, 256 numbers).  Us, packed | as they are, with weights from memory:
+//   1,024 x 4,608    1,000 rows 22.6 | 23.8, 1,300 31.1 | 29.7, 1,500 31.5 | 32.8, 1,700 31.6 | 30.2, 2,048 33.0 | 35.4, 4,096 58.6 | 63.5
+//   1,024 x 1,024    600 8.4 | 8.4, 1,500 11.6 | 12.0, 2,048 12.2 | 12.5, 8,192 33.9 | 34.6
+//   2,048 x 2,048    512 13.4 | 13.9, 700 18.0 | 17.7, 1,024 19.7 | 20.0, 1,500 29.6 | 30.9, 2,048 33.2 | 34.1, 4,096 47.8 | 50.3
+//   2,048 x 8,192    512 38.4 | 39.5, 600 49.8 | 48.7, 1,024 53.2 | 52.3, 1,500 71.3 | 75.1, 2,048 77.3 | 82.2
+// (128x64, the tile of 1,024 x 4,608 from 1,025 rows on and of 2,048 x 8,192 at 513 to 1,024: only where it is on nearly all
+// compute units and K below 8,192; 64x192 and 128x192, which none of these takes, and the wide tiles: not.)
+extern "C" int celeg_gemm_tiles_packed(int M, int N, int K) {
+    if (tile_split(M, N, K).slices > 1) return 1;
     const TileShape s = tile_shape(M, N, K, 1);
+    if (s.id == 2) return K < 8192 && static_cast<long long>((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn) >= 240;
+    return s.id == 0 || s.id == 1 || s.id == 3 || s.id == 5 || s.id == 6 || s.id == 8;
+}
+extern "C" size_t celeg_gemm_tiles_split_bytes() { return TILE_SPLIT_MOST_BYTES; }
+
+// Number of partial sums of squares a row gets from the "residual" epilogue for these
+// sizes (one per tile column): the caller sizes stats_out [>= M, >= blocks].  packed: with packed weights and room
+// for a cut K's sums.
+extern "C" int celeg_gemm_tiles_blocks(int M, int N, int K, int packed) {
+    const TileShape s = tile_shape(M, N, K, 1, packed != 0);
     return (N + s.bn - 1) / s.bn;
 }
 
@@ -1007,7 +1149,7 @@ extern "C" int celeg_gemm_tiles(const TileParams* params, int epi, hipStream_t s
     const TileParams& p = *params;
     if (p.M <= 0 || p.N <= 0) return 0;
     if (p.K <= 0 || (p.K % 64) || (p.N % 4) || (p.lda % 8) || (p.ldw % 8) || (p.ldo % 4) ||
-        p.lda < p.K || p.ldw < p.K || p.ldo < p.N)
+        p.lda < p.K || (p.w_block ? p.ldw != 32 || p.w_block % 8 || p.w_block < 32LL * p.N || epi != T_RESIDUAL : p.ldw < p.K) || p.ldo < p.N)
         return static_cast<int>(hipErrorInvalidValue);
     if (p.stats && p.n_stat_blocks < 1) return static_cast<int>(hipErrorInvalidValue);
     if (reinterpret_cast<uintptr_t>(p.bias) & 15) return static_cast<int>(hipErrorInvalidValue);
@@ -1015,7 +1157,7 @@ extern "C" int celeg_gemm_tiles(const TileParams* params, int epi, hipStream_t s
     if (epi == T_SWIGLU && p.stream_rows < p.N) return static_cast<int>(hipErrorInvalidValue);
     switch (epi) {
         case T_STORE: return launch_epilogue<T_STORE>(p, stream);
-        case T_RESIDUAL: return launch_epilogue<T_RESIDUAL>(p, stream);
+        case T_RESIDUAL: return p.w_block ? launch_packed<T_RESIDUAL>(p, stream) : launch_epilogue<T_RESIDUAL>(p, stream);
         case T_SWIGLU: return launch_epilogue<T_SWIGLU>(p, stream);
         case T_QKV: {
             const auto misaligned = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) != 0; };
@@ -1030,10 +1172,10 @@ extern "C" int celeg_gemm_tiles(const TileParams* params, int epi, hipStream_t s
             // more than one for each of its compute units, as above.  In a model, 2,048 columns by
             // 1,024: 301 rows 12.4 us, 600 rows 14.4, 2,048 rows 21.3; with the last of these for all 22.4, 22.6 and 23.0)
             const auto fits = [&](int bm, int bn) { return dies_of((p.M + bm - 1) / bm, (p.N + bn - 1) / bn, p.M, p.N).per_die <= DIE_UNITS; };
-            if (fits(64, 64)) return launch_tiles<64, 64, 4, 1, 4, 0, T_QKV>(p, stream);
-            if (fits(64, 128)) return launch_tiles<64, 128, 4, 2, 4, 0, T_QKV>(p, stream);
-            if (fits(128, 128)) return launch_tiles<128, 128, 4, 2, 4, 0, T_QKV>(p, stream);
-            return launch_tiles<128, 128, 4, 2, 2, 0, T_QKV>(p, stream);
+            if (fits(64, 64)) return launch_tiles<64, 64, 4, 1, 4, 0, T_QKV, false, false>(p, stream);
+            if (fits(64, 128)) return launch_tiles<64, 128, 4, 2, 4, 0, T_QKV, false, false>(p, stream);
+            if (fits(128, 128)) return launch_tiles<128, 128, 4, 2, 4, 0, T_QKV, false, false>(p, stream);
+            return launch_tiles<128, 128, 4, 2, 2, 0, T_QKV, false, false>(p, stream);
         }
         default: return static_cast<int>(hipErrorInvalidValue);
     }

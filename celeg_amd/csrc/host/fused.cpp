@@ -211,7 +211,8 @@ void linear_into_stream(Runtime& rt, const Tensor& a, const Tensor& w, const Ten
     if (tiled_step(rt, T, width)) {
         Tensor stats = stream_stats(rt, width, T);
         Tensor xb = stream_bf16(rt, T, width);
-        rt.ops.tiled_linear(a, w, h, Epilogue::Residual, 0.f, nullptr, 0, bias, &stats, &xb);
+        const bool packed = w.dtype == DType::BF16 && Ops::tiled_packed(T, static_cast<int>(width), static_cast<int>(w.shape[1]));
+        rt.ops.tiled_linear(a, packed ? packed_weight(rt, w)->view : w, h, Epilogue::Residual, 0.f, nullptr, 0, bias, &stats, &xb);
         rt.stream_stat_blocks = rt.ops.last_stat_blocks;
         rt.stream_has_bf16 = true;
         return;

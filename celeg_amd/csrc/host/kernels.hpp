@@ -150,9 +150,11 @@ int celeg_gemv_fused(const GemvParams* params, int amode, int epi, int shape, hi
 int celeg_embed_stats(const void* table, const int* ids, float* out, float* stats, int stats_ld, int rows, int width,
                       int vocab, hipStream_t stream);
 // gemm_tiles.hip: the fused products of many rows
-int celeg_gemm_tiles_blocks(int M, int N, int K);
+int celeg_gemm_tiles_blocks(int M, int N, int K, int packed);
 int celeg_gemm_tiles_params_size();
 int celeg_gemm_tiles(const TileParams* params, int epi, hipStream_t stream);
+int celeg_gemm_tiles_packed(int M, int N, int K);
+size_t celeg_gemm_tiles_split_bytes();
 // norm_step.hip
 int celeg_norm_step(float* h, const void* y, int y_dtype, CelegNorm post, CelegNorm pre, void* out, int out_dtype,
                     const int* rows, int n_rows, int width, int write_back, hipStream_t stream);

@@ -1994,7 +1994,8 @@ bool Ops::tiled_linear_ok(int rows, int n, std::initializer_list<long long> inne
     return true;
 }
 
-int Ops::tiled_stat_blocks(int rows, int n, int k) const { return celeg_gemm_tiles_blocks(rows, n, k); }
+int Ops::tiled_stat_blocks(int rows, int n, int k, bool packed) const { return celeg_gemm_tiles_blocks(rows, n, k, packed ? 1 : 0); }
+bool Ops::tiled_packed(int rows, int n, int k) { return celeg_gemm_tiles_packed(rows, n, k) != 0; }
 
 // out = epilogue(scale * (a w^T) + bias) for many bfloat16 rows (any number; made for more than
 // 64), inner size a multiple of 64, columns a multiple of 4.  With stat_blocks > 0, a is the
@@ -2002,7 +2003,8 @@ int Ops::tiled_stat_blocks(int rows, int n, int k) const { return celeg_gemm_til
 // and stats[row, :stat_blocks] are partial sums of squares of its rows, from which the rows'
 // 1/rms (with eps) scales the sums.  Epilogues: Store (bfloat16 [M, N]), Residual (out is the
 // 32-bit stream, added to in place; out_bf16 receives its bfloat16 copy and stats_out the partial
-// sums of squares of the new rows; last_stat_blocks says how many a row), Swiglu (w is [2N, K]).
+// sums of squares of the new rows; last_stat_blocks says how many a row; w as it is or packed, [K/32, N, 32]),
+// Swiglu (w is [2N, K]).
 bool Ops::tiled_qkv_ok(int head_dim, const Tensor* inv_freq, int rotary_dim, int pairing, const KVView& kv) const {
     if (!use_qkv_tail) return false;
     if (head_dim != 64 || kv.dtype != DType::BF16 || kv.head_dim != 64 || (kv.v_head_dim && kv.v_head_dim != 64)) return false;
@@ -2018,10 +2020,11 @@ void Ops::tiled_linear(const Tensor& a, const Tensor& w, const Tensor& out, Epil
     dev(a, "a", DType::BF16, false);
     dev(w, "w", DType::BF16);
     const int streams = epi == Epilogue::Swiglu ? 2 : 1;
-    need(a.ndim == 2 && w.ndim == 2, "tiled_linear: a and w must be 2-D");
-    const long long M = a.shape[0], K = a.shape[1];
-    need(w.shape[1] == K && w.shape[0] % streams == 0, "tiled_linear: a and w do not fit");
-    const long long N = w.shape[0] / streams;
+    const bool packed = w.ndim == 3 && w.shape[2] == 32 && epi == Epilogue::Residual;
+    need(a.ndim == 2 && (w.ndim == 2 || packed), "tiled_linear: a and w must be 2-D");
+    const long long M = a.shape[0], K = a.shape[1], w_rows = w.shape[packed ? 1 : 0];
+    need((packed ? w.shape[0] * 32 : w.shape[1]) == K && w_rows % streams == 0, "tiled_linear: a and w do not fit");
+    const long long N = w_rows / streams;
     need(K % 64 == 0 && N % 4 == 0, "tiled_linear: inner size " + std::to_string(K) + " must be a multiple of 64 and " +
                                         std::to_string(N) + " columns a multiple of 4");
     const int lda = rows_of(a, "a");
@@ -2035,8 +2038,18 @@ void Ops::tiled_linear(const Tensor& a, const Tensor& w, const Tensor& out, Epil
     prm.a = a.as<bf16>();
     prm.lda = lda;
     prm.w = w.as<bf16>();
-    prm.ldw = static_cast<int>(K);
+    prm.ldw = packed ? 32 : static_cast<int>(K);
+    prm.w_block = packed ? 32 * w_rows : 0;
     prm.stream_rows = static_cast<int>(N);
+    if (packed) {
+        if (!tile_parts_.ptr()) {      // (a recorded step has run once before it is recorded)
+            tile_counts_ = DeviceBuffer(256 * sizeof(int), true);
+            CELEG_HIP(hipStreamSynchronize(nullptr));      // (the zeros are there before this stream goes on)
+            tile_parts_ = DeviceBuffer(celeg_gemm_tiles_split_bytes());
+        }
+        prm.parts = tile_parts_.as<float>();
+        prm.arrived = tile_counts_.as<int>();
+    }
     if (bias) {
         dev(*bias, "bias", DType::F32);
         need(bias->numel() == streams * N, "tiled_linear: bias does not fit");
@@ -2058,7 +2071,7 @@ void Ops::tiled_linear(const Tensor& a, const Tensor& w, const Tensor& out, Epil
     prm.out = out.data;
     prm.ldo = ldo;
     if (epi == Epilogue::Residual) {
-        last_stat_blocks = tiled_stat_blocks(static_cast<int>(M), static_cast<int>(N), static_cast<int>(K));
+        last_stat_blocks = tiled_stat_blocks(static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), packed);
         if (out_bf16) {
             dev(*out_bf16, "out_bf16", DType::BF16, false);
             const int ldb = rows_of(*out_bf16, "out_bf16");

@@ -424,7 +424,9 @@ public:
     void fused_linear_f32(const Tensor& a, const Tensor& w, const Tensor& out, const FusedArgs& args);
     // fused products of many rows
     bool tiled_linear_ok(int rows, int n, std::initializer_list<long long> inner) const;
-    int tiled_stat_blocks(int rows, int n, int k) const;
+    int tiled_stat_blocks(int rows, int n, int k, bool packed = false) const;
+    // whether a product into the stream of many rows is better given packed weights ([K/32, rows, 32])
+    static bool tiled_packed(int rows, int n, int k);
     void tiled_linear(const Tensor& a, const Tensor& w, const Tensor& out, Epilogue epilogue, float eps,
                       const Tensor* stats, int stat_blocks, const Tensor* bias, const Tensor* stats_out,
                       const Tensor* out_bf16, const QkvTail* qkv = nullptr);
@@ -440,6 +442,9 @@ public:
     void forget_rope_tables(const void* inv_freq);
 
 private:
+    // sums of tiled products whose K is cut over workgroups, and the tiles' counts of them (of this stream's launches,
+    // which come one after the other)
+    DeviceBuffer tile_parts_, tile_counts_;
     std::unique_ptr<BlasLt> blaslt_;
     DeviceBuffer argmax_state_;
     std::map<std::pair<const void*, int>, std::shared_ptr<DeviceTensor>> rope_tables_;

@@ -8,6 +8,7 @@ struct TileParams {
     const bf16* w;          // [streams * stream_rows, ldw]; stream s starts at row s * stream_rows
     int ldw;
     int stream_rows;
+    long long w_block;      // 0; or (residual) w is packed, [K/32, rows, 32], w_block values from one block of 32 values of k to the next
     const float* bias;      // optional [streams * stream_rows]
     const float* stats;     // optional partial sums of squares [M, stats_ld], n_stat_blocks valid a row
     int n_stat_blocks, stats_ld;
@@ -19,6 +20,9 @@ struct TileParams {
     int ld_bf16;
     float* stats_out;       // residual: [M, stats_ld_out], one partial sum per tile column and row; or null
     int stats_ld_out;
+    float* parts;           // residual, packed weights: room for the sums of slices of K (celeg_gemm_tiles_split_bytes), and
+    int* arrived;           // 256 zeros that the launch leaves as zeros; or null.  Of one stream's launches.
+    int k_slices;           // (set by the launch)
     // The q/k/v epilogue: the columns are heads of 64, q_heads query heads, then kv_heads key
     // heads, then kv_heads value heads.  Query heads are normalised (weight, eps; null: not),
     // turned by their row's position (cos_sin [positions, 32, 2]; null: not) and stored to out;
