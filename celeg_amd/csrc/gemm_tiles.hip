@@ -938,7 +938,8 @@ extern "C" void celeg_gemm_tiles_force_dies(int dies_m) { g_force_dies_m = dies_
     X(7, 128, 192, 4, 2, 3, 0) \
     X(8, 128, 128, 4, 2, 2, 0) \
     X(9, 256, 192, 4, 2, 2, 64) \
-    X(10, 256, 288, 4, 2, 2, 64)
+    X(10, 256, 288, 4, 2, 2, 64) \
+    X(11, 256, 256, 4, 2, 2, 64)
 
 #define TILE_ROWS(ID, BM, BN, WGM, WGN, STAGES, KB) BM,
 #define TILE_COLUMNS(ID, BM, BN, WGM, WGN, STAGES, KB) BN,
@@ -947,7 +948,7 @@ static const int k_shape_bn[] = {TILE_SHAPES(TILE_COLUMNS)};
 #undef TILE_ROWS
 #undef TILE_COLUMNS
 static constexpr int N_TILE_SHAPES = sizeof(k_shape_bm) / sizeof(k_shape_bm[0]);
-extern "C" int celeg_gemm_tiles_shapes() { return N_TILE_SHAPES; }      // (how many there are to force)
+extern "C" int celeg_gemm_tiles_shapes() { return N_TILE_SHAPES - 1; }      // (how many there are to force, ahead of the square one)
 
 // How the dies share the grid of tiles: every row of tiles of A is read by 8 / m dies, every column of
 // tiles of W by m of them; the split with the fewest bytes read of those that leave no die more tiles than it
@@ -1023,33 +1024,37 @@ static TileShape tile_shape(int M, int N, int K, int streams, bool may_split = f
         //   64x128 on 4 wavefronts, two a compute unit, before 128x128 on 8, one: 2 to 6 % faster, up to 10 Mi weights;
         //   with more than the dies' L2s hold beside the rows (2,048 x 8,192, 4,096 x 4,096) 10 to 25 % slower
         //   128x128, two a compute unit, before 256x192: w1 with w3 at 800 rows 23.2 us against 27.5
-        //   256x192 before more than two of 128x128: 1 to 27 % faster in all of 45
-        //   256x288 likewise, where the work of a round pays for its long first loads and its end: values of k x tiles
-        //   of 128x128 from 1,152 Ki on 12 % faster to 2 % slower (29), below 5 to 20 % slower (12; w1 with w3 at
-        //   1,400 rows 39.7 us against 37.1)
-        const auto tiles = [&](int bm, int bn) {
-            return static_cast<long long>((M + bm - 1) / bm) * ((static_cast<long long>(N) * streams + bn - 1) / bn);
-        };
-        const auto fits = [&](int bm, int bn, int on_a_unit) {
-            return dies_of((M + bm - 1) / bm, (N * streams + bn - 1) / bn, M, N * streams).per_die <= DIE_UNITS * on_a_unit;
+        const auto fits = [&](int bm, int bn) {
+            return dies_of((M + bm - 1) / bm, (N * streams + bn - 1) / bn, M, N * streams).per_die <= DIE_UNITS;
         };
         const long long weights = static_cast<long long>(N) * streams * K;
-        if (fits(32, 64, 1)) id = 0;
-        else if (fits(64, 64, 1)) id = 1;
-        else if (K >= 2048 && fits(128, 64, 1)) id = 2;
-        else if (fits(64, 128, 1)) id = 3;
-        else if (fits(64, 192, 1)) id = 4;
-        else if (fits(128, 128, 1)) id = weights <= (10 << 20) ? 5 : 6;
-        else if (fits(128, 192, 1)) id = 7;
-        else if (fits(128, 128, 2)) id = 8;
-        else if (fits(256, 192, 1)) id = 9;
-        else if (fits(256, 288, 1) && K * tiles(128, 128) >= (1152 << 10)) id = 10;
+        if (fits(32, 64)) id = 0;
+        else if (fits(64, 64)) id = 1;
+        else if (K >= 2048 && fits(128, 64)) id = 2;
+        else if (fits(64, 128)) id = 3;
+        else if (fits(64, 192)) id = 4;
+        else if (fits(128, 128)) id = weights <= (10 << 20) ? 5 : 6;
         else {
-            // More than a round: 128x128 with two workgroups a compute unit, or 256x288, one a compute unit, where
-            // the rounds of them (2.2 times as long as a round of 128x128 tiles, measured at 1,024 and 2,048 values
-            // of k) cover the product in less time.
-            const long long rounds288 = (tiles(256, 288) + 255) / 256, rounds128 = (tiles(128, 128) + 511) / 512;
-            id = rounds288 * 22 < rounds128 * 10 ? 10 : 8;
+            // Beyond that the tile whose rounds cover the product in the least time.  A round (on the die with the most
+            // tiles) takes, in us, SwiGLU at 1,024 | 2,048 values of k: 128x192 17.5 | 29.5, 128x128, two a compute unit,
+            // 20.5 | 38.5, 256x192 26 | 45, 256x256 30.8 | 56, 256x288 34 | 60.  Of these five, at 512 to 4,096 rows of
+            // 6,144 x 2,048, 9,216 x 1,024, 12,288 x 1,536 and 16,384 x 2,048, the sums choose the fastest or one within 3 %
+            // in all of 36.  16,384 x 2,048: 2,048 rows 111.9 us in two rounds of 256x256 (128x128 150, 256x288 119.3), 1,200
+            // rows 87.0 in two of 256x192 (100), 4,096 rows 228 (322, 245); 9,216 x 1,024 at 1,500 rows 31.5 in one of 256x256
+            // (39.4 in two of 128x128).
+            struct Cost { int id, on_a_unit; long long fixed, per_k; };      // tenths of us a round and 1,024 values of k
+            static constexpr Cost costs[] = {{7, 1, 55, 120}, {8, 2, 25, 180}, {9, 1, 70, 190}, {11, 1, 85, 230}, {10, 1, 110, 240}};
+            long long best = -1;
+            for (const Cost& c : costs) {
+                const int bm = k_shape_bm[c.id], bn = k_shape_bn[c.id];
+                const int per_die = dies_of((M + bm - 1) / bm, (N * streams + bn - 1) / bn, M, N * streams).per_die;
+                const long long rounds = (per_die + DIE_UNITS * c.on_a_unit - 1) / (DIE_UNITS * c.on_a_unit);
+                const long long cost = rounds * (1024 * c.fixed + c.per_k * K);
+                if (best < 0 || cost < best) {
+                    best = cost;
+                    id = c.id;
+                }
+            }
         }
     }
     return TileShape{id, k_shape_bm[id], k_shape_bn[id], 1};

@@ -478,10 +478,9 @@ struct Runtime {
     // through the tiled products with the norm, SwiGLU and residual sum folded in, wider ones
     // through the library's products with separate norm and activation kernels.  The default is
     // what was measured on whole prefills of 2,048 tokens: at a width of 1,024 the tiled path
-    // takes 2.33 ms against 2.72 ms, at 2,048 the library's products run at 1.2 PFLOP/s and win
-    // (5.5 against 6.2 ms and 9.3 against 11.0 ms for 16 and 30 layers).  0: always the library;
-    // a large number: always the tiles.
+    // takes 2.33 ms against 2.72 ms.  0: always the library; a large number: always the tiles.
     long long tiled_max_width = 1024;
+    bool tiled_by_rows = false;         // wider streams by the step's rows (fused::tiled_step); where nobody has chosen one or the other
     int fused_max_rows = -1;            // -1: by the kernels' own limits
     // how many partial sums of squares of the stream's rows are valid (0: none), and whether
     // the stream's bfloat16 copy is; whoever writes the stream another way resets them
