@@ -596,6 +596,7 @@ const std::vector<Knob>& knobs() {
         {"portion_graph_min_tokens", [](LoadedModel& m) { return m.runner->portion_graph_min_tokens; },
          [](LoadedModel& m, int v) { m.runner->portion_graph_min_tokens = v; }},
         {"use_fused", [](LoadedModel& m) { return m.rt->use_fused ? 1 : 0; }, [](LoadedModel& m, int v) { m.rt->use_fused = v != 0; }},
+        {"wanted_rows_only", [](LoadedModel& m) { return m.rt->wanted_rows_only ? 1 : 0; }, [](LoadedModel& m, int v) { m.rt->wanted_rows_only = v != 0; }},
         {"defer_prologue", [](LoadedModel& m) { return m.rt->defer_prologue ? 1 : 0; }, [](LoadedModel& m, int v) { m.rt->defer_prologue = v != 0; }},
         // (use_tiled_products: 1 = always, 0 = never; tiled_max_width is the rule itself)
         {"use_tiled_products", [](LoadedModel& m) { return m.model->spec.hidden_size <= m.rt->tiled_max_width ? 1 : 0; },

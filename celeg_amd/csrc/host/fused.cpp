@@ -208,9 +208,35 @@ void norm_linear(Runtime& rt, const Tensor& h, const Norm::Foldable& norm, const
     rt.ops.fused_linear(h, w, out, args);
 }
 
+// Leaves all rows but the wanted ones (Runtime::wanted): rt.wanted.stream gets theirs of h, and the result is theirs of `a`
+// (nothing where there is no `a`), laid out as products of so few rows read them where `operand` says that one does.
+Tensor keep_wanted_rows(Runtime& rt, const Tensor& h, const Tensor& a, bool operand) {
+    Runtime::WantedRows& wanted = rt.wanted;
+    wanted.pending = false;
+    const long long width = h.shape[1], room = std::max(wanted.n, STAT_COLUMNS);     // (one size for all steps of few)
+    wanted.stream = rt.ws.buf("wanted_stream", DType::F32, {room, width}).rows(0, wanted.n);
+    rt.stream_stat_blocks = 0;
+    rt.stream_has_bf16 = false;
+    Tensor few;
+    if (a.defined() && operand && rt.dtype == DType::BF16) few = operand_rows(rt, "wanted_operand", wanted.n, a.shape[1], {});
+    else if (a.defined()) few = rt.ws.buf("wanted_branch", rt.dtype, {room, a.shape[1]}).rows(0, wanted.n);
+    rt.ops.gather_rows(h, a.defined() ? &a : nullptr, wanted.rows, wanted.n, wanted.stream, few.defined() ? &few : nullptr);
+    return few;
+}
+
 void linear_into_stream(Runtime& rt, const Tensor& a, const Tensor& w, const Tensor& h, const Tensor* bias) {
     const int T = static_cast<int>(h.shape[0]);
     const long long width = h.shape[1];
+    if (rt.wanted.pending && a.ndim == 2) {
+        if (rt.wanted.n == 0) return;
+        StepBatch few;
+        few.n_tokens = rt.wanted.n;
+        if (fused_rows_ok(rt, few, {width, a.shape[1]}) || fused_f32_ok(rt, few, {width, a.shape[1]})) {
+            const Tensor rows = keep_wanted_rows(rt, h, a, true);
+            linear_into_stream(rt, rows, w, rt.wanted.stream, bias);
+            return;
+        }
+    }
     if (rt.dtype == DType::F32) {
         FusedArgs args;
         args.epilogue = Epilogue::Residual;

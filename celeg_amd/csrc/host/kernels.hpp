@@ -209,6 +209,8 @@ int celeg_normed_mean(const void* a, int lda, const float* wa, const void* b, in
                       void* out, int dtype, int rows, int width, hipStream_t stream);
 int celeg_depth_mix(float* history, size_t entry_stride, float* h, const float* w, int n, int rows, int width, hipStream_t stream);
 int celeg_stream_add(float* h, const float* rows, const float* vec, int n_rows, int width, hipStream_t stream);
+int celeg_gather_rows(const int* rows, int n, const float* h, float* h_out, int width, const void* a, long long lda, void* a_out,
+                      long long lda_out, long long k8_stride, int inner, int dtype, hipStream_t stream);
 int celeg_softcap(float* x, size_t n, float cap, hipStream_t stream);
 // conv_rope.hip
 int celeg_conv_rope_store(const void* proj, int ld, int dtype, const float* conv_w, const float* conv_state, size_t state_stride,

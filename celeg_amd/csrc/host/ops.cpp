@@ -144,6 +144,32 @@ void Ops::scale(const Tensor& x, float factor) {
 }
 
 // ---------------------------------------------------------------------------- several residual streams
+// Rows rows[0 .. n) of h to h_out and of a, if given, to a_out (rows one after the other, or side by side inside every group of 8
+// values).  The row numbers are the caller's: below the number of rows of h.
+void Ops::gather_rows(const Tensor& h, const Tensor* a, const int* rows, int n, const Tensor& h_out, const Tensor* a_out) {
+    dev(h, "h", DType::F32);
+    dev(h_out, "h_out", DType::F32);
+    need(rows && n > 0 && h.ndim == 2 && h_out.ndim == 2 && h.shape[1] == h_out.shape[1] && h_out.shape[0] >= n && !a == !a_out,
+         "gather_rows: the rows do not fit");
+    long long lda = 0, lda_out = 0, k8 = 8, inner = 0;
+    if (a) {
+        dev(*a, "a", a->dtype, false);
+        dev(*a_out, "a_out", a->dtype, false);
+        inner = a->shape[1];
+        const bool side = a_out->ndim == 3;
+        need(a->ndim == 2 && a->shape[0] == h.shape[0] && a->stride[1] == 1 && a_out->shape[0] >= n &&
+             (side ? a_out->shape[1] * 8 == inner && a_out->shape[2] == 8 && a_out->stride[2] == 1
+                   : a_out->ndim == 2 && a_out->shape[1] == inner && a_out->stride[1] == 1),
+             "gather_rows: a and its rows do not fit");
+        lda = a->stride[0];
+        lda_out = a_out->stride[0];
+        if (side) k8 = a_out->stride[1];
+    }
+    kernel_check(celeg_gather_rows(rows, n, h.as<float>(), h_out.as<float>(), static_cast<int>(h.shape[1]), a ? a->data : nullptr, lda,
+                                   a ? a_out->data : nullptr, lda_out, k8, static_cast<int>(inner), a ? dt(*a, "a") : CELEG_F32, stream),
+                 "gather_rows");
+}
+
 void Ops::streams_spread(const Tensor& h, const Tensor& xs, int streams) {
     dev(h, "h", DType::F32);
     dev(xs, "xs", DType::F32);

@@ -163,6 +163,7 @@ public:
                      const Tensor& out, const Tensor* xb, const Tensor* stats);
     void scale(const Tensor& x, float factor);     // x *= factor, 32-bit x
     // several residual streams: xs [rows, streams * width] 32-bit
+    void gather_rows(const Tensor& h, const Tensor* a, const int* rows, int n, const Tensor& h_out, const Tensor* a_out);
     void streams_spread(const Tensor& h, const Tensor& xs, int streams);
     void streams_sum(const Tensor& xs, const Tensor& h, int streams);
     // One sub-layer boundary of a row's streams: if y is given, every stream becomes
@@ -493,6 +494,17 @@ struct Runtime {
     bool leave_sum = false;
     PendingSum pending_sum;
     PendingSum take_pending_sum() { return std::exchange(pending_sum, PendingSum{}); }
+    // The last entry of the run order: of what its mixer adds and of its feed-forward, only the rows whose logits the step
+    // wants are looked at by anyone.  pending: nobody has left the other rows yet; stream: the wanted rows' stream [n, width],
+    // defined once somebody has (whoever does goes on with it instead of the step's rows).
+    struct WantedRows {
+        bool pending = false;
+        const int* rows = nullptr;
+        int n = 0;
+        Tensor stream;
+    };
+    WantedRows wanted;
+    bool wanted_rows_only = true;
     // the step's prologue, left by the runner for the embedding's kernel to take along
     // (defer_prologue); whoever cannot take it along calls flush_prologue() before its own work
     bool defer_prologue = true;

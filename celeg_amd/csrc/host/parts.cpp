@@ -1225,6 +1225,7 @@ public:
         const Norm::Foldable* fold1 = mixer_norm_->foldable();
         const Norm::Foldable* fold2 = has_ffn_ ? ffn_norm_->foldable() : nullptr;
         const bool fusable = fold1 && (fold2 || !has_ffn_);
+        const bool only_wanted = rt.wanted.pending;
         Tensor mixed;
         if (fusable && !delta.defined() && mixer_->forward_fused(h, *fold1, batch, cache, rt)) {
             // the stream holds the mixer's sum already
@@ -1235,18 +1236,27 @@ public:
         }
         rt.mark("mixer " + mixer_->spec.kind);
         if (!has_ffn_) return mixed;          // (undefined where the mixer wrote the stream itself)
-        if (fusable && !mixed.defined() && ffn_->forward_fused(h, *fold2, batch, rt)) {
-            rt.mark("ffn " + ffn_->spec.kind);
-            return Tensor();
+        if (!only_wanted) return feed(h, mixed, normed, fusable ? fold2 : nullptr, batch, rt);
+        if (rt.wanted.n == 0) return Tensor();          // (nobody looks at the stream any more)
+        if (rt.wanted.pending) mixed = fused::keep_wanted_rows(rt, h, mixed, false);      // (the mixer has not)
+        StepBatch few;
+        few.n_tokens = few.n_seqs = rt.wanted.n;
+        return feed(rt.wanted.stream, mixed, normed.rows(0, rt.wanted.n), fusable ? fold2 : nullptr, few, rt);
+    }
+    bool takes_wanted_rows() const override { return has_ffn_; }
+
+private:
+    // the feed-forward on the rows of h (mixed: what the mixer adds to them, where it has not done so itself)
+    Tensor feed(const Tensor& h, const Tensor& mixed, const Tensor& normed, const Norm::Foldable* fold, const StepBatch& batch, Runtime& rt) {
+        Tensor out;
+        if (!(fold && !mixed.defined() && ffn_->forward_fused(h, *fold, batch, rt))) {
+            rt.stream_stat_blocks = 0;
+            ffn_norm_->forward(h, normed, rt, mixed.defined() ? &mixed : nullptr, nullptr);
+            out = ffn_->forward(normed, batch, rt);
         }
-        rt.stream_stat_blocks = 0;
-        ffn_norm_->forward(h, normed, rt, mixed.defined() ? &mixed : nullptr, nullptr);
-        Tensor out = ffn_->forward(normed, batch, rt);
         rt.mark("ffn " + ffn_->spec.kind);
         return out;
     }
-
-private:
     std::unique_ptr<Norm> mixer_norm_;
     std::unique_ptr<Mixer> mixer_;
     bool has_ffn_;

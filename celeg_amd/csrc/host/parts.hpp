@@ -166,6 +166,8 @@ public:
     virtual Tensor forward(const Tensor& h, const Tensor& delta, const StepBatch& batch, const LayerCache& cache, Runtime& rt) = 0;
     // whether forward() makes the addition that the block before it left in rt.pending_sum
     virtual bool takes_pending_sum() const { return false; }
+    // whether the block, as the last entry of the run order, goes on with the wanted rows alone (Runtime::wanted)
+    virtual bool takes_wanted_rows() const { return false; }
 };
 
 // ---------------------------------------------------------------------------- registries
@@ -233,6 +235,7 @@ void norm_linear(Runtime& rt, const Tensor& h, const Norm::Foldable& norm, const
 // h += a w^T, leaving the partial sums of squares of the new rows (and, for few rows, the
 // stream's bfloat16 copy)
 void linear_into_stream(Runtime& rt, const Tensor& a, const Tensor& w, const Tensor& h, const Tensor* bias = nullptr);
+Tensor keep_wanted_rows(Runtime& rt, const Tensor& h, const Tensor& a, bool operand);
 }  // namespace fused
 
 }  // namespace celeg

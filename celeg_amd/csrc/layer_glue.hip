@@ -98,6 +98,31 @@ __global__ void depth_mix_kernel(float* __restrict__ history, size_t entry_strid
     h[at] = fmaf(w[n - 1], last, sum);
 }
 
+// Row rows[r] of h to row r of h_out and, where there is an a, its row likewise (in groups of 8 values k8_stride apart); one
+// workgroup a row.  8 values a piece: every load of a row of up to 2,048 values is asked for at once.  What bounds it is one trip
+// to memory for the row's number and one for the row (one row of 1,024 values and 1,024 of the branch: 3.0 us with its launch).
+template <typename T, bool WIDE>
+__global__ __launch_bounds__(256) void gather_rows_kernel(const int* __restrict__ rows, const float* __restrict__ h, float* __restrict__ h_out,
+                                                          int width, const T* __restrict__ a, size_t lda, T* __restrict__ a_out,
+                                                          size_t lda_out, size_t k8_stride, int inner) {
+    const int r = blockIdx.x;
+    const size_t from = rows[r];
+    const float* const hr = h + from * width;
+    float* const ho = h_out + static_cast<size_t>(r) * width;
+    const T* const ar = a + from * lda;
+    T* const ao = a_out + r * lda_out;
+    if constexpr (WIDE) {
+        typedef float f32x4 __attribute__((ext_vector_type(4)));
+        struct alignas(16) Eight { T v[8]; };
+        for (int i = threadIdx.x; i < width / 4; i += 256) reinterpret_cast<f32x4*>(ho)[i] = reinterpret_cast<const f32x4*>(hr)[i];
+        for (int i = threadIdx.x; i < inner / 8; i += 256)
+            *reinterpret_cast<Eight*>(ao + i * k8_stride) = *reinterpret_cast<const Eight*>(ar + 8 * i);
+    } else {
+        for (int i = threadIdx.x; i < width; i += 256) ho[i] = hr[i];
+        for (int i = threadIdx.x; i < inner; i += 256) ao[(i >> 3) * k8_stride + (i & 7)] = ar[i];
+    }
+}
+
 // h[t, :] += (rows[t, :] +) vec, all 32-bit: what a stream takes in before a run of a looped range
 __global__ void stream_add_kernel(float* __restrict__ h, const float* __restrict__ rows, const float* __restrict__ vec, int width) {
     const int t = blockIdx.y;
@@ -186,6 +211,27 @@ extern "C" int celeg_stream_add(float* h, const float* rows, const float* vec, i
     if (n_rows <= 0 || (!rows && !vec)) return 0;
     dim3 grid((width + 255) / 256, n_rows), block(256);
     hipLaunchKernelGGL(stream_add_kernel, grid, block, 0, stream, h, rows, vec, width);
+    return CELEG_LAUNCH_RESULT();
+}
+
+extern "C" int celeg_gather_rows(const int* rows, int n, const float* h, float* h_out, int width, const void* a, long long lda, void* a_out,
+                                 long long lda_out, long long k8_stride, int inner, int dtype, hipStream_t stream) {
+    if (n <= 0) return 0;
+    if (width <= 0 || inner < 0 || (inner > 0 && (!a || !a_out))) return static_cast<int>(hipErrorInvalidValue);
+    dim3 grid(n), block(256);
+    const auto on16 = [](const void* p, long long row_bytes) { return ((reinterpret_cast<uintptr_t>(p) | static_cast<uintptr_t>(row_bytes)) & 15) == 0; };
+    const long long size = dtype == CELEG_F32 ? 4 : 2;
+    const bool wide = on16(h, width * 4LL) && on16(h_out, 0) && inner % 8 == 0 && on16(a, lda * size) && on16(a_out, lda_out * size) &&
+                      on16(nullptr, k8_stride * size);
+#define LG_GATHER(T, WIDE)                                                                                                     \
+    hipLaunchKernelGGL((gather_rows_kernel<T, WIDE>), grid, block, 0, stream, rows, h, h_out, width, static_cast<const T*>(a),     \
+                       static_cast<size_t>(lda), static_cast<T*>(a_out), static_cast<size_t>(lda_out), static_cast<size_t>(k8_stride), inner)
+    if (dtype == CELEG_F32) {
+        if (wide) LG_GATHER(float, true); else LG_GATHER(float, false);
+    } else {
+        if (wide) LG_GATHER(bf16, true); else LG_GATHER(bf16, false);
+    }
+#undef LG_GATHER
     return CELEG_LAUNCH_RESULT();
 }
 

@@ -1,0 +1,79 @@
+"""The last layer's feed-forward for the wanted rows of a step alone: the logits against the plain implementation and against
+the pass over all rows, and the kernel that takes the rows out."""
+import ctypes
+
+import pytest
+import torch
+
+import plain_lfm2 as plain
+from helpers import assert_close, random_tokens
+from kernel_ops import HipOps
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,n,width,inner,side", [(70, 1, 64, 64, False), (70, 33, 64, 192, True), (9, 4, 1024, 4608, True), (65, 65, 6, 10, False),
+                                                  (3, 5, 2052, 8, False), (300, 64, 1028, 2056, True)])
+def test_rows_taken_out(dtype, T, n, width, inner, side):
+    lib = HipOps()._lib("layer_glue")
+    gen = torch.Generator().manual_seed(T * n)
+    h = torch.randn(T, width, generator=gen).to(DEV)
+    a = torch.randn(T, inner + 8, generator=gen).to(dtype).to(DEV)[:, :inner]       # (rows of a wider matrix)
+    rows = torch.randint(0, T, (n,), generator=gen, dtype=torch.int32).to(DEV)
+    h_out = torch.full((n + 1, width), 7.0, device=DEV)
+    a_out = torch.full((inner // 8, n + 1, 8) if side else (n + 1, inner), 7.0, dtype=dtype, device=DEV)
+    ld, k8 = (8, (n + 1) * 8) if side else (inner, 8)
+    p, ll = ctypes.c_void_p, ctypes.c_longlong
+    rc = lib.celeg_gather_rows(p(rows.data_ptr()), n, p(h.data_ptr()), p(h_out.data_ptr()), width, p(a.data_ptr()), ll(inner + 8),
+                               p(a_out.data_ptr()), ll(ld), ll(k8), inner, 0 if dtype == torch.float32 else 1,
+                               p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0
+    got = a_out.permute(1, 0, 2).reshape(n + 1, inner) if side else a_out
+    assert torch.equal(h_out[:n], h[rows.long()]) and bool((h_out[n] == 7).all())
+    assert torch.equal(got[:n], a[rows.long()]) and bool((got[n] == 7).all())
+
+
+# entries (tokens, wanted places from the end) of the steps of one run: portions without wanted rows, single tokens beside
+# prompts, several places of one entry, and (65 rows, 33 wanted) a step that keeps all rows
+STEPS = [[(0, 70, [])], [(0, 66, [1]), (1, 40, [1, 2, 40])], [(2, 129, [129, 1]), (0, 1, [1]), (1, 1, [1])], [(3, 65, list(range(1, 34)))],
+         [(3, 160, list(range(1, 77)))]]
+
+
+@pytest.mark.parametrize("dtype,last,width,backend", [("bfloat16", "conv", 128, "auto"), ("bfloat16", "full_attention", 128, "auto"),
+                                                      ("bfloat16", "conv", 128, "library"), ("float32", "full_attention", 128, "auto"),
+                                                      ("float32", "conv", 192, "auto")])
+def test_logits_of_the_wanted_rows(tmp_path, dtype, last, width, backend):
+    from celeg_amd.engine import StepEntry, load_model
+    from celeg_amd.weights import write_random_model
+    config = {"architectures": ["Lfm2ForCausalLM"], "vocab_size": 320, "hidden_size": width, "num_hidden_layers": 3,
+              "layer_types": ["conv", "full_attention", last], "num_attention_heads": width // 64, "num_key_value_heads": 1, "head_dim": 64,
+              "intermediate_size": 448, "block_auto_adjust_ff_dim": False, "rope_theta": 10000.0, "conv_L_cache": 3, "conv_bias": False,
+              "tie_word_embeddings": True, "norm_eps": 1e-5, "max_position_embeddings": 512, "eos_token_id": 7}
+    folder = write_random_model(config, str(tmp_path), seed=5, dtype=getattr(torch, dtype), std=0.05)
+    cfg, W = plain.load_model_folder(folder)
+    results = []
+    for only in (0, 1):
+        lm = load_model(folder, dtype=dtype, page_tokens=16, n_pages=80, max_requests=4, max_batched_tokens=512, gemm_backend=backend)
+        lm.set_knob("wanted_rows_only", only)
+        slots, tokens, seen = {}, {i: random_tokens(320, 400, seed=60 + i) for i in range(4)}, {}
+        for step in STEPS:
+            entries, want = [], []
+            for request, n, from_end in step:
+                slot = slots.setdefault(request, lm.cache.open() if request not in slots else None)
+                pos = seen.get(request, 0)
+                assert lm.cache.prepare(slot, pos, n)
+                entries.append(StepEntry(slot, pos, tokens[request][pos:pos + n], [n - k for k in from_end]))
+                want += [(request, pos + n - k) for k in from_end]
+                seen[request] = pos + n
+            got = lm.runner.step(entries)
+            assert got.shape[0] == len(want)
+            results.append((only, got.clone(), want))
+        lm.close()
+    whole = {r: plain.model_logits(cfg, W, tokens[r]) for r in range(4)}
+    for only, got, want in results:
+        if not want:
+            continue
+        ref = torch.stack([whole[r][at] for r, at in want])
+        assert_close(got, ref, dtype, f"{dtype}/{last}/{backend}/wanted only {only}")
