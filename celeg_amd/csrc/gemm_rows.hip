@@ -8,7 +8,7 @@
 // Epilogues: store | store of an activation | 32-bit store | add into the 32-bit residual stream, refresh its
 // bfloat16 copy and leave partial sums of squares | SwiGLU of a gate and an up stream |
 // the double-gated short convolution of a B, a C and an x stream for one new token per
-// request, with its state update.
+// request, with its state update | the same over all rows of the requests of a step (E_CONV_ROWS).
 //
 // Layout.  At these sizes the weights are read once from memory and the rows of A come
 // from cache.  A workgroup owns CT tiles of 16 columns (of every weight stream), for MT tiles
@@ -46,7 +46,7 @@
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float floatx4_t __attribute__((ext_vector_type(4)));
 
-enum { E_STORE = 0, E_STORE_F32 = 1, E_RESIDUAL = 2, E_SWIGLU = 3, E_CONV = 4, E_ACT = 5 };
+enum { E_STORE = 0, E_STORE_F32 = 1, E_RESIDUAL = 2, E_SWIGLU = 3, E_CONV = 4, E_ACT = 5, E_CONV_ROWS = 6 };
 #define ROWS_MAX_TAPS 8
 #define ROWS_MAX_STAT_BLOCKS 512
 #define ROWS_MAX_LDS (128 * 1024)
@@ -57,6 +57,7 @@ __device__ __forceinline__ float round_bf16(float x) { return to_float(from_floa
 template <int EPI> struct Streams { static constexpr int n = 1; };
 template <> struct Streams<E_SWIGLU> { static constexpr int n = 2; };
 template <> struct Streams<E_CONV> { static constexpr int n = 3; };
+template <> struct Streams<E_CONV_ROWS> { static constexpr int n = 3; };
 
 // Most wavefronts of a workgroup: what LDS holds of their tiles (a power of two, up to 16).
 constexpr int rows_max_waves(int mt, int sc) {
@@ -144,6 +145,45 @@ __device__ __forceinline__ float finish_output(const GemvParams& p, int r, int n
     return 0.f;
 }
 
+// The short convolution over the rows of a step whose rows are all the workgroup's: the sums of its columns' B, C and x are
+// rounded to bfloat16, as where they are a tensor of their own; B x of every row waits in LDS for the rows behind it, and what lies
+// ahead of a request's first row comes from its state, which is written when everybody has read it.  Sums start at the bias and
+// positions before 0 add nothing, as in the kernel of the convolution alone: the same bits, but for the rows' 1/rms, whose partial
+// sums are added by as many threads as a workgroup has for a row.
+// What it saves is that kernel, at these sizes a launch and two trips to memory (24 rows of 1,024 channels 3.4 us), and
+// its rows' way to memory and back; what it costs is that every workgroup reads all rows of A for its columns, 4 of 1,024, where
+// the product alone shares rows out too (24 rows 7.2 us against 4.4 and 3.4; 64 rows no gain: conv_rows_pay).
+struct ConvRow {
+    int first, last, start;
+    float* state;           // entry 0 of the request's state at the column
+};
+__device__ __forceinline__ ConvRow conv_row(const GemvParams& p, int seq, int n) {
+    return ConvRow{p.cu_seqlens[seq], p.cu_seqlens[seq + 1], p.seq_start[seq],
+                   p.state + static_cast<size_t>(p.seq_slot[seq]) * p.state_slot_stride + n};
+}
+__device__ __forceinline__ void conv_rows_out(const GemvParams& p, const ConvRow& at, int r, int n, const float* bx, int bx_ld, float gate) {
+    float conv = p.conv_b ? p.conv_b[n] : 0.f;
+    const int i = r - at.first;
+    for (int tap = 0; tap < p.taps; ++tap) {
+        const int back = p.taps - 1 - tap;
+        if (at.start + i < back) continue;
+        const float v = i >= back ? bx[(r - back) * bx_ld] : at.state[static_cast<size_t>(i - back + p.taps) * p.N];
+        conv = fmaf(p.conv_w[static_cast<size_t>(n) * p.taps + tap], v, conv);
+    }
+    static_cast<bf16*>(p.out)[static_cast<size_t>(r) * p.ldo + static_cast<size_t>(n >> 3) * p.out_k8_stride + (n & 7)] =
+        from_float<bf16>(gate * conv);
+}
+// (entry k of the new state is B x of the request's row rows - taps + k, or an old entry that lies behind entry k)
+__device__ __forceinline__ void conv_rows_state(const GemvParams& p, const ConvRow& at, const float* bx, int bx_ld) {
+    for (int k = 0; k < p.taps; ++k) {
+        const int from = at.last - at.first - p.taps + k;
+        float v = 0.f;
+        if (from >= 0) v = bx[(at.first + from) * bx_ld];
+        else if (at.start + from >= 0) v = at.state[static_cast<size_t>(from + p.taps) * p.N];
+        at.state[static_cast<size_t>(k) * p.N] = v;
+    }
+}
+
 // MT: tiles of 16 rows; CT: tiles of 16 columns per weight stream; blockDim.x / 64
 // wavefronts split K.  LDS: [waves][MT][streams * CT][4][64] floats, then MT*16 scales.
 template <int MT, int CT, int EPI>
@@ -167,12 +207,15 @@ void gemm_rows_kernel(const void* const a_, const bf16* const w_, const int* con
     float* const s_scale = smem + static_cast<size_t>(n_waves) * MT * SC * 256;
     // (E_STORE_F32 with row_best: the best logit of every 16 columns of a row, [ROWS][CT])
     unsigned long long* const s_best = reinterpret_cast<unsigned long long*>(s_scale + ROWS);
+    float* const s_bx = s_scale + ROWS;        // (E_CONV_ROWS: B x, then C, of every row and column)
     // the wavefront's number as a scalar: the branches on its range of k are then uniform
     // ones (the matrix instructions do not honour a lane mask)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int n0 = blockIdx.x * cols;
     const int row0 = blockIdx.y * ROWS;        // the workgroup's first row
     const int c16 = lane & 15, q = lane >> 4;
+
+    const int conv_seq = EPI == E_CONV_ROWS ? p.token_seq[min(static_cast<int>(threadIdx.x) / COLS, M - 1)] : 0;
 
     // ---- operands: A rows t*16 + c16, W columns n0 + ct*16 + c16 of every stream
     const bf16* arow[MT];
@@ -224,6 +267,9 @@ void gemm_rows_kernel(const void* const a_, const bf16* const w_, const int* con
 
     // ---- what the end of this thread's first output needs (asked for behind the first weights)
     const int e0 = min(static_cast<int>(threadIdx.x), ROWS * COLS - 1);
+    // (the request of the row of this thread's first output: its number has come with the first weights)
+    ConvRow conv0{};
+    if constexpr (EPI == E_CONV_ROWS) conv0 = conv_row(p, conv_seq, min(n0 + e0 % COLS, N - 1));
     const Early<EPI> early0 = early_fetch<EPI>(p, min(row0 + e0 / COLS, M - 1), min(n0 + e0 % COLS, N - 1));
 
     // ---- the rows' 1/rms from the partial sums of squares (likewise): LPR neighbouring
@@ -285,6 +331,14 @@ void gemm_rows_kernel(const void* const a_, const bf16* const w_, const int* con
 #pragma unroll
         for (int s = 0; s < NS; ++s) sum[s] *= scale;
         float v = 0.f;
+        if constexpr (EPI == E_CONV_ROWS) {
+            float part[NS];
+#pragma unroll
+            for (int s = 0; s < NS; ++s) part[s] = round_bf16(sum[s] + (p.bias ? p.bias[static_cast<size_t>(s) * p.stream_rows + nc] : 0.f));
+            s_bx[e] = part[0] * part[2];
+            s_bx[ROWS * COLS + e] = part[1];
+            continue;
+        }
         if (e == static_cast<int>(threadIdx.x)) {
             if (ok) v = finish_output<EPI>(p, rc, nc, sum, early0);
         } else if (ok) {
@@ -299,6 +353,19 @@ void gemm_rows_kernel(const void* const a_, const bf16* const w_, const int* con
             // this loop's reads of the partial sums would wait behind); the tiles meet below
             const unsigned long long b = group_best_logit<16>(v, ok, n0 + (j & ~15));
             if (jj == 0) s_best[rl * CT + ct] = b;
+        }
+    }
+    if constexpr (EPI == E_CONV_ROWS) {
+        __syncthreads();
+        for (int pass = 0; pass < 2; ++pass) {
+            for (int e = threadIdx.x; e < ROWS * COLS; e += n_threads) {
+                const int r = e / COLS, j = e % COLS, n = n0 + j;      // (row0 is 0)
+                if (r >= M || n >= N || j >= cols) continue;
+                const ConvRow at = e == static_cast<int>(threadIdx.x) ? conv0 : conv_row(p, p.token_seq[r], n);
+                if (pass == 0) conv_rows_out(p, at, r, n, s_bx + j, COLS, s_bx[ROWS * COLS + e]);
+                else if (r == at.last - 1) conv_rows_state(p, at, s_bx + j, COLS);
+            }
+            __syncthreads();        // (every old state has been read)
         }
     }
     if (EPI == E_STORE_F32 && p.row_best) {
@@ -334,8 +401,14 @@ static int g_force_ct = 0, g_force_waves = 0, g_force_mt = 0, g_force_cols = 0;
 extern "C" void celeg_gemm_rows_force(int ct, int waves, int mt) { g_force_ct = ct; g_force_waves = waves; g_force_mt = mt; }
 extern "C" void celeg_gemm_rows_force_cols(int cols) { g_force_cols = cols; }
 
-static RowsShape rows_shape(int M, int N, int K, int streams) {
+static RowsShape rows_shape(int M, int N, int K, int streams, bool all_rows = false) {
     RowsShape s;
+    if (all_rows) {      // every workgroup all rows (three streams): columns by halves down to a workgroup a compute unit
+        s = RowsShape{M <= 16 ? 1 : (M <= 32 ? 2 : 4), 1, 8, 16};
+        while (s.cols > 4 && (N + s.cols / 2 - 1) / (s.cols / 2) <= ROWS_COMPUTE_UNITS) s.cols >>= 1;
+        while (s.waves > 1 && s.waves * 2 > K / 32) s.waves >>= 1;
+        return s;
+    }
     const int max_mt = M <= 16 ? 1 : (M <= 32 ? 2 : 4);
     s.mt = max_mt;
     const int max_ct = streams == 1 ? 4 : (streams == 2 ? 2 : 1);
@@ -395,7 +468,8 @@ static int launch_rows(const GemvParams& params, int waves, int cols, hipStream_
     GemvParams p = params;
     p.cols = cols;
     const size_t lds = static_cast<size_t>(waves) * MT * NS * CT * 1024 + MT * 16 * sizeof(float) +
-                       (p.row_best ? static_cast<size_t>(MT) * 16 * CT * sizeof(unsigned long long) : 0);
+                       (p.row_best ? static_cast<size_t>(MT) * 16 * CT * sizeof(unsigned long long) : 0) +
+                       (EPI == E_CONV_ROWS ? static_cast<size_t>(MT) * 16 * CT * 16 * 2 * sizeof(float) : 0);
     static bool raised = false;              // once per instantiation: more LDS than the default limit
     if (lds > 48 * 1024 && !raised) {
         hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_rows_kernel<MT, CT, EPI>),
@@ -414,7 +488,7 @@ static int launch_rows(const GemvParams& params, int waves, int cols, hipStream_
 template <int EPI>
 static int launch_epilogue(const GemvParams& p, hipStream_t stream) {
     constexpr int NS = Streams<EPI>::n;
-    const RowsShape s = rows_shape(p.M, p.N, p.K, NS);
+    const RowsShape s = rows_shape(p.M, p.N, p.K, NS, EPI == E_CONV_ROWS);
 #define ROWS_CASE(MT_, CT_) \
     if (s.mt == MT_ && s.ct == CT_) return launch_rows<MT_, CT_, EPI>(p, s.waves, s.cols, stream);
     ROWS_CASE(1, 1) ROWS_CASE(2, 1) ROWS_CASE(4, 1)
@@ -466,6 +540,11 @@ extern "C" int celeg_gemm_rows(const GemvParams* params, int epi, hipStream_t st
         case E_SWIGLU: return launch_epilogue<E_SWIGLU>(p, stream);
         case E_CONV: return launch_epilogue<E_CONV>(p, stream);
         case E_ACT: return launch_epilogue<E_ACT>(p, stream);
+        case E_CONV_ROWS:
+            // (taps: a row's way through LDS and state has no limit of its own; the operands of requests are all there)
+            if (p.taps < 1 || p.stream_rows != p.N || p.rows || !p.token_seq || !p.cu_seqlens || !p.seq_start || !p.seq_slot || !p.conv_w || !p.state)
+                return static_cast<int>(hipErrorInvalidValue);
+            return launch_epilogue<E_CONV_ROWS>(p, stream);
         default: return static_cast<int>(hipErrorInvalidValue);
     }
 }

@@ -64,6 +64,8 @@ struct GemvParams {
     //   n * w_row_stride + (k / 32) * w_kb_stride + (k % 32 / 8) * w_q_stride + k % 8
     long long a_k8_stride, out_k8_stride, bf16_k8_stride, w_q_stride;
     int row_best_ld, row_best_rows;     // (room for row_best_rows rows of row_best_ld parts: a launch that would leave more is refused)
+    // E_CONV_ROWS: every row's request, the requests' first rows [n + 1] and first positions (seq_slot is [n] then)
+    const int *token_seq, *cu_seqlens, *seq_start;
 };
 static_assert(offsetof(GemvParams, M) == 64 && offsetof(GemvParams, conv_w) == 128 && offsetof(GemvParams, a_k8_stride) == 192,
               "the fields of GemvParams are grouped by 64-byte lines");

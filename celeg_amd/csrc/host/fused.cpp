@@ -154,7 +154,7 @@ void norm_linear(Runtime& rt, const Tensor& h, const Norm::Foldable& norm, const
         return;
     }
     if (extras.qkv) throw KernelError("norm_linear: the q/k/v tail goes with steps of many rows");
-    const int streams = epilogue == Epilogue::Swiglu ? 2 : epilogue == Epilogue::Conv ? 3 : 1;
+    const int streams = epilogue == Epilogue::Swiglu ? 2 : epilogue == Epilogue::Conv || epilogue == Epilogue::ConvRows ? 3 : 1;
     const bool streamed = rt.ops.rows_kernel_ok(M, {width});
     FusedArgs args;
     args.epilogue = epilogue;

@@ -1748,6 +1748,16 @@ bool Ops::rows_kernel_ok(int rows, std::initializer_list<long long> inner) const
     return true;
 }
 
+// Every workgroup then reads all rows for its columns: worth it up to 32 rows, and up to 64 where a workgroup a compute unit has 8
+// columns (2,048 of them).  A whole step of one prompt, us, apart | inside:
+//   rows             9           16          17          24          32          33          48            64
+//   1,024 wide   541 | 505   523 | 510   530 | 523   534 | 526   548 | 536   579 | 587   597 | 602     620 | 613 (621 in another run)
+//   2,048 wide   836 | 800   820 | 801   858 | 845   866 | 851   905 | 888   997 | 976  1,021 | 1,000  1,083 | 1,065
+// (fewer than 9 rows: another kernel.)
+bool Ops::conv_rows_pay(int rows, long long width) const {
+    return use_conv_rows && rows_kernel_ok(rows, {width}) && (rows <= 32 || width >= 2048);
+}
+
 int Ops::residual_stat_blocks(int rows, int n, int k) const {
     if (rows_kernel_ok(rows, {k})) return celeg_gemm_rows_blocks(rows, n, k, static_cast<int>(Epilogue::Residual));
     if (rows <= 16 && use_sliced) return celeg_gemv_slices_blocks(rows, n, k);
@@ -1874,7 +1884,8 @@ void Ops::fused_linear_f32(const Tensor& a, const Tensor& w, const Tensor& out, 
 void Ops::fused_linear(const Tensor& a, const Tensor& w, const Tensor& out, const FusedArgs& args) {
     dev(w, "w", DType::BF16);
     const Epilogue epi = args.epilogue;
-    const int streams = epi == Epilogue::Swiglu ? 2 : epi == Epilogue::Conv ? 3 : 1;
+    const bool conv_rows = epi == Epilogue::ConvRows;
+    const int streams = epi == Epilogue::Swiglu ? 2 : epi == Epilogue::Conv || conv_rows ? 3 : 1;
     const bool packed = args.packed;
     need(!packed || (w.ndim == 3 && w.shape[2] == 32), "fused_linear: a packed weight is [K/32, rows, 32]");
     need(packed || w.ndim == 2, "fused_linear: w must be a matrix");
@@ -1962,13 +1973,18 @@ void Ops::fused_linear(const Tensor& a, const Tensor& w, const Tensor& out, cons
             prm.stats_ld_out = static_cast<int>(args.stats_out.stride[0]);
         }
     }
-    if (epi == Epilogue::Conv) {
+    if (epi == Epilogue::Conv || conv_rows) {
         need(args.conv != nullptr, "fused_linear: the convolution epilogue needs its operands");
         const ConvOperands& c = *args.conv;
         dev(c.taps, "conv taps", DType::F32);
         dev(c.state, "state", DType::F32, false);
         const long long L = c.taps.shape[1];
-        need(L <= 8, "fused_linear: the convolution epilogue holds up to 8 taps, not " + std::to_string(L));
+        need(conv_rows || L <= 8, "fused_linear: the convolution epilogue holds up to 8 taps, not " + std::to_string(L));
+        need(!conv_rows || (streamed && !args.rows && c.token_seq && c.cu_seqlens && c.seq_start),
+             "fused_linear: the convolution over the rows of a step goes with the kernel for 9 to 64 rows and the requests' places");
+        prm.token_seq = c.token_seq;
+        prm.cu_seqlens = c.cu_seqlens;
+        prm.seq_start = c.seq_start;
         need(c.taps.shape[0] == N && c.state.ndim == 3 && c.state.shape[1] == L && c.state.shape[2] == N &&
                  c.state.stride[1] == N && c.state.stride[2] == 1 && c.seq_slot,
              "fused_linear: convolution operands do not fit");

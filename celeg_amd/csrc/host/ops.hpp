@@ -22,7 +22,7 @@
 
 namespace celeg {
 
-enum class Epilogue : int { Store = 0, StoreF32 = 1, Residual = 2, Swiglu = 3, Conv = 4, Activation = 5 };
+enum class Epilogue : int { Store = 0, StoreF32 = 1, Residual = 2, Swiglu = 3, Conv = 4, Activation = 5, ConvRows = 6 };
 
 // An activation behind a product (see Ops::activation_bias)
 struct Activation {
@@ -60,7 +60,8 @@ struct ConvOperands {
     Tensor taps;          // [N, L] 32-bit
     Tensor bias;          // optional [N]
     Tensor state;         // [slots, L, N] 32-bit, the slots a fixed number of elements apart
-    const int* seq_slot = nullptr;   // [M]
+    const int* seq_slot = nullptr;   // [M]; ConvRows: [requests]
+    const int *token_seq = nullptr, *cu_seqlens = nullptr, *seq_start = nullptr;     // ConvRows: of the step's rows and requests
 };
 
 struct FusedArgs {
@@ -150,6 +151,7 @@ public:
     bool use_qkv_tail = true;          // q/k/v products of many rows take norm, rotation and cache write along
     bool use_fresh_decode = true;      // decode-only steps: the attention prepares and writes the new keys and values
     bool use_head_argmax = true;       // greedy rows without a penalty: the token from what the head left beside the logits
+    bool use_conv_rows = true;           // the short convolution over the rows of a step of 9 to 64 inside the product ahead of it
     int rows_kernel_min_rows = 9, tiles_min_rows = 65, fused_linear_shape = 0;
     int last_stat_blocks = 0, last_best_parts = 0, last_best_cols = 0;
 
@@ -413,6 +415,8 @@ public:
     // fused skinny products
     bool fused_linear_ok(int rows, std::initializer_list<long long> inner) const;
     bool rows_kernel_ok(int rows, std::initializer_list<long long> inner) const;
+    // whether the short convolution over the rows of a step goes into the product ahead of it (Epilogue::ConvRows)
+    bool conv_rows_pay(int rows, long long width) const;
     int residual_stat_blocks(int rows, int n, int k) const;
     void stream_prepare(const Tensor& h, const Tensor& xb, const Tensor& stats);
     // (with `prologue`: the step's block-table updates and token ids from the device in the same launch)

@@ -730,8 +730,8 @@ public:
         rt.ops.linear(y, w_out_->view, out, b_out_ ? &b_out_->view : nullptr, rt.ws);
         return out;
     }
-    // h += mixer(norm(h)) with the norm, the convolution (for one new token per request) and the
-    // residual addition folded into the two products
+    // h += mixer(norm(h)) with the norm, the convolution (for one new token per request, and for the rows of steps of
+    // 9 to 64) and the residual addition folded into the two products
     bool forward_fused(const Tensor& h, const Norm::Foldable& norm, const StepBatch& batch, const LayerCache& cache,
                        Runtime& rt) override {
         if (!(fused::fused_rows_ok(rt, batch, {width_}) || fused::fused_f32_ok(rt, batch, {width_})) || w_in_->view.dtype != rt.dtype ||
@@ -741,15 +741,20 @@ public:
         fused::LinearExtras extras;
         if (b_in_) extras.bias = b_in_->view;
         Tensor y;
-        if (batch.decode_only && batch.n_seqs == T && taps_ <= 8 && !fused::tiled_step(rt, T, width_)) {   // the fused form holds 8 taps
+        const bool singles = batch.decode_only && batch.n_seqs == T && taps_ <= 8;      // (that form holds 8 taps)
+        const bool rows = !singles && rt.dtype == DType::BF16 && rt.ops.conv_rows_pay(T, width_);
+        if ((singles || rows) && !fused::tiled_step(rt, T, width_)) {
             y = rt.dtype == DType::F32 ? rt.ws.buf("conv_y", rt.dtype, {T, width_}) : fused::operand_rows(rt, "conv_y_fused", T, width_, {width_});
             ConvOperands conv;
             conv.taps = taps_view_;
             if (b_conv_) conv.bias = b_conv_->view;
             conv.state = cache.states.at("bx");
             conv.seq_slot = batch.seq_slot;
+            conv.token_seq = batch.token_seq;
+            conv.cu_seqlens = batch.cu_seqlens;
+            conv.seq_start = batch.seq_start;
             extras.conv = &conv;
-            fused::norm_linear(rt, h, norm, w_in_->view, y, Epilogue::Conv, extras);
+            fused::norm_linear(rt, h, norm, w_in_->view, y, rows ? Epilogue::ConvRows : Epilogue::Conv, extras);
         } else {
             y = rt.ws.buf("conv_y", rt.dtype, {T, width_});
             Tensor bcx = rt.ws.buf("conv_bcx", rt.dtype, {T, 3 * width_});
