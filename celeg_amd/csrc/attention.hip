@@ -103,11 +103,14 @@ __global__ __launch_bounds__(ROPE_WAVES * CELEG_WAVE) void qk_norm_rope_store_ke
     }
 }
 
-// The same for head sizes 32, 64 and 128 with rotation over the whole head (or none) and
+// The same for head sizes 32, 64 and 128 with rotation by halves over the whole head (or none) and
 // the table of cosines and sines: LPH = head_dim / 4 lanes share a head, a lane holds 4
 // neighbouring values, a wavefront 64 / LPH heads of one row.  The sum of squares is
 // reduced inside the LPH lanes, and the rotation's partner (the value half a head away) sits
 // in lane ^ (LPH / 2), so nothing goes through LDS.
+// PART: the rotation takes the head's first 2 * `half` values (a multiple of 8: a lane's four are all of one half or all behind);
+// a partner then sits half / 4 lanes away.  The kernel above has a wavefront a head and two bytes a lane, for any rotation: 2,048 rows
+// of 16 + 8 + 8 heads of 64, half of a head rotated, 23 us there and 10.4 to 12 here; 4 rows 2.5 and 2.2.
 template <typename T> struct Quad;
 template <> struct Quad<float> {
     typedef float raw __attribute__((ext_vector_type(4)));
@@ -136,15 +139,16 @@ template <> struct Quad<bf16> {
 // anything is used: a row's chain of position -> page -> address is three trips to memory, and a
 // thread that has one row only spends its time waiting for them (2,048 rows: 13.6 us a layer
 // with one row a thread).
-template <typename T, int LPH, int TOKENS>
+template <typename T, int LPH, int TOKENS, bool PART>
 __global__ __launch_bounds__(ROPE_WAVES * CELEG_WAVE) void qk_norm_rope_store_quad_kernel(
     T* __restrict__ q, int ldq, const T* __restrict__ k, int ldk, const T* __restrict__ v, int ldv,
     const float* __restrict__ q_weight, const float* __restrict__ k_weight, float eps,
     const float* __restrict__ cos_sin, const int* __restrict__ positions,
     const int* __restrict__ token_slot, const int* __restrict__ table, int table_stride,
     T* __restrict__ k_pool, T* __restrict__ v_pool, int n_layers, int layer, int page_tokens,
-    int q_heads, int kv_heads, int n_heads, int n_tokens) {
-    constexpr int HD = 4 * LPH, HPW = CELEG_WAVE / LPH, HALF = HD / 2;
+    int q_heads, int kv_heads, int n_heads, int n_tokens, int half) {
+    constexpr int HD = 4 * LPH, HPW = CELEG_WAVE / LPH;
+    const int HALF = PART ? half : HD / 2;
     const int wave = threadIdx.x / CELEG_WAVE, lane = threadIdx.x % CELEG_WAVE;
     const int head_raw = (blockIdx.y * ROPE_WAVES + wave) * HPW + lane / LPH;
     const bool live_head = head_raw < n_heads;
@@ -156,7 +160,9 @@ __global__ __launch_bounds__(ROPE_WAVES * CELEG_WAVE) void qk_norm_rope_store_qu
     const float* weight = is_q ? q_weight : (is_k ? k_weight : nullptr);
     float w[4] = {1.f, 1.f, 1.f, 1.f};
     if (weight) Quad<float>::load(weight + d0, w);
-    const bool rotate = cos_sin && (is_q || is_k);
+    const bool rotate = cos_sin && (is_q || is_k) && (!PART || d0 < 2 * HALF);
+    const bool first = d0 < HALF;
+    const int partner = PART ? lane + (rotate ? (first ? HALF / 4 : -HALF / 4) : 0) : 0;
 
     int t[TOKENS], pos[TOKENS], page[TOKENS];
     float x[TOKENS][4], cs[TOKENS][8];
@@ -215,9 +221,9 @@ __global__ __launch_bounds__(ROPE_WAVES * CELEG_WAVE) void qk_norm_rope_store_qu
         float y[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const float other = __shfl_xor(x[i][e], LPH / 2, CELEG_WAVE);
+            const float other = PART ? __shfl(x[i][e], partner, CELEG_WAVE) : __shfl_xor(x[i][e], LPH / 2, CELEG_WAVE);
             // first half: a c - b s with b the partner; second half: b c + a s with a the partner
-            y[e] = rotate ? (l < LPH / 2 ? x[i][e] * cs[i][2 * e] - other * cs[i][2 * e + 1]
+            y[e] = rotate ? (first ? x[i][e] * cs[i][2 * e] - other * cs[i][2 * e + 1]
                                          : x[i][e] * cs[i][2 * e] + other * cs[i][2 * e + 1])
                           : x[i][e];
         }
@@ -236,26 +242,26 @@ __global__ __launch_bounds__(ROPE_WAVES * CELEG_WAVE) void qk_norm_rope_store_qu
     }
 }
 
-template <typename T, int LPH>
+template <typename T, int LPH, bool PART>
 static int launch_rope_quad(T* q, int ldq, const T* k, int ldk, const T* v, int ldv,
                             const float* q_weight, const float* k_weight, float eps,
                             const float* cos_sin, const int* positions, const int* token_slot,
                             const int* table, int table_stride, T* k_pool, T* v_pool, int n_layers,
                             int layer, int page_tokens, int n_tokens, int q_heads, int kv_heads,
-                            int n_heads, hipStream_t stream) {
+                            int n_heads, int half, hipStream_t stream) {
     const int per_block = ROPE_WAVES * (CELEG_WAVE / LPH);
     const unsigned head_blocks = (n_heads + per_block - 1) / per_block;
     // four rows a thread once there are enough of them to fill the chip that way
     if (static_cast<long long>(n_tokens) * head_blocks >= 4 * 1024) {
-        hipLaunchKernelGGL((qk_norm_rope_store_quad_kernel<T, LPH, 4>), dim3((n_tokens + 3) / 4, head_blocks),
+        hipLaunchKernelGGL((qk_norm_rope_store_quad_kernel<T, LPH, 4, PART>), dim3((n_tokens + 3) / 4, head_blocks),
                            dim3(ROPE_WAVES * CELEG_WAVE), 0, stream, q, ldq, k, ldk, v, ldv, q_weight, k_weight, eps,
                            cos_sin, positions, token_slot, table, table_stride, k_pool, v_pool, n_layers, layer,
-                           page_tokens, q_heads, kv_heads, n_heads, n_tokens);
+                           page_tokens, q_heads, kv_heads, n_heads, n_tokens, half);
     } else {
-        hipLaunchKernelGGL((qk_norm_rope_store_quad_kernel<T, LPH, 1>), dim3(n_tokens, head_blocks),
+        hipLaunchKernelGGL((qk_norm_rope_store_quad_kernel<T, LPH, 1, PART>), dim3(n_tokens, head_blocks),
                            dim3(ROPE_WAVES * CELEG_WAVE), 0, stream, q, ldq, k, ldk, v, ldv, q_weight, k_weight, eps,
                            cos_sin, positions, token_slot, table, table_stride, k_pool, v_pool, n_layers, layer,
-                           page_tokens, q_heads, kv_heads, n_heads, n_tokens);
+                           page_tokens, q_heads, kv_heads, n_heads, n_tokens, half);
     }
     return CELEG_LAUNCH_RESULT();
 }
@@ -266,17 +272,21 @@ static int rope_quad_dispatch(void* q, int ldq, const void* k, int ldk, const vo
                               const float* cos_sin, const int* positions, const int* token_slot,
                               const int* table, int table_stride, void* k_pool, void* v_pool,
                               int n_layers, int layer, int page_tokens, int n_tokens, int q_heads,
-                              int kv_heads, int head_dim, int n_heads, hipStream_t stream) {
-#define CELEG_ROPE_QUAD(LPH_)                                                                     \
-    return launch_rope_quad<T, LPH_>(static_cast<T*>(q), ldq, static_cast<const T*>(k), ldk,      \
+                              int kv_heads, int head_dim, int n_heads, int half, hipStream_t stream) {
+#define CELEG_ROPE_QUAD_OF(LPH_, PART_)                                                           \
+    return launch_rope_quad<T, LPH_, PART_>(static_cast<T*>(q), ldq, static_cast<const T*>(k), ldk,      \
                                      static_cast<const T*>(v), ldv, q_weight, k_weight, eps,      \
                                      cos_sin, positions, token_slot, table, table_stride,         \
                                      static_cast<T*>(k_pool), static_cast<T*>(v_pool), n_layers,  \
-                                     layer, page_tokens, n_tokens, q_heads, kv_heads, n_heads, stream)
+                                     layer, page_tokens, n_tokens, q_heads, kv_heads, n_heads, half, stream)
+#define CELEG_ROPE_QUAD(LPH_)                                                                     \
+    if (cos_sin && 2 * half != head_dim) { CELEG_ROPE_QUAD_OF(LPH_, true); }                       \
+    CELEG_ROPE_QUAD_OF(LPH_, false)
     if (head_dim == 32) { CELEG_ROPE_QUAD(8); }
     if (head_dim == 64) { CELEG_ROPE_QUAD(16); }
     CELEG_ROPE_QUAD(32);
 #undef CELEG_ROPE_QUAD
+#undef CELEG_ROPE_QUAD_OF
 }
 
 // cos and sin of position * inv_freq[i] for positions 0 .. n_positions-1, interleaved:
@@ -312,8 +322,9 @@ extern "C" int celeg_qk_norm_rope_store(
     if (pairing != 0 && pairing != 1) return static_cast<int>(hipErrorInvalidValue);
     const int n_heads = q_heads + (store_kv ? 2 * kv_heads : 0);
     const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-    const bool whole_rotation = !inv_freq || (cos_sin && rotary_dim == head_dim && pairing == 0);
-    if ((head_dim == 32 || head_dim == 64 || head_dim == 128) && whole_rotation && ldq % 4 == 0 &&
+    // (no rotation, or by halves of which each is whole lanes of four)
+    const bool lane_rotation = !inv_freq || (cos_sin && rotary_dim > 0 && rotary_dim <= head_dim && rotary_dim % 8 == 0 && pairing == 0);
+    if ((head_dim == 32 || head_dim == 64 || head_dim == 128) && lane_rotation && ldq % 4 == 0 &&
         (!store_kv || (ldk % 4 == 0 && ldv % 4 == 0 && aligned(k) && aligned(v))) && aligned(q) &&
         aligned(k_pool) && aligned(v_pool) && (!q_weight || aligned(q_weight)) && (!k_weight || aligned(k_weight)) &&
         (!cos_sin || aligned(cos_sin))) {
@@ -322,11 +333,11 @@ extern "C" int celeg_qk_norm_rope_store(
             return rope_quad_dispatch<float>(q, ldq, k, ldk, v, ldv, q_weight, k_weight, eps, cs,
                                              positions, token_slot, table, table_stride, k_pool, v_pool,
                                              n_layers, layer, page_tokens, n_tokens, q_heads, kv_heads,
-                                             head_dim, n_heads, stream);
+                                             head_dim, n_heads, rotary_dim / 2, stream);
         return rope_quad_dispatch<bf16>(q, ldq, k, ldk, v, ldv, q_weight, k_weight, eps, cs, positions,
                                         token_slot, table, table_stride, k_pool, v_pool, n_layers,
                                         layer, page_tokens, n_tokens, q_heads, kv_heads, head_dim,
-                                        n_heads, stream);
+                                        n_heads, rotary_dim / 2, stream);
     }
     dim3 grid(n_tokens, (n_heads + ROPE_WAVES - 1) / ROPE_WAVES), block(ROPE_WAVES * CELEG_WAVE);
     const size_t lds = static_cast<size_t>(ROPE_WAVES) * head_dim * sizeof(float);
