@@ -1798,17 +1798,28 @@ public:
         else rt.ops.norm_step(h, delta.defined() ? &delta : nullptr, nullptr, &of(*mixer_norm_), &normed);
         Tensor y = mixer_->forward(normed, batch, cache, rt);
         rt.mark("mixer " + mixer_->spec.kind);
+        Tensor stream = h;
+        StepBatch few;
+        const bool only_wanted = rt.wanted.pending;
+        if (only_wanted) {
+            if (rt.wanted.n == 0) return Tensor();          // (nobody looks at the stream any more)
+            y = fused::keep_wanted_rows(rt, h, y, false);
+            stream = rt.wanted.stream;
+            normed = normed.rows(0, rt.wanted.n);
+            few.n_tokens = few.n_seqs = rt.wanted.n;
+        }
         if (has_ffn_) {
-            rt.ops.norm_step(h, &y, &of(*mixer_post_), &of(*ffn_norm_), &normed, nullptr, gain_);
-            y = ffn_->forward(normed, batch, rt);
+            rt.ops.norm_step(stream, &y, &of(*mixer_post_), &of(*ffn_norm_), &normed, nullptr, gain_);
+            y = ffn_->forward(normed, only_wanted ? few : batch, rt);
         }
         const Ops::NormParams& post = of(has_ffn_ ? *ffn_post_ : *mixer_post_);
         if (rt.leave_sum) rt.pending_sum = PendingSum{y, &post, gain_};
-        else rt.ops.norm_step(h, &y, &post, nullptr, nullptr, nullptr, gain_);
+        else rt.ops.norm_step(stream, &y, &post, nullptr, nullptr, nullptr, gain_);
         if (has_ffn_) rt.mark("ffn " + ffn_->spec.kind);
         return Tensor();
     }
     bool takes_pending_sum() const override { return true; }
+    bool takes_wanted_rows() const override { return has_ffn_; }
 
 private:
     static const Ops::NormParams& of(const Norm& norm) {
