@@ -86,6 +86,102 @@ __global__ __launch_bounds__(CELEG_WAVE) void delta_prepare_kernel(
     for (int d = lane; d < D; d += CELEG_WAVE) dst[d] *= inv;     // (a lane reads what it wrote itself)
 }
 
+// The same for keys of 16 to 256 values (a power of two) and up to four taps: a thread has four neighbouring channels of DP_TOKENS
+// rows, reads a row once for all the taps that use it, and the D / 4 lanes of a head share its sum.  A wavefront a row and head with two
+// bytes a lane (above) reads every row once a tap: 2,048 rows of 2,048 channels (24 MB read and written) 33 us there and 17.5
+// here.
+#define DP_TOKENS 4
+#define DP_TAPS 4
+// The sum of a head's squares: up to 64 values in the order of wave_sum over a wavefront that holds one a lane (far halves first), so
+// that a row's bits do not hang on how many rows its step has; more values in any order.
+template <int LPH>
+__device__ __forceinline__ float dp_head_sum(float a, float b, float c, float d) {
+#pragma clang fp contract(off)
+    float s[4] = {a * a, b * b, c * c, d * d};
+    if (LPH > 16) return lanes_sum<LPH>((s[0] + s[2]) + (s[1] + s[3]));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if (LPH == 16) {
+            s[e] += lane_move<LANES_ROTATE_8>(s[e]);
+            s[e] += lane_move<LANES_ROTATE_4>(s[e]);      // (the row of 16 repeats after 8)
+            s[e] += lane_move<LANES_XOR_2>(s[e]);
+            s[e] += lane_move<LANES_XOR_1>(s[e]);
+        } else {
+            for (int off = LPH / 2; off > 0; off >>= 1) s[e] += __shfl_xor(s[e], off, CELEG_WAVE);
+        }
+    }
+    return (s[0] + s[2]) + (s[1] + s[3]);
+}
+
+template <typename T, int LPH>
+__global__ __launch_bounds__(256) void delta_prepare_quad_kernel(
+    const T* __restrict__ proj, int ld, int col_b, int col_a, const float* __restrict__ conv_w, const float* __restrict__ a_log,
+    const float* __restrict__ dt_bias, const float* __restrict__ conv_state, size_t state_stride,
+    const int* __restrict__ positions, const int* __restrict__ token_seq, const int* __restrict__ seq_start,
+    const int* __restrict__ token_slot, float* __restrict__ qk, float* __restrict__ v_out, float* __restrict__ beta_decay, int G,
+    int H, int V, int taps, int n_tokens) {
+    constexpr int D = 4 * LPH;
+    const int t0 = blockIdx.x * DP_TOKENS, n_channels = 2 * G * D + H * V;
+    if (blockIdx.y + 1 == gridDim.y) {          // beta and the decay of every value head
+        for (int idx = threadIdx.x; idx < DP_TOKENS * H; idx += 256) {
+            const int t = t0 + idx / H, h = idx % H;
+            if (t >= n_tokens) break;
+            beta_decay[static_cast<size_t>(t) * 2 * H + h] = dr_sigmoid(to_float(proj[static_cast<size_t>(t) * ld + col_b + h]));
+            if (a_log)
+                beta_decay[static_cast<size_t>(t) * 2 * H + H + h] =
+                    expf(-expf(a_log[h]) * dr_softplus(to_float(proj[static_cast<size_t>(t) * ld + col_a + h]) + dt_bias[h]));
+        }
+        return;
+    }
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    struct alignas(4 * sizeof(T)) Four { T v[4]; };
+    const int c_raw = 4 * (blockIdx.y * 256 + static_cast<int>(threadIdx.x));
+    const bool live = c_raw < n_channels;
+    const int c = live ? c_raw : n_channels - 4;          // (n_channels % 4 == 0)
+    Four rows[DP_TOKENS + DP_TAPS - 1];
+#pragma unroll
+    for (int r = 0; r < DP_TOKENS + DP_TAPS - 1; ++r)     // (rows that no tap reads are asked for all the same, from inside the step)
+        rows[r] = *reinterpret_cast<const Four*>(proj + static_cast<size_t>(min(max(t0 - (DP_TAPS - 1) + r, 0), n_tokens - 1)) * ld + c);
+    float w[4][DP_TAPS];                                  // [channel][rows back]
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int back = 0; back < DP_TAPS; ++back)
+            w[e][back] = back < taps ? conv_w[static_cast<size_t>(c + e) * taps + taps - 1 - back] : 0.f;
+#pragma unroll
+    for (int j = 0; j < DP_TOKENS; ++j) {
+        const int t = t0 + j;
+        if (t >= n_tokens) break;
+        const int i = positions[t] - seq_start[token_seq[t]];        // the row's place among its request's in this step
+        const float* const saved = conv_state + static_cast<size_t>(token_slot[t]) * state_stride + c;
+        f32x4 y{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int back = DP_TAPS - 1; back >= 0; --back) {
+            if (back >= taps) continue;
+            f32x4 x;
+            if (i >= back) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[e] = to_float(rows[DP_TAPS - 1 + j - back].v[e]);
+            } else {
+                x = *reinterpret_cast<const f32x4*>(saved + static_cast<size_t>(taps - 1 + i - back) * n_channels);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e] = fmaf(w[e][back], x[e], y[e]);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = dr_silu(y[e]);
+        const float sum = dp_head_sum<LPH>(y[0], y[1], y[2], y[3]);
+        if (!live) continue;
+        if (c >= 2 * G * D) {
+            *reinterpret_cast<f32x4*>(v_out + static_cast<size_t>(t) * H * V + c - 2 * G * D) = y;
+        } else {          // a unit vector over the head (queries also times D^-1/2)
+            float inv = 1.0f / sqrtf(sum + 1e-6f);
+            if (c < G * D) inv *= 1.0f / sqrtf(static_cast<float>(D));
+            *reinterpret_cast<f32x4*>(qk + static_cast<size_t>(t) * 2 * G * D + c) = y * inv;
+        }
+    }
+}
+
 // per (request of the step, channel): new saved input j is old saved input j + n, or the step's
 // row j + n - (taps - 1) where that is not negative
 template <typename T>
@@ -553,6 +649,30 @@ extern "C" int celeg_delta_prepare(const void* proj, int ld, int dtype, int col_
                                    float* qk, float* v_out, float* beta_decay, int n_tokens, int G, int H, int D, int V, int taps,
                                    hipStream_t stream) {
     if (n_tokens <= 0) return 0;
+    const auto on16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    const int n_channels = 2 * G * D + H * V;
+    // (a whole step of one prompt, us, a wavefront a row and head | quads: 300 rows 809 | 810, 1,100 1,372 | 1,359, 2,048 1,726 | 1,695;
+    // four of 1,100 4,460 | 4,373)
+    if (n_tokens >= 256 && taps <= DP_TAPS && (D == 16 || D == 32 || D == 64 || D == 128 || D == 256) && V % 4 == 0 && ld % 4 == 0 &&
+        state_stride % 4 == 0 && on16(proj) && on16(conv_state) && on16(qk) && on16(v_out)) {
+        dim3 quad_grid((n_tokens + DP_TOKENS - 1) / DP_TOKENS, (n_channels / 4 + 255) / 256 + 1), quad_block(256);
+#define CELEG_DELTA_QUAD(T_, LPH_)                                                                                                   \
+    hipLaunchKernelGGL((delta_prepare_quad_kernel<T_, LPH_>), quad_grid, quad_block, 0, stream, static_cast<const T_*>(proj), ld, col_b, \
+                       col_a, conv_w, a_log, dt_bias, conv_state, state_stride, positions, token_seq, seq_start, token_slot, qk, v_out, \
+                       beta_decay, G, H, V, taps, n_tokens)
+#define CELEG_DELTA_QUADS(T_)                                                              \
+    switch (D) {                                                                           \
+        case 16: CELEG_DELTA_QUAD(T_, 4); break;                                           \
+        case 32: CELEG_DELTA_QUAD(T_, 8); break;                                           \
+        case 64: CELEG_DELTA_QUAD(T_, 16); break;                                          \
+        case 128: CELEG_DELTA_QUAD(T_, 32); break;                                         \
+        default: CELEG_DELTA_QUAD(T_, 64); break;                                          \
+    }
+        if (dtype == CELEG_F32) { CELEG_DELTA_QUADS(float) } else { CELEG_DELTA_QUADS(bf16) }
+#undef CELEG_DELTA_QUADS
+#undef CELEG_DELTA_QUAD
+        return CELEG_LAUNCH_RESULT();
+    }
     dim3 grid(n_tokens, 2 * G + H + 1), block(CELEG_WAVE);
     if (dtype == CELEG_F32)
         hipLaunchKernelGGL(delta_prepare_kernel<float>, grid, block, 0, stream, static_cast<const float*>(proj), ld, col_b, col_a,
