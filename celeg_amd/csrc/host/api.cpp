@@ -600,9 +600,9 @@ const std::vector<Knob>& knobs() {
         {"defer_prologue", [](LoadedModel& m) { return m.rt->defer_prologue ? 1 : 0; }, [](LoadedModel& m, int v) { m.rt->defer_prologue = v != 0; }},
         // (use_tiled_products: 1 = always, 0 = never; tiled_max_width is the rule itself)
         {"use_tiled_products", [](LoadedModel& m) { return m.model->spec.hidden_size <= m.rt->tiled_max_width ? 1 : 0; },
-         [](LoadedModel& m, int v) { m.rt->tiled_max_width = v ? (1LL << 40) : 0; m.rt->tiled_by_rows = false; }},
+         [](LoadedModel& m, int v) { m.rt->tiled_max_width = v ? (1LL << 40) : 0; }},
         {"tiled_max_width", [](LoadedModel& m) { return static_cast<int>(std::min<long long>(m.rt->tiled_max_width, 1 << 30)); },
-         [](LoadedModel& m, int v) { m.rt->tiled_max_width = v; m.rt->tiled_by_rows = false; }},
+         [](LoadedModel& m, int v) { m.rt->tiled_max_width = v; }},
         {"fused_max_rows", [](LoadedModel& m) { return m.rt->fused_max_rows; }, [](LoadedModel& m, int v) { m.rt->fused_max_rows = v; }},
         OPS_INT(attention_decode_whole), OPS_BOOL(use_blaslt), OPS_INT(attention_rows_per_tile), OPS_INT(attention_rows_form),
         OPS_BOOL(attention_general), OPS_BOOL(use_rope_table), OPS_BOOL(use_argmax_parts), OPS_BOOL(use_head_argmax), OPS_BOOL(decode_parts_fill), OPS_BOOL(use_sliced),

@@ -8,21 +8,12 @@ namespace fused {
 // Whether products of `rows` rows that read a stream of this width take the fused path through
 // the tiled products (otherwise they run the library's products with separate norm and activation
 // kernels).  The choice is by the sizes of the products, not by the model: Runtime::tiled_max_width
-// holds the widest stream for which the tiled products were measured faster at any number of rows.
-// Wider streams take them where the step's rows do: the whole prompt of a model with 16 layers, ms with the tiles | the library:
-//   rows           70            300           512          700         1,024       1,300       1,500       1,700       2,048
-//   width 1,536  0.97 | 1.20   1.31 | 1.54  1.55 | 1.78  2.03 | 2.15  2.24 | 2.46             3.18 | 3.42  3.34 | 3.37  3.61 | 3.73
-//   width 2,048  1.20 | 1.42   1.74 | 1.91  2.11 | 2.22  2.68 | 2.75  2.93 | 3.21  4.35 | 4.18 4.56 | 4.28  4.61 | 4.79  4.89 | 5.08
-//   width 2,560  1.43 | 1.59   2.27 | 2.22  2.92 | 2.73  3.10 | 3.24  4.01 | 4.02  5.05 | 4.92             5.84 | 5.95  6.19 | 6.34
-static bool tiled_wide_step(int rows, long long width) {
-    if (width <= 1536) return true;
-    if (width <= 2048) return rows <= 1024 || rows >= 1600;      // (1,100: 3.94 | 3.83; 1,600 4.50 | 4.52)
-    return width <= 2560 && rows <= 256;
-}
-
+// holds the widest stream for which the tiled products were measured faster.  (Whole prompts of wider models are faster on the tiles
+// too at some numbers of rows, width 2,048 2 to 16 % up to 1,024 rows and from 1,600 on; but the weights with a norm's folded in
+// are rounded to bfloat16 once more: logits of three prompts of 1,000 to 2,000 tokens 0.016 of the result away from 64 bits with
+// them and 0.0147 without.  So they stay with the library.)
 bool tiled_step(const Runtime& rt, int rows, long long width) {
-    if (rows <= FUSED_MAX_ROWS || rt.dtype != DType::BF16 || !rt.use_fused) return false;
-    return width <= rt.tiled_max_width || (rt.tiled_by_rows && tiled_wide_step(rows, width));
+    return rows > FUSED_MAX_ROWS && width <= rt.tiled_max_width && rt.dtype == DType::BF16 && rt.use_fused;
 }
 
 // Whether this step's rows can take the fused path through products with these inner sizes.

@@ -685,7 +685,6 @@ std::unique_ptr<LoadedModel> load_model(const std::string& model_dir, const Load
     CELEG_HIP(hipStreamCreate(&lm->stream));
     lm->rt = std::make_unique<Runtime>(dtype, lm->stream);
     // "auto" keeps the runtime's own rule, which goes by the sizes of the products
-    lm->rt->tiled_by_rows = options.gemm_backend == "auto";
     if (options.gemm_backend == "tiles") lm->rt->tiled_max_width = 1LL << 40;
     if (options.gemm_backend == "library") lm->rt->tiled_max_width = 0;
     lm->model = std::make_unique<Model>(described.spec);

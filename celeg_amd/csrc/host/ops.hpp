@@ -485,7 +485,6 @@ struct Runtime {
     // what was measured on whole prefills of 2,048 tokens: at a width of 1,024 the tiled path
     // takes 2.33 ms against 2.72 ms.  0: always the library; a large number: always the tiles.
     long long tiled_max_width = 1024;
-    bool tiled_by_rows = false;         // wider streams by the step's rows (fused::tiled_step); where nobody has chosen one or the other
     int fused_max_rows = -1;            // -1: by the kernels' own limits
     // how many partial sums of squares of the stream's rows are valid (0: none), and whether
     // the stream's bfloat16 copy is; whoever writes the stream another way resets them
