@@ -743,6 +743,8 @@ public:
         Tensor y;
         const bool singles = batch.decode_only && batch.n_seqs == T && taps_ <= 8;      // (that form holds 8 taps)
         const bool rows = !singles && rt.dtype == DType::BF16 && rt.ops.conv_rows_pay(T, width_);
+        // (the operand of steps of 9 to 64 rows exists from any step on: made later, it would have recorded steps recorded again)
+        if (rt.dtype == DType::BF16) fused::operand_rows(rt, "conv_y_fused", fused::FUSED_MAX_ROWS, width_, {width_});
         if ((singles || rows) && !fused::tiled_step(rt, T, width_)) {
             y = rt.dtype == DType::F32 ? rt.ws.buf("conv_y", rt.dtype, {T, width_}) : fused::operand_rows(rt, "conv_y_fused", T, width_, {width_});
             ConvOperands conv;
