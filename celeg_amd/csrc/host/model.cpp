@@ -192,7 +192,7 @@ void Model::bind_cache(const CacheManager& cache) {
 // us).  A whole step, us, all rows | the wanted ones (requests x tokens, one row of each wanted):
 //                1x65         1x128        1x300        1x1,024        8x16         32x4           64x4
 //   350M      777 | 764    820 | 805    953 | 933    1,434 | 1,387   867 | 853   1,170 | 1,151   1,760 | 1,753
-//   1.2B    1,212 | 1,184  1,294 | 1,268  1,760 | 1,707  2,986 | 2,882  1,354 | 1,316  1,739 | 1,712   2,343 | 2,362 (runs differ by 2 %)
+//   1.2B    1,425 | 1,416  1,508 | 1,500  1,949 | 1,911  3,198 | 3,116  1,595 | 1,576   1,990 | 1,996   2,664 | 2,660 (runs differ by 0.5 %)
 // Kifetar, four prompts of 1,100 tokens 4,540 | 4,460.  A prompt of 2,048 tokens 2,112 -> 2,031, 20,001 tokens (whose portions but the last want no row) 27,640 -> 26,700, 64 requests
 // served 122,080 -> 119,250.
 static bool wanted_rows_pay(const Runtime& rt, long long T, long long R) { return rt.wanted_rows_only && T > 64 && 2 * R <= T; }
