@@ -16,9 +16,8 @@ bool tiled_step(const Runtime& rt, int rows, long long width) {
     return rows > FUSED_MAX_ROWS && width <= rt.tiled_max_width && rt.dtype == DType::BF16 && rt.use_fused;
 }
 
-// Whether this step's rows can take the fused path through products with these inner sizes.
-bool fused_rows_ok(const Runtime& rt, const StepBatch& batch, std::initializer_list<long long> inner) {
-    const int rows = batch.n_tokens;
+// Whether so many rows can take the fused path through products with these inner sizes.
+bool rows_ok(const Runtime& rt, int rows, std::initializer_list<long long> inner) {
     long long widest = 0;
     for (long long k : inner) widest = std::max(widest, k);
     if (rows > FUSED_MAX_ROWS)
@@ -31,6 +30,8 @@ bool fused_rows_ok(const Runtime& rt, const StepBatch& batch, std::initializer_l
     if (limit < 0) limit = rt.ops.rows_kernel_ok(rows, inner) ? FUSED_MAX_ROWS : FUSED_MAX_ROWS_OLD_KERNEL;
     return rows <= limit;
 }
+
+bool fused_rows_ok(const Runtime& rt, const StepBatch& batch, std::initializer_list<long long> inner) { return rows_ok(rt, batch.n_tokens, inner); }
 
 bool fused_f32_ok(const Runtime& rt, const StepBatch& batch, std::initializer_list<long long> inner) {
     return rt.dtype == DType::F32 && rt.use_fused && Ops::fused_linear_f32_ok(batch.n_tokens, inner);
@@ -159,7 +160,16 @@ void norm_linear(Runtime& rt, const Tensor& h, const Norm::Foldable& norm, const
     args.row_best_ld = extras.row_best_ld;
     args.row_best_rows = extras.row_best_rows;
     rt.ops.last_best_parts = 0;
-    if (sliced(rt, M, width) && w.dtype == DType::BF16 && (streamed || w.shape[0] / streams <= SLICED_MAX_COLUMNS)) {
+    const bool folds = sliced(rt, M, width) && w.dtype == DType::BF16 && (streamed || w.shape[0] / streams <= SLICED_MAX_COLUMNS);
+    if (folds && extras.as_stored) {
+        const Tensor normed = rt.ws.buf("normed_as_stored", DType::BF16, {STAT_COLUMNS, width}).rows(0, M);
+        rt.ops.rmsnorm(h, norm.weight, norm.eps, normed, nullptr, extras.rows);
+        args.rows = nullptr;
+        args.plain = true;
+        rt.ops.fused_linear(normed, w, out, args);
+        return;
+    }
+    if (folds) {
         // the stream's bfloat16 copy times the weight with the norm's weight folded in, scaled
         // by the rows' 1/rms at the end
         Tensor stats = stream_stats(rt, width);
@@ -187,11 +197,11 @@ void norm_linear(Runtime& rt, const Tensor& h, const Norm::Foldable& norm, const
     if (blocks) args.stats = stream_stats(rt, width);
     args.stat_blocks = blocks;
     if (w.dtype == DType::BF16 && w.ndim == 2 && w.shape[1] % 32 == 0 && w.shape[1] >= 2048 &&
-        w.shape[0] / streams > SLICED_MAX_COLUMNS) {
+        w.shape[0] / streams > SLICED_MAX_COLUMNS && !extras.as_stored) {
         // a product of very many long weight rows (the output head of a wide model): a copy of w in
         // blocks of 32 values of k with the rows side by side, which the kernel reads whole kilobytes
         // of; made once and kept (65,536 rows of 2,048 values at 8 rows: 54.6 against 62.4 us; of 1,024
-        // values: 29.3 against 29.5, not worth a second copy of the table)
+        // values: 29.3 against 29.5, not worth a second copy of the table; nor is a prompt's one product)
         args.packed = true;
         rt.ops.fused_linear(h, packed_weight(rt, w)->view, out, args);
         return;

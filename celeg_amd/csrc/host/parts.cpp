@@ -1105,12 +1105,15 @@ private:
 bool head_fused(const Tensor& h, const Norm::Foldable& norm, const StepBatch& batch, const Tensor& out, Runtime& rt,
                 const Tensor& weight) {
     const int R = batch.n_logit_rows;
-    if (!(weight.defined() && weight.dtype == DType::BF16 && fused::fused_rows_ok(rt, batch, {h.shape[1]}) && R > 0 && R <= 64 &&
+    if (!(weight.defined() && weight.dtype == DType::BF16 && fused::rows_ok(rt, batch.n_tokens, {h.shape[1]}) && R > 0 && R <= 64 &&
           !fused::tiled_step(rt, batch.n_tokens, h.shape[1])))
         return false;
     fused::LinearExtras extras;
     extras.rows = batch.logit_rows;
     extras.n_rows = R;
+    // (steps of many rows read the output table as it is: the rows that are left of one do so too.  With the final norm folded in, the
+    // table is rounded to bfloat16 once more, and there is a second copy of it, also in programs that only classify)
+    extras.as_stored = rt.wanted.stream.defined();
     // beside the logits: the best (logit, index) of every share of a row's columns, from which a
     // greedy row's token follows without the logits being read again
     const int room = Ops::head_best_parts(weight.shape[0]);

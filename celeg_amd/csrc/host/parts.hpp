@@ -206,6 +206,7 @@ constexpr int TILED_MAX_STAT_BLOCKS = 128;
 constexpr int SLICED_MAX_ROWS = 16, SLICED_MAX_STAT_BLOCKS = 512, SLICED_MAX_COLUMNS = 16384;
 
 bool tiled_step(const Runtime& rt, int rows, long long width);
+bool rows_ok(const Runtime& rt, int rows, std::initializer_list<long long> inner);
 bool fused_rows_ok(const Runtime& rt, const StepBatch& batch, std::initializer_list<long long> inner);
 // The same in 32-bit: up to 16 rows, for parts that ask for products with a norm in front (stored, SwiGLU or the short
 // convolution behind) and products into the stream, and nothing else of what is below.
@@ -224,6 +225,7 @@ struct LinearExtras {
     const QkvTail* qkv = nullptr;          // steps of many rows: what follows a q/k/v product, inside its kernel
     unsigned long long* row_best = nullptr;   // an output head's 32-bit store: see FusedArgs
     int row_best_ld = 0, row_best_rows = 0;
+    bool as_stored = false;                // w neither with the norm folded in nor laid out anew: the norm has a kernel of its own there
 };
 // whether norm_linear would take a q/k/v tail for a step of this many rows
 bool qkv_tail_ok(const Runtime& rt, int rows, long long width);

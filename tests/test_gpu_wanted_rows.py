@@ -77,3 +77,71 @@ def test_logits_of_the_wanted_rows(tmp_path, dtype, last, width, backend):
             continue
         ref = torch.stack([whole[r][at] for r, at in want])
         assert_close(got, ref, dtype, f"{dtype}/{last}/{backend}/wanted only {only}")
+
+
+def one_prompt(folder, wanted, T=150, backend="auto"):
+    """One step of a prompt of T tokens with its last `wanted` rows wanted: their logits and what each kernel family launched."""
+    from celeg_amd.engine import StepEntry, load_model
+    lm = load_model(folder, dtype="bfloat16", page_tokens=16, n_pages=40, max_requests=4, max_batched_tokens=512, gemm_backend=backend)
+    tokens = random_tokens(320, T, seed=wanted)
+    slot = lm.cache.open()
+    assert lm.cache.prepare(slot, 0, T)
+    before = lm.knobs()["paths"]
+    got = lm.runner.step([StepEntry(slot, 0, tokens, list(range(T - wanted, T)))]).clone()
+    after = lm.knobs()["paths"]
+    lm.close()
+    return got.double().cpu(), tokens, {k: after[k] - before[k] for k in after}
+
+
+def small_config(width, vocab=320, tied=True, ff=448):
+    return {"architectures": ["Lfm2ForCausalLM"], "vocab_size": vocab, "hidden_size": width, "num_hidden_layers": 2,
+            "layer_types": ["conv", "full_attention"], "num_attention_heads": max(1, width // 64), "num_key_value_heads": 1, "head_dim": 64,
+            "intermediate_size": ff, "block_auto_adjust_ff_dim": False, "rope_theta": 10000.0, "conv_L_cache": 3, "conv_bias": False,
+            "tie_word_embeddings": tied, "norm_eps": 1e-5, "max_position_embeddings": 512, "eos_token_id": 7}
+
+
+# (8 and fewer, 9 to 64 and more rows have kernels of their own; 16,400 columns are more than those of up to 16 rows fold a norm into)
+@pytest.mark.parametrize("wanted", [1, 8, 9, 16, 33, 64, 75])
+@pytest.mark.parametrize("vocab", [320, 16400])
+def test_the_head_reads_the_output_table_as_it_is(tmp_path, wanted, vocab):
+    """Every entry of the table is 1.5 times a power of two and every weight of the final norm 1 + 2^-7: their product lies half way
+    between two bfloat16 numbers and rounds to 1.515625 of that power, 2^-8.6 too much.  Logits from the table as it is have no
+    such bias: what the roundings of the layers leave of one, 2^-8 a value over 128 values of a row and more, is a tenth of it."""
+    from celeg_amd.weights import write_random_model, write_safetensors
+    config = small_config(128, vocab, tied=False)
+    folder = write_random_model(config, str(tmp_path), seed=3, dtype=torch.bfloat16, std=0.05)
+    cfg, W = plain.load_model_folder(folder)
+    gen = torch.Generator().manual_seed(4)
+    signs = torch.randint(0, 2, W["lm_head.weight"].shape, generator=gen) * 2.0 - 1.0
+    W["lm_head.weight"] = (signs * 1.5 * 2.0 ** -torch.randint(3, 6, signs.shape, generator=gen)).double()
+    W["model.embedding_norm.weight"] = torch.full_like(W["model.embedding_norm.weight"], 1 + 2.0 ** -7)
+    write_safetensors(f"{folder}/model.safetensors", {k: v.to(torch.bfloat16) for k, v in W.items()}, metadata={"format": "pt"})
+    got, tokens, _ = one_prompt(folder, wanted)
+    ref = plain.model_logits(cfg, W, tokens)[-wanted:]
+    assert got.shape == ref.shape
+    bias = float((got * ref).sum() / (ref * ref).sum()) - 1
+    assert abs(bias) < 1e-3, bias
+
+
+@pytest.mark.parametrize("dtype,last", [("bfloat16", "conv"), ("bfloat16", "full_attention"), ("float32", "full_attention")])
+@pytest.mark.parametrize("wanted", [9, 16, 17, 33, 64, 65])
+def test_logits_of_9_to_64_wanted_rows(tmp_path, dtype, last, wanted):
+    """As ragged prompts and a server have them: one row of each of so many prompts of 2 to 5 tokens, and a step behind."""
+    from celeg_amd.engine import StepEntry, load_model
+    from celeg_amd.weights import write_random_model
+    config = small_config(128)
+    config["layer_types"] = ["full_attention", last]
+    folder = write_random_model(config, str(tmp_path), seed=6, dtype=getattr(torch, dtype), std=0.05)
+    cfg, W = plain.load_model_folder(folder)
+    lm = load_model(folder, dtype=dtype, page_tokens=16, n_pages=80, max_requests=72, max_batched_tokens=512)
+    tokens = [random_tokens(320, 2 + i % 4 + 2 + (70 if i == 0 else 0), seed=80 + i) for i in range(wanted)]
+    slots, seen = [lm.cache.open() for _ in tokens], [0] * wanted
+    for n in ([len(t) - 2 for t in tokens], [1] * wanted):
+        entries = []
+        for i, slot in enumerate(slots):
+            assert lm.cache.prepare(slot, seen[i], n[i])
+            entries.append(StepEntry(slot, seen[i], tokens[i][seen[i]:seen[i] + n[i]], [n[i] - 1]))
+            seen[i] += n[i]
+        got = lm.runner.step(entries)
+        assert_close(got, torch.stack([plain.model_logits(cfg, W, t[:s])[-1] for t, s in zip(tokens, seen)]), dtype, f"{dtype}/{last}/{wanted}")
+    lm.close()
