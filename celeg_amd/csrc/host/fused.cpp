@@ -31,7 +31,13 @@ bool rows_ok(const Runtime& rt, int rows, std::initializer_list<long long> inner
     return rows <= limit;
 }
 
-bool fused_rows_ok(const Runtime& rt, const StepBatch& batch, std::initializer_list<long long> inner) { return rows_ok(rt, batch.n_tokens, inner); }
+// The same for the rows of a step.  Rows that are left of a step of many (Runtime::wanted) take it only where all of that step's rows
+// do: the fused path multiplies a norm's weight into the product's, which rounds that to bfloat16 once more, and what a prompt's
+// logits are made of does not hang on how many of them are wanted.
+bool fused_rows_ok(const Runtime& rt, const StepBatch& batch, std::initializer_list<long long> inner) {
+    if (rt.wanted.stream.defined() && !rows_ok(rt, rt.wanted.step_rows, inner)) return false;
+    return rows_ok(rt, batch.n_tokens, inner);
+}
 
 bool fused_f32_ok(const Runtime& rt, const StepBatch& batch, std::initializer_list<long long> inner) {
     return rt.dtype == DType::F32 && rt.use_fused && Ops::fused_linear_f32_ok(batch.n_tokens, inner);
@@ -232,7 +238,7 @@ void linear_into_stream(Runtime& rt, const Tensor& a, const Tensor& w, const Ten
         if (rt.wanted.n == 0) return;
         StepBatch few;
         few.n_tokens = rt.wanted.n;
-        if (fused_rows_ok(rt, few, {width, a.shape[1]}) || fused_f32_ok(rt, few, {width, a.shape[1]})) {
+        if (rows_ok(rt, few.n_tokens, {width, a.shape[1]}) || fused_f32_ok(rt, few, {width, a.shape[1]})) {
             const Tensor rows = keep_wanted_rows(rt, h, a, true);
             linear_into_stream(rt, rows, w, rt.wanted.stream, bias);
             return;

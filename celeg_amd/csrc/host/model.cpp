@@ -205,6 +205,7 @@ Tensor Model::forward(const StepBatch& batch, Runtime& rt) {
     rt.stream_stat_blocks = 0;
     rt.stream_has_bf16 = false;
     rt.head_best = HeadBest{};
+    rt.wanted = Runtime::WantedRows{};
     if (!embedding_->takes_step_prologue()) rt.flush_prologue();
     embedding_->forward(batch.token_ids, h, rt, &batch, embedding_cache_);
     rt.flush_prologue();      // (an embedding that said it would and did not)
@@ -236,7 +237,6 @@ Tensor Model::forward(const StepBatch& batch, Runtime& rt) {
     // A block's last addition can wait for the norm of the block behind it, or for the final norm, where nothing
     // else looks at the stream in between.
     rt.pending_sum = PendingSum{};
-    rt.wanted = Runtime::WantedRows{};
     auto norm_follows = [&](size_t i, size_t layer) {
         if (S > 1 || rt.after_layer || token_inputs_[layer] || depth_mixes_[layer] || history.defined()) return false;
         if (i + 1 == spec.order.size()) return final_norm_->params() && !final_norm_->foldable();
@@ -259,6 +259,7 @@ Tensor Model::forward(const StepBatch& batch, Runtime& rt) {
             rt.wanted.pending = true;
             rt.wanted.rows = batch.logit_rows;
             rt.wanted.n = static_cast<int>(R);
+            rt.wanted.step_rows = static_cast<int>(T);
         }
         delta = blocks_[layer]->forward(hs, delta, batch, caches_[i], rt);
         if (token_inputs_[layer] || depth_mixes_[layer] || (history.defined() && static_cast<int>(i) + 1 < history_entries_)) {

@@ -503,7 +503,7 @@ struct Runtime {
     struct WantedRows {
         bool pending = false;
         const int* rows = nullptr;
-        int n = 0;
+        int n = 0, step_rows = 0;
         Tensor stream;
     };
     WantedRows wanted;

@@ -123,6 +123,24 @@ def test_the_head_reads_the_output_table_as_it_is(tmp_path, wanted, vocab):
     assert abs(bias) < 1e-3, bias
 
 
+# (480: the products of many rows want a multiple of 64, those of few rows one of 32; a single layer, whose mixer takes the norm along)
+@pytest.mark.parametrize("width,ff,backend", [(128, 448, "library"), (1152, 448, "auto"), (128, 480, "auto")])
+@pytest.mark.parametrize("wanted", [1, 8, 9, 33, 64])
+def test_no_norm_is_folded_where_the_whole_step_folds_none(tmp_path, width, ff, backend, wanted):
+    """Feed-forwards of many rows that the library's products make read every weight as it is stored; so do the rows that are left
+    of such a step.  (Of the fused products the one into the stream behind the mixer, which has no norm, remains.)"""
+    from celeg_amd.weights import write_random_model
+    config = small_config(width, ff=ff)
+    if ff == 480:
+        config.update(num_hidden_layers=1, layer_types=["full_attention"])
+    folder = write_random_model(config, str(tmp_path), seed=5, dtype=torch.bfloat16, std=0.05 if width < 1000 else 0.03)
+    got, tokens, paths = one_prompt(folder, wanted, backend=backend)
+    cfg, W = plain.load_model_folder(folder)
+    assert_close(got, plain.model_logits(cfg, W, tokens)[-wanted:], "bfloat16", f"{width}/{ff}/{backend}/{wanted}")
+    assert paths["linear_few_rows"] > 0
+    assert paths["fused_rows"] + paths["fused_sliced"] <= (1 if ff == 480 else 0), paths
+
+
 @pytest.mark.parametrize("dtype,last", [("bfloat16", "conv"), ("bfloat16", "full_attention"), ("float32", "full_attention")])
 @pytest.mark.parametrize("wanted", [9, 16, 17, 33, 64, 65])
 def test_logits_of_9_to_64_wanted_rows(tmp_path, dtype, last, wanted):
