@@ -1612,10 +1612,6 @@ void Ops::depth_mix(const Tensor& history, const Tensor& h, const Tensor& w, int
 // parts rather than hundreds of them, and at short lengths workgroups of 4 once there are enough
 // of them for half the compute units (1, 2, 4 and 16 requests at 2,048 tokens: 0.5 to 1.4 % faster
 // than single wavefronts).  Measured at 1 to 16 requests, 2,048 and 8,192 tokens.
-// One workgroup a (request, key/value head), its wavefronts taking the rounds in turn and no second
-// kernel, once there are enough of them: 192 (24 requests of 8 key/value heads) at any length, 96 at
-// contexts up to 4,096 tokens (12 and 16 requests at 2,048 tokens: 1 and 3 % of a decode step
-// faster than in parts; 16 requests at 8,192: 3 % slower).
 // Up to how many rounds of 64 keys one workgroup a (request, key/value head) is faster than parts and the kernel that joins
 // them, however few they are: its 16 wavefronts have a round each, and what a compute unit pulls alone (16 KB a round) stays
 // below what the second kernel costs.  16 heads over 8, in a recorded chain, us (one workgroup | parts):
@@ -1626,9 +1622,16 @@ void Ops::depth_mix(const Tensor& history, const Tensor& h, const Tensor& w, int
 // (groups of 4 heads the same within 0.2; heads of 128 have not been measured.)
 int Ops::decode_short_rounds(long long groups, int head_dim) { return head_dim != 64 ? 0 : groups >= 64 ? 16 : 10; }
 
-bool Ops::decode_whole(long long groups, int rounds, int head_dim) const {
-    if (attention_decode_whole >= 0) return attention_decode_whole > 0;
+// One workgroup a (request, key/value head), its wavefronts taking the rounds in turn and no second
+// kernel, once there are enough of them: 192 (24 requests of 8 key/value heads) at any length, 96 at
+// contexts up to 4,096 tokens (12 and 16 requests at 2,048 tokens: 1 and 3 % of a decode step
+// faster than in parts; 16 requests at 8,192: 3 % slower).
+bool Ops::decode_whole_by_sizes(long long groups, int rounds, int head_dim) {
     return groups >= 192 || (groups >= 96 && rounds <= 64) || rounds <= decode_short_rounds(groups, head_dim);
+}
+
+bool Ops::decode_whole(long long groups, int rounds, int head_dim) const {
+    return attention_decode_whole >= 0 ? attention_decode_whole > 0 : decode_whole_by_sizes(groups, rounds, head_dim);
 }
 
 int Ops::decode_split_rounds(long long groups, int rounds) const {

@@ -133,6 +133,7 @@ public:
     bool decode_parts_fill = true;       // parts of 16 rounds where they are one workgroup a compute unit
     int decode_split_rounds(long long groups, int rounds) const;
     bool decode_whole(long long groups, int rounds, int head_dim) const;
+    static bool decode_whole_by_sizes(long long groups, int rounds, int head_dim);
     static int decode_short_rounds(long long groups, int head_dim);
     bool attention_general = false;      // always the general attention kernel
     bool delta_general = false;          // the delta rule's recurrence always by the kernel for any dim

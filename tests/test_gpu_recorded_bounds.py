@@ -1,0 +1,39 @@
+"""How often single tokens' steps are recorded: once for every bound on the context at which their launches change."""
+import pytest
+import torch
+
+from helpers import random_tokens
+
+pytestmark = pytest.mark.gpu
+
+
+def recordings(lm, requests, contexts):
+    """Recordings made behind the one for contexts[0], after a step of `requests` single tokens at each of these contexts.  (Nobody
+    reads what the pages hold ahead of the tokens.  The first step brings so many pages that their list gets a buffer of its own,
+    behind which it is recorded once more.)"""
+    from celeg_amd.engine import StepEntry
+    slots = [lm.cache.open() for _ in range(requests)]
+    for slot in slots:
+        assert lm.cache.prepare(slot, 0, max(contexts))
+    seen = []
+    for context in [contexts[0]] + contexts:
+        lm.runner.step([StepEntry(slot, context - 1, random_tokens(60, 1, seed=slot), [0]) for slot in slots])
+        seen.append(lm.runner.counters()["captures"])
+    return [n - seen[1] for n in seen[1:]]
+
+
+# pairs of request and key/value head: 8 and 56 (one workgroup each up to 640 keys), 64 (1,024), 96 and 128 (4,096); and 128
+# requests, whose attention prepares the new keys itself up to 2,048 keys
+@pytest.mark.parametrize("requests,kv_heads,after", [(1, 8, [0, 0, 1, 1]), (8, 7, [0, 0, 1, 1]), (8, 8, [0, 0, 0, 1]),
+                                                     (16, 6, [0, 0, 0, 0]), (16, 8, [0, 0, 0, 0]), (128, 1, [0, 0, 0, 1])])
+def test_softmax_attention(tmp_path, requests, kv_heads, after):
+    from celeg_amd.engine import load_model
+    from celeg_amd.weights import write_random_model
+    config = {"architectures": ["Lfm2ForCausalLM"], "vocab_size": 60, "hidden_size": 64 * kv_heads, "num_hidden_layers": 1, "layer_types": ["full_attention"],
+              "num_attention_heads": kv_heads, "num_key_value_heads": kv_heads, "head_dim": 64, "intermediate_size": 64,
+              "block_auto_adjust_ff_dim": False, "rope_theta": 10000.0, "conv_L_cache": 3, "conv_bias": False, "tie_word_embeddings": True,
+              "norm_eps": 1e-5, "max_position_embeddings": 2048, "eos_token_id": 7}
+    folder = write_random_model(config, str(tmp_path), seed=2, dtype=torch.bfloat16, std=0.05)
+    lm = load_model(folder, dtype="bfloat16", page_tokens=16, n_pages=requests * 66 + 2, max_requests=requests, max_batched_tokens=256)
+    assert recordings(lm, requests, [600, 640, 641, 1030]) == after
+    lm.close()
