@@ -1656,7 +1656,9 @@ void Ops::attention_decode(const Tensor& q, const Tensor& out, int heads, int kv
     const int split_rounds = decode_split_rounds(static_cast<long long>(kv_heads) * chunks * T, rounds);
     const int n_parts = (rounds + split_rounds - 1) / split_rounds;
     const size_t parts = static_cast<size_t>(T) * heads * n_parts;
-    float* workspace = static_cast<float*>(ws.raw("attention_decode_parts", parts * (head_dim + 2) * sizeof(float)));
+    // (room for parts of 4,096 keys also where there are fewer, or no parts: made later, it would have recorded steps recorded again)
+    const size_t room = static_cast<size_t>(T) * heads * std::max<size_t>(n_parts, (std::min(4096, max_context) + 63) / 64);
+    float* workspace = static_cast<float*>(ws.raw("attention_decode_parts", room * (head_dim + 2) * sizeof(float)));
     if (fresh) {
         need(fresh->k && fresh->v, "attention_decode: fresh keys and values are missing");
         const long long kvw = static_cast<long long>(kv_heads) * head_dim;

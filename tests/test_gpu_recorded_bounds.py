@@ -24,8 +24,8 @@ def recordings(lm, requests, contexts):
 
 # pairs of request and key/value head: 8 and 56 (one workgroup each up to 640 keys), 64 (1,024), 96 and 128 (4,096); and 128
 # requests, whose attention prepares the new keys itself up to 2,048 keys
-@pytest.mark.parametrize("requests,kv_heads,after", [(1, 8, [0, 0, 1, 1]), (8, 7, [0, 0, 1, 1]), (8, 8, [0, 0, 0, 1]),
-                                                     (16, 6, [0, 0, 0, 0]), (16, 8, [0, 0, 0, 0]), (128, 1, [0, 0, 0, 1])])
+@pytest.mark.parametrize("requests,kv_heads,after", [(1, 8, [0, 0, 1, 1, 1]), (8, 7, [0, 0, 1, 1, 1]), (8, 8, [0, 0, 0, 1, 1]),
+                                                     (16, 6, [0, 0, 0, 0, 0]), (16, 8, [0, 0, 0, 0, 0]), (128, 1, [0, 0, 0, 1, 1])])
 def test_softmax_attention(tmp_path, requests, kv_heads, after):
     from celeg_amd.engine import load_model
     from celeg_amd.weights import write_random_model
@@ -35,5 +35,5 @@ def test_softmax_attention(tmp_path, requests, kv_heads, after):
               "norm_eps": 1e-5, "max_position_embeddings": 2048, "eos_token_id": 7}
     folder = write_random_model(config, str(tmp_path), seed=2, dtype=torch.bfloat16, std=0.05)
     lm = load_model(folder, dtype="bfloat16", page_tokens=16, n_pages=requests * 66 + 2, max_requests=requests, max_batched_tokens=256)
-    assert recordings(lm, requests, [600, 640, 641, 1030]) == after
+    assert recordings(lm, requests, [600, 640, 641, 1030, 600]) == after
     lm.close()
