@@ -55,14 +55,14 @@ Model::Model(ModelSpec s) : spec(std::move(s)) {
     for (const auto& np : named_parts()) visit(np.second);
 }
 
-int Model::short_context(int requests, DType dtype) const {
-    int longest = 0;
+std::vector<int> Model::short_contexts(int requests, DType dtype) const {
+    std::set<int> borders;
     std::function<void(const Part*)> visit = [&](const Part* p) {
-        longest = std::max(longest, p->short_context(requests, dtype));
+        if (const int border = p->short_context(requests, dtype)) borders.insert(border);
         for (const Part* c : p->children()) visit(c);
     };
     for (const auto& np : const_cast<Model*>(this)->named_parts()) visit(np.second);
-    return longest;
+    return {borders.begin(), borders.end()};
 }
 
 void Model::resolve_cache_sharing() {
@@ -329,7 +329,7 @@ ModelRunner::ModelRunner(Model& m, CacheManager& c, Runtime& r, int max_tokens)
     std::set<int> buckets;
     for (int i = 0; i < 12; ++i) buckets.insert(std::min(1 << i, S));
     buckets_.assign(buckets.begin(), buckets.end());
-    for (int bucket : buckets_) short_contexts_[bucket] = model.short_context(bucket, rt.dtype);
+    for (int bucket : buckets_) short_contexts_[bucket] = model.short_contexts(bucket, rt.dtype);
 }
 
 ModelRunner::~ModelRunner() { drop_graphs(); }
@@ -485,11 +485,13 @@ bool ModelRunner::graph_applies(const std::vector<StepEntry>& entries) const {
 // the context: a graph is therefore good up to a bound on the context, and there is one per
 // (batch-size bucket, bound).  The first step beyond a bound makes the next one's graph in the middle of a request:
 // a pass over padding rows, recording and instantiation, 0.9 to 1.0 ms at the 350M shape for 1 to 8 requests.  A short bound
-// (Part::short_context) costs that once more for every bucket that gets both.
+// (Part::short_context; every part's is one) costs that once more for every bucket that gets both.
 int ModelRunner::context_bound(const std::vector<StepEntry>& entries, int bucket) const {
     int longest = 0;
     for (const StepEntry& e : entries) longest = std::max(longest, e.start_pos + static_cast<int>(e.tokens.size()));
-    for (int bound : {short_contexts_.at(bucket), 4096, 16384, 65536})
+    for (int bound : short_contexts_.at(bucket))
+        if (longest <= bound) return std::min(bound, cache.max_context);
+    for (int bound : {4096, 16384, 65536})
         if (longest <= bound) return std::min(bound, cache.max_context);
     return cache.max_context;
 }

@@ -26,7 +26,8 @@ public:
 
     // whether a recorded step of this model may be replayed from a HIP graph
     bool graph_safe() const { return graph_safe_; }
-    int short_context(int requests, DType dtype) const;
+    // the parts' borders (Part::short_context), in order
+    std::vector<int> short_contexts(int requests, DType dtype) const;
     std::vector<std::pair<std::string, Part*>> named_parts();
     // checkpoint tensor name -> what is expected of it
     ExpectedTensors expected_tensors();
@@ -103,7 +104,7 @@ private:
     void validate(const std::vector<StepEntry>& entries) const;
     bool graph_applies(const std::vector<StepEntry>& entries) const;
     int context_bound(const std::vector<StepEntry>& entries, int bucket) const;
-    std::map<int, int> short_contexts_;      // by the bucket of a recorded step: Model::short_context
+    std::map<int, std::vector<int>> short_contexts_;      // by the bucket of a recorded step
     Tensor step_from_graph(const std::vector<StepEntry>& entries);
     Captured& capture(int bucket, const std::vector<int>& caps, int bound);
     Captured& record(std::pair<int, int> key, const StepBatch& batch);

@@ -37,3 +37,34 @@ def test_softmax_attention(tmp_path, requests, kv_heads, after):
     lm = load_model(folder, dtype="bfloat16", page_tokens=16, n_pages=requests * 66 + 2, max_requests=requests, max_batched_tokens=256)
     assert recordings(lm, requests, [600, 640, 641, 1030, 600]) == after
     lm.close()
+
+
+def test_two_kinds_of_attention(tmp_path):
+    """Sigmoid attention is cut into parts beyond 640 keys, softmax attention of 64 pairs beyond 1,024: steps of a model with both are
+    recorded for each."""
+    from celeg_amd.config import LayerSpec, ModelSpec, PartSpec, RunStep, register_architecture, registered_architectures
+    from celeg_amd.engine import load_model
+    from celeg_amd.weights import write_random_model
+
+    def build_spec(cfg, shapes):
+        width = cfg["width"]
+        norm = lambda name: PartSpec("rmsnorm", {"width": width, "eps": 1e-5}, {"weight": name})
+        rope = PartSpec("rope", {"theta": 100.0, "head_dim": 64})
+        sizes = {"width": width, "heads": 8, "kv_heads": 8, "head_dim": 64, "qk_norm": False}
+        layers = []
+        for i, mixer in enumerate((PartSpec("gqa_attention", dict(sizes, position=rope),
+                                            {"q_proj": "0.q", "k_proj": "0.k", "v_proj": "0.v", "out_proj": "0.o"}),
+                                   PartSpec("sigmoid_attention", dict(sizes, position=rope), {"q": "1.q", "k": "1.k", "v": "1.v", "o": "1.o"}))):
+            ffn = PartSpec("swiglu", {"width": width, "ff": 64}, {"gate": f"{i}.g", "up": f"{i}.u", "down": f"{i}.d"})
+            layers.append(LayerSpec(mixer, norm(f"{i}.n1"), ffn, norm(f"{i}.n2")))
+        return ModelSpec("BothAttentions", cfg["vocab"], width, 2048, PartSpec("embedding", {"vocab": cfg["vocab"], "width": width}, {"table": "emb"}),
+                         tuple(layers), tuple(RunStep(i) for i in range(len(layers))), norm("final"),
+                         PartSpec("tied_head", {"vocab": cfg["vocab"], "width": width}))
+
+    if "BothAttentions" not in registered_architectures():
+        register_architecture("BothAttentions", build_spec)
+    folder = write_random_model({"architectures": ["BothAttentions"], "width": 64, "vocab": 60}, str(tmp_path), seed=2, dtype=torch.bfloat16,
+                                std=0.05)
+    lm = load_model(folder, dtype="bfloat16", page_tokens=16, n_pages=8 * 66 + 2, max_requests=8, max_batched_tokens=256)
+    assert recordings(lm, 8, [600, 640, 641, 1024, 1030]) == [0, 0, 1, 1, 2]
+    lm.close()
