@@ -77,6 +77,12 @@ Tensor operand_rows(Runtime& rt, const std::string& name, int rows, long long wi
     return rt.ws.buf(name, DType::BF16, {STAT_COLUMNS, width}).rows(0, rows);
 }
 
+// Both layouts of such an operand for up to 64 rows: made at one's first need, they would have recorded steps recorded again.
+void operand_room(Runtime& rt, const std::string& name, long long width, std::initializer_list<long long> producer_inner) {
+    operand_rows(rt, name, 1, width, producer_inner);
+    operand_rows(rt, name, FUSED_MAX_ROWS, width, producer_inner);
+}
+
 // The bfloat16 copy of the residual stream that products behind a norm read.
 Tensor stream_bf16(Runtime& rt, int rows, long long width) { return operand_rows(rt, "stream_bf16", rows, width, {}); }
 
@@ -110,6 +116,8 @@ std::shared_ptr<DeviceTensor> packed_weight(Runtime& rt, const Tensor& w) {
     if (it == rt.packed_weights.end()) it = rt.packed_weights.emplace(w.data, rt.ops.fold_weight(w, nullptr, true)).first;
     return it->second;
 }
+// the rows of a product that reads its weights as they are stored, behind their norm
+Tensor rows_as_stored(Runtime& rt, long long width) { return rt.ws.buf("normed_as_stored", DType::BF16, {STAT_COLUMNS, width}); }
 }  // namespace
 
 bool qkv_tail_ok(const Runtime& rt, int rows, long long width) { return tiled_step(rt, rows, width); }
@@ -168,7 +176,7 @@ void norm_linear(Runtime& rt, const Tensor& h, const Norm::Foldable& norm, const
     rt.ops.last_best_parts = 0;
     const bool folds = sliced(rt, M, width) && w.dtype == DType::BF16 && (streamed || w.shape[0] / streams <= SLICED_MAX_COLUMNS);
     if (folds && extras.as_stored) {
-        const Tensor normed = rt.ws.buf("normed_as_stored", DType::BF16, {STAT_COLUMNS, width}).rows(0, M);
+        const Tensor normed = rows_as_stored(rt, width).rows(0, M);
         rt.ops.rmsnorm(h, norm.weight, norm.eps, normed, nullptr, extras.rows);
         args.rows = nullptr;
         args.plain = true;
@@ -220,13 +228,23 @@ void norm_linear(Runtime& rt, const Tensor& h, const Norm::Foldable& norm, const
 Tensor keep_wanted_rows(Runtime& rt, const Tensor& h, const Tensor& a, bool operand) {
     Runtime::WantedRows& wanted = rt.wanted;
     wanted.pending = false;
-    const long long width = h.shape[1], room = std::max(wanted.n, STAT_COLUMNS);     // (one size for all steps of few)
+    // Sizes that go by the step's rows, as those of all its buffers do, and not by how many are wanted: the first step of many rows
+    // makes what later ones of no more rows need, and steps recorded behind it stay good.
+    const long long width = h.shape[1], room = std::max<long long>(wanted.step_rows / 2, STAT_COLUMNS);
     wanted.stream = rt.ws.buf("wanted_stream", DType::F32, {room, width}).rows(0, wanted.n);
     rt.stream_stat_blocks = 0;
     rt.stream_has_bf16 = false;
+    if (rt.dtype == DType::BF16) rows_as_stored(rt, width);      // (the head's)
     Tensor few;
-    if (a.defined() && operand && rt.dtype == DType::BF16) few = operand_rows(rt, "wanted_operand", wanted.n, a.shape[1], {});
-    else if (a.defined()) few = rt.ws.buf("wanted_branch", rt.dtype, {room, a.shape[1]}).rows(0, wanted.n);
+    if (a.defined() && operand && rt.dtype == DType::BF16) {
+        operand_room(rt, "wanted_operand", a.shape[1], {});
+        operand_room(rt, "stream_bf16", width, {});
+        stream_stats(rt, width);
+        few = rt.ws.buf("wanted_operand_many", DType::BF16, {room, a.shape[1]}).rows(0, wanted.n);
+        if (wanted.n <= FUSED_MAX_ROWS) few = operand_rows(rt, "wanted_operand", wanted.n, a.shape[1], {});
+    } else if (a.defined()) {
+        few = rt.ws.buf("wanted_branch", rt.dtype, {room, a.shape[1]}).rows(0, wanted.n);
+    }
     rt.ops.gather_rows(h, a.defined() ? &a : nullptr, wanted.rows, wanted.n, wanted.stream, few.defined() ? &few : nullptr);
     return few;
 }

@@ -846,6 +846,7 @@ public:
             return false;
         // (32-bit rows have one layout: the buffer of longer steps, so that a step of few rows makes none of its own, upon which
         // recorded steps would be recorded again)
+        if (rt.wanted.stream.defined() && rt.dtype == DType::BF16) fused::operand_room(rt, "ffn_act_fused", ff_, {width_});
         Tensor act = rt.dtype == DType::F32 ? rt.ws.buf("ffn_act", rt.dtype, {batch.n_tokens, ff_})
                                             : fused::operand_rows(rt, "ffn_act_fused", batch.n_tokens, ff_, {width_});
         fused::norm_linear(rt, h, norm, w_gate_up_->view, act, Epilogue::Swiglu);
@@ -2615,6 +2616,7 @@ public:
         // few rows: the activation too, in the same kernel
         const int rows = batch.n_tokens;
         const bool in_product = fused::activation_ok(rt, rows, width_, ff_);
+        if (rt.wanted.stream.defined()) fused::operand_room(rt, "mlp_up_fused", ff_, {width_});
         Tensor up = in_product ? fused::operand_rows(rt, "mlp_up_fused", rows, ff_, {width_}) : rt.ws.buf("mlp_up", rt.dtype, {rows, ff_});
         fused::LinearExtras extras;
         if (in_product) {

@@ -213,6 +213,7 @@ bool fused_rows_ok(const Runtime& rt, const StepBatch& batch, std::initializer_l
 bool fused_f32_ok(const Runtime& rt, const StepBatch& batch, std::initializer_list<long long> inner);
 Tensor stream_stats(Runtime& rt, long long width, int rows = 0);
 Tensor operand_rows(Runtime& rt, const std::string& name, int rows, long long width, std::initializer_list<long long> producer_inner);
+void operand_room(Runtime& rt, const std::string& name, long long width, std::initializer_list<long long> producer_inner);
 Tensor stream_bf16(Runtime& rt, int rows, long long width);
 bool sliced(const Runtime& rt, int rows, long long inner);
 

@@ -163,3 +163,34 @@ def test_logits_of_9_to_64_wanted_rows(tmp_path, dtype, last, wanted):
         got = lm.runner.step(entries)
         assert_close(got, torch.stack([plain.model_logits(cfg, W, t[:s])[-1] for t, s in zip(tokens, seen)]), dtype, f"{dtype}/{last}/{wanted}")
     lm.close()
+
+
+@pytest.mark.parametrize("dtype,last,backend", [("bfloat16", "conv", "auto"), ("bfloat16", "full_attention", "auto"),
+                                                ("bfloat16", "conv", "library"), ("float32", "conv", "auto")])
+def test_recorded_steps_stay_good_however_many_rows_are_wanted(tmp_path, dtype, last, backend):
+    """Twelve requests decoded together between steps of 200 rows: the first of these makes every buffer of the others."""
+    from celeg_amd.engine import StepEntry, load_model
+    from celeg_amd.weights import write_random_model
+    config = small_config(128)
+    config["layer_types"] = ["full_attention", last]
+    folder = write_random_model(config, str(tmp_path), seed=8, dtype=getattr(torch, dtype), std=0.05)
+    lm = load_model(folder, dtype=dtype, page_tokens=16, n_pages=400, max_requests=12, max_batched_tokens=256, gemm_backend=backend)
+    slots, seen = [lm.cache.open() for _ in range(12)], [0] * 12
+
+    def step(*entries):
+        batch = []
+        for i, n, wanted in entries:
+            assert lm.cache.prepare(slots[i], seen[i], n)
+            batch.append(StepEntry(slots[i], seen[i], random_tokens(320, n, seed=seen[i]), list(range(n - wanted, n))))
+            seen[i] += n
+        lm.runner.step(batch)
+        return lm.runner.counters()["captures"]
+    singles = [(i, 1, 1) for i in range(12)]
+    step((0, 120, 60), (1, 80, 40))
+    step(*singles)
+    recorded = step(*singles)
+    for wanted in (1, 9, 33, 70, 100):
+        step((2 + wanted % 5, 50, wanted // 2), (8, 150, wanted - wanted // 2))
+        assert step(*singles) == recorded, wanted
+        seen[8] = 0
+    lm.close()
