@@ -948,7 +948,7 @@ static const int k_shape_bn[] = {TILE_SHAPES(TILE_COLUMNS)};
 #undef TILE_ROWS
 #undef TILE_COLUMNS
 static constexpr int N_TILE_SHAPES = sizeof(k_shape_bm) / sizeof(k_shape_bm[0]);
-extern "C" int celeg_gemm_tiles_shapes() { return N_TILE_SHAPES - 1; }      // (how many there are to force, ahead of the square one)
+extern "C" int celeg_gemm_tiles_shapes() { return N_TILE_SHAPES; }      // (how many there are to force)
 
 // How the dies share the grid of tiles: every row of tiles of A is read by 8 / m dies, every column of
 // tiles of W by m of them; the split with the fewest bytes read of those that leave no die more tiles than it
@@ -1041,7 +1041,12 @@ static TileShape tile_shape(int M, int N, int K, int streams, bool may_split = f
             // 6,144 x 2,048, 9,216 x 1,024, 12,288 x 1,536 and 16,384 x 2,048, the sums choose the fastest or one within 3 %
             // in all of 36.  16,384 x 2,048: 2,048 rows 111.9 us in two rounds of 256x256 (128x128 150, 256x288 119.3), 1,200
             // rows 87.0 in two of 256x192 (100), 4,096 rows 228 (322, 245); 9,216 x 1,024 at 1,500 rows 31.5 in one of 256x256
-            // (39.4 in two of 128x128).
+            // (39.4 in two of 128x128).  The costs hold for the other epilogues too, though 256x256 into the stream has 40 registers
+            // too few behind its loop (164 bytes of scratch a lane) and pays for it once a tile.  Into the stream, us,
+            // 256x256 | 256x288 | 128x128 | 256x192: 1,024 columns, 1,024 values of k, 10,400 rows 58.8 | 61.8 | 64.0 | 66.4, 16,000 rows
+            // 74.1 | 74.4 | 77.0 | 86.9; 4,608 values of k 136 | 142 | 161 | 194 and 158 | 162 | 180 | 223; 2,048 columns, 5,300 rows,
+            // 2,048 values of k 84.8 | 85.3 | 91.5 | 109 and 8,192 211 | 218 | 243 | 318; 8,000 rows 99.8 | 99.5 | 108 | 126 and 244 | 252 |
+            // 288 | 337.  Where another tile is faster (8,192 rows of 1,024: 52.4 | 53.1 | 39.0 | 40.9) the sums choose that.
             struct Cost { int id, on_a_unit; long long fixed, per_k; };      // tenths of us a round and 1,024 values of k
             static constexpr Cost costs[] = {{7, 1, 55, 120}, {8, 2, 25, 180}, {9, 1, 70, 190}, {11, 1, 85, 230}, {10, 1, 110, 240}};
             long long best = -1;
@@ -1090,6 +1095,9 @@ static int launch_tiles(const TileParams& p, hipStream_t stream) {
     hipLaunchKernelGGL(kernel, grid, block, lds, stream, p, tiles_m, tiles_n, dies_m);
     return CELEG_LAUNCH_RESULT();
 }
+
+// (for tests: which of the shapes a product of weights as they are takes)
+extern "C" int celeg_gemm_tiles_chosen(int M, int N, int K, int epi) { return tile_shape(M, N, K, epi == T_SWIGLU ? 2 : 1).id; }
 
 template <int EPI>
 static int launch_epilogue(const TileParams& p, hipStream_t stream) {

@@ -6,7 +6,7 @@ import torch
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 BF = torch.bfloat16
-N_SHAPES = 11
+N_SHAPES = 12
 
 
 @pytest.fixture(scope="module")
@@ -92,7 +92,7 @@ def swiglu_of(ops, gates, ups):
     return out.cpu()
 
 
-@pytest.mark.parametrize("shape", [0, 9, 10])
+@pytest.mark.parametrize("shape", [0, 9, 10, 11])
 def test_swiglu_of_every_gate(ops, shape):
     """Every normal gate, those whose 1 + e^-g has a reciprocal below the normal numbers among them."""
     ops._lib("gemm_tiles").celeg_gemm_tiles_force(shape)
@@ -109,7 +109,7 @@ def test_swiglu_of_every_gate(ops, shape):
     assert float(got[g < -88.75].abs().max()) == 0
 
 
-@pytest.mark.parametrize("shape", [0, 9, 10])
+@pytest.mark.parametrize("shape", [0, 9, 10, 11])
 def test_swiglu_divides_as_32_bit_division_does(ops, shape):
     """The quotient is rounded correctly: where no error of the exponential within its bound can change 1 + e^-g, the result's
     bits follow from it (among them 5.9375, whose quotient lies beside the middle of two bfloat16 numbers)."""
