@@ -1753,14 +1753,23 @@ bool Ops::rows_kernel_ok(int rows, std::initializer_list<long long> inner) const
     return true;
 }
 
-// Every workgroup then reads all rows for its columns: worth it up to 32 rows, and up to 64 where a workgroup a compute unit has 8
-// columns (2,048 of them).  A whole step of one prompt, us, apart | inside:
-//   rows             9           16          17          24          32          33          48            64
-//   1,024 wide   541 | 505   523 | 510   530 | 523   534 | 526   548 | 536   579 | 587   597 | 602     620 | 613 (621 in another run)
-//   2,048 wide   836 | 800   820 | 801   858 | 845   866 | 851   905 | 888   997 | 976  1,021 | 1,000  1,083 | 1,065
-// (fewer than 9 rows: another kernel.)
+// Every workgroup then reads all rows for its columns: worth it up to 16 rows, up to 32 where a workgroup has eight
+// wavefronts (512 values of k; four below), and up to 64 where a workgroup a compute unit has 8 columns (2,048 of them).  Of a whole step of one prompt
+// through 16 convolution layers, us a layer more or less inside than apart (negative: faster; runs of one side differ by 0.2):
+//   rows            9       16      17      24      32      33      48      64
+//     64 wide    -0.6     +1.7    +4.1    +5.2    +6.6
+//    128         -2.2     -0.5    +1.6    +1.6    +2.5
+//    256         -3.3     -1.2    +0.5    +0.3    +0.4
+//    448         -2.9     -0.8    +1.0    +1.0    +1.0
+//    512         -3.2     -1.0    -0.7    -0.6    -0.5
+//  1,024         -3.6     -1.6    -1.2    -1.4    -1.5    +0.8    +0.5    -0.7
+//  1,536         -3.9     -1.9    -1.7    -1.8    -2.3
+//  2,048         -4.7     -2.8    -2.4    -2.6    -2.8    -2.6    -2.7    -2.4
+//  3,072         -7.1     -6.7    -6.9    -7.2    -7.8   -12.0   -11.5   -10.9
+//  4,096        -14.1    -13.2   -14.1   -14.3   -16.3   -19.3   -22.9   -26.2
+// (1,024 wide beyond 32 rows in another run, ten layers; between 1,024 and 2,048 not measured there.  Fewer than 9 rows: another kernel.)
 bool Ops::conv_rows_pay(int rows, long long width) const {
-    return use_conv_rows && rows_kernel_ok(rows, {width}) && (rows <= 32 || width >= 2048);
+    return use_conv_rows && rows_kernel_ok(rows, {width}) && width >= (rows <= 16 ? 128 : rows <= 32 ? 512 : 2048);
 }
 
 int Ops::residual_stat_blocks(int rows, int n, int k) const {

@@ -275,6 +275,8 @@ Json call(celeg_ops& h, const std::string& op, const Json& a) {
     } else if (op == "rows_kernel_ok") {
         const int rows = static_cast<int>(a["rows"].as_int());
         out.set("ok", all_sizes(ints_of(a["inner"]), [&](long long k) { return ops.rows_kernel_ok(rows, {k}); }));
+    } else if (op == "conv_rows_pay") {
+        out.set("ok", ops.conv_rows_pay(static_cast<int>(a["rows"].as_int()), a["width"].as_int()));
     } else if (op == "tiled_linear_ok") {
         const int rows = static_cast<int>(a["rows"].as_int()), n = static_cast<int>(a["n"].as_int());
         out.set("ok", all_sizes(ints_of(a["inner"]), [&](long long k) { return ops.tiled_linear_ok(rows, n, {k}); }));

@@ -376,6 +376,10 @@ class HipOps:
         return out
 
     # ------------------------------------------------------------------ fused products of many rows
+    def conv_rows_pay(self, rows: int, width: int) -> bool:
+        """Whether a step of so many rows has its short convolutions inside the products ahead of them."""
+        return bool(self._call("conv_rows_pay", rows=int(rows), width=int(width))["ok"])
+
     def tiled_linear_ok(self, rows: int, n: int, *inner_sizes: int) -> bool:
         """Whether the fused bfloat16 product for many rows takes these sizes."""
         return bool(self._call("tiled_linear_ok", rows=int(rows), n=int(n), inner=[int(k) for k in inner_sizes])["ok"])

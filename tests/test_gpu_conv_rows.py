@@ -14,7 +14,8 @@ STEPS = [[(0, 9)], [(1, 2), (0, 14)], [(2, 1), (1, 1), (0, 15)], [(2, 1), (3, 31
          [(3, 62), (2, 1)], [(0, 1), (1, 3), (2, 2), (3, 58)], [(0, 65)], [(0, 10), (1, 33), (3, 1), (2, 2)]]
 
 
-@pytest.mark.parametrize("width,taps,bias", [(128, 3, False), (192, 2, True), (1152, 4, False), (2304, 3, True), (64, 9, False)])
+@pytest.mark.parametrize("width,taps,bias", [(128, 3, False), (192, 2, True), (1152, 4, False), (2304, 3, True), (64, 9, False),
+                                             (512, 9, False), (544, 2, True)])
 def test_conv_rows(tmp_path, width, taps, bias):
     from celeg_amd.engine import StepEntry, load_model
     from celeg_amd.weights import write_random_model
@@ -45,3 +46,12 @@ def test_conv_rows(tmp_path, width, taps, bias):
         assert_close_bf16(inside, torch.stack([plain.model_logits(cfg, W, tokens[r][:at + 1])[-1] for r, at in want]))
         if width <= 192:       # (K is cut alike and a row has few partial sums of squares: the same bits)
             assert torch.equal(apart, inside)
+
+
+def test_where_the_convolution_is_inside():
+    """Up to 16 rows from a width of 128 on, up to 32 from 512 and up to 64 from 2,048; elsewhere it is slower there."""
+    from kernel_ops import HipOps
+    ops = HipOps()
+    for width, most in ((64, 0), (96, 0), (128, 16), (480, 16), (512, 32), (1024, 32), (2016, 32), (2048, 64), (4096, 64)):
+        for rows in (1, 8, 9, 16, 17, 32, 33, 64, 65):
+            assert ops.conv_rows_pay(rows, width) == (9 <= rows <= most), (rows, width)
