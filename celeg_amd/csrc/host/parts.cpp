@@ -817,6 +817,7 @@ public:
         if (act == "clamped") read_clamp(s.params, "swiglu", limit_, alpha_);
     }
     bool graph_safe() const override { return true; }
+    bool rows_alone() const override { return true; }
     WeightSpecs weight_specs() const override {
         return {{"gate", matrix(ff_, width_)}, {"up", matrix(ff_, width_)}, {"down", matrix(width_, ff_)}};
     }
@@ -926,6 +927,7 @@ public:
         rule_.score = score_;
     }
     bool graph_safe() const override { return !shared_ || shared_->graph_safe(); }
+    bool rows_alone() const override { return !shared_ || shared_->rows_alone(); }
     std::vector<const Part*> children() const override {
         return shared_ ? std::vector<const Part*>{shared_.get()} : std::vector<const Part*>{};
     }
@@ -1005,6 +1007,7 @@ class NoFeedForward final : public FeedForward {
 public:
     explicit NoFeedForward(const PartSpec& s) : FeedForward(s) {}
     bool graph_safe() const override { return true; }
+    bool rows_alone() const override { return true; }
     Tensor forward(const Tensor& x, const StepBatch&, Runtime& rt) override { return NoMixer::zeros(rt, x.shape[0], x.shape[1]); }
 };
 
@@ -1257,7 +1260,7 @@ public:
         few.n_tokens = few.n_seqs = rt.wanted.n;
         return feed(rt.wanted.stream, mixed, normed.rows(0, rt.wanted.n), fusable ? fold2 : nullptr, few, rt);
     }
-    bool takes_wanted_rows() const override { return has_ffn_; }
+    bool takes_wanted_rows() const override { return has_ffn_ && ffn_->rows_alone(); }
 
 private:
     // the feed-forward on the rows of h (mixed: what the mixer adds to them, where it has not done so itself)
@@ -1828,7 +1831,7 @@ public:
         return Tensor();
     }
     bool takes_pending_sum() const override { return true; }
-    bool takes_wanted_rows() const override { return has_ffn_; }
+    bool takes_wanted_rows() const override { return has_ffn_ && ffn_->rows_alone(); }
 
 private:
     static const Ops::NormParams& of(const Norm& norm) {
@@ -2577,6 +2580,7 @@ public:
         bias_ = s.params.get_bool("bias", true);
     }
     bool graph_safe() const override { return true; }
+    bool rows_alone() const override { return true; }
     WeightSpecs weight_specs() const override {
         WeightSpecs specs{{"up", matrix(ff_, width_)}, {"down", matrix(width_, ff_)}};
         if (bias_) {

@@ -130,6 +130,9 @@ public:
     using Part::Part;
     virtual Tensor forward(const Tensor& x, const StepBatch& batch, Runtime& rt) = 0;
     virtual bool forward_fused(const Tensor& h, const Norm::Foldable& norm, const StepBatch& batch, Runtime& rt) { return false; }
+    // Whether a row's result hangs on that row alone and of `batch` only the number of rows is looked at: such a part may be given
+    // some of a step's rows (Runtime::wanted), with nothing else of the step.  Any other one sees every step whole.
+    virtual bool rows_alone() const { return false; }
 };
 
 class Embedding : public Part {

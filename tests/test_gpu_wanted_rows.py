@@ -194,3 +194,65 @@ def test_recorded_steps_stay_good_however_many_rows_are_wanted(tmp_path, dtype, 
         assert step(*singles) == recorded, wanted
         seen[8] = 0
     lm.close()
+
+
+@pytest.mark.parametrize("arrangement", ["pre_norm", "sandwich_norm"])
+@pytest.mark.parametrize("shared", [False, True])
+def test_a_feed_forward_that_reads_the_step_is_given_all_of_it(tmp_path, arrangement, shared):
+    """A feed-forward from outside goes by its rows' tokens, places and requests, as the last layer's and as what routed experts
+    share: it is given every row and the step's arrays, however few rows are wanted."""
+    from celeg_amd.config import LayerSpec, ModelSpec, PartSpec, RunStep, register_architecture, registered_architectures
+    from celeg_amd.engine import StepEntry, load_model
+    from celeg_amd.parts import as_tensor, int_array, on_stream, register_part, registered_parts
+    from celeg_amd.weights import write_random_model
+
+    class ByToken:
+        def __init__(self, spec):
+            pass
+
+        def describe(self):
+            return {"graph_safe": False}
+
+        def forward(self, args):
+            step, rows = args.step, int(args.x.shape[0])
+            if rows != step.n_tokens or not (step.token_ids and step.positions and step.host_seq_start and step.host_cu_seqlens) or \
+                    step.host_cu_seqlens[step.n_seqs] != rows:
+                raise RuntimeError("the step is not whole")
+            with on_stream(args):
+                by = int_array(step.token_ids, rows).float() + 0.5 * int_array(step.positions, rows).float()
+                as_tensor(args.out).copy_(as_tensor(args.x) * (0.01 * by)[:, None])
+
+    if "by_token" not in registered_parts("ffn"):
+        register_part("ffn", "by_token", ByToken)
+
+    def build(cfg, shapes):
+        H, V = cfg["width"], cfg["vocab"]
+        norm = lambda name: PartSpec("rmsnorm", {"width": H, "eps": 1e-5}, {"weight": name})
+        ffn = PartSpec("by_token")
+        if cfg["shared"]:
+            names = {"router": "router"}
+            for e in range(2):
+                names.update({f"gate.{e}": f"{e}.g", f"up.{e}": f"{e}.u", f"down.{e}": f"{e}.d"})
+            ffn = PartSpec("routed_experts", {"width": H, "ff": 32, "experts": 2, "top": 1, "shared": ffn}, names)
+        layer = LayerSpec(PartSpec("none", {"width": H}), norm("n1"), ffn, norm("n2"), cfg["arrangement"],
+                          **({"mixer_post_norm": norm("n3"), "ffn_post_norm": norm("n4")} if cfg["arrangement"] == "sandwich_norm" else {}))
+        return ModelSpec("ByToken", V, H, 256, PartSpec("embedding", {"vocab": V, "width": H}, {"table": "emb"}), (layer,), (RunStep(0),),
+                         norm("final"), PartSpec("hidden", {"width": H}))
+
+    if "ByToken" not in registered_architectures():
+        register_architecture("ByToken", build)
+    config = {"architectures": ["ByToken"], "width": 32, "vocab": 90, "shared": shared, "arrangement": arrangement}
+    folder = write_random_model(config, str(tmp_path), seed=7, dtype=torch.float32, std=0.3)
+    lm = load_model(folder, dtype="float32", page_tokens=16, n_pages=40, max_requests=4, max_batched_tokens=256)
+    tokens = random_tokens(90, 80, seed=3)
+
+    def step(wanted):
+        slot = lm.cache.open()
+        assert lm.cache.prepare(slot, 0, 80)
+        got = lm.runner.step([StepEntry(slot, 0, tokens, wanted)]).clone()
+        lm.cache.close(slot)
+        return got
+    whole = step(list(range(80)))
+    for wanted in ([79], [3, 70, 79], []):
+        assert torch.equal(step(wanted), whole[wanted])
+    lm.close()
