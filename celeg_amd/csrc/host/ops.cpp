@@ -1652,13 +1652,20 @@ void Ops::attention_decode(const Tensor& q, const Tensor& out, int heads, int kv
     const int bound = hint ? std::min(hint, max_context) : max_context;
     const int rounds = (bound + 63) / 64;
     const int chunks = (heads / kv_heads + 15) / 16;
-    const int whole = decode_whole(static_cast<long long>(kv_heads) * chunks * T, rounds, head_dim) ? 1 : 0;
-    const int split_rounds = decode_split_rounds(static_cast<long long>(kv_heads) * chunks * T, rounds);
+    const long long groups = static_cast<long long>(kv_heads) * chunks * T;
+    const int whole = decode_whole(groups, rounds, head_dim) ? 1 : 0;
+    const int split_rounds = decode_split_rounds(groups, rounds);
     const int n_parts = (rounds + split_rounds - 1) / split_rounds;
     const size_t parts = static_cast<size_t>(T) * heads * n_parts;
-    // (room for parts of 4,096 keys also where there are fewer, or no parts: made later, it would have recorded steps recorded again)
-    const size_t room = static_cast<size_t>(T) * heads * std::max<size_t>(n_parts, (std::min(4096, max_context) + 63) / 64);
-    float* workspace = static_cast<float*>(ws.raw("attention_decode_parts", room * (head_dim + 2) * sizeof(float)));
+    // Room for parts, where there are any, and for those that the same rows have at 4,096 keys: made later, it would have recorded
+    // steps recorded again.  (Whole pairs of request and key/value head need none.)
+    size_t room = whole ? 0 : n_parts;
+    const int rounds_later = (std::min(4096, max_context) + 63) / 64;
+    if (!decode_whole(groups, rounds_later, head_dim)) {
+        const int split_later = decode_split_rounds(groups, rounds_later);
+        room = std::max<size_t>(room, (rounds_later + split_later - 1) / split_later);
+    }
+    float* workspace = static_cast<float*>(ws.raw("attention_decode_parts", static_cast<size_t>(T) * heads * room * (head_dim + 2) * sizeof(float)));
     if (fresh) {
         need(fresh->k && fresh->v, "attention_decode: fresh keys and values are missing");
         const long long kvw = static_cast<long long>(kv_heads) * head_dim;

@@ -68,3 +68,24 @@ def test_two_kinds_of_attention(tmp_path):
     lm = load_model(folder, dtype="bfloat16", page_tokens=16, n_pages=8 * 66 + 2, max_requests=8, max_batched_tokens=256)
     assert recordings(lm, 8, [600, 640, 641, 1024, 1030]) == [0, 0, 1, 1, 2]
     lm.close()
+
+
+def test_room_for_parts_is_what_parts_need(tmp_path):
+    """1,024 requests of 16 heads take their pairs whole at any context: no room for parts, of which 64 a head would be 277 MB.  (The
+    rest of a step of so many rows, recorded, is 124 MB.)"""
+    from celeg_amd.engine import load_model
+    from celeg_amd.weights import write_random_model
+    config = {"architectures": ["Lfm2ForCausalLM"], "vocab_size": 60, "hidden_size": 1024, "num_hidden_layers": 1, "layer_types": ["full_attention"],
+              "num_attention_heads": 16, "num_key_value_heads": 8, "head_dim": 64, "intermediate_size": 64,
+              "block_auto_adjust_ff_dim": False, "rope_theta": 10000.0, "conv_L_cache": 3, "conv_bias": False, "tie_word_embeddings": True,
+              "norm_eps": 1e-5, "max_position_embeddings": 4096, "eos_token_id": 7}
+    folder = write_random_model(config, str(tmp_path), seed=2, dtype=torch.bfloat16, std=0.05)
+    lm = load_model(folder, dtype="bfloat16", page_tokens=16, n_pages=4200, max_requests=1024, max_batched_tokens=1024)
+    recordings(lm, 1, [40])          # (the kernels' code and what a step of one request needs)
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    recordings(lm, 1000, [40])
+    torch.cuda.synchronize()
+    taken = before - torch.cuda.mem_get_info()[0]
+    lm.close()
+    assert taken < 200 << 20, taken
