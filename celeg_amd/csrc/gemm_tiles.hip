@@ -983,6 +983,7 @@ static Dies dies_of(int tiles_m, int tiles_n, int M, int weight_rows) {
 //   2,048 x 8,192            18.1 | 28.6   24.6 | 28.8   24.7 | 28.9   29.0 | 36.5   (35.4 | 35.9)
 // (2,048 x 2,048 and less: the same or slower; tiles that fill the compute units, cut: 2 to 20 % slower; a second round of
 // workgroups on one die, 772 x 5,120 at 700 rows: 31.5 us against 26.3.)
+// The number of slices, and with it the order of a sum, goes by the rows of the step: other tiles all give the same bits.
 static TileShape tile_split(int M, int N, int K) {
     const auto fits = [&](int id, int slices) {
         return dies_of((M + k_shape_bm[id] - 1) / k_shape_bm[id], (N + k_shape_bn[id] - 1) / k_shape_bn[id], M, N).per_die * slices <= DIE_UNITS;

@@ -148,7 +148,7 @@ celeg_status celeg_model_create(const char* model_dir, const celeg_engine_option
 void celeg_model_destroy(celeg_model* model);
 /* JSON: {"config": typed configuration, "spec": model description, "cache_layout": .., "vocab_size", "max_context",
  *        "page_tokens", "max_requests", "graph_safe", "logit_width", "gemm_backend": "library" | "tiles" (what
- *        CELEG_GEMM_AUTO became; "library": for the steps whose rows do not make the tiles faster)} */
+ *        CELEG_GEMM_AUTO became)} */
 const char* celeg_model_describe(celeg_model* model);
 celeg_status celeg_model_open_slot(celeg_model* model, int32_t* slot);      /* -1: every slot is taken */
 celeg_status celeg_model_close_slot(celeg_model* model, int32_t slot);

@@ -99,8 +99,9 @@ __global__ void depth_mix_kernel(float* __restrict__ history, size_t entry_strid
 }
 
 // Row rows[r] of h to row r of h_out and, where there is an a, its row likewise (in groups of 8 values k8_stride apart); one
-// workgroup a row.  8 values a piece: every load of a row of up to 2,048 values is asked for at once.  What bounds it is one trip
-// to memory for the row's number and one for the row (one row of 1,024 values and 1,024 of the branch: 3.0 us with its launch).
+// workgroup a row.  A thread takes four values of h and eight of a at a time: every load of 1,024 values of h and of 2,048 of a is
+// asked for at once.  What bounds it is one trip to memory for the row's number and one for the row (one row of 1,024 values and 1,024
+// of the branch: 3.0 us with its launch).
 template <typename T, bool WIDE>
 __global__ __launch_bounds__(256) void gather_rows_kernel(const int* __restrict__ rows, const float* __restrict__ h, float* __restrict__ h_out,
                                                           int width, const T* __restrict__ a, size_t lda, T* __restrict__ a_out,
